@@ -234,3 +234,68 @@ def tolerance(case):
     # Against the same attention in 64 bits these cases are off by 2.1e-4 to 3.0e-4 in float16 and by 1.6e-3 to
     # 2.7e-3 in bfloat16: four times that.
     return {"rel": 1.2e-3 if case["dtype"] == "float16" else 1e-2}
+
+
+def _rotated(x, cos, sin):
+    """Rotary embedding in 64 bits (cos and sin are inputs, in 16 bits as the model holds them)."""
+    a = x.double()
+    half = a.shape[-1] // 2
+    turned = torch.cat((-a[..., half:], a[..., :half]), dim=-1)
+    return a * cos.double()[:, None] + turned * sin.double()[:, None]
+
+
+def _exact_prompt_attention(q, k, v, scale, spans):
+    """Block-sparse causal attention in 64 bits, a head and some query blocks at a time: [B, N, Hq, D]."""
+    B, Hq, N, D = q.shape
+    group = Hq // k.shape[1]
+    out = torch.empty(B, N, Hq, D, dtype=torch.float64, device=q.device)
+    col = torch.arange(N, device=q.device)[None, :]
+    step = 2048
+    for b in range(B):
+        for h in range(Hq):
+            kd, vd = k[b, h // group].double(), v[b, h // group].double()
+            for lo in range(0, N, step):
+                hi = min(N, lo + step)
+                row = torch.arange(lo, hi, device=q.device)[:, None]
+                live = (col[:, :hi] <= row) & ((col[:, :hi] < SINK) |
+                                               (row // 64 - col[:, :hi] // 64 < spans[h // group] // 64))
+                score = (q[b, h, lo:hi].double() @ kd[:hi].t()) * scale
+                out[b, lo:hi, h] = torch.softmax(score.masked_fill_(~live, -math.inf), dim=-1) @ vd[:hi]
+    return out
+
+
+def exact(case, seed):
+    """What ``run`` returns, by torch in 64 bits.  Rotated keys are rounded to the 16 bits of the rings they are kept
+    in; None stands for what is bookkeeping or a copy of other outputs."""
+    state = prepare(case, seed)
+    scale, group, D = state["sm_scale"], case["heads"] // case["kv_heads"], case["head_dim"]
+    if case["kind"] == "attention":
+        q, k, v = state["qkv"][0]
+        return _exact_prompt_attention(q, k, v, scale, _spans(case, 0))
+    results = []
+    for layer, (q, k, v) in enumerate(state["qkv"]):
+        if case["kind"] == "prompt" or case["fused"]:
+            q, k = (_rotated(x, state["cos"], state["sin"]) for x in (q, k))
+        if case["kind"] == "prompt":
+            if case["attend"]:
+                q, k = q.to(v.dtype), k.to(v.dtype)
+                results.append([_exact_prompt_attention(q, k, v, scale, _spans(case, layer))] + [None] * 5)
+            else:
+                results.append([q, k] + [None] * 5)
+            continue
+        q, k = q.to(v.dtype), k.to(v.dtype)
+        cache = state["cache"]
+        keys, values = cache.key_cache[layer].clone(), cache.value_cache[layer].clone()
+        slot, valid = cache.cache_update_index[layer], cache.cache_valid_length[layer]
+        start, room = cache.cache_head_start_index[layer], cache.cache_max_length[layer]
+        each = torch.arange(case["batch"], device=keys.device)[:, None]
+        keys[each, slot], values[each, slot] = k[:, :, 0], v[:, :, 0]
+        out = torch.empty(case["batch"], 1, case["heads"], D, dtype=torch.float64, device=keys.device)
+        for h in range(case["kv_heads"]):   # no padding here: the rows of a batch are filled alike
+            first = int(start[0, h])
+            rows = slice(first, first + min(int(valid[0, h]) + 1, int(room[h])))
+            heads = slice(h * group, (h + 1) * group)
+            score = q[:, heads, 0].double() @ keys[:, rows].double().transpose(1, 2).contiguous() * scale
+            out[:, 0, heads] = torch.softmax(score, dim=-1) @ values[:, rows].double()
+        results.append([out, keys, values, None, None, None])
+    return results
