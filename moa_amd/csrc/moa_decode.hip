@@ -95,6 +95,15 @@ struct DecInt {
   static constexpr int value = N;
 };
 
+// Sixteen bytes of a cache row, which a step reads once.  NT marks the load non-temporal: it leaves no line
+// behind in the caches, which a launch that reads more than they hold only pays for (see kNtBytes).
+template <bool NT>
+__device__ __forceinline__ u32x4 load_once16(const uint16_t* p) {
+  const u32x4* s = reinterpret_cast<const u32x4*>(p);
+  if constexpr (NT) return __builtin_nontemporal_load(s);
+  else return *s;
+}
+
 // Chunk table of one batch row: prefix[h] = number of chunks of heads < h, and every head's segment
 // (first row, length) clamped into the row, so that a bad index cannot fault and a work-group finds a
 // chunk's segment in LDS instead of behind another memory latency.
@@ -233,7 +242,7 @@ __device__ __forceinline__ int build_prefix_even(const int64_t* __restrict__ val
 // one is consumed) instead of loading a full batch, waiting for it and consuming it.  Measured at
 // the 7B decode shape: 8 % faster at batch 4, 2 % at 8-16, 0.7 % at 64; at batch 1-2 (about one
 // work-group per CU, the call is launch-latency bound) the plain loop is 2-4 % faster.
-template <typename T, int D, int CHUNK, int G, bool PIPE>
+template <typename T, int D, int CHUNK, int G, bool PIPE, bool NT>
 __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     uint16_t* __restrict__ o, float* __restrict__ part_acc, float* __restrict__ part_ml,
@@ -300,8 +309,8 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
         const int64_t row = r0 + i * RPL + sub;
         const bool ok = row < r_end;
         const int64_t rr = ok ? row : r_begin;  // any valid row: keeps the load in bounds
-        kr[i] = *reinterpret_cast<const u32x4*>(kbase + rr * D);
-        vr[i] = *reinterpret_cast<const u32x4*>(vbase + rr * D);
+        kr[i] = load_once16<NT>(kbase + rr * D);
+        vr[i] = load_once16<NT>(vbase + rr * D);
       }
     };
     // online-softmax update with those rows
@@ -549,7 +558,7 @@ template <> struct MfmaElem<BF16> { typedef PBF16 type; };
 template <int D>
 constexpr size_t gqa_lds_bytes() { return (size_t)kGqaWaves * kGqaStages * 2 * kGqaTile * D * 2; }
 
-template <typename T, int D>
+template <typename T, int D, bool NT>
 __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     uint16_t* __restrict__ o, float* __restrict__ part_acc, float* __restrict__ part_ml,
@@ -658,16 +667,16 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
       const int last = n_rows - 1 - t * kGqaTile;   // last valid row of the tile, >= 0
       if (last >= kGqaTile - 1) {
 #pragma unroll
-        for (int i = 0; i < NCP; ++i) async_copy16(ksrc, koff[i], dst + i * 1024);
+        for (int i = 0; i < NCP; ++i) async_copy16<NT>(ksrc, koff[i], dst + i * 1024);
 #pragma unroll
-        for (int i = 0; i < NCP; ++i) async_copy16(vsrc, voff[i], dst + TILE_B + i * 1024);
+        for (int i = 0; i < NCP; ++i) async_copy16<NT>(vsrc, voff[i], dst + TILE_B + i * 1024);
       } else {
 #pragma unroll
         for (int i = 0; i < NCP; ++i)
-          async_copy16(ksrc, koff[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + i * 1024);
+          async_copy16<NT>(ksrc, koff[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + i * 1024);
 #pragma unroll
         for (int i = 0; i < NCP; ++i)
-          async_copy16(vsrc, voff[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + TILE_B + i * 1024);
+          async_copy16<NT>(vsrc, voff[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + TILE_B + i * 1024);
       }
     };
     if (n_t > 0) issue(0);
@@ -793,6 +802,17 @@ constexpr int kDecBlocksPerCu = 16;   // work-groups per CU over the whole grid
 constexpr int kDecSmallBelow = 2;     // work-groups per CU below which the chunks are half as long
 constexpr int kDecPipeFrom = 3;       // work-groups per CU from which the waves pipeline their own loads
 
+// From this many bytes of K and V per launch on they are read non-temporally.  What a step reads of one layer
+// is read again a token later, after the rings of all other layers: with several layers of this size that is
+// past the 256 MB of the last-level cache, and lines kept for it only cost.  Measured with graphs of 16
+// layers, ordinary against non-temporal loads: one query head per ring, D = 128, 67 MB a layer 21.2 -> 19.7 us,
+// 268 MB 55.4 -> 51.0 us, 2.1 GB 382 -> 337 us (6.4 TB/s); eight query heads 134 MB 36.1 -> 34.7 us, 268 MB
+// 57.5 -> 53.9 us.  Below, the rings of some layers do stay cached and ordinary loads win: 16.8 MB a layer
+// 14.1 against 15.1 us.  (The same single layer of 134 MB read over and over, which stays cached whole, loses
+// 7 %; a decoder has more layers than one.)
+constexpr int64_t kNtBytes = (int64_t)64 << 20;
+static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_t)B * sumC * D * 4 >= kNtBytes; }
+
 constexpr int kSmallChunk = kChunk / 2;   // chunk length of the one-query-head kernel when the grid is small
 
 // partial slots per batch row: at most this many chunks exist when the rings do not overlap (sized
@@ -819,29 +839,25 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
   const bool small = (int64_t)B * chunks < (int64_t)256 * kDecSmallBelow;
   constexpr int GROUPS = kDecThreads / D;
   const int mx = (H * G + GROUPS - 1) / GROUPS;
-  if (small) {
-    hipLaunchKernelGGL((decode_split_kernel<T, D, kSmallChunk, G, false>), dim3(bx, B), dim3(kDecThreads), 0, st,
-                       (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (uint16_t*)o,
-                       part_acc, part_ml, head_start, head_valid, H, sumC, sm_scale * kLog2e, cap);
-    int rc = check_launch("moa_decode_fwd(split)");
-    if (rc) return rc;
-    hipLaunchKernelGGL((decode_merge_kernel<T, D, kSmallChunk>), dim3(mx, B), dim3(kDecThreads), 0, st,
-                       (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, G, sumC, cap, 0);
+  auto launch = [&](auto split, auto merge) {
+    hipLaunchKernelGGL(split, dim3(bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
+                       (const uint16_t*)vc, (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, sumC,
+                       sm_scale * kLog2e, cap);
+    if (int rc = check_launch("moa_decode_fwd(split)")) return rc;
+    hipLaunchKernelGGL(merge, dim3(mx, B), dim3(kDecThreads), 0, st, (uint16_t*)o, part_acc, part_ml, head_start,
+                       head_valid, H, G, sumC, cap, 0);
     return check_launch("moa_decode_fwd(merge)");
+  };
+  const bool nt = read_nontemporal(B, sumC, D);
+  if (small) {
+    if (nt) return launch(&decode_split_kernel<T, D, kSmallChunk, G, false, true>, &decode_merge_kernel<T, D, kSmallChunk>);
+    return launch(&decode_split_kernel<T, D, kSmallChunk, G, false, false>, &decode_merge_kernel<T, D, kSmallChunk>);
   }
-  if (pipe)
-    hipLaunchKernelGGL((decode_split_kernel<T, D, kChunk, G, true>), dim3(bx, B), dim3(kDecThreads), 0, st,
-                       (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (uint16_t*)o,
-                       part_acc, part_ml, head_start, head_valid, H, sumC, sm_scale * kLog2e, cap);
-  else
-    hipLaunchKernelGGL((decode_split_kernel<T, D, kChunk, G, false>), dim3(bx, B), dim3(kDecThreads), 0, st,
-                       (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (uint16_t*)o,
-                       part_acc, part_ml, head_start, head_valid, H, sumC, sm_scale * kLog2e, cap);
-  int rc = check_launch("moa_decode_fwd(split)");
-  if (rc) return rc;
-  hipLaunchKernelGGL((decode_merge_kernel<T, D, kChunk>), dim3(mx, B), dim3(kDecThreads), 0, st,
-                     (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, G, sumC, cap, 0);
-  return check_launch("moa_decode_fwd(merge)");
+  // the pipelined kernel's launches are past kNtBytes but for short rings of 64-element rows
+  if (pipe && nt) return launch(&decode_split_kernel<T, D, kChunk, G, true, true>, &decode_merge_kernel<T, D, kChunk>);
+  if (pipe) return launch(&decode_split_kernel<T, D, kChunk, G, true, false>, &decode_merge_kernel<T, D, kChunk>);
+  if (nt) return launch(&decode_split_kernel<T, D, kChunk, G, false, true>, &decode_merge_kernel<T, D, kChunk>);
+  return launch(&decode_split_kernel<T, D, kChunk, G, false, false>, &decode_merge_kernel<T, D, kChunk>);
 }
 
 
@@ -873,10 +889,12 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
   if (bx > cap) bx = cap;
   if (bx < 1) bx = 1;
   constexpr size_t lds = gqa_lds_bytes<D>();
-  static bool lds_reserved[kMaxDevices] = {};   // per template instance
-  if (int rc = reserve_lds(reinterpret_cast<const void*>(&decode_gqa_kernel<T, D>), lds, lds_reserved, "moa_decode_fwd"))
+  static bool lds_reserved[2][kMaxDevices] = {};   // per template instance
+  const bool nt = read_nontemporal(B, sumC, D);
+  const auto kernel = nt ? &decode_gqa_kernel<T, D, true> : &decode_gqa_kernel<T, D, false>;
+  if (int rc = reserve_lds(reinterpret_cast<const void*>(kernel), lds, lds_reserved[nt], "moa_decode_fwd"))
     return rc;
-  hipLaunchKernelGGL((decode_gqa_kernel<T, D>), dim3((unsigned)bx, B), dim3(kGqaThreads), lds, st,
+  hipLaunchKernelGGL(kernel, dim3((unsigned)bx, B), dim3(kGqaThreads), lds, st,
                      (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (uint16_t*)o,
                      part_acc, part_ml, head_start, head_valid, H, G, sumC, mfma_softmax_scale(sm_scale), cap,
                      (int)target);

@@ -44,14 +44,25 @@ struct PBF16 {
 // full vmcnt(0) wait in front of every LDS read; completion is tracked by hand with wait_vm().
 // Loads complete in order, so the compiler's own vmcnt bookkeeping for ordinary loads stays safe
 // (it can only wait longer than it planned).
+// NT: non-temporal, for bytes that are read once.
+template <bool NT = false>
 __device__ __forceinline__ void async_copy16(const void* base, uint32_t byte_off, uint32_t lds_addr) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1"
-      :
-      : "v"(byte_off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
-      : "memory");
+  if constexpr (NT)
+    asm volatile(
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, %1 nt"
+        :
+        : "v"(byte_off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
+        : "memory");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, %1"
+        :
+        : "v"(byte_off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
+        : "memory");
 }
 // max of a value with its twin in the other half of the wave (lane ^ 32), without going through LDS
 __device__ __forceinline__ float max_with_other_half(float x) {

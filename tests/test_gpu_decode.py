@@ -122,6 +122,43 @@ def test_partial_fill_with_a_large_grid(dev, D, B):
     _close(out, ref, ("large grid", D))
 
 
+@pytest.mark.parametrize("G,B,sizes,D", [
+    (1, 1, [40000, 64, 90001], 128),            # half-length chunks, just under 64 MiB of K and V
+    (1, 1, [40000, 64, 91043], 128),            # the same just over it: non-temporal loads from here on
+    (1, 3, [30000, 64, 15777], 128),
+    (1, 3, [30000, 64, 15777], 64),
+    (1, 9, [20000, 30, 10999, 513], 128),       # full-length chunks
+    (1, 9, [40000, 30, 10999, 513], 64),        # the load-pipelined loop
+    (2, 2, [60000, 33, 30001], 128),            # grouped query, non-temporal copies
+    (7, 5, [60000, 33, 30001], 64),
+])
+def test_large_rings_of_both_load_kinds(dev, G, B, sizes, D):
+    """Launches on both sides of the size from which the rings are read non-temporally: ragged rings with rows
+    outside the valid part that must not be looked at, against the oracle."""
+    rng = np.random.default_rng(sum(sizes) + B)
+    g = torch.Generator(device=dev).manual_seed(B)
+    H, sumc = len(sizes), sum(sizes)
+    start = np.concatenate([[0], np.cumsum(sizes)[:-1]])
+    kc, vc = (torch.randn(B, sumc, D, generator=g, device=dev, dtype=torch.float16) for _ in range(2))
+    q = torch.randn(B, H * G, 1, D, generator=g, device=dev, dtype=torch.float16)
+    hs = np.broadcast_to(start, (B, H)).astype(np.int64).copy()
+    hv = np.array([[n - int(rng.integers(0, min(n, 700))) for n in sizes] for _ in range(B)], dtype=np.int64)
+    hv[0] = sizes
+    for b in range(B):
+        for h in range(H):
+            kc[b, start[h] + hv[b, h]:start[h] + sizes[h]] = float("nan")
+            vc[b, start[h] + hv[b, h]:start[h] + sizes[h]] = float("inf")
+    from moa_amd import mixture_of_sparse_attention
+    out = mixture_of_sparse_attention(q, kc, vc, D ** -0.5, head_start_index=torch.from_numpy(hs).to(dev),
+                                      head_valid_length=torch.from_numpy(hv).to(dev))
+    if G > 1:
+        _close_grouped(out[:, 0], q[:, :, 0], kc, vc, hs, hv, D ** -0.5, G, ("large", G, B))
+    else:
+        ref = decode_segments(q[:, :, 0].float().cpu().numpy(), kc.float().cpu().numpy(), vc.float().cpu().numpy(),
+                              hs, hv, D ** -0.5)
+        _close(out[:, 0].float().cpu().numpy(), ref, ("large", G, B))
+
+
 def test_peaked_softmax(dev):
     """Large score range: the running max must carry across chunks and waves."""
     rng = np.random.default_rng(11)
