@@ -434,94 +434,160 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   }
 }
 
-// Merge of the per-chunk partials of heads with more than one chunk, and the
-// zero output of empty heads.  A group of D threads takes one query head at a time: its lanes load
-// the (max, sum) pairs of the chunks side by side, the factors go through LDS, then thread d sums
-// column d of the partial accumulators with several loads in flight.
+__device__ __forceinline__ int wave_sum(int x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
+}
+__device__ __forceinline__ float wave_sum(float x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
+}
+
+// One head's entries of the chunk table (build_prefix, or build_prefix_even when even_target > 0: the same
+// arithmetic), worked out by a single wave without LDS or barriers: the first chunk and the number of chunks.
+struct HeadChunks {
+  int first, count;
+};
+template <int CHUNK>
+__device__ __forceinline__ HeadChunks chunks_of_head(const int64_t* __restrict__ valid_row,
+                                                     const int64_t* __restrict__ start_row, int H, int64_t sumC,
+                                                     int cap, int even_target, int h) {
+  constexpr int kGroups = kMaxHeads / 64;
+  const int lane = threadIdx.x & 63;
+  int len[kGroups];
+#pragma unroll
+  for (int k = 0; k < kGroups; ++k) {
+    const int i = k * 64 + lane;
+    int64_t l = 0;
+    if (i < H) {
+      l = valid_row[i];
+      const int64_t seg0 = start_row[i];
+      if (l < 0 || seg0 < 0 || seg0 >= sumC) l = 0;
+      if (l > sumC - seg0) l = sumC - seg0;
+    }
+    len[k] = (int)l;
+  }
+  int c = CHUNK;
+  if (even_target > 0) {
+    int steps = 0;
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k)
+      if (k * 64 < H) steps += (len[k] + kEvenStep - 1) / kEvenStep;
+    c = max(kEvenMinChunk, ((wave_sum(steps) + even_target - 1) / even_target) * kEvenStep);
+    for (int t = 0; t < kEvenTries; ++t) {
+      int n = 0;
+#pragma unroll
+      for (int k = 0; k < kGroups; ++k)
+        if (k * 64 < H) n += (len[k] + c - 1) / c;
+      if (wave_sum(n) <= even_target) break;
+      c += kEvenStep;
+    }
+  }
+  int before = 0, mine = 0;
+#pragma unroll
+  for (int k = 0; k < kGroups; ++k) {
+    if (k * 64 >= H) break;
+    int n = (len[k] + c - 1) / c;
+    if (even_target > 0 && n > 0) {
+      const int clen = (((len[k] + n - 1) / n + kEvenStep - 1) / kEvenStep) * kEvenStep;
+      n = (len[k] + clen - 1) / clen;
+    }
+    const int i = k * 64 + lane;
+    before += (i < h) ? n : 0;
+    mine += (i == h) ? n : 0;
+  }
+  before = wave_sum(before);
+  mine = wave_sum(mine);
+  HeadChunks r;
+  r.first = min(before, cap);
+  r.count = min(before + mine, cap) - r.first;
+  return r;
+}
+
+// Merge of the per-chunk partials of heads with more than one chunk, and the zero output of empty heads.
+// Latency is all there is to it (a few MB at most): one work-group per query head, each of its waves finds the
+// head's chunks by itself (one memory latency), then asks for the (max, sum) pairs of all chunks, a lane each,
+// and for its share of the accumulators, every fourth chunk, before it looks at any of them (a second one);
+// the waves meet once, in LDS, for the final sum.  {MEASURED}
 template <typename T, int D, int CHUNK>
 __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
     uint16_t* __restrict__ o, const float* __restrict__ part_acc, const float* __restrict__ part_ml,
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
     int G /* query heads per ring */, int64_t sumC, int cap,
     int even_target /* > 0: the split kernel used build_prefix_even with this target */) {
-  constexpr int GROUPS = kDecThreads / D;
-  constexpr int kFactors = 64;   // chunks whose factors are staged at a time
-  __shared__ HeadTable s_tab;
-  const int* const s_prefix = s_tab.prefix;
-  __shared__ float s_f[GROUPS][kFactors];
-  __shared__ int s_n[GROUPS];
-  const int b = blockIdx.y;
-  const int tid = threadIdx.x;
-  if (even_target > 0)
-    build_prefix_even<kDecWaves>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, even_target, &s_tab);
-  else
-    build_prefix<CHUNK>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, &s_tab);
-  const int grp = tid / D;
-  const int d = tid % D;
-  // every group runs the same number of rounds so that the barriers below are uniform
-  const int rounds = (H * G + gridDim.x * GROUPS - 1) / (gridDim.x * GROUPS);
-  for (int r = 0; r < rounds; ++r) {
-    const int hq = (r * gridDim.x + blockIdx.x) * GROUPS + grp;
-    const bool on = hq < H * G;
-    const int h = on ? hq / G : 0, g = on ? hq % G : 0;
-    const int w0 = s_prefix[h];
-    const int n = on ? s_prefix[h + 1] - w0 : 1;
-    const int64_t bhq = (int64_t)b * H * G + hq;
-    const int64_t slot0 = (int64_t)b * cap + w0;
-    if (on && n == 0) o[bhq * D + d] = 0;
-    // n == 1: written by the split kernel
-    float M = -INFINITY;
-    if (n > 1)
-      for (int i = d; i < n; i += D) M = fmaxf(M, part_ml[((slot0 + i) * G + g) * 2]);
-    // max over the group's lanes (D = 64: one wave; D = 128: two waves, through LDS)
+  constexpr int VEC = D / 64;      // columns per lane
+  constexpr int kFirst = 8;        // chunks per wave asked for at once (32 of the head; more are rare)
+  constexpr int kMore = 4;
+  typedef float fvec __attribute__((ext_vector_type(VEC)));
+  __shared__ float s_a[kDecWaves][D];
+  const int hq = blockIdx.x, b = blockIdx.y;
+  const int h = hq / G, g = hq % G;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const HeadChunks hc = chunks_of_head<CHUNK>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap,
+                                              even_target, h);
+  const int n = __builtin_amdgcn_readfirstlane(hc.count);
+  if (n == 1) return;   // written by the split kernel
+  uint16_t* const out = o + ((int64_t)b * H * G + hq) * D;
+  if (n == 0) {
+    if (tid < D) out[tid] = 0;
+    return;
+  }
+  const int64_t slot0 = ((int64_t)b * cap + __builtin_amdgcn_readfirstlane(hc.first)) * G + g;
+  const float* const acc = part_acc + slot0 * D + lane * VEC;
+  const f32x2* const ml = reinterpret_cast<const f32x2*>(part_ml) + slot0;
+  const int64_t step = (int64_t)G * D;   // from a chunk's accumulator to the next one's
+
+  fvec x[kFirst];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-    if (D > 64) {
-      if ((tid & 63) == 0) s_f[grp][(d >> 6)] = M;
-      __syncthreads();
-      M = fmaxf(s_f[grp][0], s_f[grp][1]);
-      __syncthreads();
-    }
-    const float m_use = (M == -INFINITY) ? 0.f : M;
-    float L = 0.f, a = 0.f;
-    // the groups of a block walk their chunks in lockstep (work-group barriers inside): as many
-    // rounds as the longest of them needs
-    const int n_eff = (n > 1) ? n : 0;
-    if (d == 0) s_n[grp] = n_eff;
-    __syncthreads();
-    int n_loop = 0;
+  for (int j = 0; j < kFirst; ++j)
+    if (wave + kDecWaves * j < n) x[j] = *reinterpret_cast<const fvec*>(acc + (wave + kDecWaves * j) * step);
+  f32x2 mine = {-INFINITY, 0.f};   // chunk `lane`
+  if (lane < n) mine = ml[(int64_t)lane * G];
+  float M = mine.x;
+  for (int i = 64 + lane; i < n; i += 64) M = fmaxf(M, ml[(int64_t)i * G].x);
 #pragma unroll
-    for (int k = 0; k < GROUPS; ++k) n_loop = max(n_loop, s_n[k]);
-    for (int i0 = 0; i0 < n_loop; i0 += kFactors) {
-      const int cnt = max(0, min(kFactors, n_eff - i0));
-      if (d < cnt) {
-        const int64_t slot = (slot0 + i0 + d) * G + g;
-        const float f = fast_exp2(part_ml[slot * 2] - m_use);
-        s_f[grp][d] = f;
-        L += part_ml[slot * 2 + 1] * f;
+  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+  const float m_use = (M == -INFINITY) ? 0.f : M;
+  float f = fast_exp2(mine.x - m_use);   // the factor of chunk `lane`
+  float L = mine.y * f;
+  auto factor = [&](int i) __attribute__((always_inline)) {   // of the chunk at lane i (uniform)
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), i));
+  };
+  fvec a = {};
+#pragma unroll
+  for (int j = 0; j < kFirst; ++j)
+    if (wave + kDecWaves * j < n) a += x[j] * factor(wave + kDecWaves * j);
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    if (i0 > 0) {
+      f = 0.f;
+      if (i0 + lane < n) {
+        const f32x2 v = ml[(int64_t)(i0 + lane) * G];
+        f = fast_exp2(v.x - m_use);
+        L += v.y * f;
       }
-      __syncthreads();
-      const float* acc = part_acc + ((slot0 + i0) * G + g) * D + d;
-      int i = 0;
-      for (; i + 4 <= cnt; i += 4) {
-        const float x0 = acc[(int64_t)(i + 0) * G * D], x1 = acc[(int64_t)(i + 1) * G * D];
-        const float x2 = acc[(int64_t)(i + 2) * G * D], x3 = acc[(int64_t)(i + 3) * G * D];
-        a += x0 * s_f[grp][i] + x1 * s_f[grp][i + 1] + x2 * s_f[grp][i + 2] + x3 * s_f[grp][i + 3];
-      }
-      for (; i < cnt; ++i) a += acc[(int64_t)i * G * D] * s_f[grp][i];
-      __syncthreads();
     }
-    // the sum of the group's partial L values
+    const int end = min(64, n - i0);
+    for (int i = (i0 == 0 ? kFirst * kDecWaves : 0) + wave; i < end; i += kMore * kDecWaves) {
+      fvec y[kMore];
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) L += __shfl_xor(L, off, 64);
-    if (D > 64) {
-      if ((tid & 63) == 0) s_f[grp][(d >> 6)] = L;
-      __syncthreads();
-      L = s_f[grp][0] + s_f[grp][1];
-      __syncthreads();
+      for (int j = 0; j < kMore; ++j)
+        if (i + kDecWaves * j < end) y[j] = *reinterpret_cast<const fvec*>(acc + (int64_t)(i0 + i + kDecWaves * j) * step);
+#pragma unroll
+      for (int j = 0; j < kMore; ++j)
+        if (i + kDecWaves * j < end) a += y[j] * factor(i + kDecWaves * j);
     }
-    if (on && n > 1) o[bhq * D + d] = pack1<T>((L > 0.f) ? a / L : 0.f);
-    __syncthreads();   // s_n and s_f are written again in the next round
+  }
+  L = wave_sum(L);
+  *reinterpret_cast<fvec*>(&s_a[wave][lane * VEC]) = a;
+  __syncthreads();
+  if (tid < D) {
+    float t = s_a[0][tid];
+#pragma unroll
+    for (int w = 1; w < kDecWaves; ++w) t += s_a[w][tid];
+    out[tid] = pack1<T>((L > 0.f) ? t / L : 0.f);
   }
 }
 
@@ -837,14 +903,12 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
   const bool pipe = (int64_t)B * chunks >= (int64_t)256 * kDecPipeFrom;
   // fewer than two work-groups per CU: half-length chunks give every CU something to do
   const bool small = (int64_t)B * chunks < (int64_t)256 * kDecSmallBelow;
-  constexpr int GROUPS = kDecThreads / D;
-  const int mx = (H * G + GROUPS - 1) / GROUPS;
   auto launch = [&](auto split, auto merge) {
     hipLaunchKernelGGL(split, dim3(bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
                        (const uint16_t*)vc, (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, sumC,
                        sm_scale * kLog2e, cap);
     if (int rc = check_launch("moa_decode_fwd(split)")) return rc;
-    hipLaunchKernelGGL(merge, dim3(mx, B), dim3(kDecThreads), 0, st, (uint16_t*)o, part_acc, part_ml, head_start,
+    hipLaunchKernelGGL(merge, dim3(H * G, B), dim3(kDecThreads), 0, st, (uint16_t*)o, part_acc, part_ml, head_start,
                        head_valid, H, G, sumC, cap, 0);
     return check_launch("moa_decode_fwd(merge)");
   };
@@ -900,9 +964,7 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
                      (int)target);
   int rc = check_launch("moa_decode_fwd(grouped split)");
   if (rc) return rc;
-  constexpr int GROUPS = kDecThreads / D;
-  int mx = (H * G + GROUPS - 1) / GROUPS;
-  hipLaunchKernelGGL((decode_merge_kernel<T, D, kGqaChunk>), dim3(mx, B), dim3(kDecThreads), 0, st,
+  hipLaunchKernelGGL((decode_merge_kernel<T, D, kGqaChunk>), dim3(H * G, B), dim3(kDecThreads), 0, st,
                      (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, G, sumC, cap, (int)target);
   return check_launch("moa_decode_fwd(merge)");
 }
