@@ -42,25 +42,33 @@ __global__ __launch_bounds__(kCacheThreads) void cache_append_kernel(
   const int b = (int)(bh / H);
   const int h = (int)(bh % H);
 
-  const int64_t idx = update_index[bh];
-  const bool in_range = idx >= 0 && idx < sumC;
-  if (in_range && kc != nullptr) {
-    const int units = row_bytes / 16;
-    const size_t dst = ((size_t)b * sumC + idx) * row_bytes;
-    copy_row16(k_new + b * kn_sb + h * kn_sh, kc + dst, units, lane);
-    copy_row16(v_new + b * vn_sb + h * vn_sh, vc + dst, units, lane);
+  // Every load goes out before the first one is waited for: the launch is three memory latencies otherwise (the
+  // slot, the rows, the bookkeeping).
+  const int units = row_bytes / 16;
+  const char* const ksrc = k_new + b * kn_sb + h * kn_sh;
+  const char* const vsrc = v_new + b * vn_sb + h * vn_sh;
+  u32x4 k0 = {}, v0 = {};
+  if (kc != nullptr && lane < units) {
+    k0 = *reinterpret_cast<const u32x4*>(ksrc + (size_t)lane * 16);
+    v0 = *reinterpret_cast<const u32x4*>(vsrc + (size_t)lane * 16);
   }
+  int64_t idx = update_index[bh], vl = valid_len[bh], ml = max_len[h], ss = static_size[h], ch = circ_head[h],
+          csz = circ_size[h];
+  asm volatile("" : "+v"(idx), "+v"(vl), "+v"(ml), "+v"(ss), "+v"(ch), "+v"(csz));   // keeps the loads up here
+  const bool in_range = idx >= 0 && idx < sumC;
   if (lane == 0) {
     if (in_range && mask_cache != nullptr) mask_cache[(size_t)b * sumC + idx] = 1;
-    const int64_t vl = valid_len[bh];
-    valid_len[bh] = vl + (vl < max_len[h] ? 1 : 0);
-    const bool is_circular = (kv_len + 1) > static_size[h];
-    int64_t next = idx + 1;
-    if (is_circular) {
-      const int64_t ch = circ_head[h];
-      next = py_mod(idx + 1 - ch, circ_size[h]) + ch;
+    valid_len[bh] = vl + (vl < ml ? 1 : 0);
+    update_index[bh] = next_slot(idx, (kv_len + 1) > ss, ch, csz);
+  }
+  if (in_range && kc != nullptr) {
+    const size_t dst = ((size_t)b * sumC + idx) * row_bytes;
+    if (lane < units) {
+      *reinterpret_cast<u32x4*>(kc + dst + (size_t)lane * 16) = k0;
+      *reinterpret_cast<u32x4*>(vc + dst + (size_t)lane * 16) = v0;
     }
-    update_index[bh] = next;
+    copy_row16(ksrc, kc + dst, units, lane + kRowLanes);
+    copy_row16(vsrc, vc + dst, units, lane + kRowLanes);
   }
 }
 

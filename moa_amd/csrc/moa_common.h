@@ -58,6 +58,16 @@ __device__ __forceinline__ int64_t py_mod(int64_t a, int64_t m) {
   return (r != 0 && ((r < 0) != (m < 0))) ? r + m : r;
 }
 
+// The slot after `idx` in a head's segment (cache_utils.py:1041-1045): the next row until the head has left its
+// static part, then the next ring row.  The pointer of a ring in use lies in the ring, so its step is one compare;
+// anything else a caller may hold there takes the division.
+__device__ __forceinline__ int64_t next_slot(int64_t idx, bool is_circular, int64_t ch, int64_t csz) {
+  const int64_t off = idx + 1 - ch;
+  if (!is_circular || (off >= 0 && off < csz)) return idx + 1;
+  if (off == csz) return ch;
+  return py_mod(off, csz) + ch;
+}
+
 // DPP lane exchanges inside a row of 16 lanes.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float x) {

@@ -93,21 +93,35 @@ __device__ __forceinline__ void rope_pair(const u32x4& lo, const u32x4& hi, cons
   }
 }
 
+// The six chunks a pair needs.
+struct PairIn {
+  u32x4 lo, hi, cl, ch, sl, sh;
+};
+__device__ __forceinline__ PairIn load_pair(const char* src, const char* __restrict__ cos_row,
+                                            const char* __restrict__ sin_row, int pair, int half_bytes) {
+  const size_t o_lo = (size_t)pair * 16, o_hi = o_lo + half_bytes;
+  PairIn x;
+  x.lo = *reinterpret_cast<const u32x4*>(src + o_lo);
+  x.hi = *reinterpret_cast<const u32x4*>(src + o_hi);
+  x.cl = *reinterpret_cast<const u32x4*>(cos_row + o_lo);
+  x.ch = *reinterpret_cast<const u32x4*>(cos_row + o_hi);
+  x.sl = *reinterpret_cast<const u32x4*>(sin_row + o_lo);
+  x.sh = *reinterpret_cast<const u32x4*>(sin_row + o_hi);
+  return x;
+}
+template <typename E>
+__device__ __forceinline__ void store_pair(const PairIn& x, char* dst, int pair, int half_bytes) {
+  const size_t o_lo = (size_t)pair * 16, o_hi = o_lo + half_bytes;
+  u32x4 out_lo, out_hi;
+  rope_pair<E>(x.lo, x.hi, x.cl, x.sl, x.ch, x.sh, out_lo, out_hi);
+  *reinterpret_cast<u32x4*>(dst + o_lo) = out_lo;
+  *reinterpret_cast<u32x4*>(dst + o_hi) = out_hi;
+}
 template <typename E>
 __device__ __forceinline__ void rope_row_pair(const char* src, char* dst,
                                               const char* __restrict__ cos_row, const char* __restrict__ sin_row,
                                               int pair, int half_bytes) {
-  const size_t o_lo = (size_t)pair * 16, o_hi = o_lo + half_bytes;
-  const u32x4 lo = *reinterpret_cast<const u32x4*>(src + o_lo);
-  const u32x4 hi = *reinterpret_cast<const u32x4*>(src + o_hi);
-  const u32x4 cl = *reinterpret_cast<const u32x4*>(cos_row + o_lo);
-  const u32x4 ch = *reinterpret_cast<const u32x4*>(cos_row + o_hi);
-  const u32x4 sl = *reinterpret_cast<const u32x4*>(sin_row + o_lo);
-  const u32x4 sh = *reinterpret_cast<const u32x4*>(sin_row + o_hi);
-  u32x4 out_lo, out_hi;
-  rope_pair<E>(lo, hi, cl, sl, ch, sh, out_lo, out_hi);
-  *reinterpret_cast<u32x4*>(dst + o_lo) = out_lo;
-  *reinterpret_cast<u32x4*>(dst + o_hi) = out_hi;
+  store_pair<E>(load_pair(src, cos_row, sin_row, pair, half_bytes), dst, pair, half_bytes);
 }
 
 struct RopeTensor {
@@ -179,29 +193,34 @@ __global__ __launch_bounds__(kRopeThreads) void rope_append_kernel(
     for (int p = lane; p < pairs; p += kRopeRowLanes) rope_row_pair<E>(src, dst, cos_row, sin_row, p, half_bytes);
     return;
   }
+  // Every load goes out before the first one is waited for: the launch is three memory latencies otherwise (the
+  // slot, the rows, the bookkeeping).
   const int h = r - Hq;
   const int64_t bh = (int64_t)b * Hkv + h;
-  const int64_t idx = update_index[bh];
+  const int units = row_bytes / 16;
+  const char* const ksrc = k_new + b * kn_sb + h * kn_sh;
+  const char* const vsrc = v_new + b * vn_sb + h * vn_sh;
+  PairIn k0 = {};
+  u32x4 v0 = {};
+  if (lane < pairs) k0 = load_pair(ksrc, cos_row, sin_row, lane, half_bytes);
+  if (lane < units) v0 = *reinterpret_cast<const u32x4*>(vsrc + (size_t)lane * 16);
+  int64_t idx = update_index[bh], vl = valid_len[bh], ml = max_len[h], ss = static_size[h], chd = circ_head[h],
+          csz = circ_size[h];
+  asm volatile("" : "+v"(idx), "+v"(vl), "+v"(ml), "+v"(ss), "+v"(chd), "+v"(csz));   // keeps the loads up here
   const bool in_range = idx >= 0 && idx < sumC;
-  if (in_range) {
-    const size_t dst = ((size_t)b * sumC + idx) * row_bytes;
-    for (int p = lane; p < pairs; p += kRopeRowLanes)
-      rope_row_pair<E>(k_new + b * kn_sb + h * kn_sh, kc + dst, cos_row, sin_row, p, half_bytes);
-    const char* vsrc = v_new + b * vn_sb + h * vn_sh;
-    for (int u = lane; u < row_bytes / 16; u += kRopeRowLanes)
-      *reinterpret_cast<u32x4*>(vc + dst + (size_t)u * 16) = *reinterpret_cast<const u32x4*>(vsrc + (size_t)u * 16);
-  }
   if (lane == 0) {
     if (in_range && mask_cache != nullptr) mask_cache[(size_t)b * sumC + idx] = 1;
-    const int64_t vl = valid_len[bh];
-    valid_len[bh] = vl + (vl < max_len[h] ? 1 : 0);
-    const bool is_circular = (kv_len + 1) > static_size[h];
-    int64_t next = idx + 1;
-    if (is_circular) {
-      const int64_t chd = circ_head[h];
-      next = py_mod(idx + 1 - chd, circ_size[h]) + chd;
-    }
-    update_index[bh] = next;
+    valid_len[bh] = vl + (vl < ml ? 1 : 0);
+    update_index[bh] = next_slot(idx, (kv_len + 1) > ss, chd, csz);
+  }
+  if (in_range) {
+    const size_t dst = ((size_t)b * sumC + idx) * row_bytes;
+    if (lane < pairs) store_pair<E>(k0, kc + dst, lane, half_bytes);
+    if (lane < units) *reinterpret_cast<u32x4*>(vc + dst + (size_t)lane * 16) = v0;
+    for (int p = lane + kRopeRowLanes; p < pairs; p += kRopeRowLanes)
+      rope_row_pair<E>(ksrc, kc + dst, cos_row, sin_row, p, half_bytes);
+    for (int u = lane + kRopeRowLanes; u < units; u += kRopeRowLanes)
+      *reinterpret_cast<u32x4*>(vc + dst + (size_t)u * 16) = *reinterpret_cast<const u32x4*>(vsrc + (size_t)u * 16);
   }
 }
 
