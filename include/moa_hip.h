@@ -234,6 +234,30 @@ int moa_cache_prefill_insert(const void* k, const void* v,
                              int64_t sumC, int64_t max_cache_size, int dtype,
                              void* stream);
 
+/*
+ * Rotary embedding of a prompt and its bulk insert in one pass: what moa_rope_fwd
+ * (q -> q_out, k -> k_out) followed by moa_cache_prefill_insert (of k_out and v) give,
+ * bit for bit.  Replaces modeling_llama.py:252 and :262 for a prompt.
+ * q, k, v, q_out, k_out: host strides (order B,H,S,D; D stride 1); outputs do not overlap
+ * inputs.  kc, vc are required, max_cache_size is the largest head's segment
+ * (static_size + circ_size); with zero_rest != 0 (rings just allocated, not filled) the
+ * rows of every head's segment that the insert does not write are set to zero.
+ * workspace: as for moa_cache_prefill_insert.  Hkv <= 64; head rows of 64, 128, 256 or 512 bytes; at most
+ * 2^31 - 1 tokens (B * S) and cache rows.
+ */
+int moa_rope_prefill_insert(const void* q, const void* k, const void* v, void* q_out,
+                            void* k_out, const int64_t* q_strides, const int64_t* k_strides,
+                            const int64_t* v_strides, const int64_t* qo_strides,
+                            const int64_t* ko_strides, const void* cos, const void* sin,
+                            const int64_t* cs_strides, void* kc, void* vc,
+                            int64_t* mask_cache, int64_t* update_index, int64_t* valid_len,
+                            const int64_t* circ_head, const int64_t* circ_size,
+                            const int64_t* static_size, const int64_t* attention_mask,
+                            int64_t am_stride, void* workspace, size_t workspace_bytes,
+                            int64_t kv_len, int B, int Hq, int Hkv, int S, int D,
+                            int64_t sumC, int64_t max_cache_size, int zero_rest, int dtype,
+                            void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -54,6 +54,9 @@ SIGNATURES = {
                                       c_int64, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                       c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int, c_int, c_int,
                                       c_int, c_int64, c_int, c_void_p]),
+    "moa_rope_prefill_insert": (c_int, [c_void_p] * 5 + [_I64P] * 5 + [c_void_p, c_void_p, _I64P] + [c_void_p] * 9
+                                + [c_int64, c_void_p, c_size_t, c_int64, c_int, c_int, c_int, c_int, c_int, c_int64,
+                                   c_int64, c_int, c_int, c_void_p]),
 }
 
 _lib: Optional[ctypes.CDLL] = None

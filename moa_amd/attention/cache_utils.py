@@ -153,7 +153,9 @@ class StaticCircularCache:
         return groups
 
     # ------------------------------------------------------------------
-    def _to_device(self, layer_idx: int, device: torch.device) -> None:
+    def _to_device(self, layer_idx: int, device: torch.device, zeroed: bool = True) -> None:
+        """Places a layer on the device of its first update.  ``zeroed=False``: the caller's launch writes every
+        row of the rings."""
         if self._ready_on[layer_idx] == device:
             return
         for name in ("mask_cache", "cache_update_index", "cache_head_start_index",
@@ -164,8 +166,9 @@ class StaticCircularCache:
                 lst[layer_idx] = lst[layer_idx].to(device=device)
         if self.update_cache_content and self.key_cache[layer_idx] is None:
             shape = (self.batch_size, self.layer_cache_size[layer_idx], self.head_dim)
-            self.key_cache[layer_idx] = torch.zeros(shape, dtype=self.dtype, device=device)
-            self.value_cache[layer_idx] = torch.zeros(shape, dtype=self.dtype, device=device)
+            make = torch.zeros if zeroed else torch.empty
+            self.key_cache[layer_idx] = make(shape, dtype=self.dtype, device=device)
+            self.value_cache[layer_idx] = make(shape, dtype=self.dtype, device=device)
         self._ready_on[layer_idx] = device
         self._step_args[layer_idx] = None
 
@@ -212,6 +215,9 @@ class StaticCircularCache:
 
         seq_len = key_states.shape[-2]
         if seq_len != 1 or not self.update_cache_content:
+            if self._prompt_fits_one_launch(query_states, key_states, value_states, cos, sin, layer_idx, attention_mask):
+                return self._rope_insert_prompt(query_states, key_states, value_states, cos, sin, layer_idx,
+                                                attention_mask)
             q_embed, k_embed = apply_rotary_pos_emb(query_states, key_states, cos, sin)
             keys, values = self.update(k_embed, value_states, layer_idx, attention_mask)
             return q_embed, keys, values
@@ -289,6 +295,78 @@ class StaticCircularCache:
             self.cache_position += 1
         self._kv_len[layer_idx] += 1
         return q_view, self.key_cache[layer_idx], self.value_cache[layer_idx]
+
+    def _prompt_fits_one_launch(self, q, k, v, cos, sin, layer_idx, attention_mask) -> bool:
+        """Is this prompt one for ``_rope_insert_prompt``?  Anything out of the ordinary goes through the two steps it
+        replaces, which say what is wrong with it."""
+        if not self.update_cache_content or not 0 <= layer_idx < self.num_layers:
+            return False
+        device, H, D = k.device, self.num_head_for_each_layer[layer_idx], self.head_dim
+        if device.type != "cuda" or any(t.device != device or t.dtype != self.dtype for t in (q, k, v, cos, sin)):
+            return False
+        if k.dim() != 4 or q.dim() != 4 or v.shape != k.shape or k.shape[:2] != (self.batch_size, H) or k.shape[3] != D:
+            return False
+        N = k.shape[2]
+        if N < 2 or q.shape[0] != self.batch_size or q.shape[2:] != k.shape[2:] or q.shape[1] == 0 or H == 0:
+            return False
+        if cos.dim() != 3 or cos.shape != sin.shape or cos.shape[0] not in (1, self.batch_size) or cos.shape[1:] != k.shape[2:]:
+            return False
+        if attention_mask is not None and (attention_mask.device != device or attention_mask.dim() != 2
+                                           or attention_mask.shape[0] != self.batch_size or attention_mask.shape[1] < N):
+            return False
+        # What the kernel is made for: a wave walks the heads of a token, so these have to lie side by side (views of
+        # [B, N, H, D] projections) and be enough for its lanes; slots of all kv heads fit its lanes.  Else the two
+        # steps, which walk memory in either order a row at a time.
+        row_bytes = D * k.element_size()
+        if (row_bytes not in (64, 128, 256, 512) or H > 64 or q.shape[1] + H < 8 or self.batch_size > 65535
+                or q.stride(1) >= q.stride(2) or k.stride(1) >= k.stride(2)
+                or self.batch_size * N >= 2 ** 31 or self.layer_cache_size[layer_idx] >= 2 ** 31):
+            return False
+        # rings that exist, or that this call allocates
+        return (self.key_cache[layer_idx] is None) == (self._ready_on[layer_idx] is None)
+
+    def _rope_insert_prompt(self, q, k, v, cos, sin, layer_idx, attention_mask):
+        """Rotary embedding and insert of a prompt in one pass over q, k and v (moa_rope_prefill_insert)."""
+        from ..kernels.rotary import _cos_sin_strides
+
+        device = k.device
+        B, Hq, N, D = q.shape
+        H = k.shape[1]
+        cos, sin, css = _cos_sin_strides(cos, sin, B, N, D)
+        q_out, k_out = torch.empty_like(q), torch.empty_like(k)
+        q, k, v_in = (t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
+        am_ptr, am_stride, ws_ptr, ws_bytes = None, 0, None, 0
+        lib = _lib.load()
+        if attention_mask is not None:
+            am = attention_mask[:, -N:]
+            if am.dtype != torch.int64 or am.stride(-1) != 1:
+                am = am.to(torch.int64).contiguous()
+            am_ptr, am_stride = am.data_ptr(), am.stride(0)
+            ws_bytes = lib.moa_cache_prefill_workspace_bytes(B, N)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+            ws_ptr = ws.data_ptr()
+        fresh = self.key_cache[layer_idx] is None
+        self._to_device(layer_idx, device, zeroed=False)
+        upd = self.cache_update_index[layer_idx]
+        assert upd.is_contiguous() and self.cache_valid_length[layer_idx].is_contiguous()
+        kc, vc = self.key_cache[layer_idx], self.value_cache[layer_idx]
+        rc = lib.moa_rope_prefill_insert(
+            q.data_ptr(), k.data_ptr(), v_in.data_ptr(), q_out.data_ptr(), k_out.data_ptr(), _lib.i64_array(q.stride()),
+            _lib.i64_array(k.stride()), _lib.i64_array(v_in.stride()), _lib.i64_array(q_out.stride()),
+            _lib.i64_array(k_out.stride()), cos.data_ptr(), sin.data_ptr(), css, kc.data_ptr(), vc.data_ptr(),
+            self.mask_cache[layer_idx].data_ptr(), upd.data_ptr(), self.cache_valid_length[layer_idx].data_ptr(),
+            self.circular_cache_head_index[layer_idx].data_ptr(), self.circular_cache_size[layer_idx].data_ptr(),
+            self.static_cache_size[layer_idx].data_ptr(), am_ptr, am_stride, ws_ptr, ws_bytes, self._kv_len[layer_idx],
+            B, Hq, H, N, D, self.layer_cache_size[layer_idx], self._max_cache_size[layer_idx], int(fresh),
+            _lib.dtype_code(self.dtype), _lib.current_stream_ptr(device))
+        if rc != 0 and fresh:   # refused: the rings are what an update that failed would have left
+            kc.zero_()
+            vc.zero_()
+        _lib.check(rc)
+        if layer_idx == 0:
+            self.cache_position += N
+        self._kv_len[layer_idx] += N
+        return q_out, k_out, v
 
     def update(
         self,

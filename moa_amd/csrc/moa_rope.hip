@@ -15,13 +15,18 @@
 // Both kernels are HBM/latency bound byte work: 128-bit accesses, no LDS.  One
 // thread owns a PAIR of 16-byte chunks (elements e..e+7 and e+D/2..e+D/2+7 of
 // one head row), reads both and writes both, which makes in-place use safe.
-#include "moa_common.h"
+#include "moa_ring.h"
 
 // Every product and sum below is rounded on its own, as torch does.  This file must be compiled
 // with -ffp-contract=off (the build does): otherwise the compiler contracts the rounded products
 // and the sum into v_fma_f16 / v_pk_fma_f16, which rounds once.
 
 namespace moa {
+
+template <int V>
+struct IC {
+  static constexpr int value = V;
+};
 
 constexpr int kRopeThreads = 256;
 constexpr int kRopeRowLanes = 16;   // lanes that share one head row in the fused kernel
@@ -224,6 +229,206 @@ __global__ __launch_bounds__(kRopeThreads) void rope_append_kernel(
   }
 }
 
+// cos and sin chunks of one pair, and the rotation of a row's pair by them: what rope_pair computes, bit for bit, in
+// the fewest instructions, for a kernel that keeps the coefficients over the heads of a token.
+template <typename E>
+struct Coef {
+  u32x4 cl, sl, ch, sh;
+  __device__ __forceinline__ void rotate(const u32x4& lo, const u32x4& hi, u32x4& out_lo, u32x4& out_hi) const {
+    rope_pair<E>(lo, hi, cl, sl, ch, sh, out_lo, out_hi);
+  }
+};
+// f16: packed f16 products and sums.  A product of two f16 is exact in fp32 and a sum of two f16 rounded to fp32 and
+// then to f16 is the sum rounded once (24 >= 2 * 11 + 2 bits), so these are the fp32 evaluation's bits.
+template <>
+struct Coef<EF16> {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  u32x4 cl, sl, ch, sh;
+  __device__ __forceinline__ void rotate(const u32x4& lo, const u32x4& hi, u32x4& out_lo, u32x4& out_hi) const {
+    const h8 x1 = __builtin_bit_cast(h8, lo), x2 = __builtin_bit_cast(h8, hi);
+    const h8 a1 = x1 * __builtin_bit_cast(h8, cl), b1 = x2 * __builtin_bit_cast(h8, sl);
+    const h8 a2 = x2 * __builtin_bit_cast(h8, ch), b2 = x1 * __builtin_bit_cast(h8, sh);
+    out_lo = __builtin_bit_cast(u32x4, a1 - b1);
+    out_hi = __builtin_bit_cast(u32x4, a2 + b2);
+  }
+};
+// bf16: fp32 arithmetic, two values to a conversion
+template <>
+struct Coef<EBF16> {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  u32x4 cl, sl, ch, sh;
+  static __device__ __forceinline__ uint32_t pack(float x, float y) {
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{x, y}), b2));
+  }
+  static __device__ __forceinline__ float even(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+  static __device__ __forceinline__ float odd(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+  __device__ __forceinline__ void rotate(const u32x4& lo, const u32x4& hi, u32x4& out_lo, u32x4& out_hi) const {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = even(lo[i]), q = odd(lo[i]), r = even(hi[i]), t = odd(hi[i]);
+      const uint32_t a1 = pack(__fmul_rn(p, even(cl[i])), __fmul_rn(q, odd(cl[i])));
+      const uint32_t b1 = pack(__fmul_rn(r, even(sl[i])), __fmul_rn(t, odd(sl[i])));
+      const uint32_t a2 = pack(__fmul_rn(r, even(ch[i])), __fmul_rn(t, odd(ch[i])));
+      const uint32_t c2 = pack(__fmul_rn(p, even(sh[i])), __fmul_rn(q, odd(sh[i])));
+      out_lo[i] = pack(__fsub_rn(even(a1), even(b1)), __fsub_rn(odd(a1), odd(b1)));
+      out_hi[i] = pack(__fadd_rn(even(a2), even(c2)), __fadd_rn(odd(a2), odd(c2)));
+    }
+  }
+};
+
+// The start of a generation in one pass over the projections: q and k of a whole prompt rotated into q_out and k_out,
+// kept rows of k stored into their ring slots on the way.  HBM bound, with the vector ALU close behind it: a thread
+// per chunk pair that works out its own row and slot takes 1160 us at the size below, so a wave owns a piece of a
+// token here, kRopeAtOnce wave-wide loads of its q heads or of its kv heads (consecutive memory): cos and sin are
+// fetched once for all of them, and in a kv piece the lanes work out the slots of all kv heads side by side.  A
+// rotated row is in registers when its slot is known, so the rings of k cost their writes only.
+// The first work-groups walk the rings' rows instead: they fetch the v row that belongs into each, and in rings that
+// have just been allocated (FRESH) zero the rows no token goes to, so no fill runs in front.
+// Batch 8, 32 heads of 128, 16384 tokens, bf16, a third of the tokens kept (4.9 GB): 970 us (5.1 TB/s) against 743 us
+// rotary + 87 us fill + 268 us insert in separate launches; 64 query heads on 8 rings, batch 1: 103 us.
+struct RingArgs {
+  const char* v;
+  int64_t v_sb, v_sh, v_sn;   // byte strides of v
+  char *kc, *vc;
+  int64_t *mask_cache;
+  const int64_t *update_index, *circ_head, *circ_size, *static_size;
+  const int32_t *tok_of, *rank_of, *n_valid;   // with an attention mask, else null
+  int64_t kv_len, sumC;
+};
+constexpr int kRingRows = 256;      // segment rows per work-group of the ring part
+constexpr int kRingAtOnce = 4;      // rows a group of 16 lanes has under way
+// Wave-wide row loads a wave has under way, and all it does.  Measured at the two sizes above: 2: 970 and 103 us,
+// 4: 1000 and 106 us, 8: 950 and 110 us; a whole token (q and k heads in turn) to a wave: 960 and 118 us.
+constexpr int kRopeAtOnce = 2;
+// From this many bytes of q and k on they are read, and their rotated copies written, non-temporally: the copies
+// are past what the last-level cache (256 MB) could keep for the attention that reads them next, and lines held for
+// them only cost (2.1 GB: 1015 -> 975 us a launch).
+constexpr int64_t kRopeNtBytes = (int64_t)256 << 20;
+template <bool NT>
+__device__ __forceinline__ u32x4 load16(const char* p) {
+  const u32x4* s = reinterpret_cast<const u32x4*>(p);
+  if constexpr (NT) return __builtin_nontemporal_load(s);
+  else return *s;
+}
+template <bool NT>
+__device__ __forceinline__ void store16(char* p, u32x4 x) {
+  if constexpr (NT) __builtin_nontemporal_store(x, reinterpret_cast<u32x4*>(p));
+  else *reinterpret_cast<u32x4*>(p) = x;
+}
+template <typename E, int P /* chunk pairs per row: 64 % P == 0 */, bool FRESH, bool NT>
+__global__ __launch_bounds__(kRopeThreads) void rope_insert_kernel(
+    RopeTensor tq, RopeTensor tk, const char* __restrict__ cos, const char* __restrict__ sin, int64_t cs_sb,
+    int64_t cs_sn, RingArgs ra, int B, int Hq, int Hkv, int N, unsigned ring_blocks, int ring_slices /* per head */,
+    int pieces /* of a token's heads */) {
+  constexpr int half_bytes = P * 16;
+  if (blockIdx.x < ring_blocks) {
+    const unsigned bh = blockIdx.x / (unsigned)ring_slices, slice = blockIdx.x % (unsigned)ring_slices;
+    const int b = (int)(bh / (unsigned)Hkv), h = (int)(bh % (unsigned)Hkv);
+    const HeadRing g = load_ring(ra.update_index, ra.circ_head, ra.circ_size, ra.static_size, ra.kv_len, bh, h);
+    const int64_t nv = ra.n_valid ? (int64_t)ra.n_valid[b] : (int64_t)N;
+    const int64_t first = g.ch - g.s, rows = min(g.s + g.csz, (int64_t)(slice + 1) * kRingRows);
+    const int lane = threadIdx.x % kRopeRowLanes;
+    const int row_bytes = 2 * half_bytes, units = row_bytes / 16;
+    for (int64_t r0 = (int64_t)slice * kRingRows + threadIdx.x / kRopeRowLanes; r0 < rows;
+         r0 += kRopeRowsPerBlock * kRingAtOnce) {
+      const char* src[kRingAtOnce];
+      size_t dst[kRingAtOnce];
+      bool in[kRingAtOnce], keep[kRingAtOnce];
+#pragma unroll
+      for (int j = 0; j < kRingAtOnce; ++j) {
+        const int64_t r = r0 + j * kRopeRowsPerBlock, row = first + r;
+        in[j] = r < rows && row >= 0 && row < ra.sumC;
+        int64_t t = in[j] ? token_of_row(g, row, nv) : -1;
+        keep[j] = t >= 0;
+        if (keep[j] && ra.tok_of) t = ra.tok_of[(int64_t)b * N + t];
+        src[j] = ra.v + b * ra.v_sb + h * ra.v_sh + t * ra.v_sn;
+        dst[j] = ((size_t)b * ra.sumC + row) * row_bytes;
+        if (keep[j] && lane == 0 && ra.mask_cache != nullptr) ra.mask_cache[(size_t)b * ra.sumC + row] = 1;
+      }
+      for (int u = lane; u < units; u += kRopeRowLanes) {
+        u32x4 x[kRingAtOnce];
+#pragma unroll
+        for (int j = 0; j < kRingAtOnce; ++j) {
+          x[j] = u32x4{0, 0, 0, 0};
+          if (keep[j]) x[j] = *reinterpret_cast<const u32x4*>(src[j] + (size_t)u * 16);
+        }
+#pragma unroll
+        for (int j = 0; j < kRingAtOnce; ++j) {
+          if (keep[j] || (FRESH && in[j])) *reinterpret_cast<u32x4*>(ra.vc + dst[j] + (size_t)u * 16) = x[j];
+          if (FRESH && in[j] && !keep[j]) *reinterpret_cast<u32x4*>(ra.kc + dst[j] + (size_t)u * 16) = x[j];
+        }
+      }
+    }
+    return;
+  }
+  constexpr int R = 64 / P;           // rows per wave-wide load
+  const int lane = threadIdx.x & 63;
+  const unsigned unit = (blockIdx.x - ring_blocks) * (kRopeThreads / 64) +
+                        (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned token = unit / (unsigned)pieces, piece = unit % (unsigned)pieces;
+  if (token >= (unsigned)B * (unsigned)N) return;
+  const int b = (int)(token / (unsigned)N), n = (int)(token % (unsigned)N);
+  const int sub = lane / P;
+  const size_t o_lo = (size_t)(lane % P) * 16;
+
+  Coef<E> w;
+  {
+    const char* c = cos + b * cs_sb + n * cs_sn + o_lo;
+    const char* s = sin + b * cs_sb + n * cs_sn + o_lo;
+    w.cl = *reinterpret_cast<const u32x4*>(c);
+    w.ch = *reinterpret_cast<const u32x4*>(c + half_bytes);
+    w.sl = *reinterpret_cast<const u32x4*>(s);
+    w.sh = *reinterpret_cast<const u32x4*>(s + half_bytes);
+  }
+  auto walk = [&](const RopeTensor& t, int h0, int H, auto RING) __attribute__((always_inline)) {
+    const char* const src = t.src + b * t.sb + n * t.sn + o_lo;
+    char* const dst = t.dst + b * t.db + n * t.dn + o_lo;
+    u32x4 lo[kRopeAtOnce], hi[kRopeAtOnce];
+#pragma unroll
+    for (int j = 0; j < kRopeAtOnce; ++j) {
+      const int h = h0 + j * R + sub;
+      if (h < H) {
+        const char* p = src + h * t.sh;
+        lo[j] = load16<NT>(p);
+        hi[j] = load16<NT>(p + half_bytes);
+      }
+    }
+    int slot = -1;   // ring row of the token in head `lane`, -1 if it is not kept
+    if (decltype(RING)::value && lane < Hkv) {
+      const HeadRing g = load_ring(ra.update_index, ra.circ_head, ra.circ_size, ra.static_size, ra.kv_len,
+                                   (int64_t)b * Hkv + lane, lane);
+      const int64_t a = ra.rank_of ? (int64_t)ra.rank_of[token] : (int64_t)n;
+      const int64_t nv = ra.n_valid ? (int64_t)ra.n_valid[b] : (int64_t)N;
+      // ring tokens older than the last csz are dropped whatever their slot (:1122-1133)
+      if (a >= 0 && (nv - a <= g.csz || g.kv0 + a <= g.s)) {
+        const int64_t at = slot_of(g, a);
+        if (keep_of(g, at, nv - a) && at >= 0 && at < ra.sumC) slot = (int)at;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kRopeAtOnce; ++j) {
+      const int h = h0 + j * R + sub;
+      const int row = decltype(RING)::value ? __shfl(slot, h & 63, 64) : -1;
+      if (h < H) {
+        u32x4 out_lo, out_hi;
+        w.rotate(lo[j], hi[j], out_lo, out_hi);
+        char* p = dst + h * t.dh;
+        store16<NT>(p, out_lo);
+        store16<NT>(p + half_bytes, out_hi);
+        if (decltype(RING)::value && row >= 0) {
+          char* ring = ra.kc + ((size_t)b * ra.sumC + row) * (2 * half_bytes) + o_lo;
+          *reinterpret_cast<u32x4*>(ring) = out_lo;
+          *reinterpret_cast<u32x4*>(ring + half_bytes) = out_hi;
+        }
+      }
+    }
+  };
+  const int first = (int)piece * (R * kRopeAtOnce), q_pieces = (Hq + R * kRopeAtOnce - 1) / (R * kRopeAtOnce);
+  if ((int)piece < q_pieces) walk(tq, first, Hq, IC<0>{});
+  else walk(tk, first - q_pieces * (R * kRopeAtOnce), Hkv, IC<1>{});
+}
+
 static int check_rope_rows(const char* who, const char* name, int D, int eb, const int64_t* strides, int nstr,
                            const void* p) {
   if (!p) return fail(MOA_ERR_ARG, "%s: null %s", who, name);
@@ -333,4 +538,92 @@ extern "C" int moa_rope_cache_append(const void* q_new, const void* k_new, const
   else MOA_ROPE_APPEND_LAUNCH(EF32);
 #undef MOA_ROPE_APPEND_LAUNCH
   return check_launch(who);
+}
+
+extern "C" int moa_rope_prefill_insert(const void* q, const void* k, const void* v, void* q_out, void* k_out,
+                                       const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                       const int64_t* qo_strides, const int64_t* ko_strides, const void* cos,
+                                       const void* sin, const int64_t* cs_strides, void* kc, void* vc,
+                                       int64_t* mask_cache, int64_t* update_index, int64_t* valid_len,
+                                       const int64_t* circ_head, const int64_t* circ_size,
+                                       const int64_t* static_size, const int64_t* attention_mask, int64_t am_stride,
+                                       void* workspace, size_t workspace_bytes, int64_t kv_len, int B, int Hq,
+                                       int Hkv, int S, int D, int64_t sumC, int64_t max_cache_size, int zero_rest,
+                                       int dtype, void* stream) {
+  const char* who = "moa_rope_prefill_insert";
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || S <= 0 || sumC <= 0)
+    return fail(MOA_ERR_ARG, "%s: B, Hq, Hkv, S, sumC must be positive", who);
+  if (Hkv > 64 || B > 65535) return fail(MOA_ERR_UNSUPPORTED, "%s: Hkv <= 64, B <= 65535", who);
+  if (sumC > 0x7fffffffLL) return fail(MOA_ERR_UNSUPPORTED, "%s: at most 2^31 - 1 cache rows per batch row", who);
+  if (!update_index || !valid_len || !circ_head || !circ_size || !static_size)
+    return fail(MOA_ERR_ARG, "%s: null index array", who);
+  if (!kc || !vc || !aligned16(kc) || !aligned16(vc))
+    return fail(MOA_ERR_ARG, "%s: kc and vc must be set and 16-byte aligned", who);
+  if (max_cache_size <= 0) return fail(MOA_ERR_ARG, "%s: max_cache_size must be positive", who);
+  int eb = 0, rc;
+  if ((rc = check_head_dim(who, D, dtype, &eb))) return rc;
+  if ((rc = check_rope_rows(who, "q", D, eb, q_strides, 4, q))) return rc;
+  if ((rc = check_rope_rows(who, "k", D, eb, k_strides, 4, k))) return rc;
+  if ((rc = check_rope_rows(who, "v", D, eb, v_strides, 4, v))) return rc;
+  if ((rc = check_rope_rows(who, "q_out", D, eb, qo_strides, 4, q_out))) return rc;
+  if ((rc = check_rope_rows(who, "k_out", D, eb, ko_strides, 4, k_out))) return rc;
+  if ((rc = check_rope_rows(who, "cos", D, eb, cs_strides, 3, cos))) return rc;
+  if ((rc = check_rope_rows(who, "sin", D, eb, cs_strides, 3, sin))) return rc;
+  const int half_bytes = D * eb / 2;
+  const int pairs = half_bytes / 16;
+  if (pairs != 2 && pairs != 4 && pairs != 8 && pairs != 16)
+    return fail(MOA_ERR_UNSUPPORTED, "%s: a head row of %d bytes (64, 128, 256 or 512)", who, 2 * half_bytes);
+  const int64_t tokens = (int64_t)B * S;
+  const int per_piece = 64 / pairs * kRopeAtOnce;   // heads a wave takes
+  const int pieces = (Hq + per_piece - 1) / per_piece + (Hkv + per_piece - 1) / per_piece;
+  const int64_t units = tokens * pieces;
+  const int64_t unit_blocks = (units + kRopeThreads / 64 - 1) / (kRopeThreads / 64);
+  const int64_t slices = (max_cache_size + kRingRows - 1) / kRingRows;
+  const int64_t ring_blocks = (int64_t)B * Hkv * slices;
+  const int64_t blocks = unit_blocks + ring_blocks;
+  if (units > 0x7fffffffLL || blocks > 0x7fffffffLL) return fail(MOA_ERR_UNSUPPORTED, "%s: too many tokens", who);
+  hipStream_t st = (hipStream_t)stream;
+  RingArgs ra = {(const char*)v, v_strides[0] * eb, v_strides[1] * eb, v_strides[2] * eb, (char*)kc, (char*)vc, mask_cache,
+                 update_index, circ_head, circ_size, static_size, nullptr, nullptr, nullptr, kv_len, sumC};
+  if (attention_mask != nullptr) {
+    const size_t need = moa_cache_prefill_workspace_bytes(B, S);
+    if (workspace == nullptr || workspace_bytes < need)
+      return fail(MOA_ERR_WORKSPACE, "%s: workspace %zu < %zu bytes", who, workspace_bytes, need);
+    int32_t* tok_of = reinterpret_cast<int32_t*>(workspace);
+    int32_t* rank_of = tok_of + (size_t)B * (size_t)S;
+    int32_t* n_valid = rank_of + (size_t)B * (size_t)S;
+    if ((rc = launch_mask_scan(attention_mask, am_stride, B, S, tok_of, n_valid, rank_of, st))) return rc;
+    ra.tok_of = tok_of;
+    ra.rank_of = rank_of;
+    ra.n_valid = n_valid;
+  }
+  const RopeTensor tq = {(const char*)q, (char*)q_out, q_strides[0] * eb, q_strides[1] * eb, q_strides[2] * eb,
+                         qo_strides[0] * eb, qo_strides[1] * eb, qo_strides[2] * eb};
+  const RopeTensor tk = {(const char*)k, (char*)k_out, k_strides[0] * eb, k_strides[1] * eb, k_strides[2] * eb,
+                         ko_strides[0] * eb, ko_strides[1] * eb, ko_strides[2] * eb};
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kRopeThreads), 0, st, tq, tk, (const char*)cos,
+                       (const char*)sin, cs_strides[0] * eb, cs_strides[1] * eb, ra, B, Hq, Hkv, S, (unsigned)ring_blocks,
+                       (int)slices, pieces);
+    return check_launch(who);
+  };
+  const bool nt = (int64_t)B * S * (Hq + Hkv) * D * eb >= kRopeNtBytes;
+  auto by_options = [&](auto e, auto p) {
+    typedef decltype(e) E;
+    constexpr int P = decltype(p)::value;
+    if (nt) return zero_rest ? launch(&rope_insert_kernel<E, P, true, true>) : launch(&rope_insert_kernel<E, P, false, true>);
+    return zero_rest ? launch(&rope_insert_kernel<E, P, true, false>) : launch(&rope_insert_kernel<E, P, false, false>);
+  };
+  auto by_row = [&](auto e) {
+    switch (pairs) {
+      case 2: return by_options(e, IC<2>{});
+      case 4: return by_options(e, IC<4>{});
+      case 8: return by_options(e, IC<8>{});
+      default: return by_options(e, IC<16>{});
+    }
+  };
+  rc = dtype == MOA_DTYPE_F16 ? by_row(EF16{}) : dtype == MOA_DTYPE_BF16 ? by_row(EBF16{}) : by_row(EF32{});
+  if (rc) return rc;
+  // behind the copy on the same stream: it overwrites update_index, which the copy reads
+  return launch_prefill_index(update_index, valid_len, circ_head, circ_size, static_size, ra.n_valid, kv_len, B, Hkv, S, st);
 }

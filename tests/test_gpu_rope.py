@@ -116,6 +116,48 @@ def test_rope_update_decode_steps(dev, dtype):
     assert cache._kv_len[0] == S + steps == o.kv_len
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.float16, 128), (torch.bfloat16, 64), (torch.bfloat16, 128),
+                                     (torch.float16, 32), (torch.float32, 128), (torch.float16, 80)])
+@pytest.mark.parametrize("S", [2, 63, 64, 65, 150, 701])   # inside the static part, around it, past every ring
+@pytest.mark.parametrize("padded", [False, True])
+def test_prompt_in_one_launch_equals_the_two_steps(dev, dtype, D, S, padded):
+    """rope_update of a prompt (one pass) against apply_rotary_pos_emb followed by update: every output and the
+    whole rings bit for bit, on rings that are allocated by the call in memory full of NaN, then once more on rings
+    in use; heads side by side (the one pass) and apart (the two steps), a row size that takes the two steps, grouped
+    heads, a head without a ring, one without a static part, a row of padding only."""
+    from moa_amd import StaticCircularCache
+    from moa_amd.kernels.rotary import apply_rotary_pos_emb
+    B, Hq, cache_size, static = 3, 8, [128, 64, 640, 333], [64, 64, 0, 64]
+    H, sumc = len(cache_size), sum(cache_size)
+
+    def make():
+        return StaticCircularCache([cache_size], static_size=[static], batch_size=B, head_dim=D, device=dev, dtype=dtype)
+
+    one, two = make(), make()
+    for step, heads_inner in enumerate([True, True, False]):
+        q, k, v = (_rand((B, S, n, D) if heads_inner else (B, n, S, D), dtype, 7 * S + i + step).to(dev)
+                   for i, n in enumerate((Hq, H, H)))
+        if heads_inner:
+            q, k, v = (t.transpose(1, 2) for t in (q, k, v))
+        cos, sin = (t.to(dev) for t in rope_cos_sin(torch.arange(S)[None, :] + step * S, D, dtype=dtype))
+        mask = None
+        if padded:   # left padding, holes, and a row without a valid token
+            mask = (torch.rand(B, S, generator=torch.Generator().manual_seed(S)) < 0.7).to(torch.int64).to(dev)
+            mask[0, : S // 3] = 0
+            mask[2] = 0
+        poison = [torch.full((B, sumc, D), float("nan"), dtype=dtype, device=dev) for _ in range(4)]
+        del poison   # the allocator hands this memory to the rings
+        got = one.rope_update(q, k, v, cos, sin, 0, mask)
+        qe, ke = apply_rotary_pos_emb(q, k, cos, sin)
+        want = (qe,) + two.update(ke, v, 0, mask)
+        for a, b in zip(got, want):
+            assert a.stride() == b.stride() and _same_bits(a, b), step
+        for name in ("key_cache", "value_cache", "mask_cache", "cache_update_index", "cache_valid_length"):
+            a, b = getattr(one, name)[0], getattr(two, name)[0]
+            assert torch.equal(a, b), (name, step)
+        assert one.get_seq_length() == two.get_seq_length() and one.cache_position == two.cache_position
+
+
 def test_fused_step_feeds_the_decode_kernel(dev):
     """rope_update (one launch) + mixture_of_sparse_attention against the oracle's decode on the
     oracle's cache: what a decoder layer sees."""
