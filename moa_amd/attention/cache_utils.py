@@ -13,6 +13,7 @@ from __future__ import annotations
 import math
 from typing import Any, Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 from torch import Tensor
 
@@ -59,33 +60,44 @@ class StaticCircularCache:
             for c, s in zip(cache_size[layer_id], static_size[layer_id]):
                 assert 0 <= s <= c, "static size must lie within the cache size"
 
-        def i64(x):
-            return torch.tensor(x, device=device, dtype=torch.int64)
-
-        self.cache_max_length: List[Tensor] = [i64(c) for c in cache_size]
-        self.static_cache_size: List[Tensor] = [i64(s) for s in static_size]
-        self.circular_cache_size: List[Tensor] = [
-            c - s for c, s in zip(self.cache_max_length, self.static_cache_size)]
         self.layer_cache_size: List[int] = [sum(c) for c in cache_size]
         self._max_cache_size: List[int] = [max(c) for c in cache_size]
         self._max_static_size: List[int] = [max(x) for x in static_size]
 
-        starts = []
-        for c in cache_size:
-            acc, row = 0, []
-            for x in c:
-                row.append(acc)
-                acc += x
-            starts.append(row)
-        self.cache_head_start_index: List[Tensor] = [
-            i64(starts[l])[None, :].expand(batch_size, -1).contiguous() for l in range(self.num_layers)]
-        self.head_index: List[Tensor] = [
-            i64(starts[l] + [starts[l][-1] + cache_size[l][-1]]) for l in range(self.num_layers)]
-        self.circular_cache_head_index: List[Tensor] = [
-            i64([a + s for a, s in zip(starts[l], static_size[l])]) for l in range(self.num_layers)]
+        # The int64 tables of all layers are laid out in one buffer that goes to the device in one copy, from pinned
+        # memory and so without a synchronisation (a copy and a wait for the GPU per table cost 50 us a layer); the
+        # tables are views of it.
+        place = torch.empty(0, device=device).device
+        if place.type == "cuda" and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("StaticCircularCache: a cache cannot be made while a HIP graph is being captured")
+        B = batch_size
+        heads = self.num_head_for_each_layer
+        packed = torch.empty(sum((4 + 3 * B) * h + h + 1 for h in heads), dtype=torch.int64, device="cpu",
+                             pin_memory=place.type == "cuda")
+        flat, at = packed.numpy(), 0
+        for c, s in zip(cache_size, static_size):
+            h = len(c)
+            rows = flat[at:at + (4 + 3 * B) * h].reshape(4 + 3 * B, h)
+            ends = flat[at + rows.size:at + rows.size + h + 1]   # head_index
+            at += rows.size + h + 1
+            rows[0], rows[1] = c, s
+            rows[2] = rows[0] - rows[1]
+            ends[0] = 0
+            np.cumsum(rows[0], out=ends[1:])
+            rows[3] = ends[:-1] + rows[1]
+            rows[4:4 + 2 * B] = ends[:-1]   # where every head starts, and the slot of its next token
+            rows[4 + 2 * B:] = 0
+        tables = packed.to(device=place, non_blocking=True).split(
+            [n for h in heads for n in (h, h, h, h, B * h, B * h, B * h, h + 1)])
+        self.cache_max_length: List[Tensor] = list(tables[0::8])
+        self.static_cache_size: List[Tensor] = list(tables[1::8])
+        self.circular_cache_size: List[Tensor] = list(tables[2::8])
+        self.circular_cache_head_index: List[Tensor] = list(tables[3::8])
+        self.cache_head_start_index: List[Tensor] = [t.view(B, h) for t, h in zip(tables[4::8], heads)]
         # materialised [B, H]: the append kernel advances it in place
-        self.cache_update_index: List[Tensor] = [
-            i64(starts[l])[None, :].expand(batch_size, -1).contiguous() for l in range(self.num_layers)]
+        self.cache_update_index: List[Tensor] = [t.view(B, h) for t, h in zip(tables[5::8], heads)]
+        self.cache_valid_length: List[Tensor] = [t.view(B, h) for t, h in zip(tables[6::8], heads)]
+        self.head_index: List[Tensor] = list(tables[7::8])
 
         self.cache_position = 0
         self._kv_len = [0 for _ in range(self.num_layers)]
@@ -98,9 +110,6 @@ class StaticCircularCache:
         self.value_cache: List[Optional[Tensor]] = [None] * self.num_layers
         self.mask_cache: List[Tensor] = [
             torch.zeros(batch_size, n, dtype=torch.int64, device=device) for n in self.layer_cache_size]
-        self.cache_valid_length: List[Tensor] = [
-            torch.zeros((batch_size, h), dtype=torch.int64, device=device)
-            for h in self.num_head_for_each_layer]
 
     def __getstate__(self):
         """Copies (copy.deepcopy, pickling) do not take the per-layer call arguments along: those hold
