@@ -83,6 +83,18 @@ int moa_prefill_fwd(const void* q, const void* k, const void* v, void* o,
                     float sm_scale, int dtype, void* stream);
 
 /*
+ * moa_prefill_fwd with the spans as the caller's wrapper holds them
+ * (mixture_of_attention.py:416-444): sink_size and local_size are int64 [Hkv] TOKEN
+ * counts, of which whole blocks of 64 count (rounded down).
+ */
+int moa_prefill_fwd_tokens(const void* q, const void* k, const void* v, void* o,
+                           const int64_t* q_strides, const int64_t* k_strides,
+                           const int64_t* v_strides, const int64_t* o_strides,
+                           int B, int Hq, int Hkv, int N, int D,
+                           const int64_t* sink_size, const int64_t* local_size,
+                           float sm_scale, int dtype, void* stream);
+
+/*
  * Bytes of scratch moa_decode_fwd needs for these sizes (split-K partials).
  */
 size_t moa_decode_workspace_bytes(int B, int Hq, int Hkv, int D, int64_t sumC);

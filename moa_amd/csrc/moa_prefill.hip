@@ -88,7 +88,8 @@ struct PrefillArgs {
   const uint16_t *q, *k, *v;
   uint16_t* o;
   Strides4 qs, ks, vs, os;
-  const int64_t *sink_blocks, *local_blocks;
+  const int64_t *sink_blocks, *local_blocks;   // spans per kv head: blocks, or tokens with span_shift = 6
+  int span_shift;
   PrefillQueue* queue;
   int BH, Hq, group, N, n_qtiles;
   int per_head, Hkv;   // (BH / Hq) * group pairs per kv head in the sorted list; Hq / group
@@ -141,10 +142,11 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     const int nb = (a0->N + kKV - 1) / kKV;
     const int64_t* sink_blocks = a0->sink_blocks;
     const int64_t* local_blocks = a0->local_blocks;
+    const int shift = a0->span_shift;
     if (Hkv <= kMaxSortedHeads) {
       for (int h = tid; h < Hkv; h += kPfThreads) {
-        s_ns[h] = (int)max((int64_t)0, min((int64_t)nb, sink_blocks[h]));
-        s_nl[h] = (int)max((int64_t)0, min((int64_t)nb, local_blocks[h]));
+        s_ns[h] = (int)max((int64_t)0, min((int64_t)nb, sink_blocks[h] >> shift));
+        s_nl[h] = (int)max((int64_t)0, min((int64_t)nb, local_blocks[h] >> shift));
       }
       __syncthreads();
       for (int h = tid; h < Hkv; h += kPfThreads) {
@@ -216,8 +218,8 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     const int hk = sorted ? s_head_of_rank[ph.q] : ph.q;
     const int b = bg.q;
     const int hq = hk * group + bg.r;
-    const int ns = sorted ? s_ns[hk] : (int)max((int64_t)0, min((int64_t)nb, ap->sink_blocks[hk]));
-    const int nl = sorted ? s_nl[hk] : (int)max((int64_t)0, min((int64_t)nb, ap->local_blocks[hk]));
+    const int ns = sorted ? s_ns[hk] : (int)max((int64_t)0, min((int64_t)nb, ap->sink_blocks[hk] >> ap->span_shift));
+    const int nl = sorted ? s_nl[hk] : (int)max((int64_t)0, min((int64_t)nb, ap->local_blocks[hk] >> ap->span_shift));
     const int mb0 = kQBlocks * qt;                              // first query block of the group
     const int mbl = min(kQBlocks * qt + kQBlocks - 1, nb - 1);  // last one that exists
     // tiles of the work-group: sinks [0, hi1], then band [lo2, mbl]
@@ -758,7 +760,7 @@ template <typename T, int D>
 static int launch_prefill(const void* q, const void* k, const void* v, void* o, const int64_t* qs,
                           const int64_t* ks, const int64_t* vs, const int64_t* os, int B, int Hq,
                           int Hkv, int N, const int64_t* sink_blocks, const int64_t* local_blocks,
-                          float sm_scale, hipStream_t st) {
+                          int span_shift, float sm_scale, hipStream_t st) {
   constexpr int NW = 8, S = 4;
   constexpr int kQRows = NW * kWRows;
   const int n_qtiles = (N + kQRows - 1) / kQRows;
@@ -785,7 +787,7 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* o, 
   PrefillArgs args;
   args.q = (const uint16_t*)q; args.k = (const uint16_t*)k; args.v = (const uint16_t*)v; args.o = (uint16_t*)o;
   args.qs = sq; args.ks = sk; args.vs = sv; args.os = so;
-  args.sink_blocks = sink_blocks; args.local_blocks = local_blocks; args.queue = queue;
+  args.sink_blocks = sink_blocks; args.local_blocks = local_blocks; args.span_shift = span_shift; args.queue = queue;
   args.BH = BH; args.Hq = Hq; args.group = Hq / Hkv; args.N = N; args.n_qtiles = n_qtiles;
   args.per_head = B * (Hq / Hkv); args.Hkv = Hkv;
   args.scale_log2_signed = mfma_softmax_scale(sm_scale);
@@ -808,14 +810,11 @@ static int check_strides(const char* name, const int64_t* s, const void* p) {
 
 using namespace moa;
 
-
-
-
-extern "C" int moa_prefill_fwd(const void* q, const void* k, const void* v, void* o,
-                               const int64_t* q_strides, const int64_t* k_strides,
-                               const int64_t* v_strides, const int64_t* o_strides, int B, int Hq,
-                               int Hkv, int N, int D, const int64_t* sink_blocks,
-                               const int64_t* local_blocks, float sm_scale, int dtype, void* stream) {
+static int prefill_fwd(const void* q, const void* k, const void* v, void* o,
+                       const int64_t* q_strides, const int64_t* k_strides,
+                       const int64_t* v_strides, const int64_t* o_strides, int B, int Hq,
+                       int Hkv, int N, int D, const int64_t* sink_blocks,
+                       const int64_t* local_blocks, int span_shift, float sm_scale, int dtype, void* stream) {
   if (!q || !k || !v || !o || !sink_blocks || !local_blocks)
     return fail(MOA_ERR_ARG, "moa_prefill_fwd: null pointer");
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || N <= 0) return fail(MOA_ERR_ARG, "moa_prefill_fwd: B, H, N must be positive");
@@ -830,9 +829,25 @@ extern "C" int moa_prefill_fwd(const void* q, const void* k, const void* v, void
   if ((rc = check_strides("o", o_strides, o))) return rc;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MOA_DTYPE_F16) {
-    if (D == 128) return launch_prefill<PF16, 128>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, sm_scale, st);
-    return launch_prefill<PF16, 64>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, sm_scale, st);
+    if (D == 128) return launch_prefill<PF16, 128>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, span_shift, sm_scale, st);
+    return launch_prefill<PF16, 64>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, span_shift, sm_scale, st);
   }
-  if (D == 128) return launch_prefill<PBF16, 128>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, sm_scale, st);
-  return launch_prefill<PBF16, 64>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, sm_scale, st);
+  if (D == 128) return launch_prefill<PBF16, 128>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, span_shift, sm_scale, st);
+  return launch_prefill<PBF16, 64>(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, sink_blocks, local_blocks, span_shift, sm_scale, st);
+}
+
+extern "C" int moa_prefill_fwd(const void* q, const void* k, const void* v, void* o, const int64_t* q_strides,
+                               const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides, int B,
+                               int Hq, int Hkv, int N, int D, const int64_t* sink_blocks,
+                               const int64_t* local_blocks, float sm_scale, int dtype, void* stream) {
+  return prefill_fwd(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, D, sink_blocks, local_blocks, 0,
+                     sm_scale, dtype, stream);
+}
+
+extern "C" int moa_prefill_fwd_tokens(const void* q, const void* k, const void* v, void* o, const int64_t* q_strides,
+                                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
+                                      int B, int Hq, int Hkv, int N, int D, const int64_t* sink_size,
+                                      const int64_t* local_size, float sm_scale, int dtype, void* stream) {
+  return prefill_fwd(q, k, v, o, q_strides, k_strides, v_strides, o_strides, B, Hq, Hkv, N, D, sink_size, local_size,
+                     6 /* kKV = 64 tokens */, sm_scale, dtype, stream);
 }

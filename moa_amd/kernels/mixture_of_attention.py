@@ -64,6 +64,11 @@ def moa_prefill(
     ``[Hkv]`` block counts.  Returns ``[B, N, Hq, D]`` contiguous.  Argument
     meaning follows the call at MoA/kernels/mixture_of_attention.py:435-444.
     """
+    return _prefill(q, k, v, causal, num_global_blocks, num_band_blocks, kv_layout, sm_scale, False)
+
+
+def _prefill(q, k, v, causal, num_global_blocks, num_band_blocks, kv_layout, sm_scale, in_tokens: bool) -> Tensor:
+    """``moa_prefill``; ``in_tokens``: the spans are token counts, of which whole blocks count."""
     assert causal, "only causal attention is defined for MoA prefill"
     assert kv_layout == "HND", "k and v are expected as [B, H, N, D]"
     _require_gpu(q, "moa_prefill")
@@ -96,9 +101,9 @@ def moa_prefill(
     vs = _lib.i64_array(v.stride())
     os_ = _lib.i64_array([o.stride(0), o.stride(2), o.stride(1), o.stride(3)])
     lib = _lib.load()
-    rc = lib.moa_prefill_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), qs, ks, vs, os_,
-                             B, Hq, Hkv, N, D, sink.data_ptr(), local.data_ptr(), float(sm_scale),
-                             _lib.dtype_code(q.dtype), _lib.current_stream_ptr(dev))
+    fwd = lib.moa_prefill_fwd_tokens if in_tokens else lib.moa_prefill_fwd
+    rc = fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), qs, ks, vs, os_, B, Hq, Hkv, N, D, sink.data_ptr(),
+             local.data_ptr(), float(sm_scale), _lib.dtype_code(q.dtype), _lib.current_stream_ptr(dev))
     _lib.check(rc)
     return o
 
@@ -234,6 +239,9 @@ def mixture_of_sparse_attention(
             band_blocks = torch.ones(H, dtype=torch.int64, device=query.device)
         else:
             assert sink_size is not None and local_size is not None
+            if all(torch.is_tensor(t) and t.dtype == torch.int64 and t.device == query.device for t in (sink_size, local_size)):
+                # token counts go to the kernel as they are: no launches to divide them
+                return _prefill(query.transpose(1, 2), key, value, True, sink_size, local_size, "HND", sm_scale, True)
             sink_blocks = sink_size // BLOCK_N
             band_blocks = local_size // BLOCK_N
         # query arrives [B, H, N, D], usually a transposed view of [B, N, H, D]: pass the view

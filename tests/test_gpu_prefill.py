@@ -234,6 +234,24 @@ def test_more_heads_than_the_sorted_schedule_covers(dev):
     _close(out, ref, "520 heads")
 
 
+@pytest.mark.parametrize("H", [6, 520])   # heads sorted by span; more than that schedule covers
+def test_spans_in_tokens_equal_their_whole_blocks(dev, H):
+    """The wrapper hands token counts to the kernel: whole blocks of 64 count, rounded down as torch's ``//`` does."""
+    from moa_amd import mixture_of_sparse_attention
+    from moa_amd.kernels.mixture_of_attention import moa_prefill
+    N, D = 200, 64
+    g = torch.Generator().manual_seed(H)
+    q, k, v = (torch.randn(1, H, N, D, generator=g).to(dev, torch.float16) for _ in range(3))
+    pick = torch.tensor([-65, -1, 0, 63, 64, 65, 127, 128, 200, 1 << 40])
+    sink, local = (pick[torch.randint(0, len(pick), (H,), generator=g)].to(dev) for _ in range(2))
+    out = mixture_of_sparse_attention(q, k, v, 0.1, sink_size=sink, local_size=local)
+    want = moa_prefill(q.transpose(1, 2), k, v, num_global_blocks=sink // 64, num_band_blocks=local // 64, sm_scale=0.1)
+    assert torch.equal(out, want)
+    # other integer types are divided by torch, as before
+    out = mixture_of_sparse_attention(q, k, v, 0.1, sink_size=sink.clamp(max=999).int(), local_size=local.clamp(max=999).int())
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_peaked_and_drifting_scores(dev, dtype):
     """Scores in the hundreds (one-hot-like softmax) and a row maximum that keeps growing along the
