@@ -17,7 +17,7 @@
 //     hands work-groups to the XCDs strictly round-robin, so with one
 //     work-group per item a CU that falls free waits until it is its XCD's turn
 //     (measured: 7 % of CU time at the benchmark shape);
-//   * thread 0 turns a queue ticket into an item descriptor (base pointers, tile
+//   * wave 0 turns a queue ticket into an item descriptor (base pointers, tile
 //     schedule) once and leaves it in LDS; it does so for item i+1 a few
 //     iterations before item i ends, and item i's last iteration starts the
 //     first copies of item i+1;
@@ -90,7 +90,7 @@ struct PrefillArgs {
   Strides4 qs, ks, vs, os;
   const int64_t *sink_blocks, *local_blocks;   // spans per kv head: blocks, or tokens with span_shift = 6
   int span_shift;
-  PrefillQueue* queue;
+  PrefillQueue* queue;   // null: one item per work-group, by its place in the grid
   int BH, Hq, group, N, n_qtiles;
   int per_head, Hkv;   // (BH / Hq) * group pairs per kv head in the sorted list; Hq / group
   float scale_log2_signed;
@@ -98,7 +98,7 @@ struct PrefillArgs {
 typedef const PrefillArgs __attribute__((address_space(4)))* PrefillArgsPtr;
 
 // x / d and x % d for 0 <= x < 2^22, 0 < d < 2^22, through the float reciprocal and one correction step
-// each way (the compiler's general 32-bit division is four times as many instructions, and thread 0 does
+// each way (the compiler's general 32-bit division is four times as many instructions, and wave 0 does
 // a dozen of these per work item on the critical path).
 struct DivMod {
   int q, r;
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     const int64_t* sink_blocks = a0->sink_blocks;
     const int64_t* local_blocks = a0->local_blocks;
     const int shift = a0->span_shift;
-    if (Hkv <= kMaxSortedHeads) {
+    if (Hkv <= kMaxSortedHeads && a0->queue != nullptr) {
       for (int h = tid; h < Hkv; h += kPfThreads) {
         s_ns[h] = (int)max((int64_t)0, min((int64_t)nb, sink_blocks[h] >> shift));
         s_nl[h] = (int)max((int64_t)0, min((int64_t)nb, local_blocks[h] >> shift));
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   uint32_t q_touch = 0;              // landing place of the load that pulls the next item's Q rows into L2
 
   // ---- the work queue ---------------------------------------------------------------------------
-  // Thread 0 takes a ticket for the item after the one under way (from the own XCD's list while that has
+  // Wave 0 takes a ticket for the item after the one under way (from the own XCD's list while that has
   // items, from the other lists then), turns it into an item descriptor once and leaves it in LDS; every wave
   // reads it from there.  The ticket is taken kTakeLead iterations before the item under way ends, not at its
   // start: a ticket held through a long item starts late, behind tickets handed out after it, and the items
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   //   [8,9] K base  [10,11] V base  [12,13] Q base (row 0 of the head)  [14,15] O base
   const int my_xcd = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 7;   // XCC_ID
   __shared__ __attribute__((aligned(16))) int s_item[2][16];
-  bool own_alive = true;     // thread 0: the own list still had items when last asked
+  bool own_alive = true;     // wave 0: the own list still had items when last asked
   auto take = [&](int slot) __attribute__((always_inline)) {
     PrefillArgsPtr ap = a0;
     asm volatile("" : "+s"(ap));
@@ -192,21 +192,44 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     };
     int list = -1;
     unsigned sq = 0;
-    if (own_alive) {
-      sq = atomicAdd(&ap->queue->next[my_xcd], 1u);
-      if (sq < list_items(my_xcd)) list = my_xcd; else own_alive = false;
-    }
-    if (list < 0) {
-      for (int a = 1; a < 8; ++a) {
-        const int x = (my_xcd + a) & 7;
-        sq = atomicAdd(&ap->queue->next[x], 1u);
-        if (sq < list_items(x)) { list = x; break; }
+    const int lane = threadIdx.x & 63;
+    int* d = s_item[slot];
+    if (ap->queue == nullptr) {   // an item to every work-group: its number is its place, and there is no second one
+      if (own_alive) {
+        list = blockIdx.x & 7;
+        sq = blockIdx.x >> 3;
+        own_alive = false;
+      }
+    } else {
+      // lane 8 asks for a ticket of the own list, lanes 0 to 7 how far the lists are handed out: one round trip to
+      // memory, also where there is nothing left (asking the lists one after the other is eight of them, in which
+      // the whole work-group stands still at the end of its last item)
+      unsigned got = 0;
+      if (lane < 8) got = atomicAdd(&ap->queue->next[lane], 0u);
+      if (lane == 8 && own_alive) got = atomicAdd(&ap->queue->next[my_xcd], 1u);
+      const unsigned long long left = __ballot(lane < 8 && got < list_items(lane & 7)) & ~(1ull << my_xcd);
+      const unsigned mine = (unsigned)__builtin_amdgcn_readlane((int)got, 8);
+      if (own_alive && mine < list_items(my_xcd)) {
+        list = my_xcd;
+        sq = mine;
+      } else {
+        own_alive = false;
+        for (int i = 1; i < 8; ++i) {
+          const int x = (my_xcd + i) & 7;
+          if (!((left >> x) & 1)) continue;
+          unsigned t = 0;
+          if (lane == 0) t = atomicAdd(&ap->queue->next[x], 1u);
+          t = (unsigned)__builtin_amdgcn_readfirstlane((int)t);
+          if (t < list_items(x)) { list = x; sq = t; break; }
+        }
       }
     }
-    int* d = s_item[slot];
-    if (list < 0) { d[0] = -1; return; }
+    if (list < 0) {
+      if (lane == 0) d[0] = -1;
+      return;
+    }
     const int nb = (N + kKV - 1) / kKV;
-    const bool sorted = Hkv <= kMaxSortedHeads;
+    const bool sorted = Hkv <= kMaxSortedHeads && ap->queue != nullptr;
     // A list walks its pairs one after the other, late (long) query tiles first.
     const DivMod rq = divmod_small((int)sq, n_qtiles);
     const int round = rq.q;
@@ -239,6 +262,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
       band_rot = n_band - divmod_small(lo2, n_band).r;   // in [1, n_band]
       if (band_rot == n_band) band_rot = 0;
     }
+    if (lane != 0) return;
     d[0] = n_tiles; d[1] = qt; d[2] = ns; d[3] = nl; d[4] = lo2; d[5] = n_sink; d[6] = n_band; d[7] = band_rot;
     const uint64_t kb = (uint64_t)(ap->k + b * ap->ks.b + hk * ap->ks.h);
     const uint64_t vb = (uint64_t)(ap->v + b * ap->vs.b + hk * ap->vs.h);
@@ -248,8 +272,14 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     d[12] = (int)(uint32_t)qb; d[13] = (int)(uint32_t)(qb >> 32); d[14] = (int)(uint32_t)ob; d[15] = (int)(uint32_t)(ob >> 32);
   };
   __syncthreads();   // the sorted heads
-  if (threadIdx.x == 0) take(0);
+  if (threadIdx.x < 64) take(0);
   __syncthreads();
+
+  // Thread 0 counts its work-group out once it has found the lists empty (it takes no ticket after that).
+  unsigned left_before = ~0u;   // work-groups that were out already; ~0: not counted out yet
+  auto sign_off = [&]() __attribute__((always_inline)) {
+    if (threadIdx.x == 0 && a0->queue != nullptr && left_before == ~0u) left_before = atomicAdd(&a0->queue->done, 1u);
+  };
 
   // An item as the waves see it.
   struct Item {
@@ -383,6 +413,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   // The touched word lands in q_touch, which is kept allocated until the next pass has waited for it.
   auto prefetch_next = [&](uint32_t r0) __attribute__((always_inline)) {
     const Item ni = read_item(par ^ 1);
+    if (ni.n_tiles < 0) sign_off();   // the count comes back while the last item is finished
     if (ni.n_tiles <= 0) return false;
     start_copies(ni, r0);
     const int64_t m_row = min((int64_t)ni.qt * kQRows + wave * kWRows + mcol, (int64_t)N - 1);
@@ -411,23 +442,23 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   int kd_prev = (rst == 0) ? -(kStages - 1) * TILE_B : TILE_B;   // how far the K read addresses moved in the previous step
 
   if (n_tiles == 0) {   // nothing is visible from this query tile: zeros (nobody prefetches for such an item)
-    if (threadIdx.x == 0) take(par ^ 1);
+    if (wave == 0) take(par ^ 1);
     if (wave_has_rows && m_glob < N) {
       uint16_t* orow = it.obase + m_glob * os_n;
       u32x2 z = {0, 0};
 #pragma unroll
       for (int i = 0; i < D / 8; ++i) *reinterpret_cast<u32x2*>(orow + 8 * i + 4 * g) = z;
     }
-    __syncthreads();   // the next descriptor, written by thread 0 above
+    __syncthreads();   // the next descriptor, written by wave 0 above
     prefetched = false;
     continue;
   }
   if (!prefetched) start_copies(it, rst);
-  // the item after this one: thread 0 works its descriptor out kTakeLead iterations before this item's last
+  // the item after this one: wave 0 works its descriptor out kTakeLead iterations before this item's last
   // one (every wave sees it after the next barrier), or here when the item is that short
   constexpr int kTakeLead = 6;
   const int t_take = n_tiles - kTakeLead;
-  if (threadIdx.x == 0 && t_take < 1) take(par ^ 1);
+  if (wave == 0 && t_take < 1) take(par ^ 1);
 
   int jt[S];   // tiles of steps t .. t+S-1
   jt[0] = first_tile(it);
@@ -650,7 +681,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   {
     int t = 1;
     for (; t < t_take; ++t) iteration(t, IC<0>{});
-    if (threadIdx.x == 0 && t_take >= 1) take(par ^ 1);
+    if (wave == 0 && t_take >= 1) take(par ^ 1);
     for (; t < n_tiles; ++t) iteration(t, IC<0>{});
   }
 
@@ -713,13 +744,11 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   }
   }   // item loop
   // the last work-group to leave clears the queue for the next launch that uses this slot
-  if (threadIdx.x == 0) {
+  sign_off();
+  if (threadIdx.x == 0 && a0->queue != nullptr && left_before == gridDim.x - 1) {
     PrefillQueue* queue = a0->queue;
-    const unsigned d = atomicAdd(&queue->done, 1u);
-    if (d == gridDim.x - 1) {
-      for (int x = 0; x < 8; ++x) atomicExch(&queue->next[x], 0u);
-      atomicExch(&queue->done, 0u);
-    }
+    for (int x = 0; x < 8; ++x) atomicExch(&queue->next[x], 0u);
+    atomicExch(&queue->done, 0u);
   }
 }
 
@@ -784,6 +813,9 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* o, 
   int cus = 0;
   if (int rc = prefill_queue(&queue, &cus)) return rc;
   const int64_t groups = items < cus ? items : cus;
+  // No queue where every work-group has one item and the eight lists are equally long: place i is item i / 8 of list
+  // i % 8, the XCD the dispatcher hands work-group i to.
+  if (items <= cus && pairs % 8 == 0) queue = nullptr;
   PrefillArgs args;
   args.q = (const uint16_t*)q; args.k = (const uint16_t*)k; args.v = (const uint16_t*)v; args.o = (uint16_t*)o;
   args.qs = sq; args.ks = sk; args.vs = sv; args.os = so;
