@@ -17,7 +17,7 @@
 //   * segments differ in length by ~80x between heads, so the unit of work is
 //     a fixed-size chunk of rows, not a head: block (x, b) walks the chunks
 //     x, x+gridDim.x, ... of batch row b, locating (head, chunk) through a
-//     prefix sum over the row's heads that it rebuilds in LDS from
+//     prefix sum over the row's heads that every wave forms from
 //     head_valid_len (no host knowledge of the lengths, no host sync);
 //   * a head with one chunk writes its output directly; otherwise chunks
 //     write fp32 partial (acc, max, sum) triples and a small second kernel
@@ -95,147 +95,133 @@ struct DecInt {
   static constexpr int value = N;
 };
 
+typedef const uint16_t __attribute__((address_space(1))) * GlobalPtr;
 // Sixteen bytes of a cache row, which a step reads once.  NT marks the load non-temporal: it leaves no line
 // behind in the caches, which a launch that reads more than they hold only pays for (see kNtBytes).
 template <bool NT>
-__device__ __forceinline__ u32x4 load_once16(const uint16_t* p) {
-  const u32x4* s = reinterpret_cast<const u32x4*>(p);
+__device__ __forceinline__ u32x4 load_once16(GlobalPtr p) {
+  typedef const u32x4 __attribute__((address_space(1))) * Global16;
+  const Global16 s = (Global16)p;
   if constexpr (NT) return __builtin_nontemporal_load(s);
   else return *s;
 }
 
-// Chunk table of one batch row: prefix[h] = number of chunks of heads < h, and every head's segment
-// (first row, length) clamped into the row, so that a bad index cannot fault and a work-group finds a
-// chunk's segment in LDS instead of behind another memory latency.
-// Built by all threads of the block (one thread per head: kDecThreads >= kMaxHeads): a shuffle
-// scan inside each wave, then the wave totals through LDS.  Returns the row's total chunk count.
-// Every entry is clamped to `cap`, the partial slots a batch row owns: with disjoint segments the clamp
-// never acts; with overlapping ones (lengths that sum to more than the row holds) the chunks past the cap
-// do not exist for any kernel that builds the table, so none of them is written, read or merged.
-struct HeadTable {
-  int prefix[kMaxHeads + 1];
-  int seg0[kMaxHeads];   // first cache row of the head's segment (rows per batch row fit 31 bits: checked on the host)
-  int len[kMaxHeads];    // valid rows, clamped to the end of the batch row
-  int clen[kMaxHeads];   // rows per chunk of this head
-};
-
-template <int CHUNK, int NWAVES = kDecWaves>
-__device__ __forceinline__ int build_prefix(const int64_t* __restrict__ valid_row, const int64_t* __restrict__ start_row,
-                                            int H, int64_t sumC, int cap, HeadTable* __restrict__ tab) {
-  __shared__ int s_wave_total[NWAVES];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  int n = 0;
-  if (tid < H) {
-    int64_t len = valid_row[tid];
-    const int64_t seg0 = start_row[tid];
-    if (len < 0 || seg0 < 0 || seg0 >= sumC) len = 0;
-    if (len > sumC - seg0) len = sumC - seg0;
-    tab->seg0[tid] = (int)(len > 0 ? seg0 : 0);
-    tab->len[tid] = (int)len;
-    tab->clen[tid] = CHUNK;
-    n = (int)((len + CHUNK - 1) / CHUNK);
-  }
-  int incl = n;   // inclusive scan inside the wave
+// Inclusive sum over the lanes of a wave, in six DPP steps (no LDS); lane 63 has the total.
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 inside rows of 16 lanes
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return x;
+}
+__device__ __forceinline__ int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
+__device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int up = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += up;
-  }
-  if (lane == 63) s_wave_total[wave] = incl;
-  __syncthreads();
-  int base = 0;
-#pragma unroll
-  for (int w = 0; w < NWAVES; ++w) base += (w < wave) ? s_wave_total[w] : 0;
-  if (tid < kMaxHeads) tab->prefix[tid + 1] = min(base + incl, cap);
-  if (tid == 0) tab->prefix[0] = 0;
-  __syncthreads();
-  return tab->prefix[H];
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+  return x;
 }
 
-// Largest h with prefix[h] <= w  (w < prefix[H]).
-__device__ __forceinline__ int find_head(const int* __restrict__ s_prefix, int H, int w) {
-  int lo = 0, hi = H;  // invariant: prefix[lo] <= w < prefix[hi]
-  while (hi - lo > 1) {
-    int mid = (lo + hi) >> 1;
-    if (s_prefix[mid] <= w) lo = mid; else hi = mid;
-  }
-  return lo;
-}
-
-// The same table with chunks of about equal length over the whole batch row instead of a fixed chunk
-// length.  With a fixed length the last chunk of every head is a remainder and the number of chunks is
-// whatever it comes to; here the caller names the number of chunks (`target`) a batch row should not
-// exceed, and the table takes the shortest chunk length c (whole steps of kEvenStep rows, at least
-// kEvenMinChunk) for which sum_h ceil(len_h / c) <= target; head h is then split evenly into
-// ceil(len_h / c) chunks.  The search starts at total / target and goes up step by step (the sum exceeds
-// the target by at most the number of heads at the start, so a few steps do), and gives up after
-// kEvenTries: the table is valid for any c, the target is a wish.  Integer arithmetic only: the split
-// and the merge kernel build this table independently and must agree on every entry.
+// The chunks of one batch row, worked out by every wave for itself: lane i holds heads i, i + 64, ... and no LDS, no
+// barrier and one memory latency stand between the launch and the first cache row (a table in LDS built by the whole
+// work-group cost 1 us of a launch).  Chunks are numbered head by head; chunk numbers are clamped to `cap`, the
+// partial slots a batch row owns: with disjoint segments the clamp never acts; with overlapping ones (lengths that sum
+// to more than the row holds) the chunks past the cap do not exist for any kernel, so none of them is written, read
+// or merged.  Segments are clamped into the row, so that a bad index cannot fault.
+//
+// Two policies.  Fixed: chunks of CHUNK rows.  Even (even_target > 0, only with EVEN): with a fixed length the last
+// chunk of every head is a remainder and the number of chunks is whatever it comes to; here the caller names the
+// number of chunks a batch row should not exceed, and the row takes the shortest chunk length c (whole steps of
+// kEvenStep rows, at least kEvenMinChunk) for which sum_h ceil(len_h / c) <= target; head h is then split evenly into
+// ceil(len_h / c) chunks.  The search starts at total / target and goes up step by step (the sum exceeds the target by
+// at most the number of heads at the start, so a few steps do), and gives up after kEvenTries: the result is valid for
+// any c, the target is a wish.  Integer arithmetic only: the split and the merge kernel must agree on every entry.
 constexpr int kEvenMinChunk = 256;   // also the chunk length the partial slots of a batch row are sized for
 constexpr int kEvenStep = 128;
 constexpr int kEvenTries = 24;
-template <int NWAVES>
-__device__ __forceinline__ int build_prefix_even(const int64_t* __restrict__ valid_row, const int64_t* __restrict__ start_row,
-                                                 int H, int64_t sumC, int cap, int target, HeadTable* __restrict__ tab) {
-  __shared__ int s_wave_total[NWAVES];
-  __shared__ int s_wave_sum[2][NWAVES];
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  int len = 0;
-  if (tid < H) {
-    int64_t l = valid_row[tid];
-    const int64_t seg0 = start_row[tid];
-    if (l < 0 || seg0 < 0 || seg0 >= sumC) l = 0;
-    if (l > sumC - seg0) l = sumC - seg0;
-    tab->seg0[tid] = (int)(l > 0 ? seg0 : 0);
-    tab->len[tid] = (int)l;
-    len = (int)l;
-  }
-  // sum over the work-group of a per-thread count (every thread gets the sum); `buf` alternates so that
-  // one barrier per call is enough
-  auto block_sum = [&](int x, int buf) {
+struct Chunk {
+  int head, index, count;   // its head, its place among the head's chunks, how many those are
+  int seg0, len, rows;      // first row and valid rows of the head's segment, rows per chunk of the head
+};
+template <int CHUNK, bool EVEN>
+struct RowChunks {
+  static constexpr int kGroups = kMaxHeads / 64;
+  int seg0[kGroups], len[kGroups], rows[kGroups], last[kGroups];   // last: chunks up to and including this head, clamped
+  int total;                                                       // chunks of the batch row, clamped
+
+  __device__ __forceinline__ RowChunks(const int64_t* __restrict__ valid_row, const int64_t* __restrict__ start_row,
+                                       int H, int64_t sumC, int cap, int even_target) {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-    if (lane == 0) s_wave_sum[buf][wave] = x;
-    __syncthreads();
-    int t = 0;
+    for (int k = 0; k < kGroups; ++k) {
+      seg0[k] = len[k] = 0;
+      const int i = k * 64 + lane;
+      if (i < H) {
+        int64_t l = valid_row[i];
+        const int64_t first = start_row[i];
+        if (l < 0 || first < 0 || first >= sumC) l = 0;
+        if (l > sumC - first) l = sumC - first;
+        seg0[k] = (int)(l > 0 ? first : 0);
+        len[k] = (int)l;
+      }
+    }
+    int c = CHUNK;
+    const bool even = EVEN && even_target > 0;
+    if (even) {
+      auto chunks = [&](int size) __attribute__((always_inline)) {
+        int n = 0;
 #pragma unroll
-    for (int w = 0; w < NWAVES; ++w) t += s_wave_sum[buf][w];
-    return t;
-  };
-  // rows of the batch row in steps (a sum of at most 256 heads of < 2^31 rows each fits 32 bits in steps)
-  const int total_steps = block_sum((len + kEvenStep - 1) / kEvenStep, 0);
-  int c = max(kEvenMinChunk, ((total_steps + target - 1) / max(target, 1)) * kEvenStep);
-  int n = 0;
-  for (int i = 0; i < kEvenTries; ++i) {
-    n = (len + c - 1) / c;
-    if (block_sum(n, (i + 1) & 1) <= target) break;   // the same for every thread
-    c += kEvenStep;
-    n = (len + c - 1) / c;   // what the table holds if this was the last try
-  }
-  int clen = kEvenStep;
-  if (n > 0) {
-    clen = (((len + n - 1) / n + kEvenStep - 1) / kEvenStep) * kEvenStep;   // even split, <= c
-    n = (len + clen - 1) / clen;
-  }
-  if (tid < kMaxHeads) tab->clen[tid] = clen;
-  int incl = n;   // inclusive scan inside the wave
+        for (int k = 0; k < kGroups; ++k)
+          if (k * 64 < H) n += (len[k] + size - 1) / size;
+        return wave_sum(n);
+      };
+      // rows in steps (a sum of at most 256 heads of < 2^31 rows each fits 32 bits in steps)
+      c = max(kEvenMinChunk, ((chunks(kEvenStep) + even_target - 1) / even_target) * kEvenStep);
+      for (int t = 0; t < kEvenTries && chunks(c) > even_target; ++t) c += kEvenStep;
+    }
+    int base = 0;
 #pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int up = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += up;
+    for (int k = 0; k < kGroups; ++k) {
+      rows[k] = c;
+      last[k] = base;
+      if (k * 64 < H) {
+        int n = (len[k] + c - 1) / c;
+        if (even && n > 0) {
+          rows[k] = (((len[k] + n - 1) / n + kEvenStep - 1) / kEvenStep) * kEvenStep;   // even split, <= c
+          n = (len[k] + rows[k] - 1) / rows[k];
+        }
+        const int incl = wave_scan(n);
+        last[k] = min(base + incl, cap);
+        base += __builtin_amdgcn_readlane(incl, 63);
+      }
+    }
+    total = min(base, cap);
   }
-  if (lane == 63) s_wave_total[wave] = incl;
-  __syncthreads();
-  int base = 0;
+  // an entry of head h (h is uniform)
+  __device__ __forceinline__ int of(const int (&x)[kGroups], int h) const {
+    int r = 0;
 #pragma unroll
-  for (int w = 0; w < NWAVES; ++w) base += (w < wave) ? s_wave_total[w] : 0;
-  if (tid < kMaxHeads) tab->prefix[tid + 1] = min(base + incl, cap);
-  if (tid == 0) tab->prefix[0] = 0;
-  __syncthreads();
-  return tab->prefix[H];
-}
+    for (int k = 0; k < kGroups; ++k) {
+      const int in_group = __builtin_amdgcn_readlane(x[k], h & 63);
+      r = (h >> 6) == k ? in_group : r;
+    }
+    return r;
+  }
+  __device__ __forceinline__ int first_of(int h) const {
+    const int before = of(last, max(h - 1, 0));
+    return h > 0 ? before : 0;
+  }
+  // chunk w, 0 <= w < total (uniform)
+  __device__ __forceinline__ Chunk at(int w, int H) const {
+    int h = 0;   // heads that end before w
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k)
+      if (k * 64 < H) h += __popcll(__ballot(last[k] <= w && k * 64 + (int)(threadIdx.x & 63) < H));
+    const int first = first_of(h);
+    return {h, w - first, of(last, h) - first, of(seg0, h), of(len, h), of(rows, h)};
+  }
+};
 
 // H: kv heads (rings) per batch row; query head hk*G + g reads ring hk.
 // PIPE: the wave keeps two half-batches of loads going (the next one is issued before the current
@@ -255,8 +241,6 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   constexpr int WCHUNK = CHUNK / kDecWaves;
   static_assert(WCHUNK % ROWS == 0, "chunk must split evenly over waves and load batches");
 
-  __shared__ HeadTable s_tab;
-  const int* const s_prefix = s_tab.prefix;
   __shared__ float s_acc[kDecWaves][G][D];
   __shared__ float s_m[kDecWaves][G];
   __shared__ float s_l[kDecWaves][G];
@@ -268,28 +252,25 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   const int col = lane % LPR;   // which 8-element slice of the row
   const int sub = lane / LPR;   // which row of a wave-wide load
 
-  // Disjoint segments give at most `cap` chunks per row; the clamp inside keeps partial
-  // slots inside the workspace if a caller hands in overlapping segments.
-  const int total = build_prefix<CHUNK>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, &s_tab);
+  const RowChunks<CHUNK, false> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, 0);
 
-  for (int w = blockIdx.x; w < total; w += gridDim.x) {
-    const int h = find_head(s_prefix, H, w);
-    const int c = w - s_prefix[h];
-    const int n_chunks = s_prefix[h + 1] - s_prefix[h];
-    const int64_t bh = (int64_t)b * H + h;
-    const int64_t seg0 = s_tab.seg0[h];
-    const int64_t len = s_tab.len[h];
-    const int64_t r_begin = (int64_t)c * CHUNK + (int64_t)wave * WCHUNK;
-    int64_t r_end = r_begin + WCHUNK;
-    if (r_end > len) r_end = len;
+  for (int w = blockIdx.x; w < row.total; w += gridDim.x) {
+    const Chunk ck = row.at(w, H);
+    const int c = ck.index, n_chunks = ck.count;
+    const int64_t bh = (int64_t)b * H + ck.head;
+    const int r_begin = c * CHUNK + wave * WCHUNK;   // rows of a segment fit 31 bits
+    const int r_end = min(r_begin + WCHUNK, ck.len);
 
     // this lane's 8 query elements of each of the G query heads, kept packed for dot2
     u32x4 qv[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) qv[g] = *reinterpret_cast<const u32x4*>(q + (bh * G + g) * D + col * 8);
 
-    const uint16_t* kbase = kc + ((int64_t)b * sumC + seg0) * D + col * 8;
-    const uint16_t* vbase = vc + ((int64_t)b * sumC + seg0) * D + col * 8;
+    GlobalPtr kbase = (GlobalPtr)kc + ((int64_t)b * sumC + ck.seg0) * D + col * 8;
+    GlobalPtr vbase = (GlobalPtr)vc + ((int64_t)b * sumC + ck.seg0) * D + col * 8;
+    // Opaque from here on: loads the compiler can prove to read constant memory are moved next to their uses, across
+    // any barrier, to save registers, and go out one at a time.
+    asm volatile("" : "+v"(kbase), "+v"(vbase));
 
     float m[G], l[G];
     float acc[G][8];
@@ -302,19 +283,19 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
     }
 
     // n wave-wide loads of K and of V starting at row r0 of the wave's share
-    auto load_rows = [&](auto N, u32x4* kr, u32x4* vr, int64_t r0) __attribute__((always_inline)) {
+    auto load_rows = [&](auto N, u32x4* kr, u32x4* vr, int r0) __attribute__((always_inline)) {
       constexpr int n = decltype(N)::value;
 #pragma unroll
       for (int i = 0; i < n; ++i) {
-        const int64_t row = r0 + i * RPL + sub;
-        const bool ok = row < r_end;
-        const int64_t rr = ok ? row : r_begin;  // any valid row: keeps the load in bounds
+        const int row = r0 + i * RPL + sub;
+        const int64_t rr = row < r_end ? row : r_begin;  // any valid row: keeps the load in bounds
         kr[i] = load_once16<NT>(kbase + rr * D);
         vr[i] = load_once16<NT>(vbase + rr * D);
       }
+      __builtin_amdgcn_sched_barrier(0);   // all of them before what uses them
     };
     // online-softmax update with those rows
-    auto consume_rows = [&](auto N, const u32x4* kr, const u32x4* vr, int64_t r0) __attribute__((always_inline)) {
+    auto consume_rows = [&](auto N, const u32x4* kr, const u32x4* vr, int r0) __attribute__((always_inline)) {
       constexpr int n = decltype(N)::value;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -352,22 +333,23 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
       }
     };
     if (!PIPE) {
-      for (int64_t r0 = r_begin; r0 < r_end; r0 += ROWS) {
+      for (int r0 = r_begin; r0 < r_end; r0 += ROWS) {
         u32x4 kr[KB], vr[KB];
         load_rows(DecInt<KB>{}, kr, vr, r0);
         consume_rows(DecInt<KB>{}, kr, vr, r0);
       }
     } else {
+      // Every half-batch is asked for without a condition (past the end: the first row again, cached): behind a
+      // branch the compiler cannot count the loads in flight and waits for all of them in front of each use.
       constexpr int KH = KB / 2, HROWS = ROWS / 2;
       u32x4 ka[KH], va[KH], kb2[KH], vb2[KH];
-      if (r_begin < r_end) load_rows(DecInt<KH>{}, ka, va, r_begin);
-      for (int64_t r0 = r_begin; r0 < r_end; r0 += ROWS) {
-        const bool second = r0 + HROWS < r_end;
-        if (second) load_rows(DecInt<KH>{}, kb2, vb2, r0 + HROWS);
-        consume_rows(DecInt<KH>{}, ka, va, r0);
-        if (second) {
-          if (r0 + ROWS < r_end) load_rows(DecInt<KH>{}, ka, va, r0 + ROWS);
-          consume_rows(DecInt<KH>{}, kb2, vb2, r0 + HROWS);
+      if (r_begin < r_end) {
+        load_rows(DecInt<KH>{}, ka, va, r_begin);
+        for (int r0 = r_begin; r0 < r_end; r0 += ROWS) {
+          load_rows(DecInt<KH>{}, kb2, vb2, r0 + HROWS);
+          consume_rows(DecInt<KH>{}, ka, va, r0);
+          load_rows(DecInt<KH>{}, ka, va, r0 + ROWS);
+          if (r0 + HROWS < r_end) consume_rows(DecInt<KH>{}, kb2, vb2, r0 + HROWS);
         }
       }
     }
@@ -434,90 +416,18 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   }
 }
 
-__device__ __forceinline__ int wave_sum(int x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
-}
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
-}
-
-// One head's entries of the chunk table (build_prefix, or build_prefix_even when even_target > 0: the same
-// arithmetic), worked out by a single wave without LDS or barriers: the first chunk and the number of chunks.
-struct HeadChunks {
-  int first, count;
-};
-template <int CHUNK>
-__device__ __forceinline__ HeadChunks chunks_of_head(const int64_t* __restrict__ valid_row,
-                                                     const int64_t* __restrict__ start_row, int H, int64_t sumC,
-                                                     int cap, int even_target, int h) {
-  constexpr int kGroups = kMaxHeads / 64;
-  const int lane = threadIdx.x & 63;
-  int len[kGroups];
-#pragma unroll
-  for (int k = 0; k < kGroups; ++k) {
-    const int i = k * 64 + lane;
-    int64_t l = 0;
-    if (i < H) {
-      l = valid_row[i];
-      const int64_t seg0 = start_row[i];
-      if (l < 0 || seg0 < 0 || seg0 >= sumC) l = 0;
-      if (l > sumC - seg0) l = sumC - seg0;
-    }
-    len[k] = (int)l;
-  }
-  int c = CHUNK;
-  if (even_target > 0) {
-    int steps = 0;
-#pragma unroll
-    for (int k = 0; k < kGroups; ++k)
-      if (k * 64 < H) steps += (len[k] + kEvenStep - 1) / kEvenStep;
-    c = max(kEvenMinChunk, ((wave_sum(steps) + even_target - 1) / even_target) * kEvenStep);
-    for (int t = 0; t < kEvenTries; ++t) {
-      int n = 0;
-#pragma unroll
-      for (int k = 0; k < kGroups; ++k)
-        if (k * 64 < H) n += (len[k] + c - 1) / c;
-      if (wave_sum(n) <= even_target) break;
-      c += kEvenStep;
-    }
-  }
-  int before = 0, mine = 0;
-#pragma unroll
-  for (int k = 0; k < kGroups; ++k) {
-    if (k * 64 >= H) break;
-    int n = (len[k] + c - 1) / c;
-    if (even_target > 0 && n > 0) {
-      const int clen = (((len[k] + n - 1) / n + kEvenStep - 1) / kEvenStep) * kEvenStep;
-      n = (len[k] + clen - 1) / clen;
-    }
-    const int i = k * 64 + lane;
-    before += (i < h) ? n : 0;
-    mine += (i == h) ? n : 0;
-  }
-  before = wave_sum(before);
-  mine = wave_sum(mine);
-  HeadChunks r;
-  r.first = min(before, cap);
-  r.count = min(before + mine, cap) - r.first;
-  return r;
-}
-
 // Merge of the per-chunk partials of heads with more than one chunk, and the zero output of empty heads.
 // Latency is all there is to it (a few MB at most): one work-group per query head, each of its waves finds the
 // head's chunks by itself (one memory latency), then asks for the (max, sum) pairs of all chunks, a lane each,
 // and for its share of the accumulators, every fourth chunk, before it looks at any of them (a second one);
-// the waves meet once, in LDS, for the final sum.  Against a table in LDS built by the whole work-group and the loads
-// behind it: four layers at batch 1 of 16k tokens 112.0 -> 108.9 us a pass, batch 4 grouped 185.0 -> 180.5 us.
+// the waves meet once, in LDS, for the final sum.  Against two heads to a work-group, a table of the row in LDS and the
+// loads behind it: four layers at batch 1 of 16k tokens 112.0 -> 108.9 us a pass, batch 4 grouped 185.0 -> 180.5 us.
 template <typename T, int D, int CHUNK>
 __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
     uint16_t* __restrict__ o, const float* __restrict__ part_acc, const float* __restrict__ part_ml,
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
     int G /* query heads per ring */, int64_t sumC, int cap,
-    int even_target /* > 0: the split kernel used build_prefix_even with this target */) {
+    int even_target /* of the split kernel's chunks */) {
   constexpr int VEC = D / 64;      // columns per lane
   constexpr int kFirst = 8;        // chunks per wave asked for at once (32 of the head; more are rare)
   constexpr int kMore = 4;
@@ -527,24 +437,23 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
   const int h = hq / G, g = hq % G;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const HeadChunks hc = chunks_of_head<CHUNK>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap,
-                                              even_target, h);
-  const int n = __builtin_amdgcn_readfirstlane(hc.count);
+  const RowChunks<CHUNK, true> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, even_target);
+  const int w0 = row.first_of(h), n = row.of(row.last, h) - w0;
   if (n == 1) return;   // written by the split kernel
   uint16_t* const out = o + ((int64_t)b * H * G + hq) * D;
   if (n == 0) {
     if (tid < D) out[tid] = 0;
     return;
   }
-  const int64_t slot0 = ((int64_t)b * cap + __builtin_amdgcn_readfirstlane(hc.first)) * G + g;
-  const float* const acc = part_acc + slot0 * D + lane * VEC;
+  const int64_t slot0 = ((int64_t)b * cap + w0) * G + g;
+  const float* const acc = part_acc + slot0 * D;   // uniform
   const f32x2* const ml = reinterpret_cast<const f32x2*>(part_ml) + slot0;
-  const int64_t step = (int64_t)G * D;   // from a chunk's accumulator to the next one's
+  const int step = G * D;   // from a chunk's accumulator to the next one's
 
-  fvec x[kFirst];
+  fvec x[kFirst];   // a chunk past the head's last repeats that one: no branch stands between the loads
 #pragma unroll
   for (int j = 0; j < kFirst; ++j)
-    if (wave + kDecWaves * j < n) x[j] = *reinterpret_cast<const fvec*>(acc + (wave + kDecWaves * j) * step);
+    x[j] = *reinterpret_cast<const fvec*>(acc + min(wave + kDecWaves * j, n - 1) * step + lane * VEC);
   f32x2 mine = {-INFINITY, 0.f};   // chunk `lane`
   if (lane < n) mine = ml[(int64_t)lane * G];
   float M = mine.x;
@@ -575,7 +484,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
       fvec y[kMore];
 #pragma unroll
       for (int j = 0; j < kMore; ++j)
-        if (i + kDecWaves * j < end) y[j] = *reinterpret_cast<const fvec*>(acc + (int64_t)(i0 + i + kDecWaves * j) * step);
+        y[j] = *reinterpret_cast<const fvec*>(acc + (int64_t)(i0 + min(i + kDecWaves * j, end - 1)) * step + lane * VEC);
 #pragma unroll
       for (int j = 0; j < kMore; ++j)
         if (i + kDecWaves * j < end) a += y[j] * factor(i + kDecWaves * j);
@@ -608,7 +517,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
 // batch 64 of the 70B shape against 612-628 us with 2-16 per CU, each walking several chunks in a fixed order.
 constexpr int kGqaBlocksPerCu = 64;
 // Largest number of cache rows per work-group step (a quarter per wave) the launch aims for; the actual
-// chunk lengths come out of an even split of every batch row (build_prefix_even).  A chunk start costs a
+// chunk lengths come out of an even split of every batch row (RowChunks).  A chunk start costs a
 // wave full memory latencies with nothing in flight, so long chunks win: with one fixed length, 2048 was
 // the best of 512..4096 at batch 64 and at batch 4.
 constexpr int kGqaChunk = 2048;
@@ -631,7 +540,7 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     uint16_t* __restrict__ o, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
     int G /* query heads per ring, <= kGqaMaxG */, int64_t sumC, float scale_log2_signed, int cap,
-    int target /* > 0: chunks a batch row is split into (build_prefix_even); 0: chunks of kGqaChunk rows */) {
+    int target /* > 0: chunks a batch row is split into (RowChunks); 0: chunks of kGqaChunk rows */) {
   typedef typename MfmaElem<T>::type M;
   // the row maximum is taken over unscaled scores: a negative softmax scale goes into Q (sign flip, exact)
   const float scale_log2 = __builtin_fabsf(scale_log2_signed);
@@ -648,8 +557,6 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
   static_assert((kEvenStep / kGqaWaves) % kGqaTile == 0, "a wave's share of a chunk is whole tiles");
 
   extern __shared__ __attribute__((aligned(1024))) char s_mem[];
-  __shared__ HeadTable s_tab;
-  const int* const s_prefix = s_tab.prefix;
   // the per-wave results (m, l, O[d] per query head) go into the first 4.5 KiB of the wave's own ring
   // once its loop is over
   __shared__ float s_m[kGqaWaves][kGqaMaxG];
@@ -689,18 +596,15 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     for (int dt = 0; dt < DT; ++dt) v_ad[dt] = ring0 + TILE_B + (v_rd ^ (uint32_t)(64 * dt));
   }
 
-  const int total = target > 0
-      ? build_prefix_even<kGqaWaves>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, target, &s_tab)
-      : build_prefix<kGqaChunk, kGqaWaves>(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, &s_tab);
+  const RowChunks<kGqaChunk, true> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, target);
 
-  for (int w = blockIdx.x; w < total; w += gridDim.x) {
-    const int h = find_head(s_prefix, H, w);
-    const int c = w - s_prefix[h];
-    const int n_chunks = s_prefix[h + 1] - s_prefix[h];
-    const int64_t bh = (int64_t)b * H + h;
-    const int64_t seg0 = s_tab.seg0[h];
-    const int64_t len = s_tab.len[h];
-    const int clen = s_tab.clen[h];            // rows of one chunk of this head
+  for (int w = blockIdx.x; w < row.total; w += gridDim.x) {
+    const Chunk ck = row.at(w, H);
+    const int c = ck.index, n_chunks = ck.count;
+    const int64_t bh = (int64_t)b * H + ck.head;
+    const int64_t seg0 = ck.seg0;
+    const int64_t len = ck.len;
+    const int clen = ck.rows;                  // rows of one chunk of this head
     const int wchunk = clen / kGqaWaves;       // a wave's share: whole tiles
     const int64_t r_begin = (int64_t)c * clen + (int64_t)wave * wchunk;
     int64_t r_end = r_begin + wchunk;
