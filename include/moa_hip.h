@@ -129,6 +129,20 @@ int moa_decode_fwd(const void* q, const void* kc, const void* vc, void* o,
                    float sm_scale, int dtype, void* stream);
 
 /*
+ * moa_decode_fwd that may merge the split-K partials inside its one launch, where few
+ * chunks make that the faster way.  counters: uint32 [n_counters] in device memory, all
+ * zero before the first call and left at zero by every call; used when n_counters >=
+ * B * Hkv and else ignored, like NULL (the call is then moa_decode_fwd).  Calls that may
+ * overlap on a GPU need counters, like workspaces, of their own.
+ */
+int moa_decode_fwd_counted(const void* q, const void* kc, const void* vc, void* o,
+                           void* workspace, size_t workspace_bytes,
+                           uint32_t* counters, size_t n_counters,
+                           const int64_t* head_start, const int64_t* head_valid_len,
+                           int B, int Hq, int Hkv, int D, int64_t sumC,
+                           float sm_scale, int dtype, void* stream);
+
+/*
  * moa_decode_fwd without a workspace argument, for callers that cannot allocate
  * device memory: code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc.  It has no counterpart in the reference.  Same

@@ -41,6 +41,9 @@ SIGNATURES = {
     "moa_decode_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int64]),
     "moa_decode_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p,
                                c_void_p, c_int, c_int, c_int, c_int, c_int64, c_float, c_int, c_void_p]),
+    "moa_decode_fwd_counted": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p,
+                                       c_size_t, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int64, c_float,
+                                       c_int, c_void_p]),
     "moa_decode_fwd_noalloc": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
                                        c_int, c_int, c_int64, c_float, c_int, c_void_p]),
     "moa_cache_append": (c_int, [c_void_p, c_void_p, _I64P, _I64P, c_void_p, c_void_p, c_void_p, c_void_p,

@@ -32,6 +32,7 @@
 #include <hip/hip_fp16.h>
 
 #include <mutex>
+#include <type_traits>
 
 namespace moa {
 
@@ -223,6 +224,131 @@ struct RowChunks {
   }
 };
 
+// What a wave knows of a head once it has gone through its share of the chunks: its VEC columns of the weighted sum
+// (of its share) and the sum of weights (of all chunks).
+template <int D>
+struct Merged {
+  static constexpr int VEC = D / 64;   // columns per lane
+  typedef float fvec __attribute__((ext_vector_type(VEC)));
+  fvec a;
+  float L;
+};
+// One wave's part of the merge of a head's n partials: chunks first, first + stride, ...  `acc` and `ml` are the head's
+// first partial (uniform), `G` partials lie between a chunk's and the next one's.  All of the wave's loads go out
+// before it looks at any of them.  COHERENT: the partials come from work-groups of this launch, on other XCDs perhaps:
+// device-scope loads.
+// A wave that takes every chunk (stride 1) sums them in kDecWaves strands, as kDecWaves waves with a stride of
+// kDecWaves and their final sum do: every way of merging gives the same bits.
+template <int D, bool COHERENT, int kFirst /* chunks asked for at once */, int kMore /* and in every round behind */,
+          bool STRANDS = false>
+__device__ __forceinline__ Merged<D> merge_wave(const float* acc, const f32x2* ml, int G, int n, int first, int stride) {
+  typedef typename Merged<D>::fvec fvec;
+  constexpr int VEC = Merged<D>::VEC;
+  static_assert(64 % kMore == 0 && kFirst % kMore == 0, "rounds do not straddle a block of 64 factors");
+  const int lane = threadIdx.x & 63;
+  const int step = G * D;          // from a chunk's accumulator to the next one's
+  auto load = [](const auto* p) __attribute__((always_inline)) {
+    typedef std::remove_cv_t<std::remove_reference_t<decltype(*p)>> V;
+    if constexpr (!COHERENT) {
+      return *p;
+    } else if constexpr (sizeof(V) == 8) {
+      return __builtin_bit_cast(V, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT));
+    } else {
+      return __builtin_bit_cast(V, __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT));
+    }
+  };
+  fvec x[kFirst];   // a chunk past the head's last repeats that one: no branch stands between the loads
+#pragma unroll
+  for (int j = 0; j < kFirst; ++j)
+    x[j] = load(reinterpret_cast<const fvec*>(acc + min(first + stride * j, n - 1) * step + lane * VEC));
+  f32x2 mine = {-INFINITY, 0.f};   // chunk `lane`
+  if (lane < n) mine = load(ml + (int64_t)lane * G);
+  float M = mine.x;
+  for (int i = 64 + lane; i < n; i += 64) M = fmaxf(M, load(ml + (int64_t)i * G).x);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
+  const float m_use = (M == -INFINITY) ? 0.f : M;
+  float f = fast_exp2(mine.x - m_use);   // the factor of chunk `lane`
+  float L = mine.y * f;
+  auto factor = [&](int i) __attribute__((always_inline)) {   // of the chunk at lane i (uniform)
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), i));
+  };
+  constexpr int kStrands = STRANDS ? kDecWaves : 1;
+  static_assert(kMore % kStrands == 0, "a round starts at strand 0");
+  fvec a[kStrands] = {};
+#pragma unroll
+  for (int j = 0; j < kFirst; ++j)
+    if (first + stride * j < n) a[j % kStrands] += x[j] * factor(first + stride * j);
+  int i = first + stride * kFirst;   // the rest; factors in blocks of 64 chunks
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    if (i0 > 0) {
+      f = 0.f;
+      if (i0 + lane < n) {
+        const f32x2 v = load(ml + (int64_t)(i0 + lane) * G);
+        f = fast_exp2(v.x - m_use);
+        L += v.y * f;
+      }
+    }
+    const int end = min(i0 + 64, n);
+    for (; i < end; i += kMore * stride) {
+      fvec y[kMore];
+#pragma unroll
+      for (int j = 0; j < kMore; ++j)
+        y[j] = load(reinterpret_cast<const fvec*>(acc + (int64_t)min(i + stride * j, end - 1) * step + lane * VEC));
+#pragma unroll
+      for (int j = 0; j < kMore; ++j)
+        if (i + stride * j < end) a[j % kStrands] += y[j] * factor(i + stride * j - i0);
+    }
+  }
+  Merged<D> r;
+  r.a = a[0];
+#pragma unroll
+  for (int k = 1; k < kStrands; ++k) r.a += a[k];
+  r.L = wave_sum(L);
+  return r;
+}
+
+// Launches of few chunks merge inside the split kernel: the work-group whose chunk is the head's last to arrive sums
+// the head's partials up, and the merge launch (4.5 us of a step's GPU time, as much again of the host's) falls away.
+// Partials are stored and read with device-scope accesses and the arrival is counted with a device-scope atomic, each
+// wave waiting for its stores before the count; no fence, which would write back and drop the XCD's whole L2.
+// `counters` holds one zero per (batch row, ring) and is left at zero.
+__device__ __forceinline__ void store_partial(float* p, float x, bool coherent) {
+  if (coherent) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = x;
+}
+// Called by the whole work-group behind its partials' stores; true for the last of the ring's n chunks to arrive.
+__device__ __forceinline__ bool arrived_last(unsigned* counter, int n) {
+  __shared__ unsigned s_before;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    s_before = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (s_before == (unsigned)n - 1) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  return s_before == (unsigned)n - 1;
+}
+// The zero output of a batch row's rings without a chunk (the merge kernel's in launches of two kernels).
+template <typename ROW>
+__device__ __forceinline__ void zero_empty_rings(const ROW& row, uint16_t* o_row, int H, int row_elems) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;   // chunks of the groups of heads so far
+#pragma unroll
+  for (int k = 0; k < ROW::kGroups; ++k) {
+    if (k * 64 >= H) break;
+    const int up = __shfl_up(row.last[k], 1, 64);
+    unsigned long long empty = __ballot(k * 64 + lane < H && row.last[k] == (lane > 0 ? up : before));
+    before = __builtin_amdgcn_readlane(row.last[k], 63);
+    for (; empty != 0; empty &= empty - 1) {
+      const int h = k * 64 + __builtin_ctzll(empty);
+      for (int i = threadIdx.x; i < row_elems; i += blockDim.x) o_row[(int64_t)h * row_elems + i] = 0;
+    }
+  }
+}
+
 // H: kv heads (rings) per batch row; query head hk*G + g reads ring hk.
 // PIPE: the wave keeps two half-batches of loads going (the next one is issued before the current
 // one is consumed) instead of loading a full batch, waiting for it and consuming it.  Measured at
@@ -233,7 +359,9 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
     uint16_t* __restrict__ o, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
-    int64_t sumC, float scale_log2, int cap /* partial slots per batch row */) {
+    int64_t sumC, float scale_log2, int cap /* partial slots per batch row */,
+    unsigned* __restrict__ counters /* one per (b, ring): merge here; null: decode_merge_kernel does */) {
+  constexpr bool MERGE = !PIPE;       // the launches that may merge inside (the code costs the others 1 %)
   constexpr int LPR = D / 8;          // lanes per row
   constexpr int RPL = 64 / LPR;       // rows per wave-wide load
   constexpr int KB = (G >= 8) ? kBatch / 2 : kBatch;   // loads in flight per tensor (registers bound it at G = 8)
@@ -248,11 +376,13 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   const int b = blockIdx.y;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane % LPR;   // which 8-element slice of the row
   const int sub = lane / LPR;   // which row of a wave-wide load
 
   const RowChunks<CHUNK, false> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, 0);
+
+  if (MERGE && counters && blockIdx.x == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
 
   for (int w = blockIdx.x; w < row.total; w += gridDim.x) {
     const Chunk ck = row.at(w, H);
@@ -404,12 +534,27 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
           o[(bh * G + g) * D + tid] = pack1<T>(out);
         } else {
           const int64_t slot = ((int64_t)b * cap + w) * G + g;
-          part_acc[slot * D + tid] = a;
+          store_partial(part_acc + slot * D + tid, a, MERGE && counters != nullptr);
           if (tid == 0) {
-            part_ml[slot * 2 + 0] = M;
-            part_ml[slot * 2 + 1] = L;
+            store_partial(part_ml + slot * 2 + 0, M, MERGE && counters != nullptr);
+            store_partial(part_ml + slot * 2 + 1, L, MERGE && counters != nullptr);
           }
         }
+      }
+    }
+    if (MERGE && counters && n_chunks > 1 && arrived_last(counters + bh, n_chunks)) {
+      float* const s_sum = &s_acc[0][0][0];   // [kDecWaves][D]
+      for (int g = 0; g < G; ++g) {
+        const int64_t slot0 = ((int64_t)b * cap + w - c) * G + g;
+        const Merged<D> m = merge_wave<D, true, 8, 4>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G,
+                                                n_chunks, wave, kDecWaves);
+        *reinterpret_cast<typename Merged<D>::fvec*>(s_sum + wave * D + lane * Merged<D>::VEC) = m.a;
+        __syncthreads();
+        if (tid < D) {
+          const float t = s_sum[tid] + s_sum[D + tid] + s_sum[2 * D + tid] + s_sum[3 * D + tid];
+          o[(bh * G + g) * D + tid] = pack1<T>((m.L > 0.f) ? t / m.L : 0.f);
+        }
+        __syncthreads();
       }
     }
     __syncthreads();  // s_acc / s_m / s_l are reused by the next chunk
@@ -428,10 +573,6 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
     int G /* query heads per ring */, int64_t sumC, int cap,
     int even_target /* of the split kernel's chunks */) {
-  constexpr int VEC = D / 64;      // columns per lane
-  constexpr int kFirst = 8;        // chunks per wave asked for at once (32 of the head; more are rare)
-  constexpr int kMore = 4;
-  typedef float fvec __attribute__((ext_vector_type(VEC)));
   __shared__ float s_a[kDecWaves][D];
   const int hq = blockIdx.x, b = blockIdx.y;
   const int h = hq / G, g = hq % G;
@@ -446,52 +587,10 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
     return;
   }
   const int64_t slot0 = ((int64_t)b * cap + w0) * G + g;
-  const float* const acc = part_acc + slot0 * D;   // uniform
-  const f32x2* const ml = reinterpret_cast<const f32x2*>(part_ml) + slot0;
-  const int step = G * D;   // from a chunk's accumulator to the next one's
-
-  fvec x[kFirst];   // a chunk past the head's last repeats that one: no branch stands between the loads
-#pragma unroll
-  for (int j = 0; j < kFirst; ++j)
-    x[j] = *reinterpret_cast<const fvec*>(acc + min(wave + kDecWaves * j, n - 1) * step + lane * VEC);
-  f32x2 mine = {-INFINITY, 0.f};   // chunk `lane`
-  if (lane < n) mine = ml[(int64_t)lane * G];
-  float M = mine.x;
-  for (int i = 64 + lane; i < n; i += 64) M = fmaxf(M, ml[(int64_t)i * G].x);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) M = fmaxf(M, __shfl_xor(M, off, 64));
-  const float m_use = (M == -INFINITY) ? 0.f : M;
-  float f = fast_exp2(mine.x - m_use);   // the factor of chunk `lane`
-  float L = mine.y * f;
-  auto factor = [&](int i) __attribute__((always_inline)) {   // of the chunk at lane i (uniform)
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), i));
-  };
-  fvec a = {};
-#pragma unroll
-  for (int j = 0; j < kFirst; ++j)
-    if (wave + kDecWaves * j < n) a += x[j] * factor(wave + kDecWaves * j);
-  for (int i0 = 0; i0 < n; i0 += 64) {
-    if (i0 > 0) {
-      f = 0.f;
-      if (i0 + lane < n) {
-        const f32x2 v = ml[(int64_t)(i0 + lane) * G];
-        f = fast_exp2(v.x - m_use);
-        L += v.y * f;
-      }
-    }
-    const int end = min(64, n - i0);
-    for (int i = (i0 == 0 ? kFirst * kDecWaves : 0) + wave; i < end; i += kMore * kDecWaves) {
-      fvec y[kMore];
-#pragma unroll
-      for (int j = 0; j < kMore; ++j)
-        y[j] = *reinterpret_cast<const fvec*>(acc + (int64_t)(i0 + min(i + kDecWaves * j, end - 1)) * step + lane * VEC);
-#pragma unroll
-      for (int j = 0; j < kMore; ++j)
-        if (i + kDecWaves * j < end) a += y[j] * factor(i + kDecWaves * j);
-    }
-  }
-  L = wave_sum(L);
-  *reinterpret_cast<fvec*>(&s_a[wave][lane * VEC]) = a;
+  const Merged<D> m = merge_wave<D, false, 8, 4>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G, n,
+                                           wave, kDecWaves);
+  const float L = m.L;
+  *reinterpret_cast<typename Merged<D>::fvec*>(&s_a[wave][lane * Merged<D>::VEC]) = m.a;
   __syncthreads();
   if (tid < D) {
     float t = s_a[0][tid];
@@ -540,11 +639,13 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     uint16_t* __restrict__ o, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
     int G /* query heads per ring, <= kGqaMaxG */, int64_t sumC, float scale_log2_signed, int cap,
-    int target /* > 0: chunks a batch row is split into (RowChunks); 0: chunks of kGqaChunk rows */) {
+    int target /* > 0: chunks a batch row is split into (RowChunks); 0: chunks of kGqaChunk rows */,
+    unsigned* __restrict__ counters /* as in decode_split_kernel */) {
   typedef typename MfmaElem<T>::type M;
   // the row maximum is taken over unscaled scores: a negative softmax scale goes into Q (sign flip, exact)
   const float scale_log2 = __builtin_fabsf(scale_log2_signed);
   const uint32_t q_sign = scale_log2_signed < 0.f ? 0x80008000u : 0u;
+  constexpr bool MERGE = !NT;                   // as in decode_split_kernel
   constexpr int KS = D / 16;                    // MFMA k-steps of Q.K^T
   constexpr int DT = D / 32;                    // 32-wide d tiles of the output
   constexpr int CPR = D / 8;                    // 16-byte chunks per cache row
@@ -597,6 +698,8 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
   }
 
   const RowChunks<kGqaChunk, true> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, target);
+
+  if (MERGE && counters && blockIdx.x == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
 
   for (int w = blockIdx.x; w < row.total; w += gridDim.x) {
     const Chunk ck = row.at(w, H);
@@ -756,12 +859,21 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
           o[(bh * G + gq) * D + tid] = pack1<T>((L > 0.f) ? a / L : 0.f);
         } else {
           const int64_t slot = ((int64_t)b * cap + w) * G + gq;
-          part_acc[slot * D + tid] = a;
+          store_partial(part_acc + slot * D + tid, a, MERGE && counters != nullptr);
           if (tid == 0) {
-            part_ml[slot * 2 + 0] = Mx;
-            part_ml[slot * 2 + 1] = L;
+            store_partial(part_ml + slot * 2 + 0, Mx, MERGE && counters != nullptr);
+            store_partial(part_ml + slot * 2 + 1, L, MERGE && counters != nullptr);
           }
         }
+      }
+    }
+    if (MERGE && counters && n_chunks > 1 && arrived_last(counters + bh, n_chunks)) {
+      for (int gq = wave; gq < G; gq += kGqaWaves) {   // a query head to a wave
+        const int64_t slot0 = ((int64_t)b * cap + w - c) * G + gq;
+        const Merged<D> m = merge_wave<D, true, 16, 16, true>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G,
+                                                n_chunks, 0, 1);
+#pragma unroll
+        for (int j = 0; j < D / 64; ++j) o[(bh * G + gq) * D + lane * (D / 64) + j] = pack1<T>((m.L > 0.f) ? m.a[j] / m.L : 0.f);
       }
     }
     __syncthreads();  // s_acc / s_m / s_l are reused by the next chunk
@@ -784,6 +896,17 @@ constexpr int kDecPipeFrom = 3;       // work-groups per CU from which the waves
 constexpr int64_t kNtBytes = (int64_t)64 << 20;
 static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_t)B * sumC * D * 4 >= kNtBytes; }
 
+// Which launches with counters merge inside the split kernel.  What is saved is a launch; what is added stands behind
+// every chunk, and where several chunks follow each other on a CU it is no longer hidden.  One query head per ring: the
+// launches that do not pipeline their loads (kDecPipeFrom).  GPU time with the merge launch and without, 32 rings of
+// 128: 256 rows 7.5 -> 5.9 us, 2048 rows 12.6 -> 11.6 us, batch 4 of 4096 rows (1152 chunks) 49.8 -> 49.6 us, batch 8
+// 90.0 -> 92.4 us; a step called from Python, bound by its launches, 24 -> 21 us.
+// Grouped kernel: only below kNtBytes, where a step called from Python waits for its launches (24 -> 21 us).  Above, the
+// GPU is behind, a chunk is alone on its CU and nothing hides the merge: batch 4 of 8 rings at 32k tokens, 8 query
+// heads, 43.9 us a layer with the merge launch, 46.2 us without.  The last work-group of a ring merges G query heads
+// alone, so their partials are bounded too: 32 chunks of 8 heads (256) 20.1 -> 22.0 us, 16 of 8 (128) 20.0 -> 20.6 us.
+constexpr int64_t kMergeInsidePartials = 128;
+
 constexpr int kSmallChunk = kChunk / 2;   // chunk length of the one-query-head kernel when the grid is small
 
 // partial slots per batch row: at most this many chunks exist when the rings do not overlap (sized
@@ -797,7 +920,7 @@ static inline size_t decode_slots(int B, int Hq, int Hkv, int64_t sumC) {
 template <typename T, int D, int G>
 static int launch_decode(const void* q, const void* kc, const void* vc, void* o, float* part_acc,
                          float* part_ml, const int64_t* head_start, const int64_t* head_valid, int B,
-                         int H, int64_t sumC, float sm_scale, hipStream_t st) {
+                         int H, int64_t sumC, float sm_scale, unsigned* counters, hipStream_t st) {
   const int cap = (int)decode_cap(sumC, H);
   const int64_t chunks = (sumC + kChunk - 1) / kChunk + H;   // per batch row, at the normal chunk length
   // 16 work-groups per CU over the whole grid (measured: 8 leaves a visible tail, 32 is no better),
@@ -811,12 +934,14 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
   auto launch = [&](auto split, auto merge) {
     hipLaunchKernelGGL(split, dim3(bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
                        (const uint16_t*)vc, (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, sumC,
-                       sm_scale * kLog2e, cap);
+                       sm_scale * kLog2e, cap, counters);
     if (int rc = check_launch("moa_decode_fwd(split)")) return rc;
+    if (counters) return MOA_OK;
     hipLaunchKernelGGL(merge, dim3(H * G, B), dim3(kDecThreads), 0, st, (uint16_t*)o, part_acc, part_ml, head_start,
                        head_valid, H, G, sumC, cap, 0);
     return check_launch("moa_decode_fwd(merge)");
   };
+  if (pipe && !small) counters = nullptr;
   const bool nt = read_nontemporal(B, sumC, D);
   if (small) {
     if (nt) return launch(&decode_split_kernel<T, D, kSmallChunk, G, false, true>, &decode_merge_kernel<T, D, kSmallChunk>);
@@ -833,7 +958,7 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
 template <typename T, int D>
 static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void* o, float* part_acc,
                              float* part_ml, const int64_t* head_start, const int64_t* head_valid, int B,
-                             int H, int G, int64_t sumC, float sm_scale, hipStream_t st) {
+                             int H, int G, int64_t sumC, float sm_scale, unsigned* counters, hipStream_t st) {
   const int cap = (int)decode_cap(sumC, H);   // partial slots per batch row the workspace was sized for
   // Chunk policy.  Chunks of kGqaChunk rows when they give at least half of the CUs a chunk: measured at
   // the 70B shape (8 rings per batch row, 104 k rows) with one fixed length, 49.8 us per call at batch 4
@@ -853,22 +978,25 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
   }
   // at most this many chunks per batch row (a work-group without a chunk still holds a CU while it finds that out)
   const int64_t chunks = target > 0 ? target + H : (sumC + kGqaChunk - 1) / kGqaChunk + H;
+  const int64_t chunk_rows = target > 0 ? (sumC / target > kEvenMinChunk ? sumC / target : kEvenMinChunk) : kGqaChunk;
+  const int64_t ring_chunks = (sumC / H + chunk_rows - 1) / chunk_rows;   // of a ring of average size
+  const bool nt = read_nontemporal(B, sumC, D);
+  if (nt || ring_chunks * G > kMergeInsidePartials) counters = nullptr;
   int64_t bx = (256 * kGqaBlocksPerCu + B - 1) / B;   // in practice one work-group per chunk (see kGqaBlocksPerCu)
   if (bx > chunks) bx = chunks;
   if (bx > cap) bx = cap;
   if (bx < 1) bx = 1;
   constexpr size_t lds = gqa_lds_bytes<D>();
   static bool lds_reserved[2][kMaxDevices] = {};   // per template instance
-  const bool nt = read_nontemporal(B, sumC, D);
   const auto kernel = nt ? &decode_gqa_kernel<T, D, true> : &decode_gqa_kernel<T, D, false>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kernel), lds, lds_reserved[nt], "moa_decode_fwd"))
     return rc;
   hipLaunchKernelGGL(kernel, dim3((unsigned)bx, B), dim3(kGqaThreads), lds, st,
                      (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (uint16_t*)o,
                      part_acc, part_ml, head_start, head_valid, H, G, sumC, mfma_softmax_scale(sm_scale), cap,
-                     (int)target);
+                     (int)target, counters);
   int rc = check_launch("moa_decode_fwd(grouped split)");
-  if (rc) return rc;
+  if (rc || counters) return rc;
   hipLaunchKernelGGL((decode_merge_kernel<T, D, kGqaChunk>), dim3(H * G, B), dim3(kDecThreads), 0, st,
                      (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, G, sumC, cap, (int)target);
   return check_launch("moa_decode_fwd(merge)");
@@ -879,14 +1007,14 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
 static int decode_dispatch(const void* q, const void* kc, const void* vc, void* o,
                            void* workspace, const int64_t* head_start, const int64_t* head_valid_len,
                            int B, int Hq, int Hkv, int D, int64_t sumC, float sm_scale, int dtype,
-                           void* stream) {
+                           unsigned* counters, void* stream) {
   const int G = Hq / Hkv;
   const size_t slots = decode_slots(B, Hq, Hkv, sumC);
   float* part_acc = reinterpret_cast<float*>(workspace);
   float* part_ml = part_acc + slots * (size_t)D;
   hipStream_t st = (hipStream_t)stream;
 #define MOA_DEC_ARGS q, kc, vc, o, part_acc, part_ml, head_start, head_valid_len, B, Hkv
-#define MOA_DEC_TAIL sumC, sm_scale, st
+#define MOA_DEC_TAIL sumC, sm_scale, counters, st
   // one query head per ring: vector ALU kernel; more: matrix-core kernel
   if (dtype == MOA_DTYPE_F16) {
     if (D == 128) return G == 1 ? launch_decode<F16, 128, 1>(MOA_DEC_ARGS, MOA_DEC_TAIL) : launch_decode_gqa<F16, 128>(MOA_DEC_ARGS, G, MOA_DEC_TAIL);
@@ -962,7 +1090,21 @@ extern "C" int moa_decode_fwd(const void* q, const void* kc, const void* vc, voi
   if (!workspace || workspace_bytes < need)
     return fail(MOA_ERR_WORKSPACE, "moa_decode_fwd: workspace %zu < %zu bytes", workspace_bytes, need);
   return decode_dispatch(q, kc, vc, o, workspace, head_start, head_valid_len, B, Hq, Hkv, D,
-                         sumC, sm_scale, dtype, stream);
+                         sumC, sm_scale, dtype, nullptr, stream);
+}
+
+extern "C" int moa_decode_fwd_counted(const void* q, const void* kc, const void* vc, void* o, void* workspace,
+                                      size_t workspace_bytes, uint32_t* counters, size_t n_counters,
+                                      const int64_t* head_start, const int64_t* head_valid_len, int B, int Hq, int Hkv,
+                                      int D, int64_t sumC, float sm_scale, int dtype, void* stream) {
+  if (int rc = decode_check_args("moa_decode_fwd_counted", q, kc, vc, o, head_start, head_valid_len, B, Hq, Hkv, D, sumC, dtype))
+    return rc;
+  const size_t need = moa_decode_workspace_bytes(B, Hq, Hkv, D, sumC);
+  if (!workspace || workspace_bytes < need)
+    return fail(MOA_ERR_WORKSPACE, "moa_decode_fwd_counted: workspace %zu < %zu bytes", workspace_bytes, need);
+  if (n_counters < (size_t)B * (size_t)Hkv) counters = nullptr;
+  return decode_dispatch(q, kc, vc, o, workspace, head_start, head_valid_len, B, Hq, Hkv, D, sumC, sm_scale, dtype, counters,
+                         stream);
 }
 
 extern "C" int moa_decode_fwd_noalloc(const void* q, const void* kc, const void* vc, void* o,
@@ -980,5 +1122,5 @@ extern "C" int moa_decode_fwd_noalloc(const void* q, const void* kc, const void*
   void* ws = nullptr;
   if (int rc = noalloc_scratch(&ws)) return rc;
   return decode_dispatch(q, kc, vc, o, ws, head_start, head_valid_len, B, Hq, Hkv, D,
-                         sumC, sm_scale, dtype, stream);
+                         sumC, sm_scale, dtype, nullptr, stream);
 }

@@ -35,6 +35,22 @@ def _workspace(device: torch.device, nbytes: int, tag: str, stream: int) -> Tens
     return ws
 
 
+_N_COUNTERS = 16384   # (batch row, ring) pairs up to which a decode launch may merge inside
+_counters: Dict[Tuple[int, int], Tensor] = {}
+
+
+def _arrival_counters(device: torch.device, stream: int) -> Optional[Tensor]:
+    """The zeroed counters of moa_decode_fwd_counted, one set per (device, stream) like the workspace; every call leaves
+    them zeroed.  Their fill must have run before a call counts on it, so none are made while a graph is recorded."""
+    key = (device.index or 0, stream)
+    counters = _counters.get(key)
+    if counters is None:
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        counters = _counters[key] = torch.zeros(_N_COUNTERS, dtype=torch.int32, device=device)
+    return counters
+
+
 def _require_gpu(t: Tensor, who: str) -> None:
     if not t.is_cuda:
         raise _lib.MoaKernelError(
@@ -145,9 +161,11 @@ def moa_decode(
     need = lib.moa_decode_workspace_bytes(B, Hq, Hkv, D, sumC)
     stream = _lib.current_stream_ptr(dev)
     ws = _workspace(dev, need, "decode", stream)
-    rc = lib.moa_decode_fwd(q3.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ws.data_ptr(),
-                            ws.numel(), hs.data_ptr(), hv.data_ptr(), B, Hq, Hkv, D, sumC,
-                            float(sm_scale), _lib.dtype_code(q.dtype), stream)
+    counters = _arrival_counters(dev, stream)
+    rc = lib.moa_decode_fwd_counted(q3.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ws.data_ptr(), ws.numel(),
+                                    None if counters is None else counters.data_ptr(),
+                                    0 if counters is None else _N_COUNTERS, hs.data_ptr(), hv.data_ptr(), B, Hq, Hkv, D,
+                                    sumC, float(sm_scale), _lib.dtype_code(q.dtype), stream)
     _lib.check(rc)
     return o
 

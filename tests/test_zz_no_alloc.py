@@ -154,3 +154,42 @@ def test_recorded_into_a_hip_graph(dev):
                                         hv_d.data_ptr(), B, Hq, Hkv, D, sumC, D ** -0.5, code, _lib.current_stream_ptr(dev))
         assert rc == 0
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("G,D,B,sizes", [
+    (1, 128, 1, [64, 3008, 576, 1344, 4160, 192, 2112, 9000]),   # 1 to 36 chunks a ring
+    (1, 64, 2, [30000, 1, 256, 257]),                            # more than 64 chunks of one ring
+    (1, 128, 5, [300, 700, 40] * 30),                            # more rings than lanes, 512-row chunks
+    (1, 128, 40, [600, 900]),
+    (2, 64, 3, [2500, 64, 5000, 700]),
+    (8, 128, 1, [4096, 3000, 100, 900]),
+    (5, 128, 2, [400] * 70),
+])
+@pytest.mark.parametrize("partial", [False, True])
+def test_merge_inside_the_launch_equals_the_merge_kernel(dev, G, D, B, sizes, partial):
+    """moa_decode_fwd_counted (the ring's last chunk to arrive merges) against moa_decode_fwd (merge kernel): the same
+    partials summed in the same order, so the same bits (a step recorded into a graph may merge the one way and the
+    eager one the other); empty rings are zero, and the counters are zero again after every call."""
+    from moa_amd import _lib
+    lib = _lib.load()
+    rng = np.random.default_rng(G + D + len(sizes))
+    q, kc, vc, hs, hv = _inputs(rng, B, sizes, G, D, torch.float16, dev, partial)
+    Hkv, sumC = len(sizes), kc.shape[1]
+    need = lib.moa_decode_workspace_bytes(B, q.shape[1], Hkv, D, sumC)
+    counters = torch.zeros(B * Hkv, dtype=torch.int32, device=dev)
+    hs_d = torch.from_numpy(hs).to(dev)
+    for shrink in (0, 1):   # a second call on shorter rings: fewer chunks arrive
+        hv_d = torch.from_numpy(hv >> shrink).to(dev)
+        outs = []
+        for n in (0, counters.numel()):
+            ws = torch.full((need,), 0xff, dtype=torch.uint8, device=dev)   # NaN partials: none is read unwritten
+            o = torch.full_like(q, float("nan"))
+            rc = lib.moa_decode_fwd_counted(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), o.data_ptr(), ws.data_ptr(), need,
+                                            counters.data_ptr(), n, hs_d.data_ptr(), hv_d.data_ptr(), B, q.shape[1], Hkv, D,
+                                            sumC, D ** -0.5, _lib.MOA_DTYPE_F16, _lib.current_stream_ptr(dev))
+            assert rc == 0, _lib.last_error()
+            outs.append(o)
+        assert torch.isfinite(outs[1]).all()
+        assert torch.equal(outs[1], outs[0])
+        assert not outs[1].view(B, Hkv, -1)[hv_d == 0].any()
+        assert not counters.any()
