@@ -351,9 +351,7 @@ __device__ __forceinline__ void zero_empty_rings(const ROW& row, uint16_t* o_row
 
 // H: kv heads (rings) per batch row; query head hk*G + g reads ring hk.
 // PIPE: the wave keeps two half-batches of loads going (the next one is issued before the current
-// one is consumed) instead of loading a full batch, waiting for it and consuming it.  Measured at
-// the 7B decode shape: 8 % faster at batch 4, 2 % at 8-16, 0.7 % at 64; at batch 1-2 (about one
-// work-group per CU, the call is launch-latency bound) the plain loop is 2-4 % faster.
+// one is consumed) instead of loading a full batch, waiting for it and consuming it (kDecPipeFrom).
 template <typename T, int D, int CHUNK, int G, bool PIPE, bool NT>
 __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vc,
@@ -882,8 +880,13 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
 
 constexpr int kChunk = 512;           // cache rows per work-group step of the one-query-head kernel
 constexpr int kDecBlocksPerCu = 16;   // work-groups per CU over the whole grid
-constexpr int kDecSmallBelow = 2;     // work-groups per CU below which the chunks are half as long
-constexpr int kDecPipeFrom = 3;       // work-groups per CU from which the waves pipeline their own loads
+// Work-groups per CU (full-length chunks by the rings' capacity) below which the chunks are half as long, and from
+// which the waves pipeline their own loads.  Half-length chunks pay only where full ones leave CUs idle: 32 rings of 128,
+// 288 chunks 17.3 us with half-length, 15.9 with full ones, 469 chunks 26.4 and 23.6, 8 rings 445 chunks 30.6 and 24.5;
+// 160 chunks 11.3 with half-length ones.  Pipelining pays where several work-groups follow each other on a CU: 814 chunks of
+// 64-element rows 23.5 us with, 22.6 without, 864 of 128 40.2 and 39.6, 1152 49.5 and 49.4, 1440 59.2 both.
+constexpr int kDecSmallBelow = 1;
+constexpr int kDecPipeFrom = 4;
 
 // From this many bytes of K and V per launch on they are read non-temporally.  What a step reads of one layer
 // is read again a token later, after the rings of all other layers: with several layers of this size that is
@@ -929,7 +932,6 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
   if (bx > cap) bx = cap;
   if (bx < 1) bx = 1;
   const bool pipe = (int64_t)B * chunks >= (int64_t)256 * kDecPipeFrom;
-  // fewer than two work-groups per CU: half-length chunks give every CU something to do
   const bool small = (int64_t)B * chunks < (int64_t)256 * kDecSmallBelow;
   auto launch = [&](auto split, auto merge) {
     hipLaunchKernelGGL(split, dim3(bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,

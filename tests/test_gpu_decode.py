@@ -128,7 +128,8 @@ def test_partial_fill_with_a_large_grid(dev, D, B):
     (1, 3, [30000, 64, 15777], 128),
     (1, 3, [30000, 64, 15777], 64),
     (1, 9, [20000, 30, 10999, 513], 128),       # full-length chunks
-    (1, 9, [40000, 30, 10999, 513], 64),        # the load-pipelined loop
+    (1, 10, [40000, 30, 10999, 513], 64),       # the load-pipelined loop
+    (1, 64, [100] * 16, 64),                    # the load-pipelined loop with ordinary loads
     (2, 2, [60000, 33, 30001], 128),            # grouped query, non-temporal copies
     (7, 5, [60000, 33, 30001], 64),
 ])
