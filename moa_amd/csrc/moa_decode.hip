@@ -21,7 +21,8 @@
 //     head_valid_len (no host knowledge of the lengths, no host sync);
 //   * a head with one chunk writes its output directly; otherwise chunks
 //     write fp32 partial (acc, max, sum) triples and a small second kernel
-//     merges them;
+//     merges them (in launches of few chunks the head's last chunk to arrive
+//     does, when the caller brings counters);
 //   * grouped-query attention (G = Hq / Hkv query heads per ring, which the
 //     reference does not have): the G query rows of a ring share every K/V
 //     row that a wave loads, so the cache is still read once.  This kernel is
