@@ -201,19 +201,19 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
         own_alive = false;
       }
     } else {
-      // lane 8 asks for a ticket of the own list, lanes 0 to 7 how far the lists are handed out: one round trip to
-      // memory, also where there is nothing left (asking the lists one after the other is eight of them, in which
-      // the whole work-group stands still at the end of its last item)
-      unsigned got = 0;
-      if (lane < 8) got = atomicAdd(&ap->queue->next[lane], 0u);
-      if (lane == 8 && own_alive) got = atomicAdd(&ap->queue->next[my_xcd], 1u);
-      const unsigned long long left = __ballot(lane < 8 && got < list_items(lane & 7)) & ~(1ull << my_xcd);
-      const unsigned mine = (unsigned)__builtin_amdgcn_readlane((int)got, 8);
-      if (own_alive && mine < list_items(my_xcd)) {
-        list = my_xcd;
-        sq = mine;
-      } else {
-        own_alive = false;
+      if (own_alive) {
+        unsigned t = 0;
+        if (lane == 0) t = atomicAdd(&ap->queue->next[my_xcd], 1u);
+        sq = (unsigned)__builtin_amdgcn_readfirstlane((int)t);
+        if (sq < list_items(my_xcd)) list = my_xcd; else own_alive = false;
+      }
+      if (list < 0) {
+        // lanes 0 to 7 ask how far the lists are handed out: one round trip to memory, also where nothing is left (asking
+        // the lists one after the other is seven of them, in which the whole work-group stands still at the end of its
+        // last item)
+        unsigned out = 0;
+        if (lane < 8) out = atomicAdd(&ap->queue->next[lane], 0u);
+        const unsigned long long left = __ballot(lane < 8 && out < list_items(lane & 7));
         for (int i = 1; i < 8; ++i) {
           const int x = (my_xcd + i) & 7;
           if (!((left >> x) & 1)) continue;
