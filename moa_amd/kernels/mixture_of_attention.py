@@ -41,12 +41,14 @@ _counters: Dict[Tuple[int, int], Tensor] = {}
 
 def _arrival_counters(device: torch.device, stream: int) -> Optional[Tensor]:
     """The zeroed counters of moa_decode_fwd_counted, one set per (device, stream) like the workspace; every call leaves
-    them zeroed.  Their fill must have run before a call counts on it, so none are made while a graph is recorded."""
+    them zeroed.  A call that is being recorded into a graph takes none (two launches, the same bits): a replay may run
+    beside eager calls of this stream or beside other graphs recorded on it, and where two launches count in the same
+    place a lost count stays for good."""
+    if torch.cuda.is_current_stream_capturing():
+        return None
     key = (device.index or 0, stream)
     counters = _counters.get(key)
     if counters is None:
-        if torch.cuda.is_current_stream_capturing():
-            return None
         counters = _counters[key] = torch.zeros(_N_COUNTERS, dtype=torch.int32, device=device)
     return counters
 

@@ -1,0 +1,104 @@
+"""The arrival counters of decode launches that merge inside: they outlive a call, so only calls that cannot overlap may
+share them.  A step recorded into a HIP graph, whose replays run on any stream, takes none of the Python path's."""
+import pytest
+import torch
+
+
+def test_a_recorded_call_takes_no_shared_counters(monkeypatch):
+    from moa_amd.kernels import mixture_of_attention as M
+    stream = -12345   # no stream of this value exists
+    kept = torch.zeros(4, dtype=torch.int32)
+    monkeypatch.setitem(M._counters, (0, stream), kept)   # as an eager call on that stream leaves them
+    dev = torch.device("cuda:0")
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    assert M._arrival_counters(dev, stream) is kept
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert M._arrival_counters(dev, stream) is None
+
+
+@pytest.fixture(scope="module")
+def dev():
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    from moa_amd import _lib
+    _lib.load()
+    return torch.device("cuda:0")
+
+
+def _rings(dev, G, D, B, sizes):
+    g = torch.Generator(device=dev).manual_seed(G * D + B)
+    H, sumC = len(sizes), sum(sizes)
+    q = torch.randn(B, H * G, 1, D, generator=g, device=dev, dtype=torch.float16)
+    kc, vc = (torch.randn(B, sumC, D, generator=g, device=dev, dtype=torch.float16) for _ in range(2))
+    start = torch.tensor([sum(sizes[:h]) for h in range(H)], device=dev).expand(B, H).contiguous()
+    valid = torch.tensor(sizes, device=dev).expand(B, H).contiguous()
+    return q, kc, vc, start, valid
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G", [1, 4])
+def test_replays_beside_eager_calls_of_the_capture_stream(dev, G):
+    """A step recorded on the stream that eager calls ran on before: replays, with eager calls in between, are right
+    and neither look at that stream's counters nor touch them."""
+    from moa_amd import mixture_of_sparse_attention
+    from moa_amd.kernels import mixture_of_attention as M
+    q, kc, vc, start, valid = _rings(dev, G, 128, 1, [700, 1100, 300, 900])
+
+    def step():
+        return mixture_of_sparse_attention(q, kc, vc, 0.1, head_start_index=start, head_valid_length=valid)
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        step()
+        counters = M._counters[(0, stream.cuda_stream)]
+        with torch.cuda.graph(graph, stream=stream):
+            recorded = step()
+        for i in range(4):
+            q.normal_(generator=torch.Generator(device=dev).manual_seed(i))
+            want = step()
+            stream.synchronize()
+            assert not counters.any(), i
+            counters.fill_(1)   # as a launch under way holds them
+            graph.replay()
+            stream.synchronize()
+            assert (counters == 1).all(), i
+            counters.zero_()
+            assert torch.equal(recorded, want), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G", [1, 4])
+def test_a_graph_with_counters_of_its_own(dev, G):
+    """Through the C entry point a graph may bring counters: every replay finds them zero and leaves them so."""
+    from moa_amd import _lib
+    lib = _lib.load()
+    B, D = 1, 128
+    q, kc, vc, start, valid = _rings(dev, G, D, B, [700, 1100, 300, 900])
+    Hq, Hkv, sumC = q.shape[1], valid.shape[1], kc.shape[1]
+    need = lib.moa_decode_workspace_bytes(B, Hq, Hkv, D, sumC)
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    counters = torch.zeros(B * Hkv, dtype=torch.int32, device=dev)
+
+    def call(o, n):
+        rc = lib.moa_decode_fwd_counted(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), o.data_ptr(), ws.data_ptr(), need,
+                                        counters.data_ptr(), n, start.data_ptr(), valid.data_ptr(), B, Hq, Hkv, D, sumC,
+                                        D ** -0.5, _lib.MOA_DTYPE_F16, _lib.current_stream_ptr(dev))
+        assert rc == 0, _lib.last_error()
+
+    recorded, want = torch.empty_like(q), torch.empty_like(q)
+    call(recorded, counters.numel())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(recorded, counters.numel())
+    for i in range(4):
+        q.normal_(generator=torch.Generator(device=dev).manual_seed(i))
+        valid.sub_(97)   # other chunk counts in every replay
+        call(want, 0)
+        recorded.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded, want), i
+        assert not counters.any(), i
