@@ -108,6 +108,25 @@ __device__ __forceinline__ u32x4 load_once16(GlobalPtr p) {
   else return *s;
 }
 
+// Rows of a segment are numbered in 32 bits, without a sign: a segment has up to 2^31 - 1 rows, and where its last
+// chunk, or the load batch at its end, would stop lies up to a chunk past that.
+constexpr __host__ __device__ __forceinline__ int chunks_of(int len, int size) {
+  return (int)(((unsigned)len + (unsigned)size - 1u) / (unsigned)size);
+}
+// first row of a wave's share of a chunk, and the first row behind it
+constexpr __host__ __device__ __forceinline__ unsigned share_begin(int chunk, int chunk_rows, int wave, int share_rows) {
+  return (unsigned)chunk * (unsigned)chunk_rows + (unsigned)wave * (unsigned)share_rows;
+}
+constexpr __host__ __device__ __forceinline__ unsigned share_end(unsigned begin, int share_rows, int len) {
+  return begin + (unsigned)share_rows < (unsigned)len ? begin + (unsigned)share_rows : (unsigned)len;
+}
+// the largest segment: whole chunks, the last one a row short (an overflow with a sign does not compile here)
+constexpr int kMaxRows = 0x7fffffff;
+static_assert(chunks_of(kMaxRows, 512) == 1 << 22 && chunks_of(kMaxRows, 2048) == 1 << 20);
+static_assert(chunks_of(0, 512) == 0 && chunks_of(1, 512) == 1 && chunks_of(512, 512) == 1 && chunks_of(513, 512) == 2);
+static_assert(share_end(share_begin((1 << 22) - 1, 512, 3, 128), 128, kMaxRows) == 0x7fffffffu);
+static_assert(share_end(share_begin((1 << 22) - 1, 512, 2, 128), 128, kMaxRows) == 0x7fffff80u);
+
 // Inclusive sum over the lanes of a wave, in six DPP steps (no LDS); lane 63 has the total.
 __device__ __forceinline__ int wave_scan(int x) {
   x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 inside rows of 16 lanes
@@ -175,7 +194,7 @@ struct RowChunks {
         int n = 0;
 #pragma unroll
         for (int k = 0; k < kGroups; ++k)
-          if (k * 64 < H) n += (len[k] + size - 1) / size;
+          if (k * 64 < H) n += chunks_of(len[k], size);
         return wave_sum(n);
       };
       // rows in steps (a sum of at most 256 heads of < 2^31 rows each fits 32 bits in steps)
@@ -188,10 +207,10 @@ struct RowChunks {
       rows[k] = c;
       last[k] = base;
       if (k * 64 < H) {
-        int n = (len[k] + c - 1) / c;
+        int n = chunks_of(len[k], c);
         if (even && n > 0) {
-          rows[k] = (((len[k] + n - 1) / n + kEvenStep - 1) / kEvenStep) * kEvenStep;   // even split, <= c
-          n = (len[k] + rows[k] - 1) / rows[k];
+          rows[k] = chunks_of(chunks_of(len[k], n), kEvenStep) * kEvenStep;   // even split, <= c
+          n = chunks_of(len[k], rows[k]);
         }
         const int incl = wave_scan(n);
         last[k] = min(base + incl, cap);
@@ -387,8 +406,8 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
     const Chunk ck = row.at(w, H);
     const int c = ck.index, n_chunks = ck.count;
     const int64_t bh = (int64_t)b * H + ck.head;
-    const int r_begin = c * CHUNK + wave * WCHUNK;   // rows of a segment fit 31 bits
-    const int r_end = min(r_begin + WCHUNK, ck.len);
+    const unsigned r_begin = share_begin(c, CHUNK, wave, WCHUNK);
+    const unsigned r_end = share_end(r_begin, WCHUNK, ck.len);
 
     // this lane's 8 query elements of each of the G query heads, kept packed for dot2
     u32x4 qv[G];
@@ -412,11 +431,11 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
     }
 
     // n wave-wide loads of K and of V starting at row r0 of the wave's share
-    auto load_rows = [&](auto N, u32x4* kr, u32x4* vr, int r0) __attribute__((always_inline)) {
+    auto load_rows = [&](auto N, u32x4* kr, u32x4* vr, unsigned r0) __attribute__((always_inline)) {
       constexpr int n = decltype(N)::value;
 #pragma unroll
       for (int i = 0; i < n; ++i) {
-        const int row = r0 + i * RPL + sub;
+        const unsigned row = r0 + i * RPL + sub;
         const int64_t rr = row < r_end ? row : r_begin;  // any valid row: keeps the load in bounds
         kr[i] = load_once16<NT>(kbase + rr * D);
         vr[i] = load_once16<NT>(vbase + rr * D);
@@ -424,7 +443,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
       __builtin_amdgcn_sched_barrier(0);   // all of them before what uses them
     };
     // online-softmax update with those rows
-    auto consume_rows = [&](auto N, const u32x4* kr, const u32x4* vr, int r0) __attribute__((always_inline)) {
+    auto consume_rows = [&](auto N, const u32x4* kr, const u32x4* vr, unsigned r0) __attribute__((always_inline)) {
       constexpr int n = decltype(N)::value;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
@@ -462,7 +481,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
       }
     };
     if (!PIPE) {
-      for (int r0 = r_begin; r0 < r_end; r0 += ROWS) {
+      for (unsigned r0 = r_begin; r0 < r_end; r0 += ROWS) {
         u32x4 kr[KB], vr[KB];
         load_rows(DecInt<KB>{}, kr, vr, r0);
         consume_rows(DecInt<KB>{}, kr, vr, r0);
@@ -474,7 +493,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
       u32x4 ka[KH], va[KH], kb2[KH], vb2[KH];
       if (r_begin < r_end) {
         load_rows(DecInt<KH>{}, ka, va, r_begin);
-        for (int r0 = r_begin; r0 < r_end; r0 += ROWS) {
+        for (unsigned r0 = r_begin; r0 < r_end; r0 += ROWS) {
           load_rows(DecInt<KH>{}, kb2, vb2, r0 + HROWS);
           consume_rows(DecInt<KH>{}, ka, va, r0);
           load_rows(DecInt<KH>{}, ka, va, r0 + ROWS);
