@@ -105,14 +105,17 @@ __device__ __forceinline__ int64_t candidate_count(const HeadRing& g, int64_t n_
 // consecutive ones, and counts the valid tokens in front of its part by itself (the row is read from L2 as often as
 // it has parts), so that nothing waits for another work-group; the counts meet in LDS once, ballots and population
 // counts give a lane the number of valid tokens in front of its four.  8 rows of
-// 16384 tokens: 8.5 us with both outputs, 18 us with one work-group per row.
+// 16384 tokens: 8.5 us with both outputs, 18 us with one work-group per row.  Rows of more than kMaskGroups parts give
+// a work-group several parts in a row, so that a row is read at most kMaskGroups times.
 // rank_of (may be null): the other direction too, rank_of[b, t] = number of valid tokens in front of t for a valid
 // token, -1 for padding, for the kernel that walks tokens.
 constexpr int kScanThreads = 1024;
 constexpr int kMaskPerLane = 4;
 constexpr int kMaskPart = kScanThreads * kMaskPerLane;
+constexpr int kMaskGroups = 512;   // work-groups per row at most
 __global__ __launch_bounds__(kScanThreads) void mask_compact_kernel(const int64_t* __restrict__ am,
                                                                      int64_t am_stride, int S,
+                                                                     unsigned group_tokens /* of a work-group: whole parts */,
                                                                      int32_t* __restrict__ tok_of,
                                                                      int32_t* __restrict__ n_valid,
                                                                      int32_t* __restrict__ rank_of) {
@@ -123,42 +126,55 @@ __global__ __launch_bounds__(kScanThreads) void mask_compact_kernel(const int64_
   const int64_t* row = am + (int64_t)b * am_stride;
   int32_t* out = tok_of + (int64_t)b * S;
   int32_t* rank = rank_of ? rank_of + (int64_t)b * S : nullptr;
-  const int part0 = blockIdx.x * kMaskPart;
-  const int t = part0 + tid * kMaskPerLane;
+  // token numbers without a sign: the last part of a row of up to 2^31 - 1 tokens ends past that
+  const unsigned n_tok = (unsigned)S, first = blockIdx.x * group_tokens, end = min(first + group_tokens, n_tok);
   bool valid[kMaskPerLane];
+  auto load_part = [&](unsigned t) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < kMaskPerLane; ++j) valid[j] = t + j < S && row[t + j] == 1;
-  int front = 0;
+    for (int j = 0; j < kMaskPerLane; ++j) valid[j] = t + j < n_tok && row[t + j] == 1;
+  };
+  load_part(first + (unsigned)(tid * kMaskPerLane));
+  int front = 0;   // this thread's share of the valid tokens in front of the work-group's
 #pragma unroll 8
-  for (int i = tid; i < part0; i += kScanThreads) front += row[i] == 1 ? 1 : 0;
+  for (unsigned i = tid; i < first; i += kScanThreads) front += row[i] == 1 ? 1 : 0;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) front += __shfl_xor(front, off, 64);
   const unsigned long long below = (1ull << lane) - 1ull;
-  int before = 0, own = 0;   // valid tokens of lower lanes; of the wave
+  int base = 0;    // valid tokens in front of the part
+  for (unsigned part0 = first;;) {
+    const unsigned t = part0 + (unsigned)(tid * kMaskPerLane);
+    int before = 0, own = 0;   // valid tokens of lower lanes; of the wave
 #pragma unroll
-  for (int j = 0; j < kMaskPerLane; ++j) {
-    const unsigned long long bal = __ballot(valid[j]);
-    before += __popcll(bal & below);
-    own += __popcll(bal);
-  }
-  if (lane == 0) {
-    s_own[wave] = own;
-    s_front[wave] = front;
-  }
-  __syncthreads();
-  int at = before, total = 0;
+    for (int j = 0; j < kMaskPerLane; ++j) {
+      const unsigned long long bal = __ballot(valid[j]);
+      before += __popcll(bal & below);
+      own += __popcll(bal);
+    }
+    if (lane == 0) {
+      s_own[wave] = own;
+      s_front[wave] = front;
+    }
+    __syncthreads();
+    int at = base + before, total = 0;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    at += s_front[w] + ((w < wave) ? s_own[w] : 0);
-    total += s_front[w] + s_own[w];
-  }
+    for (int w = 0; w < kWaves; ++w) {
+      at += s_front[w] + ((w < wave) ? s_own[w] : 0);
+      total += s_front[w] + s_own[w];
+    }
 #pragma unroll
-  for (int j = 0; j < kMaskPerLane; ++j) {
-    if (valid[j]) out[at] = t + j;
-    if (rank && t + j < S) rank[t + j] = valid[j] ? at : -1;
-    at += valid[j] ? 1 : 0;
+    for (int j = 0; j < kMaskPerLane; ++j) {
+      if (valid[j]) out[at] = (int32_t)(t + j);
+      if (rank && t + j < n_tok) rank[t + j] = valid[j] ? at : -1;
+      at += valid[j] ? 1 : 0;
+    }
+    base += total;
+    part0 += kMaskPart;
+    if (part0 >= end) break;
+    front = 0;
+    __syncthreads();   // s_own and s_front are written again
+    load_part(part0 + (unsigned)(tid * kMaskPerLane));
   }
-  if (blockIdx.x == gridDim.x - 1 && tid == 0) n_valid[b] = total;
+  if (blockIdx.x == gridDim.x - 1 && tid == 0) n_valid[b] = base;
 }
 
 constexpr int kRowsPerThread = 4;   // rows a group of 16 lanes moves: all loads go out before the first store
@@ -237,8 +253,10 @@ __global__ __launch_bounds__(256) void cache_prefill_index_kernel(
 
 int launch_mask_scan(const int64_t* attention_mask, int64_t am_stride, int B, int S, int32_t* tok_of, int32_t* n_valid,
                      int32_t* rank_of, hipStream_t st) {
-  hipLaunchKernelGGL(mask_compact_kernel, dim3((unsigned)((S + (int64_t)kMaskPart - 1) / kMaskPart), B), dim3(kScanThreads), 0, st, attention_mask, am_stride, S, tok_of, n_valid,
-                     rank_of);
+  const int64_t parts = ((int64_t)S + kMaskPart - 1) / kMaskPart;
+  const int64_t group_parts = (parts + kMaskGroups - 1) / kMaskGroups;   // parts of a work-group
+  hipLaunchKernelGGL(mask_compact_kernel, dim3((unsigned)((parts + group_parts - 1) / group_parts), B), dim3(kScanThreads),
+                     0, st, attention_mask, am_stride, S, (unsigned)(group_parts * kMaskPart), tok_of, n_valid, rank_of);
   return check_launch("prompt insert (mask scan)");
 }
 

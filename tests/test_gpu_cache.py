@@ -149,6 +149,51 @@ def test_random_against_oracle(dev, seed):
             _assert_state(cache, o, (seed, i))
 
 
+@pytest.mark.parametrize("S", [4095, 4096, 4097, 8193, 16385, 512 * 4096, 512 * 4096 + 1, 2 * 512 * 4096 + 4099])
+def test_padded_prompts_around_the_parts_of_the_mask_scan(dev, S):
+    """The scan over a padded row gives 4096 tokens to a work-group and, from 512 such parts on, several parts: rows
+    whose padding ends in another part than it begins, with holes on both sides of a part's edge, without a valid
+    token, with the last one only.  Rows carry their token's number; expected is the closed form of a first insert:
+    the first tokens in the static part, the last ones in the ring in their turn."""
+    from moa_amd import StaticCircularCache
+    rng = np.random.default_rng(S)
+    cache_size, static = [704, 64, 5000], [64, 64, 0]
+    B, H, D = 4, 3, 8
+    mask = np.ones((B, S), dtype=np.int64)
+    mask[0, :S // 3] = 0
+    mask[0, S // 3:] = rng.random(S - S // 3) < 0.9
+    mask[1] = 0
+    mask[2, :-1] = 0
+    mask[3, 4090:4100] = 0
+    k = torch.zeros(B, H, S, D, device=dev)
+    k[..., 0] = torch.arange(S, device=dev)
+    k[..., 1] = torch.arange(H, device=dev)[:, None]
+    k[..., 2] = torch.arange(B, device=dev)[:, None, None]
+    cache = StaticCircularCache([cache_size], static_size=[static], batch_size=B, head_dim=D, device=dev,
+                                dtype=torch.float32)
+    cache.update(k, -k, 0, torch.from_numpy(mask).to(dev))
+    want = np.zeros((B, sum(cache_size), D), dtype=np.float32)
+    kept, upd, valid = (np.zeros((B, n), dtype=np.int64) for n in (sum(cache_size), H, H))
+    for b in range(B):
+        tok = np.flatnonzero(mask[b])
+        n, start = len(tok), 0
+        for h, (c, s) in enumerate(zip(cache_size, static)):
+            ring = c - s
+            a = np.concatenate([np.arange(min(s, n)), np.arange(max(s, n - ring), n) if ring else np.arange(0)]).astype(int)
+            slot = start + np.where(a < s, a, s + (a - s) % max(ring, 1))
+            want[b, slot, 0], want[b, slot, 1], want[b, slot, 2] = tok[a], h, b
+            kept[b, slot] = 1
+            valid[b, h] = len(a)
+            # the slot a token after these would take
+            upd[b, h] = start + (n if n <= s else s + (n - s) % max(ring, 1))
+            start += c
+    assert np.array_equal(cache.mask_cache[0].cpu().numpy(), kept)
+    assert np.array_equal(cache.cache_valid_length[0].cpu().numpy(), valid)
+    assert np.array_equal(cache.cache_update_index[0].cpu().numpy(), upd)
+    assert np.array_equal(cache.key_cache[0].cpu().numpy(), want)
+    assert np.array_equal(cache.value_cache[0].cpu().numpy(), -want)
+
+
 def test_bookkeeping_only(dev):
     """update_cache_content=False: indices move, no payload is touched."""
     from moa_amd import StaticCircularCache
