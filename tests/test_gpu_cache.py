@@ -194,6 +194,33 @@ def test_padded_prompts_around_the_parts_of_the_mask_scan(dev, S):
     assert np.array_equal(cache.value_cache[0].cpu().numpy(), -want)
 
 
+def test_index_tables_are_complete_on_return(dev):
+    """A cache made behind work that is still under way on its stream can be read on another one at once: no table
+    waits for the copy on the constructing stream."""
+    from moa_amd import StaticCircularCache
+    cache_size, static = [[128, 64, 640], [320, 333, 96]], [[64, 64, 0], [64, 64, 64]]
+
+    def make(device):
+        return StaticCircularCache(cache_size, static_size=static, batch_size=2, head_dim=64, device=device)
+
+    names = ("cache_max_length", "static_cache_size", "circular_cache_size", "circular_cache_head_index",
+             "cache_head_start_index", "cache_update_index", "cache_valid_length", "head_index")
+    want = make("cpu")
+    other = torch.cuda.Stream()
+    junk = torch.full((1 << 16,), -1, dtype=torch.int64, device=dev)   # what the tables' memory holds before
+    a = torch.randn(8192, 8192, device=dev, dtype=torch.float16)
+    torch.cuda.synchronize()
+    del junk
+    for _ in range(20):   # some 20 ms of work
+        b = a @ a
+    cache = make(dev)
+    with torch.cuda.stream(other):
+        got = {n: [t.cpu() for t in getattr(cache, n)] for n in names}
+    torch.cuda.synchronize()
+    for n in names:
+        assert all(torch.equal(x, y) for x, y in zip(got[n], getattr(want, n))), n
+
+
 def test_bookkeeping_only(dev):
     """update_cache_content=False: indices move, no payload is touched."""
     from moa_amd import StaticCircularCache
