@@ -75,29 +75,6 @@ __global__ __launch_bounds__(kCacheThreads) void cache_append_kernel(
 // ---------------------------------------------------------------------------
 // Prompt bulk insert (cache_utils.py:1060-1164)
 // ---------------------------------------------------------------------------
-// Candidate r -> the token with advancing position a (its index among the row's valid tokens; without a
-// mask every token is valid and a is the token's position).  Only tokens that can be kept are
-// enumerated: r < csz walks the valid tokens from the last one backwards (these have
-// rap = r+1 <= csz); r >= csz walks the first ones (the only ones whose slot can lie in the static
-// part); any other token is a ring token older than the last csz and is dropped by the keep rule.
-// n_valid: valid tokens of the batch row.  Returns whether the candidate is kept, with a and its slot.
-__device__ __forceinline__ bool candidate(const HeadRing& g, int64_t r, int64_t n_valid, int64_t& a, int64_t& slot) {
-  if (r < g.csz) {
-    a = n_valid - 1 - r;
-    if (a < 0) return false;
-  } else {
-    a = r - g.csz;
-    if (a >= n_valid - g.csz || a > g.s) return false;
-  }
-  const int64_t rap = n_valid - a;   // valid tokens at or after this one (:1081-1086)
-  slot = slot_of(g, a);
-  return keep_of(g, slot, rap);
-}
-// how many candidates a head has
-__device__ __forceinline__ int64_t candidate_count(const HeadRing& g, int64_t n_valid) {
-  return min(n_valid, g.csz + g.s + 1);
-}
-
 // With an attention mask: the positions of a batch row's valid tokens (mask == 1) in order,
 // tok_of[b, a] = position of the a-th valid token, and their number n_valid[b].  This is the inverse of
 // the reference's advancing_pos = cumsum(mask) - 1 (:1075-1080); its reversed_advancing_pos of a valid

@@ -41,6 +41,29 @@ __device__ __forceinline__ bool keep_of(const HeadRing& g, int64_t slot, int64_t
   return (rap <= g.csz) || (slot < g.ch);
 }
 
+// Candidate r -> the token with advancing position a (its index among the row's valid tokens; without a
+// mask every token is valid and a is the token's position).  Only tokens that can be kept are
+// enumerated: r < csz walks the valid tokens from the last one backwards (these have
+// rap = r+1 <= csz); r >= csz walks the first ones (the only ones whose slot can lie in the static
+// part); any other token is a ring token older than the last csz and is dropped by the keep rule.
+// n_valid: valid tokens of the batch row.  Returns whether the candidate is kept, with a and its slot.
+__device__ __forceinline__ bool candidate(const HeadRing& g, int64_t r, int64_t n_valid, int64_t& a, int64_t& slot) {
+  if (r < g.csz) {
+    a = n_valid - 1 - r;
+    if (a < 0) return false;
+  } else {
+    a = r - g.csz;
+    if (a >= n_valid - g.csz || a > g.s) return false;
+  }
+  const int64_t rap = n_valid - a;   // valid tokens at or after this one (:1081-1086)
+  slot = slot_of(g, a);
+  return keep_of(g, slot, rap);
+}
+// how many candidates a head has
+__device__ __forceinline__ int64_t candidate_count(const HeadRing& g, int64_t n_valid) {
+  return min(n_valid, g.csz + g.s + 1);
+}
+
 // The advancing position of the token that the insert of n_valid tokens leaves in `row` of the head's own segment, -1
 // for none.  The inverse of slot_of and keep_of: a token in front of the ring's turn sits at upd0 + a; of the ring's
 // tokens only the last csz are kept, and exactly one of those has the row's residue.

@@ -283,8 +283,11 @@ struct Coef<EBF16> {
 // token here, kRopeAtOnce wave-wide loads of its q heads or of its kv heads (consecutive memory): cos and sin are
 // fetched once for all of them, and in a kv piece the lanes work out the slots of all kv heads side by side.  A
 // rotated row is in registers when its slot is known, so the rings of k cost their writes only.
-// The first work-groups walk the rings' rows instead: they fetch the v row that belongs into each, and in rings that
-// have just been allocated (FRESH) zero the rows no token goes to, so no fill runs in front.
+// The first work-groups take v to the rings: in rings that have just been allocated (FRESH) they walk the rows, fetch
+// the v row that belongs into each and zero the rows no token goes to, so no fill runs in front; in rings in use they
+// walk the tokens that can be kept, so that a short piece of a prompt does not cost a walk over rings of any size
+// (16 tokens into 32 x 8 rings of 8192 rows: 50.6 us by rows, 7.3 by tokens, 10.6 in two steps; 64 tokens into 8 x 32
+// rings of 4096: 31.0, 8.0, 13.5).
 // Batch 8, 32 heads of 128, 16384 tokens, bf16, a third of the tokens kept (4.9 GB): 970 us (5.1 TB/s) against 743 us
 // rotary + 87 us fill + 268 us insert in separate launches; 64 query heads on 8 rings, batch 1: 103 us.
 struct RingArgs {
@@ -296,7 +299,7 @@ struct RingArgs {
   const int32_t *tok_of, *rank_of, *n_valid;   // with an attention mask, else null
   int64_t kv_len, sumC;
 };
-constexpr int kRingRows = 256;      // segment rows per work-group of the ring part
+constexpr int kRingRows = 256;      // segment rows, or tokens, per work-group of the ring part
 constexpr int kRingAtOnce = 4;      // rows a group of 16 lanes has under way
 // Wave-wide row loads a wave has under way, and all it does.  Measured at the two sizes above: 2: 970 and 103 us,
 // 4: 1000 and 106 us, 8: 950 and 110 us; a whole token (q and k heads in turn) to a wave: 960 and 118 us.
@@ -327,7 +330,8 @@ __global__ __launch_bounds__(kRopeThreads) void rope_insert_kernel(
     const int b = (int)(bh / (unsigned)Hkv), h = (int)(bh % (unsigned)Hkv);
     const HeadRing g = load_ring(ra.update_index, ra.circ_head, ra.circ_size, ra.static_size, ra.kv_len, bh, h);
     const int64_t nv = ra.n_valid ? (int64_t)ra.n_valid[b] : (int64_t)N;
-    const int64_t first = g.ch - g.s, rows = min(g.s + g.csz, (int64_t)(slice + 1) * kRingRows);
+    const int64_t count = FRESH ? g.s + g.csz : candidate_count(g, nv);
+    const int64_t first = g.ch - g.s, rows = min(count, (int64_t)(slice + 1) * kRingRows);
     const int lane = threadIdx.x % kRopeRowLanes;
     const int row_bytes = 2 * half_bytes, units = row_bytes / 16;
     for (int64_t r0 = (int64_t)slice * kRingRows + threadIdx.x / kRopeRowLanes; r0 < rows;
@@ -337,10 +341,16 @@ __global__ __launch_bounds__(kRopeThreads) void rope_insert_kernel(
       bool in[kRingAtOnce], keep[kRingAtOnce];
 #pragma unroll
       for (int j = 0; j < kRingAtOnce; ++j) {
-        const int64_t r = r0 + j * kRopeRowsPerBlock, row = first + r;
-        in[j] = r < rows && row >= 0 && row < ra.sumC;
-        int64_t t = in[j] ? token_of_row(g, row, nv) : -1;
-        keep[j] = t >= 0;
+        const int64_t r = r0 + j * kRopeRowsPerBlock;
+        int64_t row = first + r, t = -1;
+        if (FRESH) {
+          in[j] = r < rows && row >= 0 && row < ra.sumC;
+          if (in[j]) t = token_of_row(g, row, nv);
+          keep[j] = t >= 0;
+        } else {
+          keep[j] = r < rows && candidate(g, r, nv, t, row) && row >= 0 && row < ra.sumC;
+          in[j] = keep[j];
+        }
         if (keep[j] && ra.tok_of) t = ra.tok_of[(int64_t)b * N + t];
         src[j] = ra.v + b * ra.v_sb + h * ra.v_sh + t * ra.v_sn;
         dst[j] = ((size_t)b * ra.sumC + row) * row_bytes;
@@ -578,7 +588,9 @@ extern "C" int moa_rope_prefill_insert(const void* q, const void* k, const void*
   const int pieces = (Hq + per_piece - 1) / per_piece + (Hkv + per_piece - 1) / per_piece;
   const int64_t units = tokens * pieces;
   const int64_t unit_blocks = (units + kRopeThreads / 64 - 1) / (kRopeThreads / 64);
-  const int64_t slices = (max_cache_size + kRingRows - 1) / kRingRows;
+  // with rings in use: no more candidates than tokens, or than a head's rows + 1 (see candidate())
+  const int64_t walked = zero_rest ? max_cache_size : max_cache_size < S ? max_cache_size + 1 : S;
+  const int64_t slices = (walked + kRingRows - 1) / kRingRows;
   const int64_t ring_blocks = (int64_t)B * Hkv * slices;
   const int64_t blocks = unit_blocks + ring_blocks;
   if (units > 0x7fffffffLL || blocks > 0x7fffffffLL) return fail(MOA_ERR_UNSUPPORTED, "%s: too many tokens", who);

@@ -158,6 +158,41 @@ def test_prompt_in_one_launch_equals_the_two_steps(dev, dtype, D, S, padded):
         assert one.get_seq_length() == two.get_seq_length() and one.cache_position == two.cache_position
 
 
+@pytest.mark.parametrize("H,Hq", [(4, 8), (33, 33), (64, 64)])   # one piece of kv heads to a token; several
+@pytest.mark.parametrize("padded", [False, True])
+def test_later_pieces_of_a_prompt_in_one_launch(dev, H, Hq, padded):
+    """A prompt in pieces, the later ones shorter than the rings: with rings in use the one launch walks the tokens
+    that can be kept (256 to a work-group) and must touch nothing else.  Against the two steps, whole rings bit for bit,
+    rows that no token went to holding what was there before."""
+    from moa_amd import StaticCircularCache
+    from moa_amd.kernels.rotary import apply_rotary_pos_emb
+    B, D, dtype = 2, 64, torch.float16
+    sizes = [[1500, 64, 300, 320][h % 4] for h in range(H)]
+    static = [[64, 64, 0, 64][h % 4] for h in range(H)]
+    one, two = (StaticCircularCache([sizes], static_size=[static], batch_size=B, head_dim=D, device=dev, dtype=dtype)
+                for _ in range(2))
+    at = 0
+    for step, S in enumerate([40, 2, 255, 256, 257, 700, 3, 2100]):
+        q, k, v = (_rand((B, S, n, D), dtype, 11 * step + i).to(dev).transpose(1, 2) for i, n in enumerate((Hq, H, H)))
+        cos, sin = (t.to(dev) for t in rope_cos_sin(torch.arange(S)[None, :] + at, D, dtype=dtype))
+        at += S
+        mask = None
+        if padded:
+            mask = (torch.rand(B, S, generator=torch.Generator().manual_seed(S)) < 0.7).to(torch.int64).to(dev)
+        if step:   # what lies in the rows that are free or that the piece leaves alone must stay
+            for a, b in ((one.key_cache[0], two.key_cache[0]), (one.value_cache[0], two.value_cache[0])):
+                a.normal_(generator=torch.Generator(device=dev).manual_seed(step))
+                b.copy_(a)
+        assert one._prompt_fits_one_launch(q, k, v, cos, sin, 0, mask)
+        got = one.rope_update(q, k, v, cos, sin, 0, mask)
+        qe, ke = apply_rotary_pos_emb(q, k, cos, sin)
+        want = (qe,) + two.update(ke, v, 0, mask)
+        for a, b in zip(got, want):
+            assert _same_bits(a, b), step
+        for name in ("key_cache", "value_cache", "mask_cache", "cache_update_index", "cache_valid_length"):
+            assert torch.equal(getattr(one, name)[0], getattr(two, name)[0]), (name, step)
+
+
 def test_fused_step_feeds_the_decode_kernel(dev):
     """rope_update (one launch) + mixture_of_sparse_attention against the oracle's decode on the
     oracle's cache: what a decoder layer sees."""
