@@ -230,8 +230,10 @@ class StaticCircularCache:
         seq_len = key_states.shape[-2]
         if seq_len != 1 or not self.update_cache_content:
             if self._prompt_fits_one_launch(query_states, key_states, value_states, cos, sin, layer_idx, attention_mask):
-                return self._rope_insert_prompt(query_states, key_states, value_states, cos, sin, layer_idx,
+                done = self._rope_insert_prompt(query_states, key_states, value_states, cos, sin, layer_idx,
                                                 attention_mask)
+                if done is not None:
+                    return done
             q_embed, k_embed = apply_rotary_pos_emb(query_states, key_states, cos, sin)
             keys, values = self.update(k_embed, value_states, layer_idx, attention_mask)
             return q_embed, keys, values
@@ -340,7 +342,8 @@ class StaticCircularCache:
         return (self.key_cache[layer_idx] is None) == (self._ready_on[layer_idx] is None)
 
     def _rope_insert_prompt(self, q, k, v, cos, sin, layer_idx, attention_mask):
-        """Rotary embedding and insert of a prompt in one pass over q, k and v (moa_rope_prefill_insert)."""
+        """Rotary embedding and insert of a prompt in one pass over q, k and v (moa_rope_prefill_insert).  None: more
+        than one launch holds, nothing was done; the two steps take more."""
         from ..kernels.rotary import _cos_sin_strides
 
         device = k.device
@@ -376,6 +379,8 @@ class StaticCircularCache:
         if rc != 0 and fresh:   # refused: the rings are what an update that failed would have left
             kc.zero_()
             vc.zero_()
+        if rc == _lib.MOA_ERR_UNSUPPORTED:
+            return None
         _lib.check(rc)
         if layer_idx == 0:
             self.cache_position += N

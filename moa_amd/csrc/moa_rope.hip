@@ -593,7 +593,9 @@ extern "C" int moa_rope_prefill_insert(const void* q, const void* k, const void*
   const int64_t slices = (walked + kRingRows - 1) / kRingRows;
   const int64_t ring_blocks = (int64_t)B * Hkv * slices;
   const int64_t blocks = unit_blocks + ring_blocks;
-  if (units > 0x7fffffffLL || blocks > 0x7fffffffLL) return fail(MOA_ERR_UNSUPPORTED, "%s: too many tokens", who);
+  // a launch holds less than 2^32 threads
+  if (units > 0x7fffffffLL || blocks * kRopeThreads > 0xffffffffLL)
+    return fail(MOA_ERR_UNSUPPORTED, "%s: too many tokens", who);
   hipStream_t st = (hipStream_t)stream;
   RingArgs ra = {(const char*)v, v_strides[0] * eb, v_strides[1] * eb, v_strides[2] * eb, (char*)kc, (char*)vc, mask_cache,
                  update_index, circ_head, circ_size, static_size, nullptr, nullptr, nullptr, kv_len, sumC};

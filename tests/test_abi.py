@@ -76,6 +76,18 @@ def test_prefill_size_limits_without_gpu(lib):
         assert rc == _lib.MOA_ERR_UNSUPPORTED and "too many work items" in _lib.last_error(), (B, Hq, N)
 
 
+def test_prompt_start_size_limit_without_gpu(lib):
+    """A prompt of more tokens than one launch's 2^32 threads cover is refused before anything is launched (the Python
+    path then takes the separate steps)."""
+    from moa_amd import _lib
+    p = ctypes.c_void_p(0x10000)   # never dereferenced: the call fails on the sizes
+    H, D, S = 8, 32, 1 << 25
+    st, cs = (ctypes.c_int64 * 4)(H * S * D, D, H * D, 1), (ctypes.c_int64 * 3)(0, D, 1)
+    rc = lib.moa_rope_prefill_insert(p, p, p, p, p, st, st, st, st, st, p, p, cs, p, p, p, p, p, p, p, p, None, 0, None, 0,
+                                     0, 1, H, H, S, D, 1024, 128, 0, _lib.MOA_DTYPE_F16, None)
+    assert rc == _lib.MOA_ERR_UNSUPPORTED and "too many tokens" in _lib.last_error()
+
+
 def test_no_cpu_path():
     from moa_amd import StaticCircularCache, _lib, mixture_of_sparse_attention
     q = torch.zeros(1, 2, 1, 128, dtype=torch.float16)

@@ -193,6 +193,28 @@ def test_later_pieces_of_a_prompt_in_one_launch(dev, H, Hq, padded):
             assert torch.equal(getattr(one, name)[0], getattr(two, name)[0]), (name, step)
 
 
+@pytest.mark.parametrize("fresh", [True, False])
+def test_prompt_too_large_for_one_launch_takes_the_two_steps(dev, monkeypatch, fresh):
+    """What one launch refuses for its size is done in two steps, with nothing left behind by the attempt."""
+    from moa_amd import StaticCircularCache, _lib
+    B, H, D, S, dtype = 2, 8, 64, 100, torch.float16
+    one, two = (StaticCircularCache([[128] * H], static_size=[[64] * H], batch_size=B, head_dim=D, device=dev, dtype=dtype)
+                for _ in range(2))
+    q, k, v = (_rand((B, S, H, D), dtype, i).to(dev).transpose(1, 2) for i in range(3))
+    cos, sin = (t.to(dev) for t in rope_cos_sin(torch.arange(S)[None, :], D, dtype=dtype))
+    if not fresh:
+        for c in (one, two):
+            c.rope_update(q, k, v, cos, sin, 0)
+    want = one.rope_update(q, k, v, cos, sin, 0)
+    monkeypatch.setattr(_lib.load(), "moa_rope_prefill_insert", lambda *a: _lib.MOA_ERR_UNSUPPORTED)
+    got = two.rope_update(q, k, v, cos, sin, 0)
+    for a, b in zip(got, want):
+        assert a.stride() == b.stride() and _same_bits(a, b)
+    for name in ("key_cache", "value_cache", "mask_cache", "cache_update_index", "cache_valid_length"):
+        assert torch.equal(getattr(one, name)[0], getattr(two, name)[0]), name
+    assert one.get_seq_length() == two.get_seq_length() and one.cache_position == two.cache_position
+
+
 def test_fused_step_feeds_the_decode_kernel(dev):
     """rope_update (one launch) + mixture_of_sparse_attention against the oracle's decode on the
     oracle's cache: what a decoder layer sees."""
