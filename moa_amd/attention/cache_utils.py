@@ -181,8 +181,8 @@ class StaticCircularCache:
         if self.update_cache_content and self.key_cache[layer_idx] is None:
             shape = (self.batch_size, self.layer_cache_size[layer_idx], self.head_dim)
             make = torch.zeros if zeroed else torch.empty
-            self.key_cache[layer_idx] = make(shape, dtype=self.dtype, device=device)
-            self.value_cache[layer_idx] = make(shape, dtype=self.dtype, device=device)
+            rings = [make(shape, dtype=self.dtype, device=device) for _ in range(2)]   # both or, out of memory, none
+            self.key_cache[layer_idx], self.value_cache[layer_idx] = rings
         self._ready_on[layer_idx] = device
         self._step_args[layer_idx] = None
 
@@ -338,6 +338,8 @@ class StaticCircularCache:
                 or q.stride(1) >= q.stride(2) or k.stride(1) >= k.stride(2)
                 or self.batch_size * N >= 2 ** 31 or self.layer_cache_size[layer_idx] >= 2 ** 31):
             return False
+        if not (self.cache_update_index[layer_idx].is_contiguous() and self.cache_valid_length[layer_idx].is_contiguous()):
+            return False
         # rings that exist, or that this call allocates
         return (self.key_cache[layer_idx] is None) == (self._ready_on[layer_idx] is None)
 
@@ -365,7 +367,6 @@ class StaticCircularCache:
         fresh = self.key_cache[layer_idx] is None
         self._to_device(layer_idx, device, zeroed=False)
         upd = self.cache_update_index[layer_idx]
-        assert upd.is_contiguous() and self.cache_valid_length[layer_idx].is_contiguous()
         kc, vc = self.key_cache[layer_idx], self.value_cache[layer_idx]
         rc = lib.moa_rope_prefill_insert(
             q.data_ptr(), k.data_ptr(), v_in.data_ptr(), q_out.data_ptr(), k_out.data_ptr(), _lib.i64_array(q.stride()),

@@ -167,3 +167,25 @@ def test_cache_summary_columns():
     assert model["cache_size"] == (pytest.approx(7616 / 6), 128, 2624) and model["static_size"] == (64, 64, 64)
     text = format_cache_summary(layers, model)
     assert text.splitlines()[0].split()[:2] == ["layer_id", "raw_cache_size"] and "circular_size" in text
+
+
+@pytest.mark.parametrize("zeroed", [True, False])
+def test_rings_are_allocated_both_or_not_at_all(monkeypatch, zeroed):
+    """Out of memory at the second ring: the layer stays without rings and takes them at the next try."""
+    from moa_amd import StaticCircularCache
+    cache = StaticCircularCache([[4, 6]], static_size=[[1, 2]], batch_size=1, head_dim=8)
+    name = "zeros" if zeroed else "empty"
+    make, calls = getattr(torch, name), []
+
+    def failing(*args, **kwargs):
+        calls.append(args)
+        if len(calls) == 2:
+            raise torch.OutOfMemoryError("second ring")
+        return make(*args, **kwargs)
+
+    monkeypatch.setattr(torch, name, failing)
+    with pytest.raises(torch.OutOfMemoryError):
+        cache._to_device(0, torch.device("cpu"), zeroed=zeroed)
+    assert cache.key_cache[0] is None and cache.value_cache[0] is None
+    cache._to_device(0, torch.device("cpu"), zeroed=zeroed)
+    assert cache.key_cache[0].shape == cache.value_cache[0].shape == (1, 10, 8)
