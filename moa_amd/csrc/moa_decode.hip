@@ -925,11 +925,26 @@ static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_
 // launches that do not pipeline their loads (kDecPipeFrom).  GPU time with the merge launch and without, 32 rings of
 // 128: 256 rows 7.5 -> 5.9 us, 2048 rows 12.6 -> 11.6 us, batch 4 of 4096 rows (1152 chunks) 49.8 -> 49.6 us, batch 8
 // 90.0 -> 92.4 us; a step called from Python, bound by its launches, 24 -> 21 us.
-// Grouped kernel: only below kNtBytes, where a step called from Python waits for its launches (24 -> 21 us).  Above, the
-// GPU is behind, a chunk is alone on its CU and nothing hides the merge: batch 4 of 8 rings at 32k tokens, 8 query
-// heads, 43.9 us a layer with the merge launch, 46.2 us without.  The last work-group of a ring merges G query heads
-// alone, so their partials are bounded too: 32 chunks of 8 heads (256) 20.1 -> 22.0 us, 16 of 8 (128) 20.0 -> 20.6 us.
-constexpr int64_t kMergeInsidePartials = 128;
+// Skewed rings do not change that: one of 100000 rows beside seven short ones 30.5 -> 25.4 us.
+// Grouped kernel: only below kNtBytes (above, a chunk is alone on its CU and nothing hides the merge: batch 4 of 8 rings
+// at 32k tokens, 8 query heads, 43.9 us a layer with the merge launch, 46.2 us without), and by what the last work-group
+// of a ring has to do alone.  A wave merges a query head at a time, so up to four heads take one round over the ring's
+// chunks and five to eight take two; 16 chunks are asked for at once.  GPU time with the merge launch -> without:
+//   G = 4, 8 rings of 128:  2 chunks a ring 12.8 -> 11.2 us, 8 13.5 -> 12.1, 16 14.4 -> 13.9, 32 17.9 -> 18.0
+//   G = 2, 8 rings of 128:  8 chunks 12.7 -> 11.4, 16 13.6 -> 13.0, 32 17.3 -> 17.1
+//   G = 7, 4 rings of 64:   4 chunks 11.1 -> 10.5, 8 11.2 -> 10.8, 16 11.1 -> 11.2, 32 11.8 -> 13.5
+//   G = 8, 8 rings of 128:  2 chunks 14.1 -> 14.1, 8 14.7 -> 15.2, 16 15.6 -> 17.1
+// Up to four heads the launch saved is GPU time won.  With more it is about even up to 8 chunks, and what is won is the
+// host's time for a launch (a step called from Python waits for its launches: batch 34, one ring of 7 chunks, 8 heads of
+// 64, 25.6 -> 22.0 us).
+// The rings of a plan are not equally long, and the host knows only how many rows they hold together.  So there are two
+// bounds: on the chunks of an average ring, where the gain ends, and on the chunks of a whole batch row, which is the
+// most its largest ring can have.  One ring with nearly all rows is then the worst case: G = 4, 60 chunks 14.2 -> 15.2 us;
+// G = 8, 20 chunks 14.0 -> 16.0 us; without the second bound 235 chunks 26.6 -> 31.7 us and 29.0 -> 48.9 us.
+struct MergeInside {
+  int64_t ring_chunks, row_chunks;   // at most: of a ring of average size, of a batch row
+};
+static inline MergeInside merge_inside_up_to(int G) { return G <= kGqaWaves ? MergeInside{16, 64} : MergeInside{8, 24}; }
 
 constexpr int kSmallChunk = kChunk / 2;   // chunk length of the one-query-head kernel when the grid is small
 
@@ -983,16 +998,15 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
                              float* part_ml, const int64_t* head_start, const int64_t* head_valid, int B,
                              int H, int G, int64_t sumC, float sm_scale, unsigned* counters, hipStream_t st) {
   const int cap = (int)decode_cap(sumC, H);   // partial slots per batch row the workspace was sized for
-  // Chunk policy.  Chunks of kGqaChunk rows when they give at least half of the CUs a chunk: measured at
-  // the 70B shape (8 rings per batch row, 104 k rows) with one fixed length, 49.8 us per call at batch 4
-  // with 2048-row chunks, 53.3 with 1024, 62.3 with 512 -- a chunk start costs three dependent memory
-  // latencies (ring index, query rows, first tiles).  Below that (batch 1 and 2 at that shape: 54 and 108
-  // chunks) every batch row is split evenly into its share of 256 chunks instead: 25.8 against 32.4 us at
-  // batch 1, 33.5 against 36-39 us at batch 2.  From batch 3 on the even split gains nothing (one round of
-  // 256 chunks of 1664 rows at batch 4: 50.6-52.2 us against 50.4-51.8 us with 213 chunks of 2048; whole
-  // rounds of even chunks at batch 6 to 64: between 4 % faster and 7 % slower): those launches stream at
-  // the rate of the large batches already.  The host does not know how full the rings are; it plans with
-  // their capacity.
+  // Chunk policy.  Chunks of kGqaChunk rows when they give at least half of the CUs a chunk: a chunk start costs three
+  // dependent memory latencies (ring index, query rows, first tiles).  Measured at the 70B shape (8 rings per batch
+  // row, 104 k rows) with one fixed length, before the copies were non-temporal: 49.8 us per call at batch 4 with
+  // 2048-row chunks, 53.3 with 1024, 62.3 with 512.  Below that (batch 1 and 2 at that shape: 54 and 108 chunks) every
+  // batch row is split evenly into its share of 256 chunks instead: 25.8 against 32.4 us at batch 1, 33.5 against 36-39
+  // us at batch 2.  From batch 3 on one even round of 256 chunks gains nothing at that shape, with the present copies
+  // either: 35.4 us with 2048-row chunks against 48.2 us at batch 3, 41.5 against 42.0 at 4, 71.0 against 78.8 at 6, 76.2
+  // against 75.1 at 8, 149.9 against 200.8 at 16.  The host does not know how full the rings are; it plans with their
+  // capacity.
   const int64_t fixed_chunks = (int64_t)B * (sumC / kGqaChunk + (H + 1) / 2);
   int64_t target = 0;   // 0: chunks of kGqaChunk rows
   if (fixed_chunks <= 128) {
@@ -1003,8 +1017,10 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
   const int64_t chunks = target > 0 ? target + H : (sumC + kGqaChunk - 1) / kGqaChunk + H;
   const int64_t chunk_rows = target > 0 ? (sumC / target > kEvenMinChunk ? sumC / target : kEvenMinChunk) : kGqaChunk;
   const int64_t ring_chunks = (sumC / H + chunk_rows - 1) / chunk_rows;   // of a ring of average size
+  const int64_t row_chunks = (sumC + chunk_rows - 1) / chunk_rows;        // of a ring that is all of the batch row
   const bool nt = read_nontemporal(B, sumC, D);
-  if (nt || ring_chunks * G > kMergeInsidePartials) counters = nullptr;
+  const MergeInside limit = merge_inside_up_to(G);
+  if (nt || ring_chunks > limit.ring_chunks || row_chunks > limit.row_chunks) counters = nullptr;
   int64_t bx = (256 * kGqaBlocksPerCu + B - 1) / B;   // in practice one work-group per chunk (see kGqaBlocksPerCu)
   if (bx > chunks) bx = chunks;
   if (bx > cap) bx = cap;

@@ -102,3 +102,43 @@ def test_a_graph_with_counters_of_its_own(dev, G):
         torch.cuda.synchronize()
         assert torch.equal(recorded, want), i
         assert not counters.any(), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,D,B,sizes", [
+    (4, 128, 1, [2048] * 8),                    # 64 chunks of a batch row: the most that merges inside
+    (4, 128, 1, [2048] * 7 + [2056]),           # 65
+    (2, 64, 1, [16000, 100, 100]),              # nearly all of them in one ring
+    (3, 64, 1, [4096]),                         # 16 of an average ring
+    (3, 64, 1, [4100]),                         # 17
+    (8, 128, 1, [768] * 8),                     # two rounds of query heads: 24
+    (8, 128, 1, [768] * 7 + [776]),             # 25
+    (5, 64, 2, [5500, 100, 100, 100, 100]),
+    (7, 64, 1, [2048]),                         # 8 of an average ring
+    (7, 64, 1, [2052]),                         # 9
+    (6, 128, 11, [1536] * 4),
+    (8, 64, 13, [4400, 300, 300, 300]),
+    (8, 64, 40, [700, 64]),                     # chunks of 2048 rows
+])
+def test_lines_of_the_merge_inside(dev, G, D, B, sizes):
+    """On both sides of every line of the rule for merging inside, with rings of equal length and one ring that is
+    nearly all of the batch row: the same bits as with the merge launch, and zeroed counters, call after call."""
+    from moa_amd import _lib
+    lib = _lib.load()
+    q, kc, vc, start, valid = _rings(dev, G, D, B, sizes)
+    Hq, Hkv, sumC = q.shape[1], len(sizes), kc.shape[1]
+    need = lib.moa_decode_workspace_bytes(B, Hq, Hkv, D, sumC)
+    counters = torch.zeros(B * Hkv, dtype=torch.int32, device=dev)
+    for step in range(3):
+        outs = []
+        for n in (0, counters.numel()):
+            ws = torch.full((need,), 0xff, dtype=torch.uint8, device=dev)   # NaN partials: none is read unwritten
+            o = torch.full_like(q, float("nan"))
+            rc = lib.moa_decode_fwd_counted(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), o.data_ptr(), ws.data_ptr(), need,
+                                            counters.data_ptr(), n, start.data_ptr(), valid.data_ptr(), B, Hq, Hkv, D,
+                                            sumC, D ** -0.5, _lib.MOA_DTYPE_F16, _lib.current_stream_ptr(dev))
+            assert rc == 0, _lib.last_error()
+            outs.append(o)
+        assert torch.isfinite(outs[0]).all() and torch.equal(outs[1], outs[0]), step
+        assert not counters.any(), step
+        valid = (valid * 2) // 3   # rings that are not full
