@@ -263,13 +263,14 @@ int moa_cache_prefill_insert(const void* k, const void* v,
 /*
  * Rotary embedding of a prompt and its bulk insert in one pass: what moa_rope_fwd
  * (q -> q_out, k -> k_out) followed by moa_cache_prefill_insert (of k_out and v) give,
- * bit for bit.  Replaces modeling_llama.py:252 and :262 for a prompt.
+ * bit for bit (of two NaN that meet, either may come out).  Replaces modeling_llama.py:252 and :262 for a prompt.
  * q, k, v, q_out, k_out: host strides (order B,H,S,D; D stride 1); outputs do not overlap
  * inputs.  kc, vc are required, max_cache_size is the largest head's segment
  * (static_size + circ_size); with zero_rest != 0 (rings just allocated, not filled) the
  * rows of every head's segment that the insert does not write are set to zero.
  * workspace: as for moa_cache_prefill_insert.  Hkv <= 64; head rows of 64, 128, 256 or 512 bytes; at most
- * 2^31 - 1 tokens (B * S) and cache rows.
+ * 2^31 - 1 cache rows.  A prompt that does not fit one launch of 2^32 threads (from 2^25 tokens of few, small rows on)
+ * is MOA_ERR_UNSUPPORTED, with nothing launched.
  */
 int moa_rope_prefill_insert(const void* q, const void* k, const void* v, void* q_out,
                             void* k_out, const int64_t* q_strides, const int64_t* k_strides,
