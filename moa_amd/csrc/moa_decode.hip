@@ -43,7 +43,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 constexpr int kDecThreads = 256;
 constexpr int kDecWaves = kDecThreads / 64;
 constexpr int kBatch = 8;           // wave-wide loads in flight per tensor
-constexpr int kMaxHeads = 256;     // heads per batch row the LDS prefix covers
+constexpr int kMaxHeads = 256;     // heads per batch row: four to a lane of the wave that finds the chunks
 constexpr float kLog2e = 1.4426950408889634f;
 
 struct F16 {};
@@ -915,8 +915,12 @@ constexpr int kDecPipeFrom = 4;
 // layers, ordinary against non-temporal loads: one query head per ring, D = 128, 67 MB a layer 21.2 -> 19.7 us,
 // 268 MB 55.4 -> 51.0 us, 2.1 GB 382 -> 337 us (6.4 TB/s); eight query heads 134 MB 36.1 -> 34.7 us, 268 MB
 // 57.5 -> 53.9 us.  Below, the rings of some layers do stay cached and ordinary loads win: 16.8 MB a layer
-// 14.1 against 15.1 us.  (The same single layer of 134 MB read over and over, which stays cached whole, loses
-// 7 %; a decoder has more layers than one.)
+// 14.1 against 15.1 us.
+// The launch knows its own layer only.  Where the rings of all layers together stay cached over a step (up to about
+// 270 MB, and nothing else read in between: no decoder, whose weights pass through the cache too, but a loop over one
+// or a few layers) non-temporal loads lose: one layer of 134 MB, eight query heads, 34.5 -> 37.2 us, of 268 MB 56.4 ->
+// 58.6; of 67 MB, seven heads of 64, 25.8 -> 26.8; four of 67 MB, one head, 19.4 -> 20.2.  Four layers of 134 MB already
+// win, 37.1 -> 34.9 us, and single ones from 537 MB on, 106.5 -> 93.7 us.
 constexpr int64_t kNtBytes = (int64_t)64 << 20;
 static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_t)B * sumC * D * 4 >= kNtBytes; }
 

@@ -43,8 +43,8 @@ def _arrival_counters(device: torch.device, stream: int) -> Optional[Tensor]:
     """The zeroed counters of moa_decode_fwd_counted, one set per (device, stream) like the workspace; every call leaves
     them zeroed.  A call that is being recorded into a graph takes none (two launches, the same bits): a replay may run
     beside eager calls of this stream or beside other graphs recorded on it, and where two launches count in the same
-    place a lost count stays for good."""
-    if torch.cuda.is_current_stream_capturing():
+    place a lost count stays for good.  (Stream 0 cannot be recorded and is not asked, which saves its calls 0.5 us.)"""
+    if stream != 0 and torch.cuda.is_current_stream_capturing():
         return None
     key = (device.index or 0, stream)
     counters = _counters.get(key)

@@ -14,6 +14,8 @@ def test_a_recorded_call_takes_no_shared_counters(monkeypatch):
     assert M._arrival_counters(dev, stream) is kept
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     assert M._arrival_counters(dev, stream) is None
+    monkeypatch.setitem(M._counters, (0, 0), kept)   # the stream that cannot be recorded
+    assert M._arrival_counters(dev, 0) is kept
 
 
 @pytest.fixture(scope="module")
