@@ -68,6 +68,17 @@ __device__ __forceinline__ int64_t next_slot(int64_t idx, bool is_circular, int6
   return py_mod(off, csz) + ch;
 }
 
+// Inclusive sum over the lanes of a wave, in six DPP steps (no LDS); lane 63 has the total.
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 inside rows of 16 lanes
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
 // DPP lane exchanges inside a row of 16 lanes.
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float x) {

@@ -127,16 +127,6 @@ static_assert(chunks_of(0, 512) == 0 && chunks_of(1, 512) == 1 && chunks_of(512,
 static_assert(share_end(share_begin((1 << 22) - 1, 512, 3, 128), 128, kMaxRows) == 0x7fffffffu);
 static_assert(share_end(share_begin((1 << 22) - 1, 512, 2, 128), 128, kMaxRows) == 0x7fffff80u);
 
-// Inclusive sum over the lanes of a wave, in six DPP steps (no LDS); lane 63 has the total.
-__device__ __forceinline__ int wave_scan(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 inside rows of 16 lanes
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-  return x;
-}
 __device__ __forceinline__ int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll

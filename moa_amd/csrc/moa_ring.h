@@ -24,6 +24,15 @@ __device__ __forceinline__ HeadRing load_ring(const int64_t* update_index, const
   return g;
 }
 
+// the ring that lane h of the wave holds (h is uniform, and kv0 the same in all lanes)
+__device__ __forceinline__ int64_t value_of_lane(int64_t x, int h) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, h);
+  return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), h) << 32) | lo);
+}
+__device__ __forceinline__ HeadRing ring_of_lane(const HeadRing& x, int h) {
+  return {value_of_lane(x.upd0, h), value_of_lane(x.ch, h), value_of_lane(x.csz, h), value_of_lane(x.s, h), x.kv0};
+}
+
 // py_mod(off, csz); offsets and rings of ordinary size take the 32-bit division (a fifth of the instructions).
 __device__ __forceinline__ int64_t ring_mod(int64_t off, int64_t csz) {
   if ((uint64_t)off < (1ull << 32) && (uint64_t)(csz - 1) < (1ull << 31)) return (int64_t)((uint32_t)off % (uint32_t)csz);

@@ -287,7 +287,10 @@ struct Coef<EBF16> {
 // the v row that belongs into each and zero the rows no token goes to, so no fill runs in front; in rings in use they
 // walk the tokens that can be kept, so that a short piece of a prompt does not cost a walk over rings of any size
 // (16 tokens into 32 x 8 rings of 8192 rows: 50.6 us by rows, 7.3 by tokens, 10.6 in two steps; 64 tokens into 8 x 32
-// rings of 4096: 31.0, 8.0, 13.5).
+// rings of 4096: 31.0, 8.0, 13.5).  What a head walks is cut into slices that are numbered head by head, and every wave
+// finds its slice's head with one scan over the heads, a lane each: a grid of as many slices for every head as the
+// largest has is mostly empty work-groups where heads differ (64 tokens into new rings of 8 x 16384 and 8 x 31 x 256
+// rows: 151.6 us, 34.8 by slices; fill and two steps 32.7).
 // Batch 8, 32 heads of 128, 16384 tokens, bf16, a third of the tokens kept (4.9 GB): 970 us (5.1 TB/s) against 743 us
 // rotary + 87 us fill + 268 us insert in separate launches; 64 query heads on 8 rings, batch 1: 103 us.
 struct RingArgs {
@@ -322,17 +325,31 @@ __device__ __forceinline__ void store16(char* p, u32x4 x) {
 template <typename E, int P /* chunk pairs per row: 64 % P == 0 */, bool FRESH, bool NT>
 __global__ __launch_bounds__(kRopeThreads) void rope_insert_kernel(
     RopeTensor tq, RopeTensor tk, const char* __restrict__ cos, const char* __restrict__ sin, int64_t cs_sb,
-    int64_t cs_sn, RingArgs ra, int B, int Hq, int Hkv, int N, unsigned ring_blocks, int ring_slices /* per head */,
+    int64_t cs_sn, RingArgs ra, int B, int Hq, int Hkv, int N, unsigned ring_blocks,
+    int row_blocks /* ring work-groups per batch row */, int64_t walked /* rows or tokens a head walks at most */,
     int pieces /* of a token's heads */) {
   constexpr int half_bytes = P * 16;
   if (blockIdx.x < ring_blocks) {
-    const unsigned bh = blockIdx.x / (unsigned)ring_slices, slice = blockIdx.x % (unsigned)ring_slices;
-    const int b = (int)(bh / (unsigned)Hkv), h = (int)(bh % (unsigned)Hkv);
-    const HeadRing g = load_ring(ra.update_index, ra.circ_head, ra.circ_size, ra.static_size, ra.kv_len, bh, h);
+    const int b = (int)(blockIdx.x / (unsigned)row_blocks), head_lane = threadIdx.x & 63;
     const int64_t nv = ra.n_valid ? (int64_t)ra.n_valid[b] : (int64_t)N;
-    const int64_t count = FRESH ? g.s + g.csz : candidate_count(g, nv);
-    const int64_t first = g.ch - g.s, rows = min(count, (int64_t)(slice + 1) * kRingRows);
+    HeadRing mine = {0, 0, 0, 0, ra.kv_len};   // of head `head_lane`
+    int slices = 0;
+    if (head_lane < Hkv) {
+      mine = load_ring(ra.update_index, ra.circ_head, ra.circ_size, ra.static_size, ra.kv_len, (int64_t)b * Hkv + head_lane,
+                       head_lane);
+      const int64_t count = min(FRESH ? mine.s + mine.csz : candidate_count(mine, nv), walked);
+      slices = (int)((max(count, (int64_t)0) + kRingRows - 1) / kRingRows);
+    }
+    const int upto = wave_scan(slices);   // slices of heads 0 .. head_lane
+    const int total = __builtin_amdgcn_readlane(upto, 63);
     const int lane = threadIdx.x % kRopeRowLanes;
+    const int i = (int)(blockIdx.x % (unsigned)row_blocks);   // one slice to a work-group: a loop takes 130 registers more
+    if (i >= total) return;
+    const int h = __popcll(__ballot(upto <= i));   // heads whose slices all lie in front of i
+    const int slice = i - (h > 0 ? __builtin_amdgcn_readlane(upto, h - 1) : 0);
+    const HeadRing g = ring_of_lane(mine, h);
+    const int64_t count = min(FRESH ? g.s + g.csz : candidate_count(g, nv), walked);
+    const int64_t first = g.ch - g.s, rows = min(count, (int64_t)(slice + 1) * kRingRows);
     const int row_bytes = 2 * half_bytes, units = row_bytes / 16;
     for (int64_t r0 = (int64_t)slice * kRingRows + threadIdx.x / kRopeRowLanes; r0 < rows;
          r0 += kRopeRowsPerBlock * kRingAtOnce) {
@@ -590,8 +607,11 @@ extern "C" int moa_rope_prefill_insert(const void* q, const void* k, const void*
   const int64_t unit_blocks = (units + kRopeThreads / 64 - 1) / (kRopeThreads / 64);
   // with rings in use: no more candidates than tokens, or than a head's rows + 1 (see candidate())
   const int64_t walked = zero_rest ? max_cache_size : max_cache_size < S ? max_cache_size + 1 : S;
-  const int64_t slices = (walked + kRingRows - 1) / kRingRows;
-  const int64_t ring_blocks = (int64_t)B * Hkv * slices;
+  // slices of a batch row: of all heads alike, or where heads differ as many as their rows or tokens together make
+  const int64_t slices = (int64_t)Hkv * ((walked + kRingRows - 1) / kRingRows);
+  const int64_t together = (sumC + (zero_rest ? 0 : Hkv)) / kRingRows + Hkv;
+  const int64_t row_blocks = slices < together ? slices : together;
+  const int64_t ring_blocks = (int64_t)B * row_blocks;
   const int64_t blocks = unit_blocks + ring_blocks;
   // a launch holds less than 2^32 threads
   if (units > 0x7fffffffLL || blocks * kRopeThreads > 0xffffffffLL)
@@ -618,7 +638,7 @@ extern "C" int moa_rope_prefill_insert(const void* q, const void* k, const void*
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kRopeThreads), 0, st, tq, tk, (const char*)cos,
                        (const char*)sin, cs_strides[0] * eb, cs_strides[1] * eb, ra, B, Hq, Hkv, S, (unsigned)ring_blocks,
-                       (int)slices, pieces);
+                       (int)row_blocks, walked, pieces);
     return check_launch(who);
   };
   const bool nt = (int64_t)B * S * (Hq + Hkv) * D * eb >= kRopeNtBytes;

@@ -120,6 +120,25 @@ def test_padded_prompts_past_a_part_of_the_mask_scan(dev, S):
     _check(one.rope_update(*args, 0, mask)[:2], _two_steps(two, *args, mask), one, two, S)
 
 
+@pytest.mark.parametrize("H", [1, 5, 64])
+@pytest.mark.parametrize("S", [2, 900])
+def test_heads_of_very_different_rings(dev, H, S):
+    """One ring that is most of the batch row, first, last and in the middle, among rings of a few rows, of less than
+    one and of exactly one slice, and heads without a ring: every slice finds its head."""
+    B, Hq, D, dtype = 3, 64, 64, torch.float16
+    for at in {0, H // 2, H - 1}:
+        sizes = [[3, 64, 65, 128, 129, 256, 1][h % 7] for h in range(H)]
+        static = [min(64, n) if h % 2 else n // 2 for h, n in enumerate(sizes)]
+        sizes[at], static[at] = 5001, 64
+        for mask in (None, _padding(dev, B, S)):
+            one, two = (_cache(dev, dtype, B, D, sizes, static) for _ in range(2))
+            for piece in range(2):   # new rings, then rings in use
+                args = _inputs(dev, dtype, B, Hq, H, S, D, at=piece * S, seed=piece)
+                if H > 1:
+                    assert one._prompt_fits_one_launch(*args, 0, mask)
+                _check(one.rope_update(*args, 0, mask)[:2], _two_steps(two, *args, mask), one, two, (at, piece))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("S", [8191, 8193])   # around 256 MiB of q and k, from which on they pass the caches by
 def test_large_prompts_of_both_load_kinds(dev, dtype, S):
