@@ -302,8 +302,12 @@ struct RingArgs {
   const int32_t *tok_of, *rank_of, *n_valid;   // with an attention mask, else null
   int64_t kv_len, sumC;
 };
-constexpr int kRingRows = 256;      // segment rows, or tokens, per work-group of the ring part
 constexpr int kRingAtOnce = 4;      // rows a group of 16 lanes has under way
+// Rows, or tokens, per work-group of the ring part: 16 KiB of them, once around at 256-byte rows.  Long slices are a chain
+// of memory latencies in launches too small to hide them: 2 tokens into new rings of 32 x 512 rows 12.8 us with 256 rows
+// to a slice, 9.6 with 128, 8.2 with 64 (in two steps 14); 517 tokens 13.7, 10.7, 8.9; prompt of 8 x 16384 tokens 1002, 984,
+// 983; 128-byte rows lose with shorter ones (100 tokens into 32 x 32 rings of 2048: 131, 146, 171).
+constexpr __host__ __device__ int ring_rows(int pairs /* chunk pairs per row */) { return pairs >= 8 ? 64 : 512 / pairs; }
 // Wave-wide row loads a wave has under way, and all it does.  Measured at the two sizes above: 2: 970 and 103 us,
 // 4: 1000 and 106 us, 8: 950 and 110 us; a whole token (q and k heads in turn) to a wave: 960 and 118 us.
 constexpr int kRopeAtOnce = 2;
@@ -330,6 +334,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_insert_kernel(
     int pieces /* of a token's heads */) {
   constexpr int half_bytes = P * 16;
   if (blockIdx.x < ring_blocks) {
+    constexpr int kRingRows = ring_rows(P);
     const int b = (int)(blockIdx.x / (unsigned)row_blocks), head_lane = threadIdx.x & 63;
     const int64_t nv = ra.n_valid ? (int64_t)ra.n_valid[b] : (int64_t)N;
     HeadRing mine = {0, 0, 0, 0, ra.kv_len};   // of head `head_lane`
@@ -608,8 +613,9 @@ extern "C" int moa_rope_prefill_insert(const void* q, const void* k, const void*
   // with rings in use: no more candidates than tokens, or than a head's rows + 1 (see candidate())
   const int64_t walked = zero_rest ? max_cache_size : max_cache_size < S ? max_cache_size + 1 : S;
   // slices of a batch row: of all heads alike, or where heads differ as many as their rows or tokens together make
-  const int64_t slices = (int64_t)Hkv * ((walked + kRingRows - 1) / kRingRows);
-  const int64_t together = (sumC + (zero_rest ? 0 : Hkv)) / kRingRows + Hkv;
+  const int slice_rows = ring_rows(pairs);
+  const int64_t slices = (int64_t)Hkv * ((walked + slice_rows - 1) / slice_rows);
+  const int64_t together = (sumC + (zero_rest ? 0 : Hkv)) / slice_rows + Hkv;
   const int64_t row_blocks = slices < together ? slices : together;
   const int64_t ring_blocks = (int64_t)B * row_blocks;
   const int64_t blocks = unit_blocks + ring_blocks;

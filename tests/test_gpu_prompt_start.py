@@ -139,6 +139,18 @@ def test_heads_of_very_different_rings(dev, H, S):
                 _check(one.rope_update(*args, 0, mask)[:2], _two_steps(two, *args, mask), one, two, (at, piece))
 
 
+@pytest.mark.parametrize("S,rows", [(64, 16383), (64, 16384), (4095, 16384), (4096, 16384)])
+def test_first_prompts_shorter_than_the_new_rings(dev, S, rows):
+    """On both sides of 64 MiB of rings and of a quarter of their rows: filled and walked by tokens, or walked by rows."""
+    B, H, D, dtype = 1, 8, 128, torch.bfloat16
+    sizes, static = [rows] * H, [64] * H
+    junk = [torch.full((B, rows * H, D), float("nan"), dtype=dtype, device=dev) for _ in range(4)]
+    del junk   # memory that the rings may be given
+    one, two = (_cache(dev, dtype, B, D, sizes, static) for _ in range(2))
+    args = _inputs(dev, dtype, B, H, H, S, D)
+    _check(one.rope_update(*args, 0, None)[:2], _two_steps(two, *args, None), one, two, (S, rows))
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("S", [8191, 8193])   # around 256 MiB of q and k, from which on they pass the caches by
 def test_large_prompts_of_both_load_kinds(dev, dtype, S):
