@@ -29,8 +29,8 @@ class StaticCircularCache:
     first tokens forever (the sinks) while the rest is a ring holding the most
     recent tokens.  ``update`` takes ``[batch_size, num_heads, seq_len, head_dim]``.
 
-    The index tables are complete when the constructor returns; the masks are zeroed, and the rings allocated, on
-    the streams that are current at construction and at a layer's first update.
+    The index tables and masks are complete when the constructor returns; the rings are allocated on the stream that
+    is current at a layer's first update.
 
     Unlike the reference this class does not derive from
     ``transformers.Cache``: the installed transformers release changed that base
@@ -68,10 +68,7 @@ class StaticCircularCache:
         self._max_static_size: List[int] = [max(x) for x in static_size]
 
         # The int64 tables of all layers are laid out in one buffer that goes to the device in one copy (a copy and a
-        # wait for the GPU per table cost 50 us a layer); the tables are views of it.  The copy is waited for: the tables
-        # are complete when the constructor returns, on whatever stream they are read first.  The wait costs a call that
-        # would run ahead of the GPU 10 us (prompt of 517 tokens, two layers, 204 -> 213 us a pass) to 50 us (8 x 16384
-        # tokens, 1031 -> 1081 us).
+        # wait for the GPU per table cost 50 us a layer); the tables are views of it.
         place = torch.empty(0, device=device).device
         if place.type == "cuda" and torch.cuda.is_current_stream_capturing():
             raise RuntimeError("StaticCircularCache: a cache cannot be made while a HIP graph is being captured")
@@ -92,8 +89,8 @@ class StaticCircularCache:
             rows[3] = ends[:-1] + rows[1]
             rows[4:4 + 2 * B] = ends[:-1]   # where every head starts, and the slot of its next token
             rows[4 + 2 * B:] = 0
-        tables = packed.to(device=place).split(
-            [n for h in heads for n in (h, h, h, h, B * h, B * h, B * h, h + 1)])
+        on_device = torch.empty(packed.shape, dtype=torch.int64, device=place)
+        tables = on_device.split([n for h in heads for n in (h, h, h, h, B * h, B * h, B * h, h + 1)])
         self.cache_max_length: List[Tensor] = list(tables[0::8])
         self.static_cache_size: List[Tensor] = list(tables[1::8])
         self.circular_cache_size: List[Tensor] = list(tables[2::8])
@@ -115,6 +112,11 @@ class StaticCircularCache:
         self.value_cache: List[Optional[Tensor]] = [None] * self.num_layers
         self.mask_cache: List[Tensor] = [
             torch.zeros(batch_size, n, dtype=torch.int64, device=device) for n in self.layer_cache_size]
+        # Tables and masks are complete on return, on whatever stream they are read first.  The copy waits for the work in
+        # front of it; it comes last, so that little is left to do between the wait and the next launch.  A pass without
+        # the wait and with it: prompt of 517 tokens, two layers, 206 and 215 us; 8 x 16384 tokens, one layer, 1008 and
+        # 1048 us (1054 with the copy where the tables are made).
+        on_device.copy_(packed)
 
     def __getstate__(self):
         """Copies (copy.deepcopy, pickling) do not take the per-layer call arguments along: those hold
