@@ -203,7 +203,7 @@ def test_index_tables_are_complete_on_return(dev):
     def make(device):
         return StaticCircularCache(cache_size, static_size=static, batch_size=2, head_dim=64, device=device)
 
-    names = ("cache_max_length", "static_cache_size", "circular_cache_size", "circular_cache_head_index",
+    names = ("mask_cache", "cache_max_length", "static_cache_size", "circular_cache_size", "circular_cache_head_index",
              "cache_head_start_index", "cache_update_index", "cache_valid_length", "head_index")
     want = make("cpu")
     other = torch.cuda.Stream()
