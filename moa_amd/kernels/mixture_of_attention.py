@@ -21,36 +21,41 @@ from moa_amd import _lib
 BLOCK_M = 64
 BLOCK_N = 64
 
-_workspaces: Dict[Tuple[int, int, str], Tensor] = {}
-
-
-def _workspace(device: torch.device, nbytes: int, tag: str, stream: int) -> Tensor:
-    """A per-(device, stream) scratch buffer that only ever grows, so steady
-    state calls allocate nothing."""
-    key = (device.index or 0, stream, tag)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
-    return ws
-
-
 _N_COUNTERS = 16384   # (batch row, ring) pairs up to which a decode launch may merge inside
-_counters: Dict[Tuple[int, int], Tensor] = {}
 
 
-def _arrival_counters(device: torch.device, stream: int) -> Optional[Tensor]:
-    """The zeroed counters of moa_decode_fwd_counted, one set per (device, stream) like the workspace; every call leaves
-    them zeroed.  A call that is being recorded into a graph takes none (two launches, the same bits): a replay may run
-    beside eager calls of this stream or beside other graphs recorded on it, and where two launches count in the same
-    place a lost count stays for good.  (Stream 0 cannot be recorded and is not asked, which saves its calls 0.5 us.)"""
-    if stream != 0 and torch.cuda.is_current_stream_capturing():
-        return None
+class _DecodeScratch:
+    """What the decode calls of one (device, stream) share: a workspace that only ever grows and the zeroed counters of
+    moa_decode_fwd_counted, which every call leaves zeroed.  Steady-state calls allocate nothing and take the addresses
+    from here."""
+    __slots__ = ("ws", "ws_ptr", "ws_bytes", "counters", "counters_ptr")
+
+    def __init__(self) -> None:
+        self.ws = self.ws_ptr = self.counters = self.counters_ptr = None
+        self.ws_bytes = 0
+
+
+_scratch: Dict[Tuple[int, int], _DecodeScratch] = {}
+
+
+def _decode_scratch(device: torch.device, stream: int, nbytes: int) -> Tuple[int, int, Optional[int]]:
+    """Address and size of the workspace, address of the counters or None.  A call that is being recorded into a graph
+    takes no counters (two launches, the same bits): a replay may run beside eager calls of this stream or beside other
+    graphs recorded on it, and where two launches count in the same place a lost count stays for good.  (Stream 0 cannot
+    be recorded and is not asked, which saves its calls 0.5 us.)"""
     key = (device.index or 0, stream)
-    counters = _counters.get(key)
-    if counters is None:
-        counters = _counters[key] = torch.zeros(_N_COUNTERS, dtype=torch.int32, device=device)
-    return counters
+    s = _scratch.get(key)
+    if s is None:
+        s = _scratch[key] = _DecodeScratch()
+    if s.ws_bytes < nbytes:
+        s.ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
+        s.ws_ptr, s.ws_bytes = s.ws.data_ptr(), s.ws.numel()
+    if stream != 0 and torch.cuda.is_current_stream_capturing():
+        return s.ws_ptr, s.ws_bytes, None
+    if s.counters is None:
+        s.counters = torch.zeros(_N_COUNTERS, dtype=torch.int32, device=device)
+        s.counters_ptr = s.counters.data_ptr()
+    return s.ws_ptr, s.ws_bytes, s.counters_ptr
 
 
 def _require_gpu(t: Tensor, who: str) -> None:
@@ -162,12 +167,10 @@ def moa_decode(
     lib = _lib.load()
     need = lib.moa_decode_workspace_bytes(B, Hq, Hkv, D, sumC)
     stream = _lib.current_stream_ptr(dev)
-    ws = _workspace(dev, need, "decode", stream)
-    counters = _arrival_counters(dev, stream)
-    rc = lib.moa_decode_fwd_counted(q3.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ws.data_ptr(), ws.numel(),
-                                    None if counters is None else counters.data_ptr(),
-                                    0 if counters is None else _N_COUNTERS, hs.data_ptr(), hv.data_ptr(), B, Hq, Hkv, D,
-                                    sumC, float(sm_scale), _lib.dtype_code(q.dtype), stream)
+    ws, ws_bytes, counters = _decode_scratch(dev, stream, need)
+    rc = lib.moa_decode_fwd_counted(q3.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ws, ws_bytes, counters,
+                                    _N_COUNTERS, hs.data_ptr(), hv.data_ptr(), B, Hq, Hkv, D, sumC, float(sm_scale),
+                                    _lib.dtype_code(q.dtype), stream)
     _lib.check(rc)
     return o
 

@@ -6,16 +6,17 @@ import torch
 
 def test_a_recorded_call_takes_no_shared_counters(monkeypatch):
     from moa_amd.kernels import mixture_of_attention as M
-    stream = -12345   # no stream of this value exists
-    kept = torch.zeros(4, dtype=torch.int32)
-    monkeypatch.setitem(M._counters, (0, stream), kept)   # as an eager call on that stream leaves them
-    dev = torch.device("cuda:0")
+    dev, stream = torch.device("cuda:0"), -12345   # no stream of this value exists
+    kept = M._DecodeScratch()   # as an eager call on that stream leaves it
+    kept.ws, kept.ws_ptr, kept.ws_bytes = torch.zeros(512, dtype=torch.uint8), 4096, 512
+    kept.counters, kept.counters_ptr = torch.zeros(4, dtype=torch.int32), 8192
+    monkeypatch.setitem(M._scratch, (0, stream), kept)
+    monkeypatch.setitem(M._scratch, (0, 0), kept)   # the stream that cannot be recorded
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
-    assert M._arrival_counters(dev, stream) is kept
+    assert M._decode_scratch(dev, stream, 512) == (4096, 512, 8192)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
-    assert M._arrival_counters(dev, stream) is None
-    monkeypatch.setitem(M._counters, (0, 0), kept)   # the stream that cannot be recorded
-    assert M._arrival_counters(dev, 0) is kept
+    assert M._decode_scratch(dev, stream, 512) == (4096, 512, None)
+    assert M._decode_scratch(dev, 0, 512) == (4096, 512, 8192)
 
 
 @pytest.fixture(scope="module")
@@ -53,7 +54,7 @@ def test_replays_beside_eager_calls_of_the_capture_stream(dev, G):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(stream):
         step()
-        counters = M._counters[(0, stream.cuda_stream)]
+        counters = M._scratch[(0, stream.cuda_stream)].counters
         with torch.cuda.graph(graph, stream=stream):
             recorded = step()
         for i in range(4):
