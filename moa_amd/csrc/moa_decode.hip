@@ -928,9 +928,9 @@ static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_
 //   G = 2, 8 rings of 128:  8 chunks 12.7 -> 11.4, 16 13.6 -> 13.0, 32 17.3 -> 17.1
 //   G = 7, 4 rings of 64:   4 chunks 11.1 -> 10.5, 8 11.2 -> 10.8, 16 11.1 -> 11.2, 32 11.8 -> 13.5
 //   G = 8, 8 rings of 128:  2 chunks 14.1 -> 14.1, 8 14.7 -> 15.2, 16 15.6 -> 17.1
-// Up to four heads the launch saved is GPU time won.  With more it is about even up to 8 chunks, and what is won is the
-// host's time for a launch (a step called from Python waits for its launches: batch 34, one ring of 7 chunks, 8 heads of
-// 64, 25.6 -> 22.0 us).
+// Up to four heads the launch saved is GPU time won, up to 32 chunks.  With more heads it is about even up to 8, and up
+// to 16 costs less than the host's time for a launch, which is what is won there (a step called from Python waits for
+// its launches: batch 34, one ring of 7 chunks, 8 heads of 64, 25.6 -> 22.0 us).
 // The rings of a plan are not equally long, and the host knows only how many rows they hold together.  So there are two
 // bounds: on the chunks of an average ring, where the gain ends, and on the chunks of a whole batch row, which is the
 // most its largest ring can have.  One ring with nearly all rows is then the worst case: G = 4, 60 chunks 14.2 -> 15.2 us;
@@ -938,7 +938,7 @@ static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_
 struct MergeInside {
   int64_t ring_chunks, row_chunks;   // at most: of a ring of average size, of a batch row
 };
-static inline MergeInside merge_inside_up_to(int G) { return G <= kGqaWaves ? MergeInside{16, 64} : MergeInside{8, 24}; }
+static inline MergeInside merge_inside_up_to(int G) { return G <= kGqaWaves ? MergeInside{32, 64} : MergeInside{16, 24}; }
 
 constexpr int kSmallChunk = kChunk / 2;   // chunk length of the one-query-head kernel when the grid is small
 

@@ -112,13 +112,13 @@ def test_a_graph_with_counters_of_its_own(dev, G):
     (4, 128, 1, [2048] * 8),                    # 64 chunks of a batch row: the most that merges inside
     (4, 128, 1, [2048] * 7 + [2056]),           # 65
     (2, 64, 1, [16000, 100, 100]),              # nearly all of them in one ring
-    (3, 64, 1, [4096]),                         # 16 of an average ring
-    (3, 64, 1, [4100]),                         # 17
+    (3, 64, 1, [8192]),                         # 32 of an average ring
+    (3, 64, 1, [8200]),                         # 33
     (8, 128, 1, [768] * 8),                     # two rounds of query heads: 24
     (8, 128, 1, [768] * 7 + [776]),             # 25
     (5, 64, 2, [5500, 100, 100, 100, 100]),
-    (7, 64, 1, [2048]),                         # 8 of an average ring
-    (7, 64, 1, [2052]),                         # 9
+    (7, 64, 1, [4096]),                         # 16 of an average ring
+    (7, 64, 1, [4100]),                         # 17
     (6, 128, 11, [1536] * 4),
     (8, 64, 13, [4400, 300, 300, 300]),
     (8, 64, 40, [700, 64]),                     # chunks of 2048 rows
