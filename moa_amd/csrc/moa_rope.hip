@@ -291,7 +291,7 @@ struct Coef<EBF16> {
 // finds its slice's head with one scan over the heads, a lane each: a grid of as many slices for every head as the
 // largest has is mostly empty work-groups where heads differ (64 tokens into new rings of 8 x 16384 and 8 x 31 x 256
 // rows: 151.6 us, 34.8 by slices; fill and two steps 32.7).
-// Batch 8, 32 heads of 128, 16384 tokens, bf16, a third of the tokens kept (4.9 GB): 970 us (5.1 TB/s) against 743 us
+// Batch 8, 32 heads of 128, 16384 tokens, a third of the tokens kept (4.9 GB): 983 us (5.0 TB/s) against 743 us
 // rotary + 87 us fill + 268 us insert in separate launches; 64 query heads on 8 rings, batch 1: 103 us.
 struct RingArgs {
   const char* v;
@@ -308,8 +308,8 @@ constexpr int kRingAtOnce = 4;      // rows a group of 16 lanes has under way
 // to a slice, 9.6 with 128, 8.2 with 64 (in two steps 14); 517 tokens 13.7, 10.7, 8.9; prompt of 8 x 16384 tokens 1002, 984,
 // 983; 128-byte rows lose with shorter ones (100 tokens into 32 x 32 rings of 2048: 131, 146, 171).
 constexpr __host__ __device__ int ring_rows(int pairs /* chunk pairs per row */) { return pairs >= 8 ? 64 : 512 / pairs; }
-// Wave-wide row loads a wave has under way, and all it does.  Measured at the two sizes above: 2: 970 and 103 us,
-// 4: 1000 and 106 us, 8: 950 and 110 us; a whole token (q and k heads in turn) to a wave: 960 and 118 us.
+// Wave-wide row loads a wave has under way, and all it does.  Measured at the two sizes above, with slices of 256 rows:
+// 2: 970 and 103 us, 4: 1000 and 106 us, 8: 950 and 110 us; a whole token (q and k heads in turn) to a wave: 960 and 118.
 constexpr int kRopeAtOnce = 2;
 // From this many bytes of q and k on they are read, and their rotated copies written, non-temporally: the copies
 // are past what the last-level cache (256 MB) could keep for the attention that reads them next, and lines held for
