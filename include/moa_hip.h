@@ -133,7 +133,8 @@ int moa_decode_fwd(const void* q, const void* kc, const void* vc, void* o,
  * chunks make that the faster way.  counters: uint32 [n_counters] in device memory, all
  * zero before the first call and left at zero by every call; used when n_counters >=
  * B * Hkv and else ignored, like NULL (the call is then moa_decode_fwd).  Calls that may
- * overlap on a GPU need counters, like workspaces, of their own.
+ * overlap on a GPU, replays of a graph among them, need counters, like workspaces, of their
+ * own: a count that an overlap loses stays, and later calls merge too early or never.
  */
 int moa_decode_fwd_counted(const void* q, const void* kc, const void* vc, void* o,
                            void* workspace, size_t workspace_bytes,
@@ -266,7 +267,7 @@ int moa_cache_prefill_insert(const void* k, const void* v,
  * bit for bit (of two NaN that meet, either may come out).  Replaces modeling_llama.py:252 and :262 for a prompt.
  * q, k, v, q_out, k_out: host strides (order B,H,S,D; D stride 1); outputs do not overlap
  * inputs.  kc, vc are required, max_cache_size is the largest head's segment
- * (static_size + circ_size); with zero_rest != 0 (rings just allocated, not filled) the
+ * (static_size + circ_size; segments are disjoint); with zero_rest != 0 (rings just allocated, not filled) the
  * rows of every head's segment that the insert does not write are set to zero.
  * workspace: as for moa_cache_prefill_insert.  Hkv <= 64; head rows of 64, 128, 256 or 512 bytes; at most
  * 2^31 - 1 cache rows.  A prompt that does not fit one launch of 2^32 threads (from 2^25 tokens of few, small rows on)

@@ -26,7 +26,7 @@
 //   * grouped-query attention (G = Hq / Hkv query heads per ring, which the
 //     reference does not have): the G query rows of a ring share every K/V
 //     row that a wave loads, so the cache is still read once.  This kernel is
-//     written for any G but instantiated for G = 1 only; G = 2, 4, 8 run on the
+//     written for any G but instantiated for G = 1 only; G = 2 to 8 run on the
 //     matrix cores (decode_gqa_kernel below).
 #include "moa_mfma.h"
 

@@ -12,9 +12,10 @@
 // each of the two products and one after the sum.  The kernels round at the
 // same three places, so their results are bit-identical to that evaluation.
 //
-// Both kernels are HBM/latency bound byte work: 128-bit accesses, no LDS.  One
+// All kernels are HBM/latency bound byte work: 128-bit accesses, no LDS.  One
 // thread owns a PAIR of 16-byte chunks (elements e..e+7 and e+D/2..e+D/2+7 of
-// one head row), reads both and writes both, which makes in-place use safe.
+// one head row), reads both and writes both, which makes in-place use safe in
+// the rotation alone.
 #include "moa_ring.h"
 
 // Every product and sum below is rounded on its own, as torch does.  This file must be compiled
