@@ -64,6 +64,17 @@ __device__ __forceinline__ void async_copy16(const void* base, uint32_t byte_off
         : "v"(byte_off), "s"(base), "s"(__builtin_amdgcn_readfirstlane(lds_addr))
         : "memory");
 }
+// a and b after the upper half of the wave of a and the lower half of b have changed places
+__device__ __forceinline__ u32x2 swap_halves(uint32_t a, uint32_t b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  return u32x2{r[0], r[1]};
+}
+// x of the lane's twin in the other half of the wave (lane ^ 32)
+__device__ __forceinline__ float other_half(float x) {
+  const uint32_t a = __builtin_bit_cast(uint32_t, x);
+  const u32x2 r = swap_halves(a, a);   // the lower half's x in both halves, the upper half's
+  return __builtin_bit_cast(float, (threadIdx.x & 32) ? r.x : r.y);
+}
 // max of a value with its twin in the other half of the wave (lane ^ 32), without going through LDS
 __device__ __forceinline__ float max_with_other_half(float x) {
   float a = x, b = x;
@@ -84,13 +95,6 @@ __device__ __forceinline__ void wait_vm(int n) {
   else if (n == 2) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
   else if (n == 1) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-}
-
-// The same for a count known at compile time.
-template <int N>
-__device__ __forceinline__ void wait_vm_exact() {
-  static_assert(N >= 0 && N < 64, "vmcnt holds 6 bits");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
 // Work-group barrier WITHOUT the memory fence of __syncthreads(): the fence would make every wave
@@ -115,15 +119,26 @@ struct IC {
   static constexpr int value = P;
 };
 
+// Accesses to device memory through a pointer that was an integer on the way (put together from LDS words): without the
+// address space the compiler takes flat instructions, which count as LDS accesses too and make it wait for everything.
+__device__ __forceinline__ u32x4 global_load16(const void* p) {
+  typedef const u32x4 __attribute__((address_space(1))) * global_ptr;
+  return *(global_ptr)(uintptr_t)p;
+}
+__device__ __forceinline__ void global_store16(void* p, u32x4 v) {
+  typedef u32x4 __attribute__((address_space(1))) * global_ptr;
+  *(global_ptr)(uintptr_t)p = v;
+}
+__device__ __forceinline__ void global_store8(void* p, u32x2 v) {
+  typedef u32x2 __attribute__((address_space(1))) * global_ptr;
+  *(global_ptr)(uintptr_t)p = v;
+}
+
 // LDS accesses by 32-bit LDS byte address (a VGPR) plus a compile-time offset, so that the stage
 // and row selection of an operand costs no VALU instruction.
 __device__ __forceinline__ u32x4 lds_load16(uint32_t addr, int imm) {
   typedef u32x4 __attribute__((address_space(3))) * lds_u32x4_ptr;
   return *(lds_u32x4_ptr)(uintptr_t)(addr + imm);
-}
-__device__ __forceinline__ void lds_store8(uint32_t addr, u32x2 v) {
-  typedef u32x2 __attribute__((address_space(3))) * lds_u32x2_ptr;
-  *(lds_u32x2_ptr)(uintptr_t)addr = v;
 }
 // The transposing read: 4 consecutive rows of one 16-bit column out of a row-major LDS tile.  Within
 // each group of 16 lanes, lane i must point at (row0 + i/4, col0 + 4*(i%4)); it receives rows

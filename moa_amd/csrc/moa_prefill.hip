@@ -19,8 +19,8 @@
 //     (measured: 7 % of CU time at the benchmark shape);
 //   * wave 0 turns a queue ticket into an item descriptor (base pointers, tile
 //     schedule) once and leaves it in LDS; it does so for item i+1 a few
-//     iterations before item i ends, and item i's last iteration starts the
-//     first copies of item i+1;
+//     iterations before item i ends, and item i's last iteration asks for the
+//     Q rows and starts the first copies of item i+1;
 //   * a work-group walks the union of the live 64-key tiles of its four query
 //     blocks; a wave skips the math of a tile that is dead for ITS query block;
 //   * K and V tiles are copied global -> LDS asynchronously (no registers),
@@ -165,7 +165,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   uint32_t cst = (S - 1) * TILE_B;   // ring offset of the stage K(t+S-1) is copied into; V(t+S-2) goes one stage below
   uint32_t rst = 0;                  // ring offset of the stage K(t) is read from
   bool prefetched = false;           // the previous item has started this item's first copies
-  uint32_t q_touch = 0;              // landing place of the load that pulls the next item's Q rows into L2
+  u32x4 qf[KS];                      // Q rows of this wave
 
   // ---- the work queue ---------------------------------------------------------------------------
   // Wave 0 takes a ticket for the item after the one under way (from the own XCD's list while that has
@@ -214,6 +214,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
         unsigned out = 0;
         if (lane < 8) out = atomicAdd(&ap->queue->next[lane], 0u);
         const unsigned long long left = __ballot(lane < 8 && out < list_items(lane & 7));
+#pragma unroll 1
         for (int i = 1; i < 8; ++i) {
           const int x = (my_xcd + i) & 7;
           if (!((left >> x) & 1)) continue;
@@ -226,6 +227,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     }
     if (list < 0) {
       if (lane == 0) d[0] = -1;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       return;
     }
     const int nb = (N + kKV - 1) / kKV;
@@ -270,6 +272,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     const uint64_t ob = (uint64_t)(ap->o + b * ap->os.b + hq * ap->os.h);
     d[8] = (int)(uint32_t)kb; d[9] = (int)(uint32_t)(kb >> 32); d[10] = (int)(uint32_t)vb; d[11] = (int)(uint32_t)(vb >> 32);
     d[12] = (int)(uint32_t)qb; d[13] = (int)(uint32_t)(qb >> 32); d[14] = (int)(uint32_t)ob; d[15] = (int)(uint32_t)(ob >> 32);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // in LDS before this wave's next barrier
   };
   __syncthreads();   // the sorted heads
   if (threadIdx.x < 64) take(0);
@@ -349,26 +352,27 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   const int row0 = it.qt * kQRows + wave * kWRows;            // first query row of this wave
   const int64_t m_glob = row0 + mcol;                          // this lane's query row
 
-  // the Q rows are asked for first: theirs is the longest way (the other loads of an item were started by
-  // the item before it)
-  u32x4 qf[KS];              // Q fragment (B operand): Q[m][16*ks + 8*g .. +7]
-  if (n_tiles > 0) {
-    const uint16_t* qrow = it.qbase + m_glob * qs_n + 8 * g;
-    const bool ok = m_glob < N;
+  // Q fragment (B operand): Q[m][16*ks + 8*g .. +7]; rows past N repeat row N-1 (nothing of theirs is stored)
+  auto load_q = [&](const Item& i) __attribute__((always_inline)) {
+    const int64_t m_row = min((int64_t)i.qt * kQRows + wave * kWRows + mcol, (int64_t)N - 1);
+    const uint16_t* qrow = i.qbase + m_row * qs_n + 8 * g;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      u32x4 z = {0, 0, 0, 0};
-      qf[s] = ok ? *reinterpret_cast<const u32x4*>(qrow + 16 * s) : z;
-    }
-  }
+    for (int s = 0; s < KS; ++s) qf[s] = global_load16(qrow + 16 * s);
+  };
+  // the Q rows are asked for first: theirs is the longest way
+  if (!prefetched && n_tiles > 0) load_q(it);
+  auto pin_q = [&]() __attribute__((always_inline)) {   // the Q rows have landed: no wait of the compiler's behind this
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
+  };
 
-  // ---- async tile copies: wave w, copy i fills chunks [(w*LPW+i)*64, +64) of a stage --------
+  // ---- async tile copies: wave w, copy i fills chunks [(i*NW+w)*64, +64) of a stage --------
   const uint16_t* const kbase = it.kbase;   // uniform
   const uint16_t* const vbase = it.vbase;
   uint32_t koff[LPW], voff[LPW];
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
-    const int L = (wave * LPW + i) * 64 + lane;     // chunk position inside the stage
+    const int L = (i * NW + wave) * 64 + lane;     // chunk position inside the stage
     const int row = L / CPR, pos = L % CPR;
     koff[i] = 2u * ((uint32_t)(row * ks_n) + (uint32_t)((pos ^ ((row / RSH) % CPR)) * 8));   // bytes
     voff[i] = 2u * ((uint32_t)(row * vs_n) + (uint32_t)((pos ^ (4 * ((row / RSH) % (CPR / 4)))) * 8));
@@ -383,20 +387,20 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     const char* src = reinterpret_cast<const char*>(base) + (uint64_t)(uint32_t)j * tile_bytes;
     if (j != j_ragged) {
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) async_copy16(src, off[i], dst + i * 1024);
+      for (int i = 0; i < LPW; ++i) async_copy16(src, off[i], dst + i * NW * 1024);
     } else {
       const int last = N - 1 - j * kKV;
 #pragma unroll
       for (int i = 0; i < LPW; ++i) {
-        const int L = (wave * LPW + i) * 64 + lane;
+        const int L = (i * NW + wave) * 64 + lane;
         const int row = L / CPR, pos = L % CPR;
         const int sw = is_k ? ((row / RSH) % CPR) : (4 * ((row / RSH) % (CPR / 4)));
-        async_copy16(src, 2u * ((uint32_t)(min(row, last) * stride_n) + (uint32_t)((pos ^ sw) * 8)), dst + i * 1024);
+        async_copy16(src, 2u * ((uint32_t)(min(row, last) * stride_n) + (uint32_t)((pos ^ sw) * 8)), dst + i * NW * 1024);
       }
     }
   };
-  const uint32_t k_dst0 = lds_address(s_k) + wave * LPW * 1024;      // this wave's share of stage 0
-  const uint32_t v_dst0 = lds_address(s_v) + wave * LPW * 1024;
+  const uint32_t k_dst0 = lds_address(s_k) + wave * 1024;            // this wave's share of stage 0
+  const uint32_t v_dst0 = lds_address(s_v) + wave * 1024;
   // Starts the first copies, K(0..S-2) and V(0..S-3), of item ni into the stages from ring offset r0 on.
   auto start_copies = [&](const Item& ni, uint32_t r0) __attribute__((always_inline)) {
     int j = first_tile(ni);
@@ -407,18 +411,14 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
       j = next_tile_of(ni, j, i + 1);
     }
   };
-  constexpr int kPrefetchOps = (2 * S - 3) * LPW + 1;   // vector memory operations prefetch_next starts
-  // The item after this one (its descriptor is in the other slot): its first copies go out now, and one load per
-  // lane touches both cache lines of each of its Q rows so that the real Q loads of the next pass hit in L2.
-  // The touched word lands in q_touch, which is kept allocated until the next pass has waited for it.
+  // The item after this one (its descriptor is in the other slot): its Q rows and first copies are asked for now, so that
+  // they arrive beside the rest of this item.  The Q registers are free: this item's last Q.K^T is behind.
   auto prefetch_next = [&](uint32_t r0) __attribute__((always_inline)) {
     const Item ni = read_item(par ^ 1);
     if (ni.n_tiles < 0) sign_off();   // the count comes back while the last item is finished
     if (ni.n_tiles <= 0) return false;
+    load_q(ni);
     start_copies(ni, r0);
-    const int64_t m_row = min((int64_t)ni.qt * kQRows + wave * kWRows + mcol, (int64_t)N - 1);
-    const uint16_t* qrow = ni.qbase + m_row * qs_n + (D / 2) * g;
-    asm volatile("global_load_dword %0, %1, off" : "=v"(q_touch) : "v"(qrow) : "memory");
     return true;
   };
 
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
       uint16_t* orow = it.obase + m_glob * os_n;
       u32x2 z = {0, 0};
 #pragma unroll
-      for (int i = 0; i < D / 8; ++i) *reinterpret_cast<u32x2*>(orow + 8 * i + 4 * g) = z;
+      for (int i = 0; i < D / 8; ++i) global_store8(orow + 8 * i + 4 * g, z);
     }
     __syncthreads();   // the next descriptor, written by wave 0 above
     prefetched = false;
@@ -562,7 +562,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   };
   // mask + online softmax of tile j: st -> pf, updates m_run, l_run (and rescales oacc when needed;
   // every P.V issued so far belongs to earlier tiles and has completed in this wave's matrix phase)
-  auto softmax = [&](int j) __attribute__((always_inline)) {
+  auto softmax = [&](int j, bool first) __attribute__((always_inline)) {
     if (j == mbw) {   // causal mask on the diagonal tile
       int thr = (wave & 1) * kWRows + mcol - 4 * g;   // row inside the 64-row block, minus the lane's column base
       asm volatile("" : "+v"(thr));                  // keeps the 32 compares in this branch instead of 32 hoisted lane masks
@@ -593,9 +593,10 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     // stands, and their sum tells whether that was good enough.  A lane's 32 weights are >= 0, so a sum of
     // at most 2^8 bounds each of them by 2^8 (the 16-bit types hold that with room to spare); a larger
     // sum, or the first live tile (the reference is still -inf and the sum is inf or NaN; the file is
-    // compiled without NaN semantics, so that case is asked for by name), takes the path below.
-    weights();
-    if (__builtin_expect(__any(m_run == -INFINITY || psum[0] + psum[1] > kRescaleLimit), 0)) {
+    // compiled without NaN semantics, so that case is asked for by name), takes the path below.  The item's
+    // first step goes there at once.
+    if (!first) weights();
+    if (first || __builtin_expect(__any(m_run == -INFINITY || psum[0] + psum[1] > kRescaleLimit), 0)) {
       float mx = st[0][0];
 #pragma unroll
       for (int nt = 0; nt < 2; ++nt)
@@ -656,7 +657,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     if (grp == 1) { wait_vm(n_wait); phase_barrier(); }
     // ---------------- softmax phase ----------------
     if (lc) {
-      softmax(jt[0]);
+      softmax(jt[0], kFirst);
     } else if (lp) {   // the next matrix phase this wave runs must add nothing for a dead tile
 #pragma unroll
       for (int i = 0; i < 16; ++i) pf[i] = 0;
@@ -668,21 +669,20 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     jt[S - 1] = next_tile_of(it, jt[S - 1], t + S);
     if (grp == 0) { wait_vm(n_wait); phase_barrier(); }
   };
-  wait_vm(0);
-  // the Q loads have landed too; pin that fact here so that the compiler does not put its own
-  // vmcnt(0) wait at their first use inside the loop, where it would also wait for the copies
-#pragma unroll
-  for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
+  // Q and the first copies have landed: those of an item that the one before it started were waited for there
+  if (!prefetched) {
+    wait_vm(0);
+    pin_q();
+  }
 #pragma unroll
   for (int s = 0; s < KS; ++s) qf[s] ^= u32x4{q_sign, q_sign, q_sign, q_sign};
-  asm volatile("" : "+v"(q_touch));   // the touch of the previous pass has landed as well
   phase_barrier();               // K(0..2) and V(0..1) are in LDS
   iteration(0, IC<1>{});   // no P.V yet (and no V stage to read)
-  {
-    int t = 1;
-    for (; t < t_take; ++t) iteration(t, IC<0>{});
-    if (wave == 0 && t_take >= 1) take(par ^ 1);
-    for (; t < n_tiles; ++t) iteration(t, IC<0>{});
+  for (int t = 1, stop = min(max(t_take, 1), n_tiles);;) {
+    for (; t < stop; ++t) iteration(t, IC<0>{});
+    if (t == t_take && wave == 0) take(par ^ 1);
+    if (t >= n_tiles) break;
+    stop = n_tiles;
   }
 
   // ---- iteration n_tiles: P.V of the last tile; the next item's first copies start here.
@@ -696,50 +696,35 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   advance();
   if (grp == 0) phase_barrier();
 
-  // ---- epilogue: O[m][d] = O^T[d][m] / l, written as whole rows ---------------------------------
-  // A lane holds 8-byte pieces of one row; stored as they are, a wave's store touches 32 rows with 16 bytes
-  // each.  The rows go through LDS instead, 16 at a time, into this wave's quarter of one of the two V
-  // stages that are free now (V(n_tiles-1)'s, which every wave has finished reading at the barrier above, and
-  // the one after it; the next item's V(0), V(1) are in the other two), 16-byte chunks XOR-permuted like the
-  // K tiles; then 16 lanes store one row of 2 D bytes.  The repeated copies of the last two iterations may
-  // still be under way into these stages: they are older than everything prefetch_next started.
-  if (prefetched) wait_vm_exact<kPrefetchOps>(); else wait_vm(0);
+  // ---- epilogue: O[m][d] = O^T[d][m] / l ---------------------------------------------------------
+  // A lane holds 8-byte pieces of one row; the halves of the wave swap them so that it holds 16 bytes in a row, and two
+  // lanes store 32.  Through LDS whole rows could be stored, but the way there and back costs more than the stores of
+  // 32-byte pieces.  With the Q rows of the next item asked for an iteration earlier, the accesses through flat pointers
+  // gone and a third of the code (every part of the queue was compiled in eight times): 4 x 8192 tokens, 32 heads of 128,
+  // 1237 -> 1209 us; 8192 tokens of 64-element heads 194.9 -> 183.6; 32768 tokens, 64 heads, 8453 -> 8340.
   {
-    const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+    const float l_tot = l_run + other_half(l_run);
     const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
-    const uint32_t stage = (rst + (2 + (wave >> 2)) * TILE_B) & (kRing - 1);
-    const uint32_t slice = lds_address(s_v) + stage + (wave & 3) * (TILE_B / 4);
-    const int wrow = mcol & 15;
-    const uint32_t wr = slice + wrow * ROW_B + 8 * g;
-    const uint32_t wswz = (uint32_t)((wrow / RSH) % CPR);
+    u32x4 rows[DT][2];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      if ((mcol >> 4) == r) {
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int gi = 0; gi < 4; ++gi) {
-            u32x2 w;
-            w.x = T::pack_rne(oacc[dt][4 * gi + 0] * inv, oacc[dt][4 * gi + 1] * inv);
-            w.y = T::pack_rne(oacc[dt][4 * gi + 2] * inv, oacc[dt][4 * gi + 3] * inv);
-            lds_store8(wr + ((uint32_t)(4 * dt + gi) ^ wswz) * 16, w);
-          }
+      for (int p = 0; p < 2; ++p) {
+        const f32x16& a = oacc[dt];
+        const u32x2 lo = swap_halves(T::pack_rne(a[8 * p + 0] * inv, a[8 * p + 1] * inv), T::pack_rne(a[8 * p + 4] * inv, a[8 * p + 5] * inv));
+        const u32x2 hi = swap_halves(T::pack_rne(a[8 * p + 2] * inv, a[8 * p + 3] * inv), T::pack_rne(a[8 * p + 6] * inv, a[8 * p + 7] * inv));
+        rows[dt][p] = u32x4{lo.x, hi.x, lo.y, hi.y};
+        asm volatile("" : "+v"(rows[dt][p]));
       }
-      constexpr int kReads = 16 * CPR / 64;   // 16 rows of CPR chunks, 64 lanes
-      u32x4 rowv[kReads];
+    // what the next item has been asked for lands here, before the stores: behind them it would wait for them too
+    wait_vm(0);
+    pin_q();
+    if (m_glob < N) {
+      uint16_t* const orow = it.obase + m_glob * os_n + 8 * g;
 #pragma unroll
-      for (int i = 0; i < kReads; ++i) {
-        const int idx = i * 64 + lane;
-        const int row = idx / CPR, c = idx % CPR;
-        rowv[i] = lds_load16(slice + row * ROW_B + ((uint32_t)c ^ (uint32_t)((row / RSH) % CPR)) * 16, 0);
-      }
+      for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int i = 0; i < kReads; ++i) {
-        const int idx = i * 64 + lane;
-        const int row = idx / CPR, c = idx % CPR;
-        const int64_t m_out = row0 + 16 * r + row;
-        if (wave_has_rows && m_out < N) *reinterpret_cast<u32x4*>(it.obase + m_out * os_n + 8 * c) = rowv[i];
-      }
+        for (int p = 0; p < 2; ++p) global_store16(orow + 32 * dt + 16 * p, rows[dt][p]);
     }
   }
   }   // item loop
