@@ -90,7 +90,7 @@ struct PrefillArgs {
   Strides4 qs, ks, vs, os;
   const int64_t *sink_blocks, *local_blocks;   // spans per kv head: blocks, or tokens with span_shift = 6
   int span_shift;
-  PrefillQueue* queue;   // null: one item per work-group, by its place in the grid
+  PrefillQueue* queue;
   int BH, Hq, group, N, n_qtiles;
   int per_head, Hkv;   // (BH / Hq) * group pairs per kv head in the sorted list; Hq / group
   float scale_log2_signed;
@@ -111,6 +111,183 @@ __device__ __forceinline__ DivMod divmod_small(int x, int d) {
   return {q, r};
 }
 
+// ---- what a wave does with a tile -----------------------------------------------------------------
+// st: S^T of the current tile; oacc: O^T; pf: P^T of a tile, packed pairs, B-operand order; qf: Q fragments; k_ad, v_ad:
+// operand read addresses of the lane in the stages to read.
+// Matrix phase of one iteration: P.V of the previous tile and Q.K^T of the current one,
+// alternating, operands fetched kAhead MFMAs ahead.  k_ad / v_ad point at the stages to read.
+// Slot i: even -> P.V op i/2 (k-step (i/2)/DT, d tile (i/2)%DT), odd -> Q.K^T op i/2
+// (half (i/2)%2, k-step (i/2)/2).
+template <typename T, int D>
+__device__ __forceinline__ void tile_matrix(f32x16 (&st)[2], f32x16 (&oacc)[D / 32], const uint32_t (&pf)[16], const u32x4 (&qf)[D / 16],
+                                            const uint32_t (&k_ad)[D / 16], const uint32_t (&v_ad)[D / 32]) {
+  constexpr int KS = D / 16, DT = D / 32, ROW_B = D * 2;
+  constexpr int kSlots = 4 * DT + 2 * KS;
+  constexpr int kAhead = 6;
+  u32x4 opnd[kSlots];
+  auto fetch = [&](int i) __attribute__((always_inline)) {
+    const int j = i >> 1;
+    if (i & 1) {
+      opnd[i] = lds_load16(k_ad[j >> 1], (j & 1) * 32 * ROW_B);
+    } else {
+      const int tk = j / DT, dt = j % DT;
+      const u32x2 lo = lds_load_tr16(v_ad[dt], (16 * tk) * ROW_B);
+      const u32x2 hi = lds_load_tr16(v_ad[dt], (16 * tk + 8) * ROW_B);
+      opnd[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+  };
+  auto op = [&](int i) __attribute__((always_inline)) {
+    const int j = i >> 1;
+    if (i & 1) {
+      const int nt = j & 1, s = j >> 1;
+      if (s == 0) {
+        f32x16 z;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) z[e] = 0.f;
+        st[nt] = T::mfma(opnd[i], qf[0], z);
+      } else {
+        st[nt] = T::mfma(opnd[i], qf[s], st[nt]);
+      }
+    } else {
+      const int tk = j / DT, dt = j % DT;
+      const u32x4 bfrag = {pf[4 * tk], pf[4 * tk + 1], pf[4 * tk + 2], pf[4 * tk + 3]};
+      oacc[dt] = T::mfma(opnd[i], bfrag, oacc[dt]);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) fetch(i);
+#pragma unroll
+  for (int i = 0; i < kSlots; ++i) {
+    if (i + kAhead < kSlots) fetch(i + kAhead);
+    op(i);
+    __builtin_amdgcn_sched_barrier(0);   // keeps the operand reads kAhead MFMAs ahead of their use
+  }
+}
+
+// Q.K^T only (the first iteration)
+template <typename T, int D>
+__device__ __forceinline__ void tile_qk(f32x16 (&st)[2], const u32x4 (&qf)[D / 16], const uint32_t (&k_ad)[D / 16]) {
+  constexpr int KS = D / 16, ROW_B = D * 2;
+#pragma unroll
+  for (int nt = 0; nt < 2; ++nt) {
+    u32x4 kf[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) kf[s] = lds_load16(k_ad[s], nt * 32 * ROW_B);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) st[nt][i] = 0.f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) st[nt] = T::mfma(kf[s], qf[s], st[nt]);
+  }
+}
+
+// P.V only (the last iteration)
+template <typename T, int D>
+__device__ __forceinline__ void tile_pv(f32x16 (&oacc)[D / 32], const uint32_t (&pf)[16], const uint32_t (&v_ad)[D / 32]) {
+  constexpr int DT = D / 32, ROW_B = D * 2;
+#pragma unroll
+  for (int tk = 0; tk < 4; ++tk) {
+    u32x4 vf[DT];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      const u32x2 lo = lds_load_tr16(v_ad[dt], (16 * tk) * ROW_B);
+      const u32x2 hi = lds_load_tr16(v_ad[dt], (16 * tk + 8) * ROW_B);
+      vf[dt] = u32x4{lo.x, lo.y, hi.x, hi.y};
+    }
+    const u32x4 bfrag = {pf[4 * tk], pf[4 * tk + 1], pf[4 * tk + 2], pf[4 * tk + 3]};
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] = T::mfma(vf[dt], bfrag, oacc[dt]);
+  }
+}
+
+// mask + online softmax of tile j: st -> pf, updates m_run, l_run (and rescales oacc when needed;
+// every P.V issued so far belongs to earlier tiles and has completed in this wave's matrix phase)
+template <typename T, int D>
+__device__ __forceinline__ void tile_softmax(f32x16 (&st)[2], f32x16 (&oacc)[D / 32], uint32_t (&pf)[16], float& m_run, float& l_run,
+                                             bool diagonal, int thr /* row inside the 64-row block, minus the lane's column base */,
+                                             bool first, float scale_log2) {
+  constexpr int DT = D / 32;
+  constexpr float kRescaleLimit = 256.f;   // the reference exponent is raised (and O rescaled) when a lane's 32 weights sum to more
+  if (diagonal) {   // causal mask on the diagonal tile
+    asm volatile("" : "+v"(thr));   // keeps the 32 compares in this branch instead of 32 hoisted lane masks
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (nt * 32 + 8 * (i >> 2) + (i & 3) > thr) st[nt][i] = -INFINITY;
+  }
+  // Row sums are plain fp32 adds of the unrounded weights.  (v_dot2_f32_{f16,bf16} of the packed
+  // pair with a pair of ones would halve the instruction count, but those instructions stall the
+  // MFMA stream of the wave that shares the SIMD: measured 20 % slower per iteration.)
+  float psum[2];
+  auto weights = [&]() __attribute__((always_inline)) {
+    psum[0] = psum[1] = 0.f;
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[nt][i], scale_log2, -m_run));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[nt][i + 1], scale_log2, -m_run));
+        pf[nt * 8 + (i >> 1)] = T::pack_rne(p0, p1);
+        psum[0] += p0;
+        psum[1] += p1;
+      }
+  };
+  // The common case needs no row maximum: weights are formed against the reference exponent as it
+  // stands, and their sum tells whether that was good enough.  A lane's 32 weights are >= 0, so a sum of
+  // at most 2^8 bounds each of them by 2^8 (the 16-bit types hold that with room to spare); a larger
+  // sum, or the first live tile (the reference is still -inf and the sum is inf or NaN; the file is
+  // compiled without NaN semantics, so that case is asked for by name), takes the path below.  The item's
+  // first step goes there at once.
+  if (!first) weights();
+  if (first || __builtin_expect(__any(m_run == -INFINITY || psum[0] + psum[1] > kRescaleLimit), 0)) {
+    float mx = st[0][0];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[nt][i]);
+    mx = max_with_other_half(mx);
+    const float m_cand = mx * scale_log2;   // finite: a live tile has a visible key in every row
+    // The reference exponent stays an INTEGER: a weight is then 2^frac * 2^int, and its rounding to the
+    // storage type does not depend on the power of two, so the rounded weights (relative to the row's
+    // sum) do not depend on the tile order or on how far m_run lags behind the true maximum.
+    const float m_new = __builtin_ceilf(fmaxf(m_run, m_cand));
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    l_run *= alpha;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[t][i] *= alpha;
+    m_run = m_new;
+    weights();
+  }
+  l_run += psum[0] + psum[1];
+}
+
+// A lane's pieces of its row of O, normalised: 16 bytes each, the halves of the wave having swapped 8-byte ones.
+template <typename T, int D>
+__device__ __forceinline__ void tile_rows(u32x4 (&rows)[D / 32][2], const f32x16 (&oacc)[D / 32], float l_run) {
+  const float l_tot = l_run + other_half(l_run);
+  const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const f32x16& a = oacc[dt];
+      const u32x2 lo = swap_halves(T::pack_rne(a[8 * p + 0] * inv, a[8 * p + 1] * inv), T::pack_rne(a[8 * p + 4] * inv, a[8 * p + 5] * inv));
+      const u32x2 hi = swap_halves(T::pack_rne(a[8 * p + 2] * inv, a[8 * p + 3] * inv), T::pack_rne(a[8 * p + 6] * inv, a[8 * p + 7] * inv));
+      rows[dt][p] = u32x4{lo.x, hi.x, lo.y, hi.y};
+      asm volatile("" : "+v"(rows[dt][p]));
+    }
+}
+// p: the lane's row, 8 elements on for the upper half of the wave
+template <int D>
+__device__ __forceinline__ void store_rows(uint16_t* p, const u32x4 (&rows)[D / 32][2]) {
+#pragma unroll
+  for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) global_store16(p + 32 * dt + 16 * h, rows[dt][h]);
+}
+
 template <typename T, int D>
 __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_kernarg) {
   const PrefillArgsPtr a0 = (PrefillArgsPtr)__builtin_amdgcn_kernarg_segment_ptr();   // the argument above
@@ -126,7 +303,6 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   constexpr int TILE_B = kKV * D * 2; // bytes of one K or V stage (rows unpadded)
   constexpr int ROW_B = D * 2;
   constexpr int RSH = 16 / CPR;       // rows per 256 bytes of LDS (1 at D=128, 2 at D=64)
-  constexpr float kRescaleLimit = 256.f;   // the reference exponent is raised (and O rescaled) when a lane's 32 weights sum to more
   constexpr uint32_t kRing = kStages * TILE_B;   // bytes of one tensor's ring (a power of two)
   static_assert(4 * DT == 2 * KS, "P.V and Q.K^T have the same number of MFMAs per tile");
 
@@ -143,7 +319,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     const int64_t* sink_blocks = a0->sink_blocks;
     const int64_t* local_blocks = a0->local_blocks;
     const int shift = a0->span_shift;
-    if (Hkv <= kMaxSortedHeads && a0->queue != nullptr) {
+    if (Hkv <= kMaxSortedHeads) {
       for (int h = tid; h < Hkv; h += kPfThreads) {
         s_ns[h] = (int)max((int64_t)0, min((int64_t)nb, sink_blocks[h] >> shift));
         s_nl[h] = (int)max((int64_t)0, min((int64_t)nb, local_blocks[h] >> shift));
@@ -194,35 +370,27 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     unsigned sq = 0;
     const int lane = threadIdx.x & 63;
     int* d = s_item[slot];
-    if (ap->queue == nullptr) {   // an item to every work-group: its number is its place, and there is no second one
-      if (own_alive) {
-        list = blockIdx.x & 7;
-        sq = blockIdx.x >> 3;
-        own_alive = false;
-      }
-    } else {
-      if (own_alive) {
-        unsigned t = 0;
-        if (lane == 0) t = atomicAdd(&ap->queue->next[my_xcd], 1u);
-        sq = (unsigned)__builtin_amdgcn_readfirstlane((int)t);
-        if (sq < list_items(my_xcd)) list = my_xcd; else own_alive = false;
-      }
-      if (list < 0) {
-        // lanes 0 to 7 ask how far the lists are handed out: one round trip to memory, also where nothing is left (asking
-        // the lists one after the other is seven of them, in which the whole work-group stands still at the end of its
-        // last item)
-        unsigned out = 0;
-        if (lane < 8) out = atomicAdd(&ap->queue->next[lane], 0u);
-        const unsigned long long left = __ballot(lane < 8 && out < list_items(lane & 7));
+    if (own_alive) {
+      unsigned t = 0;
+      if (lane == 0) t = atomicAdd(&ap->queue->next[my_xcd], 1u);
+      sq = (unsigned)__builtin_amdgcn_readfirstlane((int)t);
+      if (sq < list_items(my_xcd)) list = my_xcd; else own_alive = false;
+    }
+    if (list < 0) {
+      // lanes 0 to 7 ask how far the lists are handed out: one round trip to memory, also where nothing is left (asking
+      // the lists one after the other is seven of them, in which the whole work-group stands still at the end of its
+      // last item)
+      unsigned out = 0;
+      if (lane < 8) out = atomicAdd(&ap->queue->next[lane], 0u);
+      const unsigned long long left = __ballot(lane < 8 && out < list_items(lane & 7));
 #pragma unroll 1
-        for (int i = 1; i < 8; ++i) {
-          const int x = (my_xcd + i) & 7;
-          if (!((left >> x) & 1)) continue;
-          unsigned t = 0;
-          if (lane == 0) t = atomicAdd(&ap->queue->next[x], 1u);
-          t = (unsigned)__builtin_amdgcn_readfirstlane((int)t);
-          if (t < list_items(x)) { list = x; sq = t; break; }
-        }
+      for (int i = 1; i < 8; ++i) {
+        const int x = (my_xcd + i) & 7;
+        if (!((left >> x) & 1)) continue;
+        unsigned t = 0;
+        if (lane == 0) t = atomicAdd(&ap->queue->next[x], 1u);
+        t = (unsigned)__builtin_amdgcn_readfirstlane((int)t);
+        if (t < list_items(x)) { list = x; sq = t; break; }
       }
     }
     if (list < 0) {
@@ -231,7 +399,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
       return;
     }
     const int nb = (N + kKV - 1) / kKV;
-    const bool sorted = Hkv <= kMaxSortedHeads && ap->queue != nullptr;
+    const bool sorted = Hkv <= kMaxSortedHeads;
     // A list walks its pairs one after the other, late (long) query tiles first.
     const DivMod rq = divmod_small((int)sq, n_qtiles);
     const int round = rq.q;
@@ -281,7 +449,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   // Thread 0 counts its work-group out once it has found the lists empty (it takes no ticket after that).
   unsigned left_before = ~0u;   // work-groups that were out already; ~0: not counted out yet
   auto sign_off = [&]() __attribute__((always_inline)) {
-    if (threadIdx.x == 0 && a0->queue != nullptr && left_before == ~0u) left_before = atomicAdd(&a0->queue->done, 1u);
+    if (threadIdx.x == 0 && left_before == ~0u) left_before = atomicAdd(&a0->queue->done, 1u);
   };
 
   // An item as the waves see it.
@@ -485,139 +653,9 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   float m_run = -INFINITY;   // reference exponent of exp2: an integer, ceil of the row max of scale_log2 * s when it was last set; a later max may pass it by < 8
   float l_run = 0.f;         // this lane's share of the running sum (the lane+32 twin holds the rest)
 
-  // Matrix phase of one iteration: P.V of the previous tile and Q.K^T of the current one,
-  // alternating, operands fetched kAhead MFMAs ahead.  k_ad / v_ad point at the stages to read.
-  // Slot i: even -> P.V op i/2 (k-step (i/2)/DT, d tile (i/2)%DT), odd -> Q.K^T op i/2
-  // (half (i/2)%2, k-step (i/2)/2).
-  auto matrix_phase = [&]() __attribute__((always_inline)) {
-    constexpr int kSlots = 4 * DT + 2 * KS;
-    constexpr int kAhead = 6;
-    u32x4 opnd[kSlots];
-    auto fetch = [&](int i) __attribute__((always_inline)) {
-      const int j = i >> 1;
-      if (i & 1) {
-        opnd[i] = lds_load16(k_ad[j >> 1], (j & 1) * 32 * ROW_B);
-      } else {
-        const int tk = j / DT, dt = j % DT;
-        const u32x2 lo = lds_load_tr16(v_ad[dt], (16 * tk) * ROW_B);
-        const u32x2 hi = lds_load_tr16(v_ad[dt], (16 * tk + 8) * ROW_B);
-        opnd[i] = u32x4{lo.x, lo.y, hi.x, hi.y};
-      }
-    };
-    auto op = [&](int i) __attribute__((always_inline)) {
-      const int j = i >> 1;
-      if (i & 1) {
-        const int nt = j & 1, s = j >> 1;
-        if (s == 0) {
-          f32x16 z;
-#pragma unroll
-          for (int e = 0; e < 16; ++e) z[e] = 0.f;
-          st[nt] = T::mfma(opnd[i], qf[0], z);
-        } else {
-          st[nt] = T::mfma(opnd[i], qf[s], st[nt]);
-        }
-      } else {
-        const int tk = j / DT, dt = j % DT;
-        const u32x4 bfrag = {pf[4 * tk], pf[4 * tk + 1], pf[4 * tk + 2], pf[4 * tk + 3]};
-        oacc[dt] = T::mfma(opnd[i], bfrag, oacc[dt]);
-      }
-    };
-#pragma unroll
-    for (int i = 0; i < kAhead; ++i) fetch(i);
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i) {
-      if (i + kAhead < kSlots) fetch(i + kAhead);
-      op(i);
-      __builtin_amdgcn_sched_barrier(0);   // keeps the operand reads kAhead MFMAs ahead of their use
-    }
-  };
-  // Q.K^T only (the first iteration)
-  auto qk_phase = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-      u32x4 kf[KS];
-#pragma unroll
-      for (int s = 0; s < KS; ++s) kf[s] = lds_load16(k_ad[s], nt * 32 * ROW_B);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) st[nt][i] = 0.f;
-#pragma unroll
-      for (int s = 0; s < KS; ++s) st[nt] = T::mfma(kf[s], qf[s], st[nt]);
-    }
-  };
-  // P.V only (the last iteration)
-  auto pv_phase = [&]() __attribute__((always_inline)) {
-#pragma unroll
-    for (int tk = 0; tk < 4; ++tk) {
-      u32x4 vf[DT];
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const u32x2 lo = lds_load_tr16(v_ad[dt], (16 * tk) * ROW_B);
-        const u32x2 hi = lds_load_tr16(v_ad[dt], (16 * tk + 8) * ROW_B);
-        vf[dt] = u32x4{lo.x, lo.y, hi.x, hi.y};
-      }
-      const u32x4 bfrag = {pf[4 * tk], pf[4 * tk + 1], pf[4 * tk + 2], pf[4 * tk + 3]};
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) oacc[dt] = T::mfma(vf[dt], bfrag, oacc[dt]);
-    }
-  };
-  // mask + online softmax of tile j: st -> pf, updates m_run, l_run (and rescales oacc when needed;
-  // every P.V issued so far belongs to earlier tiles and has completed in this wave's matrix phase)
+  auto matrix_phase = [&]() __attribute__((always_inline)) { tile_matrix<T, D>(st, oacc, pf, qf, k_ad, v_ad); };
   auto softmax = [&](int j, bool first) __attribute__((always_inline)) {
-    if (j == mbw) {   // causal mask on the diagonal tile
-      int thr = (wave & 1) * kWRows + mcol - 4 * g;   // row inside the 64-row block, minus the lane's column base
-      asm volatile("" : "+v"(thr));                  // keeps the 32 compares in this branch instead of 32 hoisted lane masks
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (nt * 32 + 8 * (i >> 2) + (i & 3) > thr) st[nt][i] = -INFINITY;
-    }
-    // Row sums are plain fp32 adds of the unrounded weights.  (v_dot2_f32_{f16,bf16} of the packed
-    // pair with a pair of ones would halve the instruction count, but those instructions stall the
-    // MFMA stream of the wave that shares the SIMD: measured 20 % slower per iteration.)
-    float psum[2];
-    auto weights = [&]() __attribute__((always_inline)) {
-      psum[0] = psum[1] = 0.f;
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int i = 0; i < 16; i += 2) {
-          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[nt][i], scale_log2, -m_run));
-          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[nt][i + 1], scale_log2, -m_run));
-          pf[nt * 8 + (i >> 1)] = T::pack_rne(p0, p1);
-          psum[0] += p0;
-          psum[1] += p1;
-        }
-    };
-    // The common case needs no row maximum: weights are formed against the reference exponent as it
-    // stands, and their sum tells whether that was good enough.  A lane's 32 weights are >= 0, so a sum of
-    // at most 2^8 bounds each of them by 2^8 (the 16-bit types hold that with room to spare); a larger
-    // sum, or the first live tile (the reference is still -inf and the sum is inf or NaN; the file is
-    // compiled without NaN semantics, so that case is asked for by name), takes the path below.  The item's
-    // first step goes there at once.
-    if (!first) weights();
-    if (first || __builtin_expect(__any(m_run == -INFINITY || psum[0] + psum[1] > kRescaleLimit), 0)) {
-      float mx = st[0][0];
-#pragma unroll
-      for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, st[nt][i]);
-      mx = max_with_other_half(mx);
-      const float m_cand = mx * scale_log2;   // finite: a live tile has a visible key in every row
-      // The reference exponent stays an INTEGER: a weight is then 2^frac * 2^int, and its rounding to the
-      // storage type does not depend on the power of two, so the rounded weights (relative to the row's
-      // sum) do not depend on the tile order or on how far m_run lags behind the true maximum.
-      const float m_new = __builtin_ceilf(fmaxf(m_run, m_cand));
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= alpha;
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) oacc[t][i] *= alpha;
-      m_run = m_new;
-      weights();
-    }
-    l_run += psum[0] + psum[1];
+    tile_softmax<T, D>(st, oacc, pf, m_run, l_run, j == mbw, (wave & 1) * kWRows + mcol - 4 * g, first, scale_log2);
   };
 
   // Iteration t: matrix phase = P.V of tile t-1 and Q.K^T of tile t, then softmax phase = tile t.
@@ -650,7 +688,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
     issue_tile(vbase, v_tile_bytes, vs_n, voff, false, jt[S - 2], v_dst0 + ((cst - TILE_B) & (kRing - 1)));
     const bool lp = lc_prev, lc = live_tile(jt[0]);
     if (kFirst) {
-      if (lc) qk_phase();
+      if (lc) tile_qk<T, D>(st, qf, k_ad);
     } else {
       if (lp || lc) matrix_phase();
     }
@@ -691,7 +729,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   // points, which is where its iterations will look for it.  The repeated copies of the last steps
   // may still be under way into those stages: a wave's copies land in the order they were started.
   prefetched = prefetch_next((rst + TILE_B) & (kRing - 1));
-  if (lc_prev) pv_phase();
+  if (lc_prev) tile_pv<T, D>(oacc, pf, v_ad);
   if (grp == 1) phase_barrier();
   advance();
   if (grp == 0) phase_barrier();
@@ -702,39 +740,212 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(PrefillArgs args_in_ker
   // 32-byte pieces.  With the Q rows of the next item asked for an iteration earlier, the accesses through flat pointers
   // gone and a third of the code (every part of the queue was compiled in eight times): 4 x 8192 tokens, 32 heads of 128,
   // 1237 -> 1209 us; 8192 tokens of 64-element heads 194.9 -> 183.6; 32768 tokens, 64 heads, 8453 -> 8340.
-  {
-    const float l_tot = l_run + other_half(l_run);
-    const float inv = (l_tot > 0.f) ? 1.f / l_tot : 0.f;
-    u32x4 rows[DT][2];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const f32x16& a = oacc[dt];
-        const u32x2 lo = swap_halves(T::pack_rne(a[8 * p + 0] * inv, a[8 * p + 1] * inv), T::pack_rne(a[8 * p + 4] * inv, a[8 * p + 5] * inv));
-        const u32x2 hi = swap_halves(T::pack_rne(a[8 * p + 2] * inv, a[8 * p + 3] * inv), T::pack_rne(a[8 * p + 6] * inv, a[8 * p + 7] * inv));
-        rows[dt][p] = u32x4{lo.x, hi.x, lo.y, hi.y};
-        asm volatile("" : "+v"(rows[dt][p]));
-      }
-    // what the next item has been asked for lands here, before the stores: behind them it would wait for them too
-    wait_vm(0);
-    pin_q();
-    if (m_glob < N) {
-      uint16_t* const orow = it.obase + m_glob * os_n + 8 * g;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int p = 0; p < 2; ++p) global_store16(orow + 32 * dt + 16 * p, rows[dt][p]);
-    }
-  }
+  u32x4 rows[DT][2];
+  tile_rows<T, D>(rows, oacc, l_run);
+  // what the next item has been asked for lands here, before the stores: behind them it would wait for them too
+  wait_vm(0);
+  pin_q();
+  if (m_glob < N) store_rows<D>(it.obase + m_glob * os_n + 8 * g, rows);
   }   // item loop
   // the last work-group to leave clears the queue for the next launch that uses this slot
   sign_off();
-  if (threadIdx.x == 0 && a0->queue != nullptr && left_before == gridDim.x - 1) {
+  if (threadIdx.x == 0 && left_before == gridDim.x - 1) {
     PrefillQueue* queue = a0->queue;
     for (int x = 0; x < 8; ++x) atomicExch(&queue->next[x], 0u);
     atomicExch(&queue->done, 0u);
   }
+}
+
+// ---- launches of short items ----------------------------------------------------------------------
+// prefill_kernel pays about 6 us an item outside its tile loop, keeps a CU busy with one item of 256 rows, and three
+// steps of an item have only some of its four query blocks live.  Where items are short (short prompts) or few, that is
+// much of the launch.  Here a work-group of four waves does ONE item of 128 rows, the hardware dispatcher hands them out,
+// and two of them (three at D = 64, by registers) share a CU: one starts or ends beside the other's tile loop, a long
+// item runs on beside no one at the speed of a wave alone, and the code is half as long, which counts where every
+// instruction is met for the first time.  Long items stay with prefill_kernel: its loop is the faster one (every tile
+// read serves 256 rows, neighbours walk their bands in step: 32768 tokens, 64 heads: 8.2 ms there, 11.4 ms here).
+// Tile math, layouts and results are those of prefill_kernel; tiles are taken in ascending order.
+constexpr int kShortWaves = 4;
+constexpr int kShortRows = kShortWaves * kWRows;
+struct PrefillShortArgs {
+  const uint16_t *q, *k, *v;
+  uint16_t* o;
+  Strides4 qs, ks, vs, os;
+  const int64_t *sink_blocks, *local_blocks;
+  int span_shift, BH, Hq, group, N, n_qtiles;
+  int one_round;   // the chip holds all work-groups at once
+  float scale_log2_signed;
+};
+
+template <typename T, int D>
+__global__ __launch_bounds__(64 * kShortWaves, 2) void prefill_short_kernel(PrefillShortArgs a) {
+  constexpr int NW = kShortWaves;
+  constexpr int KS = D / 16, DT = D / 32;
+  constexpr int CPR = D / 8;          // 16-byte chunks per K/V row
+  constexpr int LPW = CPR / NW;       // async copies per wave per tile and tensor (64 chunks each)
+  constexpr int ROW_B = D * 2;
+  constexpr uint32_t TILE_B = kKV * ROW_B;
+  constexpr int RSH = 16 / CPR;       // rows per 256 bytes of LDS
+  constexpr int kCopyRows = 64 * NW / CPR;   // rows from a wave's copy of a tile to its next one
+  static_assert(kCopyRows % (16 * RSH) == 0, "the copies of a wave are permuted alike");
+  extern __shared__ __attribute__((aligned(1024))) char s_mem[];
+  const uint32_t s_k = lds_address(s_mem), s_v = s_k + 2 * TILE_B;   // two stages each
+
+  // ---- the item ------------------------------------------------------------------------------------
+  // Work-groups go to the XCDs in turn.  Where the (batch row, head) pairs can be shared out evenly, an XCD has its pairs
+  // to itself; late (long) query tiles of all of them come first.  In a launch that the chip holds as a whole (two
+  // work-groups to a CU, the later half beside the earlier) the early tiles come in the opposite order, so that a CU has
+  // a long item and a short one.
+  const int list = blockIdx.x & 7, n_lists = a.BH % 8 == 0 ? 8 : 1;
+  const int per_list = n_lists == 8 ? a.BH >> 3 : a.BH;
+  const DivMod place = divmod_small((int)(n_lists == 8 ? blockIdx.x >> 3 : blockIdx.x), per_list);
+  const int turn = __builtin_amdgcn_readfirstlane(place.q), pair = (n_lists == 8 ? list * per_list : 0) + __builtin_amdgcn_readfirstlane(place.r);
+  const int late = (a.n_qtiles + 1) >> 1;
+  const int qt = (a.one_round && turn >= late) ? turn - late : a.n_qtiles - 1 - turn;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int mcol = lane & 31;   // query row inside the wave's 32 (the MFMA column)
+  const int g = lane >> 5;      // half-wave
+  const int N = a.N, nb = (N + kKV - 1) / kKV;
+  const DivMod bh = divmod_small(pair, a.Hq);
+  const int b = __builtin_amdgcn_readfirstlane(bh.q), hq = __builtin_amdgcn_readfirstlane(bh.r);
+  const int hk = __builtin_amdgcn_readfirstlane(divmod_small(hq, a.group).q);
+  const int row0 = qt * kShortRows + wave * kWRows;   // first query row of this wave
+
+  u32x4 qf[KS];              // Q fragment; rows past N repeat row N-1 (nothing of theirs is stored)
+  {
+    const uint16_t* qrow = a.q + b * a.qs.b + hq * a.qs.h + (int64_t)min(row0 + mcol, N - 1) * a.qs.n + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = global_load16(qrow + 16 * s);
+  }
+  const int ns = (int)max((int64_t)0, min((int64_t)nb, a.sink_blocks[hk] >> a.span_shift));
+  const int nl = (int)max((int64_t)0, min((int64_t)nb, a.local_blocks[hk] >> a.span_shift));
+
+  // tiles of the work-group: sinks [0, hi1], then band [lo2, mbl]; of this wave: its own live set
+  const int mb0 = 2 * qt, mbl = min(mb0 + 1, nb - 1), mbw = mb0 + (wave >> 1);
+  const int hi1 = min(ns - 1, mbl), n_sink = hi1 + 1;
+  const int lo2 = max(max(0, mb0 + 1 - nl), n_sink);
+  const int n_tiles = n_sink + max(0, mbl - lo2 + 1);
+  const int w_hi1 = min(ns - 1, mbw), w_lo2 = max(0, mbw + 1 - nl);
+  auto tile_of = [&](int t) __attribute__((always_inline)) { return t < n_sink ? t : lo2 + t - n_sink; };
+  auto live_tile = [&](int j) __attribute__((always_inline)) { return mbw < nb && (j <= w_hi1 || (j >= w_lo2 && j <= mbw)); };
+
+  // ---- copies: wave w, copy i fills chunks [(i*NW+w)*64, +64) of a stage -----------------------------
+  uint32_t koff, voff;
+  const int crow = wave * (64 / CPR) + lane / CPR, cpos = lane % CPR;
+  const uint32_t ksw = (uint32_t)((cpos ^ ((crow / RSH) % CPR)) * 16), vsw = (uint32_t)((cpos ^ (4 * ((crow / RSH) % (CPR / 4)))) * 16);
+  const uint32_t k_row = (uint32_t)(2 * a.ks.n), v_row_b = (uint32_t)(2 * a.vs.n);   // bytes of a row (a tile's fit 31 bits)
+  koff = (uint32_t)crow * k_row + ksw;
+  voff = (uint32_t)crow * v_row_b + vsw;
+  const char* const kbase = reinterpret_cast<const char*>(a.k + b * a.ks.b + hk * a.ks.h);
+  const char* const vbase = reinterpret_cast<const char*>(a.v + b * a.vs.b + hk * a.vs.h);
+  const int j_ragged = (N % kKV) ? nb - 1 : -1;    // the only tile with rows past N, if any: they repeat row N-1
+  auto copy_tile = [&](const char* base, uint32_t row_bytes, uint32_t off, uint32_t swizzle, int j, uint32_t dst)
+      __attribute__((always_inline)) {
+    const char* src = base + (uint64_t)(uint32_t)j * (uint64_t)(kKV * row_bytes);
+    if (j != j_ragged) {
+#pragma unroll
+      for (int i = 0; i < LPW; ++i) async_copy16(src, off + (uint32_t)(kCopyRows * i) * row_bytes, dst + i * NW * 1024);
+    } else {
+      const int last = N - 1 - j * kKV;
+#pragma unroll
+      for (int i = 0; i < LPW; ++i)
+        async_copy16(src, (uint32_t)min(crow + kCopyRows * i, last) * row_bytes + swizzle, dst + i * NW * 1024);
+    }
+  };
+  auto copy_k = [&](int t) __attribute__((always_inline)) {
+    copy_tile(kbase, k_row, koff, ksw, tile_of(t), s_k + (t & 1) * TILE_B + wave * 1024);
+  };
+  auto copy_v = [&](int t) __attribute__((always_inline)) {
+    copy_tile(vbase, v_row_b, voff, vsw, tile_of(t), s_v + (t & 1) * TILE_B + wave * 1024);
+  };
+  if (n_tiles > 0) {
+    copy_k(0);
+    if (n_tiles > 1) copy_k(1);
+    copy_v(0);
+  }
+
+  // operand read addresses (see prefill_kernel)
+  uint32_t k_ad[KS], v_ad[DT];
+  {
+    const uint32_t k_rd = (uint32_t)(mcol * ROW_B) | (uint32_t)(((g ^ ((mcol / RSH) % CPR)) & (CPR - 1)) * 16);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) k_ad[s] = s_k + (k_rd ^ (uint32_t)(32 * s));
+    const int grp16 = lane & 15, dhalf = (lane >> 4) & 1, v_row = 4 * g + (grp16 >> 2);
+    const uint32_t v_rd = (uint32_t)(v_row * ROW_B) +
+                          (uint32_t)(((2 * dhalf + ((grp16 & 3) >> 1)) ^ (4 * ((v_row / RSH) % (CPR / 4)))) * 16 +
+                                     8 * (grp16 & 1));
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) v_ad[dt] = s_v + TILE_B + (v_rd ^ (uint32_t)(64 * dt));   // V trails K by one step
+  }
+  const float scale_log2 = __builtin_fabsf(a.scale_log2_signed);
+  const int thr = (wave & 1) * kWRows + mcol - 4 * g;
+
+  f32x16 oacc[DT], st[2];
+  uint32_t pf[16];
+  {
+    float zero = 0.f;
+    asm volatile("" : "+v"(zero));
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) oacc[t][i] = zero;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      st[0][i] = st[1][i] = zero;
+      pf[i] = __builtin_bit_cast(uint32_t, zero);
+    }
+  }
+  float m_run = -INFINITY, l_run = 0.f;
+  bool lc_prev = false;
+
+  // A stage is filled again as soon as every wave has read it: a barrier behind the matrix phase, the copies two steps
+  // ahead, the softmax, a wait for the copies of the step before, a second barrier.
+  auto step = [&](int t, auto FIRST) __attribute__((always_inline)) {
+    constexpr bool kFirst = decltype(FIRST)::value != 0;
+    const int j = tile_of(t);
+    const bool lp = lc_prev, lc = live_tile(j);
+    if (kFirst) {
+      if (lc) tile_qk<T, D>(st, qf, k_ad);
+    } else {
+      if (lp || lc) tile_matrix<T, D>(st, oacc, pf, qf, k_ad, v_ad);
+    }
+    phase_barrier();
+    const bool more_v = t + 1 < n_tiles, more_k = t + 2 < n_tiles;
+    if (more_k) copy_k(t + 2);
+    if (more_v) copy_v(t + 1);
+    if (lc) {
+      tile_softmax<T, D>(st, oacc, pf, m_run, l_run, j == mbw, thr, kFirst, scale_log2);
+    } else if (lp) {   // the next matrix phase this wave runs must add nothing for a dead tile
+#pragma unroll
+      for (int i = 0; i < 16; ++i) pf[i] = 0;
+    }
+    const uint32_t flip = (t & 1) ? -TILE_B : TILE_B;   // K(t+1), V(t)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) k_ad[s] += flip;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) v_ad[dt] -= flip;
+    lc_prev = lc;
+    if (more_k) wait_vm(2 * LPW); else if (more_v) wait_vm(LPW); else wait_vm(0);
+    phase_barrier();
+  };
+  if (n_tiles > 0) {
+    wait_vm(0);
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));   // no wait of the compiler's behind this
+    if (a.scale_log2_signed < 0.f) {   // a negative scale goes into Q (see prefill_kernel)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[s] ^= u32x4{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
+    }
+    phase_barrier();
+    step(0, IC<1>{});
+    for (int t = 1; t < n_tiles; ++t) step(t, IC<0>{});
+    if (lc_prev) tile_pv<T, D>(oacc, pf, v_ad);
+  }
+  u32x4 rows[DT][2];
+  tile_rows<T, D>(rows, oacc, l_run);
+  const int m_row = row0 + mcol;
+  if (m_row < N) store_rows<D>(a.o + b * a.os.b + hq * a.os.h + (int64_t)m_row * a.os.n + 8 * g, rows);
 }
 
 template <int D, int S>
@@ -770,6 +981,20 @@ static int prefill_queue(PrefillQueue** out, int* cus) {
   return MOA_OK;
 }
 
+// Which launches prefill_short_kernel takes: items are short by the prompt's length (the host does not know the spans), or
+// the chip holds all of them at once.  Time against prefill_kernel's on inputs that are not cached, windows of 64-256 and
+// of 64-2048 tokens + a share of the prompt, 32 to 128 (batch row, head) pairs:
+//   D = 128: 1024 tokens 0.72-0.85, 2048 0.87-0.98, 3072 0.91-1.07 (4096 1.02-1.17, 6144 1.08-1.22 cached)
+//   D = 64:  2048 tokens 0.71-0.89, 3072 0.82-0.84, 4096 0.82-0.98 (6144 0.98-1.08 cached)
+//   up to two items to a CU: 512 tokens 0.73-0.80, 3072 0.83-0.91, 8192 0.69-0.99, 32768 (1 and 2 pairs) 0.84-0.96
+// 2048 tokens, 32 heads of 64: 37.9 -> 33.2 us; 2 x 1500 tokens, 32 heads of 128: 59.5 -> 45.1; 517 tokens: 20.0 -> 15.0;
+// 130 tokens: 11.9 -> 7.9.
+static bool short_items(int D, int N, int64_t pairs, int cus) {
+  const int64_t items = pairs * ((N + kShortRows - 1) / kShortRows);
+  if (items > (1 << 21)) return false;   // divmod_small
+  return N <= (D == 64 ? 4096 : 2048) || items <= 2 * (int64_t)cus;
+}
+
 template <typename T, int D>
 static int launch_prefill(const void* q, const void* k, const void* v, void* o, const int64_t* qs,
                           const int64_t* ks, const int64_t* vs, const int64_t* os, int B, int Hq,
@@ -790,17 +1015,27 @@ static int launch_prefill(const void* q, const void* k, const void* v, void* o, 
     return fail(MOA_ERR_UNSUPPORTED, "moa_prefill_fwd: k/v token stride too large");
   Strides4 sq = {qs[0], qs[1], qs[2]}, sk = {ks[0], ks[1], ks[2]}, sv = {vs[0], vs[1], vs[2]},
            so = {os[0], os[1], os[2]};
+  PrefillQueue* queue = nullptr;
+  int cus = 0;
+  if (int rc = prefill_queue(&queue, &cus)) return rc;
+  if (short_items(D, N, pairs, cus)) {
+    PrefillShortArgs a;
+    a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.o = (uint16_t*)o;
+    a.qs = sq; a.ks = sk; a.vs = sv; a.os = so;
+    a.sink_blocks = sink_blocks; a.local_blocks = local_blocks; a.span_shift = span_shift;
+    a.BH = BH; a.Hq = Hq; a.group = Hq / Hkv; a.N = N; a.n_qtiles = (N + kShortRows - 1) / kShortRows;
+    const int64_t groups = pairs * a.n_qtiles;
+    a.one_round = groups <= 2 * (int64_t)cus;
+    a.scale_log2_signed = mfma_softmax_scale(sm_scale);
+    hipLaunchKernelGGL((prefill_short_kernel<T, D>), dim3((unsigned)groups), dim3(64 * kShortWaves),
+                       (prefill_lds_bytes<D, 2>()), st, a);
+    return check_launch("moa_prefill_fwd");
+  }
   const size_t lds = prefill_lds_bytes<D, S>();
   static bool lds_reserved[kMaxDevices] = {};   // per template instance
   if (int rc = reserve_lds(reinterpret_cast<const void*>(&prefill_kernel<T, D>), lds, lds_reserved, "moa_prefill_fwd"))
     return rc;
-  PrefillQueue* queue = nullptr;
-  int cus = 0;
-  if (int rc = prefill_queue(&queue, &cus)) return rc;
   const int64_t groups = items < cus ? items : cus;
-  // No queue where every work-group has one item and the eight lists are equally long: place i is item i / 8 of list
-  // i % 8, the XCD the dispatcher hands work-group i to.
-  if (items <= cus && pairs % 8 == 0) queue = nullptr;
   PrefillArgs args;
   args.q = (const uint16_t*)q; args.k = (const uint16_t*)k; args.v = (const uint16_t*)v; args.o = (uint16_t*)o;
   args.qs = sq; args.ks = sk; args.vs = sv; args.os = so;
