@@ -141,7 +141,9 @@ __device__ __forceinline__ float wave_sum(float x) {
 // to more than the row holds) the chunks past the cap do not exist for any kernel, so none of them is written, read
 // or merged.  Segments are clamped into the row, so that a bad index cannot fault.
 //
-// Two policies.  Fixed: chunks of CHUNK rows.  Even (even_target > 0, only with EVEN): with a fixed length the last
+// Three policies.  Fixed: chunks of CHUNK rows.  Short (kShortChunks, only with EVEN): chunks of kEvenMinChunk rows, for
+// launches whose batch rows cannot have more of them than their share of the CUs: what Even comes to there, without its
+// search and divisions (0.5 to 1 us in front of the first load).  Even (even_target > 0, only with EVEN): with a fixed length the last
 // chunk of every head is a remainder and the number of chunks is whatever it comes to; here the caller names the
 // number of chunks a batch row should not exceed, and the row takes the shortest chunk length c (whole steps of
 // kEvenStep rows, at least kEvenMinChunk) for which sum_h ceil(len_h / c) <= target; head h is then split evenly into
@@ -151,6 +153,7 @@ __device__ __forceinline__ float wave_sum(float x) {
 constexpr int kEvenMinChunk = 256;   // also the chunk length the partial slots of a batch row are sized for
 constexpr int kEvenStep = 128;
 constexpr int kEvenTries = 24;
+constexpr int kShortChunks = -1;     // instead of an even_target
 struct Chunk {
   int head, index, count;   // its head, its place among the head's chunks, how many those are
   int seg0, len, rows;      // first row and valid rows of the head's segment, rows per chunk of the head
@@ -177,8 +180,10 @@ struct RowChunks {
         len[k] = (int)l;
       }
     }
-    int c = CHUNK;
+    static_assert((CHUNK & (CHUNK - 1)) == 0 && (kEvenMinChunk & (kEvenMinChunk - 1)) == 0, "fixed chunks divide by a shift");
+    int c = EVEN && even_target == kShortChunks ? kEvenMinChunk : CHUNK;
     const bool even = EVEN && even_target > 0;
+    const int shift = __builtin_ctz(c);
     if (even) {
       auto chunks = [&](int size) __attribute__((always_inline)) {
         int n = 0;
@@ -198,7 +203,8 @@ struct RowChunks {
       rows[k] = c;
       last[k] = base;
       if (k * 64 < H) {
-        int n = chunks_of(len[k], c);
+        int n = (int)(((unsigned)len[k] + (unsigned)c - 1u) >> shift);
+        if (even) n = chunks_of(len[k], c);
         if (even && n > 0) {
           rows[k] = chunks_of(chunks_of(len[k], n), kEvenStep) * kEvenStep;   // even split, <= c
           n = chunks_of(len[k], rows[k]);
@@ -245,21 +251,26 @@ struct Merged {
   float L;
 };
 // One wave's part of the merge of a head's n partials: chunks first, first + stride, ...  `acc` and `ml` are the head's
-// first partial (uniform), `G` partials lie between a chunk's and the next one's.  All of the wave's loads go out
-// before it looks at any of them.  COHERENT: the partials come from work-groups of this launch, on other XCDs perhaps:
+// first partial (uniform), `G` partials lie between a chunk's and the next one's.  The constructor sends the wave's loads
+// out, sum() looks at them: a wave that merges several heads asks for all of theirs first.  COHERENT: the partials come from work-groups of this launch, on other XCDs perhaps:
 // device-scope loads.
 // A wave that takes every chunk (stride 1) sums them in kDecWaves strands, as kDecWaves waves with a stride of
 // kDecWaves and their final sum do: every way of merging gives the same bits.
 template <int D, bool COHERENT, int kFirst /* chunks asked for at once */, int kMore /* and in every round behind */,
           bool STRANDS = false>
-__device__ __forceinline__ Merged<D> merge_wave(const float* acc, const f32x2* ml, int G, int n, int first, int stride) {
+struct WaveMerge {
   typedef typename Merged<D>::fvec fvec;
-  constexpr int VEC = Merged<D>::VEC;
+  static constexpr int VEC = Merged<D>::VEC;
   static_assert(64 % kMore == 0 && kFirst % kMore == 0, "rounds do not straddle a block of 64 factors");
-  const int lane = threadIdx.x & 63;
-  const int step = G * D;          // from a chunk's accumulator to the next one's
-  auto load = [](const auto* p) __attribute__((always_inline)) {
-    typedef std::remove_cv_t<std::remove_reference_t<decltype(*p)>> V;
+  const float* acc;
+  const f32x2* ml;
+  int G, n, first, stride;
+  int step;          // from a chunk's accumulator to the next one's
+  fvec x[kFirst];    // a chunk past the head's last repeats that one: no branch stands between the loads
+  f32x2 mine;        // chunk `lane`
+
+  template <typename V>
+  static __device__ __forceinline__ V load(const V* p) {
     if constexpr (!COHERENT) {
       return *p;
     } else if constexpr (sizeof(V) == 8) {
@@ -269,13 +280,21 @@ __device__ __forceinline__ Merged<D> merge_wave(const float* acc, const f32x2* m
       return __builtin_bit_cast(V, __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT));
     }
-  };
-  fvec x[kFirst];   // a chunk past the head's last repeats that one: no branch stands between the loads
+  }
+  __device__ __forceinline__ WaveMerge(const float* acc_, const f32x2* ml_, int G_, int n_, int first_, int stride_)
+      : acc(acc_), ml(ml_), G(G_), n(n_), first(first_), stride(stride_), step(G_ * D) {
+    const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int j = 0; j < kFirst; ++j)
-    x[j] = load(reinterpret_cast<const fvec*>(acc + min(first + stride * j, n - 1) * step + lane * VEC));
-  f32x2 mine = {-INFINITY, 0.f};   // chunk `lane`
-  if (lane < n) mine = load(ml + (int64_t)lane * G);
+    for (int j = 0; j < kFirst; ++j)
+      x[j] = load(reinterpret_cast<const fvec*>(acc + min(first + stride * j, n - 1) * step + lane * VEC));
+    mine = f32x2{-INFINITY, 0.f};
+    if (lane < n) mine = load(ml + (int64_t)lane * G);
+  }
+  __device__ __forceinline__ Merged<D> sum() const;
+};
+template <int D, bool COHERENT, int kFirst, int kMore, bool STRANDS>
+__device__ __forceinline__ Merged<D> WaveMerge<D, COHERENT, kFirst, kMore, STRANDS>::sum() const {
+  const int lane = threadIdx.x & 63;
   float M = mine.x;
   for (int i = 64 + lane; i < n; i += 64) M = fmaxf(M, load(ml + (int64_t)i * G).x);
 #pragma unroll
@@ -555,8 +574,8 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
       float* const s_sum = &s_acc[0][0][0];   // [kDecWaves][D]
       for (int g = 0; g < G; ++g) {
         const int64_t slot0 = ((int64_t)b * cap + w - c) * G + g;
-        const Merged<D> m = merge_wave<D, true, 8, 4>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G,
-                                                n_chunks, wave, kDecWaves);
+        const Merged<D> m = WaveMerge<D, true, 8, 4>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G,
+                                                     n_chunks, wave, kDecWaves).sum();
         *reinterpret_cast<typename Merged<D>::fvec*>(s_sum + wave * D + lane * Merged<D>::VEC) = m.a;
         __syncthreads();
         if (tid < D) {
@@ -596,8 +615,8 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
     return;
   }
   const int64_t slot0 = ((int64_t)b * cap + w0) * G + g;
-  const Merged<D> m = merge_wave<D, false, 8, 4>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G, n,
-                                           wave, kDecWaves);
+  const Merged<D> m = WaveMerge<D, false, 8, 4>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G, n,
+                                                wave, kDecWaves).sum();
   const float L = m.L;
   *reinterpret_cast<typename Merged<D>::fvec*>(&s_a[wave][lane * Merged<D>::VEC]) = m.a;
   __syncthreads();
@@ -648,7 +667,7 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     uint16_t* __restrict__ o, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const int64_t* __restrict__ head_start, const int64_t* __restrict__ head_valid, int H,
     int G /* query heads per ring, <= kGqaMaxG */, int64_t sumC, float scale_log2_signed, int cap,
-    int target /* > 0: chunks a batch row is split into (RowChunks); 0: chunks of kGqaChunk rows */,
+    int target /* > 0: chunks a batch row is split into; 0 or kShortChunks: chunks of a fixed length (RowChunks) */,
     unsigned* __restrict__ counters /* as in decode_split_kernel */) {
   typedef typename MfmaElem<T>::type M;
   // the row maximum is taken over unscaled scores: a negative softmax scale goes into Q (sign flip, exact)
@@ -850,9 +869,11 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     }
     __syncthreads();
 
-    // ---- combine the waves; thread d owns output column d of every query head of the ring ----
-    if (tid < D) {
-      for (int gq = 0; gq < G; ++gq) {
+    // ---- combine the waves; a thread owns an output column of every second (fourth at D = 64) query head of the ring ----
+    {
+      const int d = tid % D;
+#pragma unroll 2
+      for (int gq = tid / D; gq < G; gq += kGqaThreads / D) {
         float Mx = s_m[0][gq];
 #pragma unroll
         for (int i = 1; i < kGqaWaves; ++i) Mx = fmaxf(Mx, s_m[i][gq]);
@@ -862,14 +883,14 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
         for (int i = 0; i < kGqaWaves; ++i) {
           const float f = fast_exp2(s_m[i][gq] - m_use);
           L += s_l[i][gq] * f;
-          a += reinterpret_cast<const float*>(s_mem + i * (kGqaStages * STAGE_B))[gq * D + tid] * f;
+          a += reinterpret_cast<const float*>(s_mem + i * (kGqaStages * STAGE_B))[gq * D + d] * f;
         }
         if (n_chunks == 1) {
-          o[(bh * G + gq) * D + tid] = pack1<T>((L > 0.f) ? a / L : 0.f);
+          o[(bh * G + gq) * D + d] = pack1<T>((L > 0.f) ? a / L : 0.f);
         } else {
           const int64_t slot = ((int64_t)b * cap + w) * G + gq;
-          store_partial(part_acc + slot * D + tid, a, MERGE && counters != nullptr);
-          if (tid == 0) {
+          store_partial(part_acc + slot * D + d, a, MERGE && counters != nullptr);
+          if (d == 0) {
             store_partial(part_ml + slot * 2 + 0, Mx, MERGE && counters != nullptr);
             store_partial(part_ml + slot * 2 + 1, L, MERGE && counters != nullptr);
           }
@@ -877,12 +898,25 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
       }
     }
     if (MERGE && counters && n_chunks > 1 && arrived_last(counters + bh, n_chunks)) {
-      for (int gq = wave; gq < G; gq += kGqaWaves) {   // a query head to a wave
+      // a wave has query heads wave and wave + 4: the loads of both go out together
+      typedef WaveMerge<D, true, 16, 16, true> HeadMerge;
+      auto part = [&](int gq) __attribute__((always_inline)) {
         const int64_t slot0 = ((int64_t)b * cap + w - c) * G + gq;
-        const Merged<D> m = merge_wave<D, true, 16, 16, true>(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G,
-                                                n_chunks, 0, 1);
+        return HeadMerge(part_acc + slot0 * D, reinterpret_cast<const f32x2*>(part_ml) + slot0, G, n_chunks, 0, 1);
+      };
+      auto finish = [&](int gq, const HeadMerge& h) __attribute__((always_inline)) {
+        const Merged<D> m = h.sum();
 #pragma unroll
         for (int j = 0; j < D / 64; ++j) o[(bh * G + gq) * D + lane * (D / 64) + j] = pack1<T>((m.L > 0.f) ? m.a[j] / m.L : 0.f);
+      };
+      static_assert(kGqaMaxG <= 2 * kGqaWaves, "two heads to a wave");
+      if (wave + kGqaWaves < G) {
+        const HeadMerge h0 = part(wave), h1 = part(wave + kGqaWaves);
+        __builtin_amdgcn_sched_barrier(0);
+        finish(wave, h0);
+        finish(wave + kGqaWaves, h1);
+      } else if (wave < G) {
+        finish(wave, part(wave));
       }
     }
     __syncthreads();  // s_acc / s_m / s_l are reused by the next chunk
@@ -1002,14 +1036,16 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
   // against 75.1 at 8, 149.9 against 200.8 at 16.  The host does not know how full the rings are; it plans with their
   // capacity.
   const int64_t fixed_chunks = (int64_t)B * (sumC / kGqaChunk + (H + 1) / 2);
-  int64_t target = 0;   // 0: chunks of kGqaChunk rows
+  int64_t target = 0;   // 0: chunks of kGqaChunk rows; kShortChunks: of kEvenMinChunk
   if (fixed_chunks <= 128) {
     target = (256 + B - 1) / B;
     if (target > cap) target = cap;
+    if ((sumC + kEvenMinChunk - 1) / kEvenMinChunk + H <= target) target = kShortChunks;
   }
   // at most this many chunks per batch row (a work-group without a chunk still holds a CU while it finds that out)
-  const int64_t chunks = target > 0 ? target + H : (sumC + kGqaChunk - 1) / kGqaChunk + H;
-  const int64_t chunk_rows = target > 0 ? (sumC / target > kEvenMinChunk ? sumC / target : kEvenMinChunk) : kGqaChunk;
+  const int64_t fixed_rows = target == kShortChunks ? kEvenMinChunk : kGqaChunk;
+  const int64_t chunks = target > 0 ? target + H : (sumC + fixed_rows - 1) / fixed_rows + H;
+  const int64_t chunk_rows = target == kShortChunks ? kEvenMinChunk : target > 0 ? (sumC / target > kEvenMinChunk ? sumC / target : kEvenMinChunk) : kGqaChunk;
   const int64_t ring_chunks = (sumC / H + chunk_rows - 1) / chunk_rows;   // of a ring of average size
   const int64_t row_chunks = (sumC + chunk_rows - 1) / chunk_rows;        // of a ring that is all of the batch row
   const bool nt = read_nontemporal(B, sumC, D);
