@@ -12,6 +12,7 @@ from typing import Optional, Sequence
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libmoa_hip.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
 
 MOA_OK = 0
 MOA_ERR_ARG = -1
@@ -66,6 +67,7 @@ SIGNATURES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
+_host = None
 
 
 class MoaKernelError(RuntimeError):
@@ -99,6 +101,30 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def host():
+    """The compiled host side of the attention and the append (csrc/moa_host.cpp), loaded once and bound to the library."""
+    global _host
+    if _host is not None:
+        return _host
+    import torch  # noqa: F401  (its libraries are what the module is linked to)
+
+    lib = load()
+    if not os.path.exists(HOST_PATH):
+        raise MoaKernelError(f"{HOST_PATH} is not built. Run `python -m moa_amd.build`.")
+    try:
+        from moa_amd import _host as module
+    except ImportError as e:  # pragma: no cover - depends on the machine
+        raise MoaKernelError(f"cannot load {HOST_PATH}: {e}; rebuild it") from e
+    from moa_amd.kernels import mixture_of_attention as attention
+
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda i: torch.cuda.current_stream(i).cuda_stream)
+    module.setup(*(ctypes.cast(getattr(lib, f), c_void_p).value for f in (
+        "moa_decode_workspace_bytes", "moa_decode_fwd_counted", "moa_rope_cache_append", "moa_cache_append",
+        "moa_prefill_fwd_tokens")), raw, check, attention._decode_scratch, attention._N_COUNTERS)
+    _host = module
+    return module
+
+
 def last_error() -> str:
     return load().moa_last_error().decode("utf-8", "replace")
 
@@ -119,7 +145,7 @@ def check(rc: int, assertion_for_arg: bool = True) -> None:
 
 
 def i64_array(values: Sequence[int]):
-    return (c_int64 * len(values))(*[int(v) for v in values])
+    return (c_int64 * len(values))(*values)
 
 
 def dtype_code(torch_dtype) -> int:

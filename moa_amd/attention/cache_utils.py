@@ -104,7 +104,7 @@ class StaticCircularCache:
         self.cache_position = 0
         self._kv_len = [0 for _ in range(self.num_layers)]
         self._ready_on: List[Optional[torch.device]] = [None] * self.num_layers   # device the layer's tensors are on
-        self._step_args: List[Optional[Dict[str, Any]]] = [None] * self.num_layers   # what rope_update keeps per layer
+        self._step_args: List[Optional[Tuple[Tensor, Tensor]]] = [None] * self.num_layers   # rope_update's q buffer, its view
         self._capturing: Optional[bool] = None   # is the stream capturing (asked once per step)
 
         # K/V are created on the device of the first update of each layer
@@ -119,8 +119,8 @@ class StaticCircularCache:
         on_device.copy_(packed)
 
     def __getstate__(self):
-        """Copies (copy.deepcopy, pickling) do not take the per-layer call arguments along: those hold
-        device addresses of THIS object's tensors."""
+        """Copies (copy.deepcopy, pickling) do not take the q buffers along: pickled, a buffer and its view are two
+        tensors."""
         state = self.__dict__.copy()
         state["_step_args"] = [None] * self.num_layers
         return state
@@ -196,15 +196,26 @@ class StaticCircularCache:
         Capturing earlier would let replays walk a head's pointer linearly out of its segment.
         (Replays do not advance ``get_seq_length()`` / ``cache_position`` either: callers that replay
         pass explicit positions.)  Called before anything is changed, so a caller that catches the error
-        can go on eagerly.  The stream is asked once per step (layer 0); the other layers of the step
-        use that answer."""
-        if layer_idx == 0 or self._capturing is None:
+        can go on eagerly.  The stream is asked at most once per step, by the first layer from layer 0 on
+        that is not past its sinks yet; the other layers of the step use that answer."""
+        if layer_idx == 0:
+            self._capturing = None
+        if self._kv_len[layer_idx] + 1 > self._max_static_size[layer_idx]:
+            return
+        if self._capturing is None:
             self._capturing = torch.cuda.is_current_stream_capturing()
-        if self._capturing and self._kv_len[layer_idx] + 1 <= self._max_static_size[layer_idx]:
+        if self._capturing:
             raise RuntimeError(
                 f"StaticCircularCache: layer {layer_idx} has seen {self._kv_len[layer_idx]} tokens, not more than its "
                 f"largest static size {self._max_static_size[layer_idx]}: a decode step captured now would be "
                 "replayed with the wrong ring decision; capture after the prompt has filled the static parts")
+
+    def _layer(self, layer_idx: int) -> Tuple[Optional[Tensor], ...]:
+        """A layer's tensors, in the order in which the compiled step takes them."""
+        return (self.key_cache[layer_idx], self.value_cache[layer_idx], self.mask_cache[layer_idx],
+                self.cache_update_index[layer_idx], self.cache_valid_length[layer_idx],
+                self.circular_cache_head_index[layer_idx], self.circular_cache_size[layer_idx],
+                self.static_cache_size[layer_idx], self.cache_max_length[layer_idx])
 
     def rope_update(
         self,
@@ -254,43 +265,17 @@ class StaticCircularCache:
         self._to_device(layer_idx, device)
         self._check_capture(layer_idx, device)
 
-        # What does not change from step to step is kept per layer: the library handle, the pointers of the
-        # cache and its index tensors, the q buffer, and the stride arrays of the last operand layout seen.
-        st = self._step_args[layer_idx]
-        layout = (query_states.stride(), key_states.stride(), value_states.stride(), cos.shape, cos.stride(),
-                  sin.stride(), Hq)
-        if st is None or st["layout"] != layout:
-            qs, ks_, vs_ = query_states.stride(), key_states.stride(), value_states.stride()
-            if qs[-1] != 1 or ks_[-1] != 1 or vs_[-1] != 1:
-                st = None   # rare: operands without a contiguous head_dim are copied, nothing is kept
-            else:
-                upd = self.cache_update_index[layer_idx]
-                assert upd.is_contiguous() and self.cache_valid_length[layer_idx].is_contiguous()
-                _, _, css = _cos_sin_strides(cos, sin, B, 1, D)
-                q_out = torch.empty((B, 1, Hq, D), dtype=self.dtype, device=device)
-                st = {
-                    "layout": layout, "lib": _lib.load(), "q_out": q_out, "q_view": q_out.transpose(1, 2),
-                    "cos_ok": cos.stride(-1) == 1 and sin.stride() == cos.stride(),
-                    "strides": (_lib.i64_array((qs[0], qs[1], qs[3])), _lib.i64_array((ks_[0], ks_[1], ks_[3])),
-                                _lib.i64_array((vs_[0], vs_[1], vs_[3])), css[0]),
-                    "tail": (q_out.data_ptr(), self.key_cache[layer_idx].data_ptr(),
-                             self.value_cache[layer_idx].data_ptr(), self.mask_cache[layer_idx].data_ptr(),
-                             upd.data_ptr(), self.cache_valid_length[layer_idx].data_ptr(),
-                             self.circular_cache_head_index[layer_idx].data_ptr(),
-                             self.circular_cache_size[layer_idx].data_ptr(),
-                             self.static_cache_size[layer_idx].data_ptr(),
-                             self.cache_max_length[layer_idx].data_ptr()),
-                    "sizes": (B, Hq, H, D, self.layer_cache_size[layer_idx], _lib.dtype_code(self.dtype)),
-                }
-                self._step_args[layer_idx] = st
-        if st is not None and st["cos_ok"]:
-            qstr, kstr, vstr, cos_b = st["strides"]
-            rc = st["lib"].moa_rope_cache_append(
-                query_states.data_ptr(), key_states.data_ptr(), value_states.data_ptr(), qstr, kstr, vstr,
-                cos.data_ptr(), sin.data_ptr(), cos_b, *st["tail"], self._kv_len[layer_idx], *st["sizes"],
-                _lib.current_stream_ptr(device))
-            q_view = st["q_view"]
-        else:
+        # The q buffer stays from step to step; the launch itself is compiled code where no operand has to be copied first
+        # (8.7 us of the host's time with ctypes).
+        kept = self._step_args[layer_idx]
+        if kept is None or kept[0].shape[2] != Hq or kept[0].device != device:
+            q_out = torch.empty((B, 1, Hq, D), dtype=self.dtype, device=device)
+            kept = self._step_args[layer_idx] = (q_out, q_out.transpose(1, 2))
+        q_out, q_view = kept
+        if not _lib.host().rope_append(query_states, key_states, value_states, cos, sin, q_out, *self._layer(layer_idx),
+                                       self._kv_len[layer_idx]):
+            assert (self.cache_update_index[layer_idx].is_contiguous()
+                    and self.cache_valid_length[layer_idx].is_contiguous())
             cos, sin, css = _cos_sin_strides(cos, sin, B, 1, D)
             qn, kn, vn = (t[:, :, -1, :] for t in (query_states, key_states, value_states))
             qn, kn, vn = (t if t.stride(-1) == 1 else t.contiguous() for t in (qn, kn, vn))
@@ -307,8 +292,8 @@ class StaticCircularCache:
                 self.cache_max_length[layer_idx].data_ptr(),
                 self._kv_len[layer_idx], B, Hq, H, D, self.layer_cache_size[layer_idx],
                 _lib.dtype_code(self.dtype), _lib.current_stream_ptr(device))
+            _lib.check(rc)
             q_view = q_out.transpose(1, 2)
-        _lib.check(rc)
         if layer_idx == 0:
             self.cache_position += 1
         self._kv_len[layer_idx] += 1
@@ -442,6 +427,10 @@ class StaticCircularCache:
             self._check_capture(layer_idx, device)   # before anything is changed
         if layer_idx == 0:
             self.cache_position += seq_len
+        if seq_len == 1 and self.update_cache_content and _lib.host().append(
+                key_states, value_states, *self._layer(layer_idx), self._kv_len[layer_idx]):
+            self._kv_len[layer_idx] += 1
+            return self.key_cache[layer_idx], self.value_cache[layer_idx]
 
         sumC = self.layer_cache_size[layer_idx]
         stream = _lib.current_stream_ptr(device)

@@ -1,4 +1,5 @@
-"""Builds moa_amd/libmoa_hip.so from moa_amd/csrc/*.hip with hipcc for gfx950.
+"""Builds moa_amd/libmoa_hip.so from moa_amd/csrc/*.hip with hipcc for gfx950, and moa_amd/_host.so, the host side of a
+decode step, from moa_amd/csrc/moa_host.cpp with g++ against torch's headers.
 
     python -m moa_amd.build            # build if sources are newer than the library
     python -m moa_amd.build --force    # always rebuild
@@ -19,6 +20,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "csrc", "build")
 LIB_PATH = os.path.join(HERE, "libmoa_hip.so")
+HOST_PATH = os.path.join(HERE, "_host.so")
+HOST_SOURCE = os.path.join(CSRC, "moa_host.cpp")
 
 SOURCES = ["moa_capi.hip", "moa_cache.hip", "moa_decode.hip", "moa_prefill.hip", "moa_rope.hip"]
 
@@ -49,13 +52,14 @@ def _hipcc() -> str:
 
 
 def _deps_mtime() -> float:
-    paths = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h"))]
+    paths = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h", ".cpp"))]
     paths.append(os.path.join(HERE, "..", "include", "moa_hip.h"))
     return max(os.path.getmtime(p) for p in paths if os.path.exists(p))
 
 
 def is_stale() -> bool:
-    return (not os.path.exists(LIB_PATH)) or os.path.getmtime(LIB_PATH) < _deps_mtime()
+    built = (LIB_PATH, HOST_PATH)
+    return not all(map(os.path.exists, built)) or min(map(os.path.getmtime, built)) < _deps_mtime()
 
 
 def _compile(src: str, extra: Sequence[str] = ()) -> str:
@@ -71,6 +75,22 @@ def _compile(src: str, extra: Sequence[str] = ()) -> str:
     return obj
 
 
+def _build_host() -> None:
+    """torch's own libraries are not found by name, nor need they be: the module is loaded where torch already is."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    include = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", *(f"-isystem{p}" for p in include),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(cpp_extension.torch._C._GLIBCXX_USE_CXX11_ABI)}", HOST_SOURCE, "-o", HOST_PATH,
+           f"-L{cpp_extension.TORCH_LIB_PATH}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed for {HOST_SOURCE}:\n{r.stdout}\n{r.stderr}")
+    if r.stderr.strip():
+        sys.stderr.write(f"[moa_amd.build] {HOST_SOURCE}:\n{r.stderr.strip()}\n")
+
+
 def build(force: bool = False, verbose: bool = True, experiment_flags: Sequence[str] = ()) -> str:
     """Compiles every source and links the library.  ``experiment_flags`` (extra hipcc arguments) are for
     measurement builds only and must be asked for explicitly: the environment never changes the build."""
@@ -82,13 +102,15 @@ def build(force: bool = False, verbose: bool = True, experiment_flags: Sequence[
     if missing:
         raise RuntimeError(f"missing sources: {sorted(missing)}")
     with ThreadPoolExecutor(max_workers=min(4, len(srcs))) as ex:
+        host = ex.submit(_build_host)
         objs = list(ex.map(lambda s: _compile(s, experiment_flags), srcs))
+        host.result()
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     if verbose:
-        print(f"[moa_amd.build] built {LIB_PATH}")
+        print(f"[moa_amd.build] built {LIB_PATH} and {HOST_PATH}")
     return LIB_PATH
 
 
