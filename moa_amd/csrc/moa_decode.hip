@@ -631,14 +631,21 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
 // ---- grouped-query decode on the matrix cores (G >= 2) ---------------------------------------
 // With G query heads per ring the vector ALU version above does G times the arithmetic per cache
 // byte and stops being HBM bound (measured: 65 % of peak at G = 2, 46 % at G = 8).  Here the G query rows of a ring are the
-// columns of a 32-wide MFMA tile (columns >= G are zero padding; the matrix pipe has the room):
+// columns of a 16-wide MFMA tile (columns >= G are zero padding; the matrix pipe has the room):
 //   S^T[key][q] = sum_d K[key][d] Q[q][d]      A = K (LDS), B = Q^T (registers)
 //   O^T[d][q]   = sum_key V[key][d] P[q][key]   A = V^T (LDS, transposing read), B = P^T
 // the same transposed pair of products as the prefill kernel, 32 keys at a time, so the softmax
-// state of a query head is lane-local.  Each wave streams its own share of the chunk through a
+// state of a query head stays in its column's four lanes (a quarter of the keys each).  v_mfma_f32_16x16x32 leaves in lane
+// 16 g + n rows 4 g + i of column n, which is the B operand of the second product as it is, when its contraction slots are
+// numbered that way.  Each wave streams its own share of the chunk through a
 // private two-stage LDS ring with asynchronous copies (16-byte chunks XOR-permuted as in the
 // prefill kernel), so no work-group barrier is needed inside the loop.  Chunks, partials and the
 // merge kernel are those of the vector version, with a longer chunk.
+// A CU has one wave per SIMD (the LDS rings fill it), so nothing hides what a wave does to a tile between two copies.  With
+// 32-wide tiles half of the matrix cycles, of the exponentials and of the packing went into padding, for up to 8 heads three
+// quarters; with 16-wide ones, and K and V waited for and copied each by itself, a call takes, before and now (GPU time):
+// batch 4 of 8 rings, 164 MB, 8 heads 34.9 -> 33.5 us; batch 2, 82 MB 23.1 -> 21.8; batch 1, 8 rings of up to 500 rows,
+// 4 heads 9.7 -> 8.7; batch 4 of 64-element rows, 66 MB, 2 heads 18.2 -> 16.5; batch 16, 655 MB 109.5 -> 107.7.
 // Work-groups per CU the grid may hold.  A CU runs one at a time (the LDS rings fill it), so the hardware
 // dispatcher hands out chunks as CUs become free when every chunk is a work-group of its own: 602 us at
 // batch 64 of the 70B shape against 612-628 us with 2-16 per CU, each walking several chunks in a fixed order.
@@ -674,8 +681,9 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
   const float scale_log2 = __builtin_fabsf(scale_log2_signed);
   const uint32_t q_sign = scale_log2_signed < 0.f ? 0x80008000u : 0u;
   constexpr bool MERGE = !NT;                   // as in decode_split_kernel
-  constexpr int KS = D / 16;                    // MFMA k-steps of Q.K^T
-  constexpr int DT = D / 32;                    // 32-wide d tiles of the output
+  constexpr int KS = D / 32;                    // MFMA k-steps of Q.K^T
+  constexpr int DT = D / 16;                    // 16-wide d tiles of the output
+  constexpr int KT = kGqaTile / 16;             // 16-key tiles of the scores
   constexpr int CPR = D / 8;                    // 16-byte chunks per cache row
   constexpr int ROW_B = D * 2;
   constexpr int RSH = 16 / CPR;                 // rows per 256 bytes of LDS
@@ -696,8 +704,8 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int mcol = lane & 31;   // query head inside the ring (the MFMA column); >= G: padding
-  const int g = lane >> 5;      // half-wave
+  const int mcol = lane & 15;   // query head inside the ring (the MFMA column); >= G: padding
+  const int g = lane >> 4;      // quarter of the wave
   const uint32_t ring0 = lds_address(s_mem) + wave * (kGqaStages * STAGE_B);   // this wave's stages
 
   // copy i of a tile moves chunks [64 i, 64 i + 64): chunk c = row * CPR + position
@@ -709,20 +717,20 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     const int row = L / CPR, pos = L % CPR;
     crow[i] = row;
     koff[i] = (uint32_t)(row * ROW_B + (pos ^ ((row / RSH) % CPR)) * 16);
-    voff[i] = (uint32_t)(row * ROW_B + (pos ^ (4 * ((row / RSH) % (CPR / 4)))) * 16);
+    voff[i] = (uint32_t)(row * ROW_B + (pos ^ (2 * ((row / RSH) % (CPR / 2)))) * 16);
   }
-  // operand read addresses inside stage 0 (see the prefill kernel for the layout)
+  // Operand read addresses inside stage 0.  K: sixteen lanes read one chunk of sixteen rows.  V: the transposing read of
+  // half a wave covers 32 bytes of each of eight rows, which the permutation spreads over all banks.
   uint32_t k_ad[KS], v_ad[DT];
   {
     const uint32_t k_rd = (uint32_t)(mcol * ROW_B) | (uint32_t)(((g ^ ((mcol / RSH) % CPR)) & (CPR - 1)) * 16);
 #pragma unroll
-    for (int s = 0; s < KS; ++s) k_ad[s] = ring0 + (k_rd ^ (uint32_t)(32 * s));
-    const int grp16 = lane & 15, dhalf = (lane >> 4) & 1, v_row = 4 * g + (grp16 >> 2);
+    for (int s = 0; s < KS; ++s) k_ad[s] = ring0 + (k_rd ^ (uint32_t)(64 * s));
+    const int v_row = 4 * g + (mcol >> 2);
     const uint32_t v_rd = (uint32_t)(v_row * ROW_B) +
-                          (uint32_t)(((2 * dhalf + ((grp16 & 3) >> 1)) ^ (4 * ((v_row / RSH) % (CPR / 4)))) * 16 +
-                                     8 * (grp16 & 1));
+                          (uint32_t)((((mcol & 3) >> 1) ^ (2 * ((v_row / RSH) % (CPR / 2)))) * 16 + 8 * (mcol & 1));
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) v_ad[dt] = ring0 + TILE_B + (v_rd ^ (uint32_t)(64 * dt));
+    for (int dt = 0; dt < DT; ++dt) v_ad[dt] = ring0 + TILE_B + (v_rd ^ (uint32_t)(32 * dt));
   }
 
   const RowChunks<kGqaChunk, true> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, target);
@@ -745,122 +753,134 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     const char* kbase = reinterpret_cast<const char*>(kc + ((int64_t)b * sumC + seg0 + r_begin) * D);
     const char* vbase = reinterpret_cast<const char*>(vc + ((int64_t)b * sumC + seg0 + r_begin) * D);
 
-    // Q^T fragments: column mcol = query head, k-step s holds Q[mcol][16 s + 8 g .. +7]
+    // Q^T fragments: column mcol = query head, k-step s holds Q[mcol][32 s + 8 g .. +7]
     u32x4 qf[KS];
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       u32x4 z = {0, 0, 0, 0};
-      qf[s] = (mcol < G) ? *reinterpret_cast<const u32x4*>(q + (bh * G + mcol) * D + 16 * s + 8 * g) : z;
+      qf[s] = (mcol < G) ? *reinterpret_cast<const u32x4*>(q + (bh * G + mcol) * D + 32 * s + 8 * g) : z;
       qf[s] ^= u32x4{q_sign, q_sign, q_sign, q_sign};
     }
-    f32x16 oacc[DT];
+    f32x4 oacc[DT];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) oacc[dt][i] = 0.f;
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
 
     // tile t: rows [32 t, 32 t + 32) of the wave's share, into stage t % kGqaStages; rows past the
     // end repeat the last row (their scores are masked)
-    auto issue = [&](int t) __attribute__((always_inline)) {
-      const char* ksrc = kbase + (int64_t)t * TILE_B;
-      const char* vsrc = vbase + (int64_t)t * TILE_B;
-      const uint32_t dst = ring0 + (t % kGqaStages) * STAGE_B;
+    auto issue = [&](const char* base, const uint32_t (&off)[NCP], uint32_t dst, int t) __attribute__((always_inline)) {
+      const char* src = base + (int64_t)t * TILE_B;
+      dst += (t % kGqaStages) * STAGE_B;
       const int last = n_rows - 1 - t * kGqaTile;   // last valid row of the tile, >= 0
       if (last >= kGqaTile - 1) {
 #pragma unroll
-        for (int i = 0; i < NCP; ++i) async_copy16<NT>(ksrc, koff[i], dst + i * 1024);
-#pragma unroll
-        for (int i = 0; i < NCP; ++i) async_copy16<NT>(vsrc, voff[i], dst + TILE_B + i * 1024);
+        for (int i = 0; i < NCP; ++i) async_copy16<NT>(src, off[i], dst + i * 1024);
       } else {
 #pragma unroll
         for (int i = 0; i < NCP; ++i)
-          async_copy16<NT>(ksrc, koff[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + i * 1024);
-#pragma unroll
-        for (int i = 0; i < NCP; ++i)
-          async_copy16<NT>(vsrc, voff[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + TILE_B + i * 1024);
+          async_copy16<NT>(src, off[i] - (uint32_t)(max(crow[i] - last, 0) * ROW_B), dst + i * 1024);
       }
     };
-    if (n_t > 0) issue(0);
-    if (kGqaStages > 1 && n_t > 1) issue(1);
+    auto issue_k = [&](int t) __attribute__((always_inline)) { issue(kbase, koff, ring0, t); };
+    auto issue_v = [&](int t) __attribute__((always_inline)) { issue(vbase, voff, ring0 + TILE_B, t); };
+    static_assert(kGqaStages == 2, "the waits below count two stages");
+    if (n_t > 0) { issue_k(0); issue_v(0); }
+    if (n_t > 1) { issue_k(1); issue_v(1); }
     // the Q loads are older than every copy: pin their arrival here
-    if (kGqaStages > 1 && n_t > 1) wait_vm(4 * NCP); else if (n_t > 0) wait_vm(2 * NCP);
+    if (n_t > 1) wait_vm(4 * NCP); else if (n_t > 0) wait_vm(2 * NCP);
 #pragma unroll
     for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
 
+    // K and V of a tile are waited for, and their stages filled again, each by itself: three or four of the wave's four
+    // half stages are in flight all the time (with whole tiles one of two stages while a tile is worked on).
     for (int t = 0; t < n_t; ++t) {
-      if (kGqaStages > 1 && t + 1 < n_t) wait_vm(2 * NCP); else wait_vm(0);   // tile t has landed; tile t+1 may be in flight
+      if (t + 1 < n_t) wait_vm(3 * NCP); else wait_vm(NCP);   // K(t) has landed; V(t), K(t+1), V(t+1) may be in flight
       const uint32_t so = (uint32_t)((t % kGqaStages) * STAGE_B);
       // ---- S^T = K . Q^T ----
-      f32x16 st;
+      f32x4 st[KT];
       {
-        u32x4 kf[KS];
+        u32x4 kf[KT][KS];
 #pragma unroll
-        for (int s = 0; s < KS; ++s) kf[s] = lds_load16(k_ad[s] + so, 0);
-        f32x16 z;
+        for (int s = 0; s < KS; ++s)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) z[i] = 0.f;
-        st = M::mfma(kf[0], qf[0], z);
+          for (int k = 0; k < KT; ++k) kf[k][s] = lds_load16(k_ad[s] + so, 16 * k * ROW_B);
 #pragma unroll
-        for (int s = 1; s < KS; ++s) st = M::mfma(kf[s], qf[s], st);
+        for (int k = 0; k < KT; ++k) st[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+          for (int k = 0; k < KT; ++k) st[k] = M::mfma16(kf[k][s], qf[s], st[k]);
       }
-      // ---- softmax over the 32 keys (element i of a lane: key 8 (i / 4) + 4 g + i % 4) ----
+      if (t + kGqaStages < n_t) {
+        wait_lds();   // this K stage has been read
+        issue_k(t + kGqaStages);
+      }
+      // ---- softmax over the 32 keys (element i of tile k: key 16 k + 4 g + i) ----
       const int n_valid = n_rows - t * kGqaTile;
       if (n_valid < kGqaTile) {
-        int thr = n_valid - 4 * g;
+        const int thr = n_valid - 4 * g;
 #pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (8 * (i >> 2) + (i & 3) >= thr) st[i] = -INFINITY;
+        for (int k = 0; k < KT; ++k)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (16 * k + i >= thr) st[k][i] = -INFINITY;
       }
-      float mx = st[0];
+      // a lane has a quarter of its column's keys: that one of them is too large is seen by the lane that has it, and
+      // the column's maximum is needed only then
+      float mx = st[0][0];
 #pragma unroll
-      for (int i = 1; i < 16; ++i) mx = fmaxf(mx, st[i]);
-      mx = max_with_other_half(mx);
-      const float m_cand = mx * scale_log2;   // finite: key 0 of the tile is valid
-      if (__any(m_cand > m_run + kRescaleStep)) {
+      for (int k = 0; k < KT; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, st[k][i]);
+      if (__any(mx * scale_log2 > m_run + kRescaleStep)) {
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = max_with_other_half(mx);
         // an integer reference exponent: the rounding of the weights below is then independent of it
-        const float m_new = __builtin_ceilf(fmaxf(m_run, m_cand));
+        const float m_new = __builtin_ceilf(fmaxf(m_run, mx * scale_log2));   // finite: key 0 of the tile is valid
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) oacc[dt][i] *= alpha;
+          for (int i = 0; i < 4; ++i) oacc[dt][i] *= alpha;
         m_run = m_new;
       }
-      uint32_t pf[8];
+      uint32_t pf[4];   // P^T in B-operand order: contraction slot 8 g + 4 k + i is key 16 k + 4 g + i
       float psum = 0.f;
 #pragma unroll
-      for (int i = 0; i < 16; i += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[i], scale_log2, -m_run));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[i + 1], scale_log2, -m_run));
-        pf[i >> 1] = M::pack_rne(p0, p1);
-        psum += p0 + p1;
-      }
-      l_run += psum;
-      // ---- O^T += V^T . P^T ----
+      for (int k = 0; k < KT; ++k)
 #pragma unroll
-      for (int tk = 0; tk < 2; ++tk) {
-        const u32x4 bfrag = {pf[4 * tk], pf[4 * tk + 1], pf[4 * tk + 2], pf[4 * tk + 3]};
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const u32x2 lo = lds_load_tr16(v_ad[dt] + so, (16 * tk) * ROW_B);
-          const u32x2 hi = lds_load_tr16(v_ad[dt] + so, (16 * tk + 8) * ROW_B);
-          oacc[dt] = M::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, bfrag, oacc[dt]);
+        for (int i = 0; i < 4; i += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i], scale_log2, -m_run));
+          const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(st[k][i + 1], scale_log2, -m_run));
+          pf[2 * k + (i >> 1)] = M::pack_rne(p0, p1);
+          psum += p0 + p1;
         }
+      l_run += psum;
+      // V(t) has landed; K(t+1), V(t+1), K(t+2) may be in flight
+      if (t + 2 < n_t) wait_vm(3 * NCP); else if (t + 1 < n_t) wait_vm(2 * NCP); else wait_vm(0);
+      // ---- O^T += V^T . P^T ----
+      const u32x4 bfrag = {pf[0], pf[1], pf[2], pf[3]};
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const u32x2 lo = lds_load_tr16(v_ad[dt] + so, 0);
+        const u32x2 hi = lds_load_tr16(v_ad[dt] + so, 16 * ROW_B);
+        oacc[dt] = M::mfma16(u32x4{lo.x, lo.y, hi.x, hi.y}, bfrag, oacc[dt]);
       }
-      if (t + kGqaStages < n_t) issue(t + kGqaStages);   // every read of this stage has returned
+      if (t + kGqaStages < n_t) {
+        wait_lds();   // this V stage has been read
+        issue_v(t + kGqaStages);
+      }
     }
 
     // ---- the wave's result per query head: (m, l, O[d]) ----
     {
-      const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+      float l_tot = l_run + __shfl_xor(l_run, 16, 64);
+      l_tot += __shfl_xor(l_tot, 32, 64);
       float* s_acc_w = reinterpret_cast<float*>(s_mem + wave * (kGqaStages * STAGE_B));
       if (mcol < G) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) s_acc_w[mcol * D + 32 * dt + 8 * (i >> 2) + 4 * g + (i & 3)] = oacc[dt][i];
+        for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<f32x4*>(s_acc_w + mcol * D + 16 * dt + 4 * g) = oacc[dt];
         if (g == 0) {
           s_m[wave][mcol] = m_run;
           s_l[wave][mcol] = l_tot;

@@ -7,6 +7,7 @@
 namespace moa {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
@@ -20,6 +21,9 @@ struct PF16 {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                   __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
   }
+  static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
   static __device__ __forceinline__ uint32_t pack_rne(float lo, float hi) {   // one v_cvt_pk_f16_f32
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     h2 r = {(_Float16)lo, (_Float16)hi};
@@ -30,6 +34,9 @@ struct PBF16 {
   static __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
                                                    __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
   }
   static __device__ __forceinline__ uint32_t pack_rne(float lo, float hi) {   // one v_cvt_pk_bf16_f32
     f32x2 x = {lo, hi};
@@ -87,7 +94,9 @@ __device__ __forceinline__ uint32_t lds_address(const char* p) {
 // Wait until at most n of this wave's global loads / async copies are outstanding.
 __device__ __forceinline__ void wait_vm(int n) {
   if (n >= 32) asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
+  else if (n >= 24) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
   else if (n >= 16) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  else if (n >= 12) asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
   else if (n >= 8) asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
   else if (n >= 6) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
   else if (n >= 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
@@ -96,6 +105,9 @@ __device__ __forceinline__ void wait_vm(int n) {
   else if (n == 1) asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
+
+// Wait until every LDS read of this wave has returned: the stage it read may be copied into again.
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 // Work-group barrier WITHOUT the memory fence of __syncthreads(): the fence would make every wave
 // wait for all of its outstanding async copies (vmcnt(0)) at each phase boundary and serialise the

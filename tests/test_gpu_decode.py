@@ -319,6 +319,24 @@ def test_grouped_query_boundaries_and_invariants(dev, G, B):
     assert (ones.float() - expect.float()).abs().max().item() <= 1e-3
 
 
+@pytest.mark.parametrize("scale", [0.09, -0.09])
+@pytest.mark.parametrize("B", [1, 33])            # chunks of 256 rows (two tiles to a wave), of 2048 (sixteen)
+@pytest.mark.parametrize("G", [2, 8])
+@pytest.mark.parametrize("D", [128, 64])
+def test_grouped_query_tile_edges(dev, D, G, B, scale):
+    """Shares of a wave that end inside, at and behind a 16-key tile of the scores and a 32-row stage, of one to several
+    stages."""
+    from moa_amd import mixture_of_sparse_attention
+    rng = np.random.default_rng(D + G + B)
+    sizes = [1, 15, 16, 17, 31, 32, 33, 65, 97, 2048 + 513]
+    q, kc, vc, hs, hv = _case(rng, B, sizes, D, torch.float16, dev)
+    q = torch.from_numpy(rng.standard_normal((B, len(sizes) * G, 1, D)).astype(np.float32)).to(dev, torch.float16)
+    out = mixture_of_sparse_attention(q, kc, vc, scale, head_start_index=torch.from_numpy(hs).to(dev),
+                                      head_valid_length=torch.from_numpy(hv).to(dev))
+    few = slice(0, 2)   # rows of the batch that the oracle does
+    _close_grouped(out[few, 0], q[few, :, 0], kc[few], vc[few], hs[few], hv[few], scale, G, (D, G, B))
+
+
 @pytest.mark.parametrize("B", [1, 2])
 def test_grouped_query_small_batch_even_split(dev, B):
     """Batch 1 and 2 at the largest config's ring sizes (8 rings of 2 k to 24 k rows, 8 query heads each,
