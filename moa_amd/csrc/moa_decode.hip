@@ -401,7 +401,8 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   __shared__ float s_m[kDecWaves][G];
   __shared__ float s_l[kDecWaves][G];
 
-  const int b = blockIdx.y;
+  const int b = PIPE ? blockIdx.x : blockIdx.y;   // see kDecPipeFrom
+  const int place = PIPE ? blockIdx.y : blockIdx.x, places = PIPE ? gridDim.y : gridDim.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -410,9 +411,9 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
 
   const RowChunks<CHUNK, false> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, 0);
 
-  if (MERGE && counters && blockIdx.x == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
+  if (MERGE && counters && place == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
 
-  for (int w = blockIdx.x; w < row.total; w += gridDim.x) {
+  for (int w = place; w < row.total; w += places) {
     const Chunk ck = row.at(w, H);
     const int c = ck.index, n_chunks = ck.count;
     const int64_t bh = (int64_t)b * H + ck.head;
@@ -649,6 +650,10 @@ __global__ __launch_bounds__(kDecThreads) void decode_merge_kernel(
 // Work-groups per CU the grid may hold.  A CU runs one at a time (the LDS rings fill it), so the hardware
 // dispatcher hands out chunks as CUs become free when every chunk is a work-group of its own: 602 us at
 // batch 64 of the 70B shape against 612-628 us with 2-16 per CU, each walking several chunks in a fixed order.
+// The grid has batch rows side by side, chunk numbers outside: a row's chunks are fewer than the host can count on, and the
+// work-groups that find none come last then.  Between the rows they delay what stands behind them, since work-groups go to
+// the XCDs strictly in turn: a chunk waits for its XCD while another has CUs free.  Batch 32 of 8 rings of up to 6800 rows,
+// 4 heads 107.1 -> 89.0 us, batch 12 of up to 17000, 8 heads 96.7 -> 87.4, batch 24 of 2 rings 25.8 -> 19.6.
 constexpr int kGqaBlocksPerCu = 64;
 // Largest number of cache rows per work-group step (a quarter per wave) the launch aims for; the actual
 // chunk lengths come out of an even split of every batch row (RowChunks).  A chunk start costs a
@@ -700,7 +705,7 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
   __shared__ float s_l[kGqaWaves][kGqaMaxG];
   static_assert(kGqaMaxG * D * 4 <= kGqaStages * STAGE_B, "the result buffer fits the wave's ring");
 
-  const int b = blockIdx.y;
+  const int b = blockIdx.x;   // batch rows side by side (see kGqaBlocksPerCu)
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -735,9 +740,9 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
 
   const RowChunks<kGqaChunk, true> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, target);
 
-  if (MERGE && counters && blockIdx.x == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
+  if (MERGE && counters && blockIdx.y == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
 
-  for (int w = blockIdx.x; w < row.total; w += gridDim.x) {
+  for (int w = blockIdx.y; w < row.total; w += gridDim.y) {
     const Chunk ck = row.at(w, H);
     const int c = ck.index, n_chunks = ck.count;
     const int64_t bh = (int64_t)b * H + ck.head;
@@ -951,6 +956,9 @@ constexpr int kDecBlocksPerCu = 16;   // work-groups per CU over the whole grid
 // 160 chunks 11.3 with half-length ones.  Pipelining pays where several work-groups follow each other on a CU: 814 chunks of
 // 64-element rows 23.5 us with, 22.6 without, 864 of 128 40.2 and 39.6, 1152 49.5 and 49.4, 1440 59.2 both.
 constexpr int kDecSmallBelow = 1;
+// These launches also have the batch rows side by side in the grid (see kGqaBlocksPerCu): batch 64 of 32 rings of 128 852.7
+// -> 825.9 us, batch 16 215.9 -> 210.7; smaller ones are as fast or faster row by row (246 chunks 10.2 and 10.4 us), with no
+// more work-groups to a row than it can have chunks (690 chunks 18.7 -> 16.9 us).
 constexpr int kDecPipeFrom = 4;
 
 // From this many bytes of K and V per launch on they are read non-temporally.  What a step reads of one layer
@@ -1010,15 +1018,15 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
                          int H, int64_t sumC, float sm_scale, unsigned* counters, hipStream_t st) {
   const int cap = (int)decode_cap(sumC, H);
   const int64_t chunks = (sumC + kChunk - 1) / kChunk + H;   // per batch row, at the normal chunk length
-  // 16 work-groups per CU over the whole grid (measured: 8 leaves a visible tail, 32 is no better),
-  // never more per batch row than chunks exist
-  int bx = (int)((256 * kDecBlocksPerCu + B - 1) / B);
-  if (bx > cap) bx = cap;
-  if (bx < 1) bx = 1;
   const bool pipe = (int64_t)B * chunks >= (int64_t)256 * kDecPipeFrom;
   const bool small = (int64_t)B * chunks < (int64_t)256 * kDecSmallBelow;
+  // 16 work-groups per CU over the whole grid (measured: 8 leaves a visible tail, 32 is no better),
+  // never more per batch row than chunks exist
+  int64_t bx = (256 * kDecBlocksPerCu + B - 1) / B;
+  if (bx > (small ? cap : chunks)) bx = small ? cap : chunks;
+  if (bx < 1) bx = 1;
   auto launch = [&](auto split, auto merge) {
-    hipLaunchKernelGGL(split, dim3(bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
+    hipLaunchKernelGGL(split, pipe && !small ? dim3(B, (unsigned)bx) : dim3((unsigned)bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
                        (const uint16_t*)vc, (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, sumC,
                        sm_scale * kLog2e, cap, counters);
     if (int rc = check_launch("moa_decode_fwd(split)")) return rc;
@@ -1046,21 +1054,22 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
                              float* part_ml, const int64_t* head_start, const int64_t* head_valid, int B,
                              int H, int G, int64_t sumC, float sm_scale, unsigned* counters, hipStream_t st) {
   const int cap = (int)decode_cap(sumC, H);   // partial slots per batch row the workspace was sized for
-  // Chunk policy.  Chunks of kGqaChunk rows when they give at least half of the CUs a chunk: a chunk start costs three
-  // dependent memory latencies (ring index, query rows, first tiles).  Measured at the 70B shape (8 rings per batch
-  // row, 104 k rows) with one fixed length, before the copies were non-temporal: 49.8 us per call at batch 4 with
-  // 2048-row chunks, 53.3 with 1024, 62.3 with 512.  Below that (batch 1 and 2 at that shape: 54 and 108 chunks) every
-  // batch row is split evenly into its share of 256 chunks instead: 25.8 against 32.4 us at batch 1, 33.5 against 36-39
-  // us at batch 2.  From batch 3 on one even round of 256 chunks gains nothing at that shape, with the present copies
-  // either: 35.4 us with 2048-row chunks against 48.2 us at batch 3, 41.5 against 42.0 at 4, 71.0 against 78.8 at 6, 76.2
-  // against 75.1 at 8, 149.9 against 200.8 at 16.  The host does not know how full the rings are; it plans with their
-  // capacity.
+  // Chunk policy.  A chunk start costs three dependent memory latencies (ring index, query rows, first tiles), so chunks of
+  // kGqaChunk rows are the rule.  Where those leave many CUs idle, all the time or in the last of few rounds, every batch row is split
+  // evenly into its share of one or two rounds of 256 chunks instead.  By the number of chunks of kGqaChunk rows, GPU time
+  // with those and with (256 chunks, 512 chunks):
+  //   D = 128: 54 32.4 (25.8)   129 30.8 us (27.3, 31.1)   140 31.8 (28.7, 32.8)   172 33.2 (33.1)   176 32.6 (33.7, 35.9)
+  //     215 37.9 (39.6, 42.0)   258 57.4 (46.2, 48.4)   344 67.6 (59.5, 59.7)   516 88.5 (85.2, 83.5)   688 108.8 (115.7, 109.5)
+  //   D = 64: 136 19.2 (17.9, 19.6)   220 21.7 (23.2, 22.3)   264 30.9 (28.9, 29.5)   280 30.2 (29.9, 28.8)
+  // The host does not know how full the rings are; it plans with their capacity.
   const int64_t fixed_chunks = (int64_t)B * (sumC / kGqaChunk + (H + 1) / 2);
   int64_t target = 0;   // 0: chunks of kGqaChunk rows; kShortChunks: of kEvenMinChunk
-  if (fixed_chunks <= 128) {
-    target = (256 + B - 1) / B;
+  if (fixed_chunks <= 160 || (fixed_chunks > 240 && fixed_chunks <= 560)) {
+    const int64_t all = fixed_chunks <= 400 ? 256 : 512;
+    target = fixed_chunks <= 128 ? (all + B - 1) / B : all / B;   // past one round by a few, those cost a round of their own
+    if (fixed_chunks > 128 && 2 * target < 3 * H) target = 0;   // short rings: a chunk or two each either way
     if (target > cap) target = cap;
-    if ((sumC + kEvenMinChunk - 1) / kEvenMinChunk + H <= target) target = kShortChunks;
+    if (target > 0 && (sumC + kEvenMinChunk - 1) / kEvenMinChunk + H <= target) target = kShortChunks;
   }
   // at most this many chunks per batch row (a work-group without a chunk still holds a CU while it finds that out)
   const int64_t fixed_rows = target == kShortChunks ? kEvenMinChunk : kGqaChunk;
@@ -1080,7 +1089,7 @@ static int launch_decode_gqa(const void* q, const void* kc, const void* vc, void
   const auto kernel = nt ? &decode_gqa_kernel<T, D, true> : &decode_gqa_kernel<T, D, false>;
   if (int rc = reserve_lds(reinterpret_cast<const void*>(kernel), lds, lds_reserved[nt], "moa_decode_fwd"))
     return rc;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)bx, B), dim3(kGqaThreads), lds, st,
+  hipLaunchKernelGGL(kernel, dim3(B, (unsigned)bx), dim3(kGqaThreads), lds, st,
                      (const uint16_t*)q, (const uint16_t*)kc, (const uint16_t*)vc, (uint16_t*)o,
                      part_acc, part_ml, head_start, head_valid, H, G, sumC, mfma_softmax_scale(sm_scale), cap,
                      (int)target, counters);

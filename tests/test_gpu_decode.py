@@ -337,6 +337,23 @@ def test_grouped_query_tile_edges(dev, D, G, B, scale):
     _close_grouped(out[few, 0], q[few, :, 0], kc[few], vc[few], hs[few], hv[few], scale, G, (D, G, B))
 
 
+@pytest.mark.parametrize("sizes,B", [([5000], 50), ([5000], 100), ([5000], 150), ([1500, 700], 70), ([300, 200, 90], 90)])
+def test_grouped_query_split_into_rounds(dev, sizes, B):
+    """Launches whose batch rows are split into their share of one round of work-groups, or of two, and one whose short
+    rings are not; rows of a batch that are filled unlike, empty ones among them."""
+    from moa_amd import mixture_of_sparse_attention
+    rng = np.random.default_rng(B)
+    G, D, scale = 3, 64, 0.12
+    q, kc, vc, hs, hv = _case(rng, B, sizes, D, torch.float16, dev, fill="partial")
+    hv[1], hv[-1] = 0, sizes
+    q = torch.from_numpy(rng.standard_normal((B, len(sizes) * G, 1, D)).astype(np.float32)).to(dev, torch.float16)
+    out = mixture_of_sparse_attention(q, kc, vc, scale, head_start_index=torch.from_numpy(hs).to(dev),
+                                      head_valid_length=torch.from_numpy(hv).to(dev))
+    assert not out[1].any()
+    few = [0, B // 2, B - 1]   # rows of the batch that the oracle does
+    _close_grouped(out[few, 0], q[few, :, 0], kc[few], vc[few], hs[few], hv[few], scale, G, (sizes, B))
+
+
 @pytest.mark.parametrize("B", [1, 2])
 def test_grouped_query_small_batch_even_split(dev, B):
     """Batch 1 and 2 at the largest config's ring sizes (8 rings of 2 k to 24 k rows, 8 query heads each,
