@@ -15,8 +15,8 @@
 //     lanes of a row; the softmax is the usual running (max, sum) in fp32,
 //     base 2, rescaled once per batch of rows;
 //   * segments differ in length by ~80x between heads, so the unit of work is
-//     a fixed-size chunk of rows, not a head: block (x, b) walks the chunks
-//     x, x+gridDim.x, ... of batch row b, locating (head, chunk) through a
+//     a fixed-size chunk of rows, not a head: a work-group walks every n-th
+//     chunk of a batch row, locating (head, chunk) through a
 //     prefix sum over the row's heads that every wave forms from
 //     head_valid_len (no host knowledge of the lengths, no host sync);
 //   * a head with one chunk writes its output directly; otherwise chunks
