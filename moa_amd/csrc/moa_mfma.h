@@ -111,7 +111,8 @@ __device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)"
 
 // Work-group barrier WITHOUT the memory fence of __syncthreads(): the fence would make every wave
 // wait for all of its outstanding async copies (vmcnt(0)) at each phase boundary and serialise the
-// copy pipeline.  What must be visible at a barrier is waited for explicitly with wait_vm().
+// copy pipeline.  What must be visible at a barrier is waited for explicitly with wait_vm(); so are LDS accesses, with
+// wait_lds(), where no use of theirs in front of the barrier is certain.
 __device__ __forceinline__ void phase_barrier() {
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_barrier();

@@ -178,6 +178,9 @@ __device__ __forceinline__ void tile_qk(f32x16 (&st)[2], const u32x4 (&qf)[D / 1
 #pragma unroll
     for (int s = 0; s < KS; ++s) st[nt] = T::mfma(kf[s], qf[s], st[nt]);
   }
+  // The next barrier lets other waves copy over this K stage.  Unlike in tile_matrix nothing else keeps the products, and
+  // with them the compiler's wait for these reads, in front of it.
+  wait_lds();
 }
 
 // P.V only (the last iteration)
