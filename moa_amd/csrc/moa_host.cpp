@@ -13,6 +13,7 @@
 #include <ATen/ATen.h>
 
 #include <climits>
+#include <initializer_list>
 
 #include "../../include/moa_hip.h"
 
@@ -64,12 +65,29 @@ PyObject* failed(int rc) {
   return nullptr;
 }
 
+// The addresses of a call's tensors.  To ask a tensor for its address can copy it (copy-on-write) and throw, so this is
+// done with the interpreter's lock held, in front of the launch that goes without.
+class Addresses {
+  void* p_[9] = {};
+
+ public:
+  explicit Addresses(std::initializer_list<const at::Tensor*> tensors) {
+    void** p = p_;
+    for (const at::Tensor* t : tensors) *p++ = t->data_ptr();
+  }
+  void* operator[](int i) const { return p_[i]; }
+  int64_t* i64(int i) const { return static_cast<int64_t*>(p_[i]); }
+};
+
 // The tensors of one layer of a cache, in the order of the calls below.
 struct Layer {
   const at::Tensor &kc, &vc, &mask, &update_index, &valid_len, &circ_head, &circ_size, &static_size, &max_len;
   explicit Layer(PyObject* const* a)
       : kc(tensor(a[0])), vc(tensor(a[1])), mask(tensor(a[2])), update_index(tensor(a[3])), valid_len(tensor(a[4])),
         circ_head(tensor(a[5])), circ_size(tensor(a[6])), static_size(tensor(a[7])), max_len(tensor(a[8])) {}
+  Addresses all() const {
+    return Addresses({&kc, &vc, &mask, &update_index, &valid_len, &circ_head, &circ_size, &static_size, &max_len});
+  }
   bool fits(at::Device device, at::ScalarType type, int64_t B, int64_t H, int64_t D) const {
     if (kc.dim() != 3) return false;
     const int64_t sumC = kc.size(1);
@@ -87,8 +105,6 @@ bool all_plain(PyObject* const* a, Py_ssize_t n) {
     if (!plain(a[i])) return false;
   return true;
 }
-int64_t* i64(const at::Tensor& t) { return static_cast<int64_t*>(t.data_ptr()); }
-
 bool number(PyObject* o, double* x) {
   if (!PyFloat_Check(o) && !PyLong_Check(o)) return false;
   *x = PyFloat_AsDouble(o);
@@ -133,11 +149,11 @@ PyObject* decode(PyObject* query, const at::Tensor& k, const at::Tensor& v, cons
   Py_DECREF(scratch);
   if (PyErr_Occurred()) return nullptr;
   at::Tensor o = at::empty({B, 1, Hq, D}, q.options());
+  const Addresses p({&q, &k, &v, &o, &start, &valid});
   int rc;
   Py_BEGIN_ALLOW_THREADS;
-  rc = decode_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ws, (size_t)ws_bytes, (uint32_t*)counters,
-                  (size_t)n_counters, i64(start), i64(valid), (int)B, (int)Hq, (int)Hkv, (int)D, sumC, (float)scale,
-                  dtype_code(type), stream);
+  rc = decode_fwd(p[0], p[1], p[2], p[3], ws, (size_t)ws_bytes, (uint32_t*)counters, (size_t)n_counters, p.i64(4), p.i64(5),
+                  (int)B, (int)Hq, (int)Hkv, (int)D, sumC, (float)scale, dtype_code(type), stream);
   Py_END_ALLOW_THREADS;
   if (rc != MOA_OK) return failed(rc);
   return THPVariable_Wrap(std::move(o));
@@ -170,11 +186,11 @@ PyObject* prefill(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
   Py_DECREF(stream_object);
   at::Tensor o = at::empty({B, N, Hq, D}, q.options());
   const int64_t os[] = {o.stride(0), o.stride(2), o.stride(1), 1};
+  const Addresses p({&q, &k, &v, &o, &sink, &local});
   int rc;
   Py_BEGIN_ALLOW_THREADS;
-  rc = prefill_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), q.strides().data(), k.strides().data(),
-                   v.strides().data(), os, (int)B, (int)Hq, (int)Hkv, (int)N, (int)D, i64(sink), i64(local), (float)scale,
-                   dtype_code(type), stream);
+  rc = prefill_fwd(p[0], p[1], p[2], p[3], q.strides().data(), k.strides().data(), v.strides().data(), os, (int)B, (int)Hq,
+                   (int)Hkv, (int)N, (int)D, p.i64(4), p.i64(5), (float)scale, dtype_code(type), stream);
   Py_END_ALLOW_THREADS;
   if (rc != MOA_OK) return failed(rc);
   return THPVariable_Wrap(std::move(o));
@@ -221,12 +237,11 @@ PyObject* rope_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Py_DECREF(stream_object);
   const int64_t qs[] = {q.stride(0), q.stride(1), q.stride(3)}, ks[] = {k.stride(0), k.stride(1), k.stride(3)},
                 vs[] = {v.stride(0), v.stride(1), v.stride(3)};
+  const Addresses p({&q, &k, &v, &cos, &sin, &q_out}), l(layer.all());
   int rc;
   Py_BEGIN_ALLOW_THREADS;
-  rc = rope_append_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), qs, ks, vs, cos.data_ptr(), sin.data_ptr(),
-                       cos.size(0) == 1 ? 0 : cos.stride(0), q_out.data_ptr(), layer.kc.data_ptr(), layer.vc.data_ptr(),
-                       i64(layer.mask), i64(layer.update_index), i64(layer.valid_len), i64(layer.circ_head),
-                       i64(layer.circ_size), i64(layer.static_size), i64(layer.max_len), kv_len, (int)B, (int)Hq, (int)H,
+  rc = rope_append_fwd(p[0], p[1], p[2], qs, ks, vs, p[3], p[4], cos.size(0) == 1 ? 0 : cos.stride(0), p[5], l[0], l[1],
+                       l.i64(2), l.i64(3), l.i64(4), l.i64(5), l.i64(6), l.i64(7), l.i64(8), kv_len, (int)B, (int)Hq, (int)H,
                        (int)D, layer.kc.size(1), dtype_code(type), stream);
   Py_END_ALLOW_THREADS;
   if (rc != MOA_OK) return failed(rc);
@@ -254,12 +269,11 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!stream_object) return nullptr;
   Py_DECREF(stream_object);
   const int64_t ks[] = {k.stride(0), k.stride(1), k.stride(3)}, vs[] = {v.stride(0), v.stride(1), v.stride(3)};
+  const Addresses p({&k, &v}), l(layer.all());
   int rc;
   Py_BEGIN_ALLOW_THREADS;
-  rc = append_fwd(k.data_ptr(), v.data_ptr(), ks, vs, layer.kc.data_ptr(), layer.vc.data_ptr(), i64(layer.mask),
-                  i64(layer.update_index), i64(layer.valid_len), i64(layer.circ_head), i64(layer.circ_size),
-                  i64(layer.static_size), i64(layer.max_len), kv_len, (int)B, (int)H, (int)D, layer.kc.size(1),
-                  dtype_code(type), stream);
+  rc = append_fwd(p[0], p[1], ks, vs, l[0], l[1], l.i64(2), l.i64(3), l.i64(4), l.i64(5), l.i64(6), l.i64(7), l.i64(8), kv_len,
+                  (int)B, (int)H, (int)D, layer.kc.size(1), dtype_code(type), stream);
   Py_END_ALLOW_THREADS;
   if (rc != MOA_OK) return failed(rc);
   Py_RETURN_TRUE;
