@@ -9,8 +9,10 @@ libmoa_hip.so; there is no Triton and no CPU path.
 """
 from __future__ import annotations
 
+import threading
 import warnings
-from typing import Dict, Optional, Tuple
+from collections import UserDict
+from typing import MutableMapping, Optional, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -25,9 +27,9 @@ _N_COUNTERS = 16384   # (batch row, ring) pairs up to which a decode launch may 
 
 
 class _DecodeScratch:
-    """What the decode calls of one (device, stream) share: a workspace that only ever grows and the zeroed counters of
-    moa_decode_fwd_counted, which every call leaves zeroed.  Steady-state calls allocate nothing and take the addresses
-    from here."""
+    """What the decode calls that a thread makes on one (device, stream) share: a workspace that only ever grows and the
+    zeroed counters of moa_decode_fwd_counted, which every call leaves zeroed.  Steady-state calls allocate nothing and
+    take the addresses from here."""
     __slots__ = ("ws", "ws_ptr", "ws_bytes", "counters", "counters_ptr")
 
     def __init__(self) -> None:
@@ -35,7 +37,13 @@ class _DecodeScratch:
         self.ws_bytes = 0
 
 
-_scratch: Dict[Tuple[int, int], _DecodeScratch] = {}
+class _ScratchOfThread(threading.local, UserDict):
+    """(device index, stream) -> _DecodeScratch, for every thread its own.  A decode is two launches or one that counts; the
+    launches of two threads on one stream may come in any order, and a thread may replace its workspace between another's
+    look at it and that one's launch.  What a thread held goes back to torch's allocator when it ends."""
+
+
+_scratch: MutableMapping[Tuple[int, int], _DecodeScratch] = _ScratchOfThread()
 
 
 def _decode_scratch(device: torch.device, stream: int, nbytes: int) -> Tuple[int, int, Optional[int]]:
@@ -44,9 +52,10 @@ def _decode_scratch(device: torch.device, stream: int, nbytes: int) -> Tuple[int
     graphs recorded on it, and where two launches count in the same place a lost count stays for good.  (Stream 0 cannot
     be recorded and is not asked, which saves its calls 0.5 us.)"""
     key = (device.index or 0, stream)
-    s = _scratch.get(key)
+    scratch = _scratch.data
+    s = scratch.get(key)
     if s is None:
-        s = _scratch[key] = _DecodeScratch()
+        s = scratch[key] = _DecodeScratch()
     if s.ws_bytes < nbytes:
         s.ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
         s.ws_ptr, s.ws_bytes = s.ws.data_ptr(), s.ws.numel()
