@@ -25,7 +25,7 @@ decltype(&moa_prefill_fwd_tokens) prefill_fwd = nullptr;
 decltype(&moa_rope_cache_append) rope_append_fwd = nullptr;
 decltype(&moa_cache_append) append_fwd = nullptr;
 PyObject* raw_stream = nullptr;       // device index -> address of torch's current stream there
-PyObject* decode_scratch = nullptr;   // (device, stream, bytes) -> workspace address, its bytes, counters' address or None
+PyObject* decode_scratch = nullptr;   // (device, stream, bytes) -> workspace address, its bytes, counters' address; None: being recorded
 PyObject* raise_error = nullptr;      // return code -> exception
 Py_ssize_t n_counters = 0;
 
@@ -131,7 +131,8 @@ PyObject* decode(PyObject* query, const at::Tensor& k, const at::Tensor& v, cons
   PyObject* const stream_object = current_stream(device, &stream);
   if (!stream_object) return nullptr;
   PyObject* const device_object = PyObject_GetAttrString(query, "device");
-  PyObject* const bytes = PyLong_FromSize_t(workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)D, sumC));
+  const size_t need = workspace_bytes((int)B, (int)Hq, (int)Hkv, (int)D, sumC);
+  PyObject* const bytes = PyLong_FromSize_t(need);
   PyObject* const request[] = {device_object, stream_object, bytes};
   PyObject* const scratch = device_object && bytes ? PyObject_Vectorcall(decode_scratch, request, 3, nullptr) : nullptr;
   Py_XDECREF(bytes);
@@ -140,14 +141,24 @@ PyObject* decode(PyObject* query, const at::Tensor& k, const at::Tensor& v, cons
   if (!scratch) return nullptr;
   void *ws = nullptr, *counters = nullptr;
   Py_ssize_t ws_bytes = 0;
+  bool recorded = false;
   if (PyTuple_Check(scratch) && PyTuple_GET_SIZE(scratch) == 3) {
-    ws = PyLong_AsVoidPtr(PyTuple_GET_ITEM(scratch, 0));
-    ws_bytes = PyLong_AsSsize_t(PyTuple_GET_ITEM(scratch, 1));
     PyObject* c = PyTuple_GET_ITEM(scratch, 2);
-    if (c != Py_None) counters = PyLong_AsVoidPtr(c);
+    recorded = c == Py_None;
+    if (!recorded) {
+      counters = PyLong_AsVoidPtr(c);
+      ws = PyLong_AsVoidPtr(PyTuple_GET_ITEM(scratch, 0));
+      ws_bytes = PyLong_AsSsize_t(PyTuple_GET_ITEM(scratch, 1));
+    }
   }
   Py_DECREF(scratch);
   if (PyErr_Occurred()) return nullptr;
+  at::Tensor own;   // a recorded call's workspace, until its launches are
+  if (recorded) {
+    own = at::empty({(int64_t)need}, q.options().dtype(at::kByte));
+    ws = own.data_ptr();
+    ws_bytes = (Py_ssize_t)need;
+  }
   at::Tensor o = at::empty({B, 1, Hq, D}, q.options());
   const Addresses p({&q, &k, &v, &o, &start, &valid});
   int rc;

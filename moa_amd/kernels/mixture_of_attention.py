@@ -46,21 +46,23 @@ class _ScratchOfThread(threading.local, UserDict):
 _scratch: MutableMapping[Tuple[int, int], _DecodeScratch] = _ScratchOfThread()
 
 
-def _decode_scratch(device: torch.device, stream: int, nbytes: int) -> Tuple[int, int, Optional[int]]:
-    """Address and size of the workspace, address of the counters or None.  A call that is being recorded into a graph
-    takes no counters (two launches, the same bits): a replay may run beside eager calls of this stream or beside other
-    graphs recorded on it, and where two launches count in the same place a lost count stays for good.  (Stream 0 cannot
-    be recorded and is not asked, which saves its calls 0.5 us.)"""
+def _decode_scratch(device: torch.device, stream: int, nbytes: int) -> Tuple[Optional[int], int, Optional[int]]:
+    """Address and size of the workspace, address of the counters.  None for the counters: the call is being recorded into
+    a graph, whose replays may run beside eager calls of this stream or beside other graphs recorded on it.  Such a call
+    takes neither from here.  Where two launches count in the same place a lost count stays for good, so it goes without
+    (two launches, the same bits); partials of two calls in the same place get mixed, and a workspace that is replaced goes
+    back to the allocator while the graph still writes to it, so it brings its own, from the graph's memory.  (Stream 0
+    cannot be recorded and is not asked, which saves its calls 0.5 us.)"""
     key = (device.index or 0, stream)
     scratch = _scratch.data
     s = scratch.get(key)
     if s is None:
         s = scratch[key] = _DecodeScratch()
+    if stream != 0 and torch.cuda.is_current_stream_capturing():
+        return s.ws_ptr, s.ws_bytes, None
     if s.ws_bytes < nbytes:
         s.ws = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=device)
         s.ws_ptr, s.ws_bytes = s.ws.data_ptr(), s.ws.numel()
-    if stream != 0 and torch.cuda.is_current_stream_capturing():
-        return s.ws_ptr, s.ws_bytes, None
     if s.counters is None:
         s.counters = torch.zeros(_N_COUNTERS, dtype=torch.int32, device=device)
         s.counters_ptr = s.counters.data_ptr()
@@ -177,6 +179,9 @@ def moa_decode(
     need = lib.moa_decode_workspace_bytes(B, Hq, Hkv, D, sumC)
     stream = _lib.current_stream_ptr(dev)
     ws, ws_bytes, counters = _decode_scratch(dev, stream, need)
+    if counters is None:   # being recorded
+        own = torch.empty(need, dtype=torch.uint8, device=dev)
+        ws, ws_bytes = own.data_ptr(), need
     rc = lib.moa_decode_fwd_counted(q3.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), ws, ws_bytes, counters,
                                     _N_COUNTERS, hs.data_ptr(), hv.data_ptr(), B, Hq, Hkv, D, sumC, float(sm_scale),
                                     _lib.dtype_code(q.dtype), stream)

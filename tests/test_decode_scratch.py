@@ -47,6 +47,23 @@ def test_threads_do_not_share_a_workspace():
     assert again1 == first1
 
 
+def test_a_recorded_call_leaves_no_workspace_behind(monkeypatch):
+    """What is allocated while a stream is recorded belongs to the graph: it is not kept for the stream's eager calls, and
+    theirs is not replaced."""
+    from moa_amd.kernels import mixture_of_attention as M
+    place, stream = torch.device("cpu"), -54321   # no stream of this value exists
+    monkeypatch.setitem(M._scratch, (0, stream), M._DecodeScratch())
+    recording = True
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: recording)
+    assert M._decode_scratch(place, stream, 512)[2] is None and M._scratch[(0, stream)].ws is None
+    recording = False
+    eager = M._decode_scratch(place, stream, 512)
+    recording = True
+    assert M._decode_scratch(place, stream, 1 << 20)[2] is None
+    recording = False
+    assert M._decode_scratch(place, stream, 512) == eager
+
+
 @pytest.fixture(scope="module")
 def dev():
     assert torch.cuda.is_available(), "these tests need the MI355X"
@@ -88,3 +105,44 @@ def test_threads_on_one_stream(dev, G, B, sizes):
     for i in range(3):
         for outs in got[i]:
             assert all(torch.equal(a, b) for a, b in zip(outs, want[i])), i
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("compiled", [True, False])
+@pytest.mark.parametrize("G,B,sizes", [(1, 40, [5000, 3000, 700]), (8, 1, [2000, 9000, 300]), (4, 1, [700, 1100, 300, 900])])
+def test_a_graph_keeps_its_workspace(dev, monkeypatch, compiled, G, B, sizes):
+    """Two graphs of one stream, the second with the longer call, and longer eager calls on it afterwards: replays of the
+    first, on another stream and beside them, are right and write to nothing of theirs."""
+    from moa_amd import _lib
+    if not compiled:
+        class Declines:
+            attend = staticmethod(lambda *args: None)
+        monkeypatch.setattr(_lib, "host", lambda: Declines)
+    small, large, larger = (_case(dev, G, b, sizes, 64, b) for b in (B, 2 * B, 4 * B))
+    want = [_attend(*c) for c in (small, large, larger)]
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graphs, recorded = [], []
+    with torch.cuda.stream(stream):
+        _attend(*small)
+        stream.synchronize()
+        for c in (small, large):
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=stream):
+                recorded.append(_attend(*c))
+        eager = _attend(*larger)   # replaces the stream's workspace
+        # what is given back is given out again
+        others = [torch.full((n << 10,), 7, dtype=torch.uint8, device=dev) for n in (64, 256, 512, 1024, 1024, 2048, 4096)]
+    torch.cuda.synchronize()
+    assert torch.equal(eager, want[2])
+    for i in range(4):
+        for r in recorded:
+            r.fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            graphs[0].replay()
+        with torch.cuda.stream(stream):
+            eager = _attend(*larger)
+            graphs[1].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(recorded[0], want[0]) and torch.equal(recorded[1], want[1]) and torch.equal(eager, want[2]), i
+        assert all((t == 7).all() for t in others), i

@@ -93,3 +93,16 @@ for name in calls():
             raise AssertionError((name, place))
         assert all(n == "moa_decode_workspace_bytes" for n, _ in seen), (name, place)
 """)
+
+
+def test_a_recorded_decode_brings_its_own_workspace(run):
+    """No counters in the scratch say that the call is being recorded: it does not take the stream's workspace."""
+    run("""
+for counters in (8192, None):
+    connect(lambda device, stream, nbytes: (4096, 256, counters))
+    call, args = calls()["decode"]
+    assert call(*args) is not None
+    name, a = seen.pop()
+    assert name == "moa_decode_fwd_counted" and a[6] == counters, a
+    assert (a[4] == 4096) == (counters is not None), a
+""")
