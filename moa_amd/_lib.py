@@ -1,12 +1,15 @@
 """ctypes binding of libmoa_hip.so (declared in include/moa_hip.h).
 
 There is no fallback: if the library is missing or does not load, every
-operator of this package raises.
+operator of this package raises.  (The compiled host side, _host.so, which
+makes the same calls of the library, may be missing: see host().)
 """
 from __future__ import annotations
 
 import ctypes
 import os
+import sys
+import warnings
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from typing import Optional, Sequence
 
@@ -101,20 +104,47 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+def host_is_built_for() -> str:
+    """What the compiled host side has to be built for to be loaded here: it uses torch's C++ classes and Python's."""
+    import torch
+
+    return f"torch {torch.__version__}, Python {sys.version_info[0]}.{sys.version_info[1]}"
+
+
+def host_fits() -> bool:
+    """Is there a compiled host side, and was it built for this torch and Python?  (Looked up in the file: one that was not is
+    not loaded.)"""
+    try:
+        with open(HOST_PATH, "rb") as f:
+            return f"moa_host was built for {host_is_built_for()};".encode() in f.read()
+    except OSError:
+        return False
+
+
+class _NoHost:
+    """Takes no call: the Python code behind it takes all of them, through ctypes."""
+    attend = rope_append = append = staticmethod(lambda *args: None)
+
+
 def host():
-    """The compiled host side of the attention and the append (csrc/moa_host.cpp), loaded once and bound to the library."""
+    """The compiled host side of the attention and the append (csrc/moa_host.cpp), loaded once and bound to the library.
+    It only saves time.  Where it is missing or was built for another torch, the calls go through the Python code."""
     global _host
     if _host is not None:
         return _host
     import torch  # noqa: F401  (its libraries are what the module is linked to)
 
     lib = load()
-    if not os.path.exists(HOST_PATH):
-        raise MoaKernelError(f"{HOST_PATH} is not built. Run `python -m moa_amd.build`.")
-    try:
-        from moa_amd import _host as module
-    except ImportError as e:  # pragma: no cover - depends on the machine
-        raise MoaKernelError(f"cannot load {HOST_PATH}: {e}; rebuild it") from e
+    module, why = None, "is not built for " + host_is_built_for()
+    if host_fits():
+        try:
+            from moa_amd import _host as module
+        except ImportError as e:
+            why = f"cannot be loaded ({e})"
+    if module is None:
+        warnings.warn(f"{HOST_PATH} {why}: small calls take the host longer. Run `python -m moa_amd.build`.", RuntimeWarning)
+        _host = _NoHost
+        return _host
     from moa_amd.kernels import mixture_of_attention as attention
 
     raw = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda i: torch.cuda.current_stream(i).cuda_stream)

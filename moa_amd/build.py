@@ -1,5 +1,5 @@
 """Builds moa_amd/libmoa_hip.so from moa_amd/csrc/*.hip with hipcc for gfx950, and moa_amd/_host.so, the host side of a
-decode step, from moa_amd/csrc/moa_host.cpp with g++ against torch's headers.
+decode step, from moa_amd/csrc/moa_host.cpp with g++ (or $CXX, or without either hipcc) against torch's headers.
 
     python -m moa_amd.build            # build if sources are newer than the library
     python -m moa_amd.build --force    # always rebuild
@@ -58,8 +58,10 @@ def _deps_mtime() -> float:
 
 
 def is_stale() -> bool:
+    from moa_amd import _lib
+
     built = (LIB_PATH, HOST_PATH)
-    return not all(map(os.path.exists, built)) or min(map(os.path.getmtime, built)) < _deps_mtime()
+    return not all(map(os.path.exists, built)) or min(map(os.path.getmtime, built)) < _deps_mtime() or not _lib.host_fits()
 
 
 def _compile(src: str, extra: Sequence[str] = ()) -> str:
@@ -77,11 +79,16 @@ def _compile(src: str, extra: Sequence[str] = ()) -> str:
 
 def _build_host() -> None:
     """torch's own libraries are not found by name, nor need they be: the module is loaded where torch already is."""
+    import shutil
     import sysconfig
 
     from torch.utils import cpp_extension
+
+    from moa_amd import _lib
     include = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", *(f"-isystem{p}" for p in include),
+    cxx = os.environ.get("CXX") or shutil.which("g++")
+    cmd = [*([cxx] if cxx else [_hipcc(), "-x", "c++"]), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           *(f"-isystem{p}" for p in include), f'-DMOA_HOST_BUILT_FOR="{_lib.host_is_built_for()}"',
            f"-D_GLIBCXX_USE_CXX11_ABI={int(cpp_extension.torch._C._GLIBCXX_USE_CXX11_ABI)}", HOST_SOURCE, "-o", HOST_PATH,
            f"-L{cpp_extension.TORCH_LIB_PATH}", "-ltorch_python", "-ltorch_cpu", "-lc10"]
     r = subprocess.run(cmd, capture_output=True, text=True)

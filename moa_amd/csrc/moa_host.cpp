@@ -19,6 +19,9 @@
 
 namespace {
 
+// What the module was built for (torch's C++ classes differ between versions), to be found in the file before it is loaded.
+__attribute__((used)) const char built_for[] = "moa_host was built for " MOA_HOST_BUILT_FOR ";";
+
 decltype(&moa_decode_workspace_bytes) workspace_bytes = nullptr;
 decltype(&moa_decode_fwd_counted) decode_fwd = nullptr;
 decltype(&moa_prefill_fwd_tokens) prefill_fwd = nullptr;

@@ -106,3 +106,32 @@ for counters in (8192, None):
     assert name == "moa_decode_fwd_counted" and a[6] == counters, a
     assert (a[4] == 4096) == (counters is not None), a
 """)
+
+
+@pytest.mark.parametrize("found", ["for another torch", "no module", "nothing"])
+def test_a_module_that_does_not_fit_is_not_loaded(tmp_path, monkeypatch, found):
+    """Torch's C++ classes differ between versions: a module that was built for another one is stale, and is not loaded. The
+    calls are left to the Python code then, as they are without any module, and it says so once."""
+    import warnings
+
+    import torch
+
+    from moa_amd import _lib, build
+    path = tmp_path / "_host.so"
+    if found == "for another torch":
+        built = open(_lib.HOST_PATH, "rb").read()
+        assert built.count(torch.__version__.encode() + b",") == 1
+        path.write_bytes(built.replace(torch.__version__.encode() + b",", b"1" * len(torch.__version__) + b","))
+    elif found == "no module":
+        path.write_bytes(b"")
+    assert _lib.host_fits()
+    for module in (_lib, build):
+        monkeypatch.setattr(module, "HOST_PATH", str(path))
+    monkeypatch.setattr(_lib, "_host", None)
+    assert build.is_stale()
+    with pytest.warns(RuntimeWarning, match="not built for torch " + torch.__version__.split("+")[0]):
+        host = _lib.host()
+    assert host.attend(*range(8)) is None and host.rope_append(*range(17)) is None and host.append(*range(12)) is None
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.host() is host
