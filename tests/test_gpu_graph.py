@@ -82,9 +82,9 @@ def test_decode_step_replays_like_eager(dev, G):
 
 
 def test_prompt_pass_replays_like_eager(dev):
-    """The prompt side recorded into a HIP graph: rotary embedding, block-sparse prefill (its work queue is
-    a slot of a device array chosen at record time: every replay of the graph reuses that slot, one after
-    the other on a stream), bulk insert into the rings.  One ordinary call comes first, as the header asks
+    """The prompt side recorded into a HIP graph: rotary embedding, block-sparse prefill (of a short prompt,
+    whose launch has no work queue; one that has is recorded in test_gpu_prefill_routes.py), bulk insert into
+    the rings.  One ordinary call comes first, as the header asks
     (the first call on a device looks up device addresses, which a capture cannot contain).  Every replay
     runs on new inputs and must equal the same calls run eagerly, bit for bit, rings and indices included."""
     import copy

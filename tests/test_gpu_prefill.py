@@ -86,9 +86,8 @@ def test_small_against_oracle(dev, dtype, D, N):
 
 @pytest.mark.parametrize("seed", range(24))
 def test_random_plans_against_oracle(dev, seed):
-    """Random lengths (ragged and long enough for several 256-row query tiles), random sink and band
-    block counts per head incl. 0 and more than there are blocks: the tile schedule (sinks, rotated
-    band, wrap, repeated last tile) against the dense masked oracle."""
+    """Random lengths (ragged and long enough for several query tiles), random sink and band block counts per
+    head incl. 0 and more than there are blocks: the tile schedule against the dense masked oracle."""
     rng = np.random.default_rng(1000 + seed)
     D = int(rng.choice([64, 128]))
     dtype = [torch.float16, torch.bfloat16][seed % 2]
@@ -161,8 +160,8 @@ def test_gqa(dev, G):
 
 
 def test_many_heads_with_equal_and_extreme_spans(dev):
-    """The span-sorted work schedule: 40 heads (13B shape, not a multiple of the 8 XCDs) with tied
-    spans, heads that see nothing, heads wider than the prompt and block counts far out of range;
+    """40 heads (13B shape) with tied spans, heads that see nothing, heads wider than the prompt and block
+    counts far out of range;
     every head against the oracle, and the result must not depend on the order of the heads."""
     B, H, N, D = 1, 40, 640, 64
     nb = N // 64
@@ -187,10 +186,9 @@ def test_many_heads_with_equal_and_extreme_spans(dev):
 
 
 def test_many_launches_in_flight_on_two_streams(dev):
-    """The work queue of a launch is one of 256 slots of a device array, handed out in turn and cleared by
-    the launch's last work-group.  600 launches of two different shapes, alternating between two streams
-    with nothing waiting in between (so launches overlap and the slots go round more than twice): every
-    result must equal that of the same call made alone, bit for bit."""
+    """600 launches of two different shapes, alternating between two streams with nothing waiting in between
+    (so launches overlap): every result must equal that of the same call made alone, bit for bit.  (Short
+    prompts: the launches have no work queue.  Those that have one: test_gpu_prefill_routes.py.)"""
     shapes = [(2, 6, 700, 64, torch.float16, [1, 0, 2, 1, 1, 3], [2, 5, 1, 11, 3, 4]),
               (1, 4, 1300, 128, torch.bfloat16, [1, 1, 0, 2], [4, 21, 2, 7])]
     cases = []
@@ -223,7 +221,8 @@ def test_gqa_70b_shape(dev):
 
 
 def test_more_heads_than_the_sorted_schedule_covers(dev):
-    """Beyond 512 kv heads the span sort is skipped and heads are taken in the given order."""
+    """More kv heads than the resident kernel sorts by their spans (512), in a prompt that is short enough for the
+    other one, which takes heads as they come.  (The resident one: test_gpu_prefill_routes.py.)"""
     B, H, N, D = 1, 520, 128, 64
     rng = np.random.default_rng(21)
     ns = [int(x) for x in rng.integers(0, 2, size=H)]
@@ -234,7 +233,7 @@ def test_more_heads_than_the_sorted_schedule_covers(dev):
     _close(out, ref, "520 heads")
 
 
-@pytest.mark.parametrize("H", [6, 520])   # heads sorted by span; more than that schedule covers
+@pytest.mark.parametrize("H", [6, 520])
 def test_spans_in_tokens_equal_their_whole_blocks(dev, H):
     """The wrapper hands token counts to the kernel: whole blocks of 64 count, rounded down as torch's ``//`` does."""
     from moa_amd import mixture_of_sparse_attention
