@@ -337,21 +337,25 @@ def test_grouped_query_tile_edges(dev, D, G, B, scale):
     _close_grouped(out[few, 0], q[few, :, 0], kc[few], vc[few], hs[few], hv[few], scale, G, (D, G, B))
 
 
-@pytest.mark.parametrize("sizes,B", [([5000], 50), ([5000], 100), ([5000], 150), ([1500, 700], 70), ([300, 200, 90], 90)])
-def test_grouped_query_split_into_rounds(dev, sizes, B):
-    """Launches whose batch rows are split into their share of one round of work-groups, or of two, and one whose short
-    rings are not; rows of a batch that are filled unlike, empty ones among them."""
+# chunks of 2048 rows by the rings' capacity: 150, 300, 450 and 140 split, 180 on neither side of a line that is, 140 of
+# rings so short that a batch row's share of one round (3) is less than 1.5 chunks to each
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("sizes,B", [([5000], 50), ([5000], 100), ([5000], 150), ([1500, 700], 70), ([300, 200, 90], 90),
+                                     ([300, 200, 90], 70)])
+def test_grouped_query_split_into_rounds(dev, sizes, B, D, dtype):
+    """Launches whose batch rows are split into their share of one round of work-groups, or of two, one between the lines
+    and one whose short rings are not; rows of a batch that are filled unlike, empty ones among them."""
     from moa_amd import mixture_of_sparse_attention
     rng = np.random.default_rng(B)
-    G, D, scale = 3, 64, 0.12
-    q, kc, vc, hs, hv = _case(rng, B, sizes, D, torch.float16, dev, fill="partial")
+    G, scale = 3, 0.12
+    q, kc, vc, hs, hv = _case(rng, B, sizes, D, dtype, dev, fill="partial")
     hv[1], hv[-1] = 0, sizes
-    q = torch.from_numpy(rng.standard_normal((B, len(sizes) * G, 1, D)).astype(np.float32)).to(dev, torch.float16)
+    q = torch.from_numpy(rng.standard_normal((B, len(sizes) * G, 1, D)).astype(np.float32)).to(dev, dtype)
     out = mixture_of_sparse_attention(q, kc, vc, scale, head_start_index=torch.from_numpy(hs).to(dev),
                                       head_valid_length=torch.from_numpy(hv).to(dev))
     assert not out[1].any()
     few = [0, B // 2, B - 1]   # rows of the batch that the oracle does
-    _close_grouped(out[few, 0], q[few, :, 0], kc[few], vc[few], hs[few], hv[few], scale, G, (sizes, B))
+    _close_grouped(out[few, 0], q[few, :, 0], kc[few], vc[few], hs[few], hv[few], scale, G, (sizes, B, D))
 
 
 @pytest.mark.parametrize("B", [1, 2])
