@@ -65,7 +65,8 @@ const char* moa_last_error(void);
  * The launch hands its (head, query tile) work items to one resident work-group
  * per CU through a few counters in a small device array that is part of the
  * library's device image (64 bytes per launch, 256 slots used in turn; a slot is
- * left cleared by the launch that used it).  The call itself allocates nothing.
+ * left cleared by the launch that used it); short prompts and launches of few
+ * items use no slot.  The call itself allocates nothing.
  * Launches may overlap on one GPU as long as fewer than 256 of them are under
  * way at once.  The first call on a device looks that array up and the first
  * call per (dtype, D) sets a kernel attribute: make one ordinary call per device

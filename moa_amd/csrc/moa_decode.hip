@@ -660,7 +660,7 @@ constexpr int kGqaBlocksPerCu = 64;
 // wave full memory latencies with nothing in flight, so long chunks win: with one fixed length, 2048 was
 // the best of 512..4096 at batch 64 and at batch 4.
 constexpr int kGqaChunk = 2048;
-constexpr int kGqaTile = 32;      // keys per MFMA tile
+constexpr int kGqaTile = 32;      // keys per stage (two MFMA tiles of scores, one contraction of P.V)
 constexpr int kGqaMaxG = 8;       // query heads per ring the per-wave result buffers are sized for
 constexpr int kGqaWaves = 4;      // waves per work-group (8 waves with one stage each measure the same)
 constexpr int kGqaThreads = 64 * kGqaWaves;
@@ -791,13 +791,13 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
     static_assert(kGqaStages == 2, "the waits below count two stages");
     if (n_t > 0) { issue_k(0); issue_v(0); }
     if (n_t > 1) { issue_k(1); issue_v(1); }
-    // the Q loads are older than every copy: pin their arrival here
-    if (n_t > 1) wait_vm(4 * NCP); else if (n_t > 0) wait_vm(2 * NCP);
+    // The Q rows are waited for here, by the compiler, which does not know of the copies behind them and waits for those too:
+    // the first two tiles have landed when the loop starts.  (Without the pin it would do so inside the loop.)
 #pragma unroll
     for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[s]));
 
-    // K and V of a tile are waited for, and their stages filled again, each by itself: three or four of the wave's four
-    // half stages are in flight all the time (with whole tiles one of two stages while a tile is worked on).
+    // K and V of a tile are waited for, and their stages filled again, each by itself: from the first refills on three or
+    // four of the wave's four half stages are in flight (with whole tiles one of two stages while a tile is worked on).
     for (int t = 0; t < n_t; ++t) {
       if (t + 1 < n_t) wait_vm(3 * NCP); else wait_vm(NCP);   // K(t) has landed; V(t), K(t+1), V(t+1) may be in flight
       const uint32_t so = (uint32_t)((t % kGqaStages) * STAGE_B);
@@ -956,9 +956,10 @@ constexpr int kDecBlocksPerCu = 16;   // work-groups per CU over the whole grid
 // 160 chunks 11.3 with half-length ones.  Pipelining pays where several work-groups follow each other on a CU: 814 chunks of
 // 64-element rows 23.5 us with, 22.6 without, 864 of 128 40.2 and 39.6, 1152 49.5 and 49.4, 1440 59.2 both.
 constexpr int kDecSmallBelow = 1;
-// These launches also have the batch rows side by side in the grid (see kGqaBlocksPerCu): batch 64 of 32 rings of 128 852.7
-// -> 825.9 us, batch 16 215.9 -> 210.7; smaller ones are as fast or faster row by row (246 chunks 10.2 and 10.4 us), with no
-// more work-groups to a row than it can have chunks (690 chunks 18.7 -> 16.9 us).
+// These launches also have the batch rows side by side in the grid (see kGqaBlocksPerCu): 32 full rings of 128, 157888 rows
+// to a batch row, batch 64 815 -> 807 us, batch 16 210 -> 204.5, batch 8 102.5 -> 101.0; smaller ones are as fast or faster
+// row by row (246 chunks 10.2 and 10.4 us), with no more work-groups to a row than it can have chunks (690 chunks 18.7 ->
+// 16.9 us).
 constexpr int kDecPipeFrom = 4;
 
 // From this many bytes of K and V per launch on they are read non-temporally.  What a step reads of one layer
@@ -983,20 +984,20 @@ static inline bool read_nontemporal(int B, int64_t sumC, int D) { return (int64_
 // 90.0 -> 92.4 us; a step called from Python, bound by its launches, 24 -> 21 us.
 // Skewed rings do not change that: one of 100000 rows beside seven short ones 30.5 -> 25.4 us.
 // Grouped kernel: only below kNtBytes (above, a chunk is alone on its CU and nothing hides the merge: batch 4 of 8 rings
-// at 32k tokens, 8 query heads, 43.9 us a layer with the merge launch, 46.2 us without), and by what the last work-group
-// of a ring has to do alone.  A wave merges a query head at a time, so up to four heads take one round over the ring's
-// chunks and five to eight take two; 16 chunks are asked for at once.  GPU time with the merge launch -> without:
-//   G = 4, 8 rings of 128:  2 chunks a ring 12.8 -> 11.2 us, 8 13.5 -> 12.1, 16 14.4 -> 13.9, 32 17.9 -> 18.0
-//   G = 2, 8 rings of 128:  8 chunks 12.7 -> 11.4, 16 13.6 -> 13.0, 32 17.3 -> 17.1
-//   G = 7, 4 rings of 64:   4 chunks 11.1 -> 10.5, 8 11.2 -> 10.8, 16 11.1 -> 11.2, 32 11.8 -> 13.5
-//   G = 8, 8 rings of 128:  2 chunks 14.1 -> 14.1, 8 14.7 -> 15.2, 16 15.6 -> 17.1
-// Up to four heads the launch saved is GPU time won, up to 32 chunks.  With more heads it is about even up to 8, and up
-// to 16 costs less than the host's time for a launch, which is what is won there (a step called from Python waits for
-// its launches: batch 34, one ring of 7 chunks, 8 heads of 64, 25.6 -> 22.0 us).
+// at 32k tokens, 8 query heads, 43.9 us a layer with the merge launch, 46.2 us without, with 32-wide tiles), and by what
+// the last work-group of a ring has to do alone.  A wave merges up to two query heads, whose partials it asks for
+// together, 16 chunks of each at once.  GPU time of a call among others in a graph, with the merge launch -> without:
+//   G = 4, 8 rings of 128:  8 chunks a ring 9.7 -> 9.3 us, 16 10.4 -> 10.2, 32 12.5 -> 13.2
+//   G = 2, 8 rings of 128:  8 chunks 9.4 -> 8.7, 16 10.2 -> 9.7, 32 12.0 -> 12.7
+//   G = 7, 4 rings of 64:   4 chunks 8.5 -> 8.1, 8 8.5 -> 8.2, 16 8.5 -> 8.6, 32 8.7 -> 10.5
+//   G = 8, 8 rings of 128:  2 chunks 10.4 -> 10.3, 4 10.4 -> 10.4, 8 10.5 -> 11.0, 16 10.5 -> 12.1
+// Up to 16 chunks of up to four heads, 8 of seven and 4 of eight the launch saved is GPU time won, or it is even; from there
+// to the lines it costs at most 0.7 us (1.5 above four heads), less than the host's time for a launch (3.5), which is
+// what is won there: a small step called from Python waits for its launches.
 // The rings of a plan are not equally long, and the host knows only how many rows they hold together.  So there are two
 // bounds: on the chunks of an average ring, where the gain ends, and on the chunks of a whole batch row, which is the
-// most its largest ring can have.  One ring with nearly all rows is then the worst case: G = 4, 60 chunks 14.2 -> 15.2 us;
-// G = 8, 20 chunks 14.0 -> 16.0 us; without the second bound 235 chunks 26.6 -> 31.7 us and 29.0 -> 48.9 us.
+// most its largest ring can have.  One ring with nearly all rows is then the worst case: G = 4, 60 chunks 10.8 -> 12.3 us;
+// G = 8, 20 chunks 10.3 -> 12.1 us; without the second bound 235 chunks 22.5 -> 29.2 us and 24.6 -> 45.5 us.
 struct MergeInside {
   int64_t ring_chunks, row_chunks;   // at most: of a ring of average size, of a batch row
 };

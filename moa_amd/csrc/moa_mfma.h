@@ -1,5 +1,5 @@
 // Device helpers shared by the MFMA kernels of libmoa_hip.so (prefill, grouped-query decode):
-// element types with their v_mfma_f32_32x32x16 wrapper, asynchronous global->LDS copies,
+// element types with their v_mfma_f32_32x32x16 and v_mfma_f32_16x16x32 wrappers, asynchronous global->LDS copies,
 // LDS operand reads (plain and transposing), small wave-level utilities.  gfx950 only.
 #pragma once
 #include "moa_common.h"

@@ -837,7 +837,7 @@ __global__ __launch_bounds__(64 * kShortWaves, 2) void prefill_short_kernel(Pref
   uint32_t koff, voff;
   const int crow = wave * (64 / CPR) + lane / CPR, cpos = lane % CPR;
   const uint32_t ksw = (uint32_t)((cpos ^ ((crow / RSH) % CPR)) * 16), vsw = (uint32_t)((cpos ^ (4 * ((crow / RSH) % (CPR / 4)))) * 16);
-  const uint32_t k_row = (uint32_t)(2 * a.ks.n), v_row_b = (uint32_t)(2 * a.vs.n);   // bytes of a row (a tile's fit 31 bits)
+  const uint32_t k_row = (uint32_t)(2 * a.ks.n), v_row_b = (uint32_t)(2 * a.vs.n);   // bytes of a row (a tile's fit 32 bits, unsigned: checked on the host)
   koff = (uint32_t)crow * k_row + ksw;
   voff = (uint32_t)crow * v_row_b + vsw;
   const char* const kbase = reinterpret_cast<const char*>(a.k + b * a.ks.b + hk * a.ks.h);
