@@ -401,8 +401,7 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
   __shared__ float s_m[kDecWaves][G];
   __shared__ float s_l[kDecWaves][G];
 
-  const int b = PIPE ? blockIdx.x : blockIdx.y;   // see kDecPipeFrom
-  const int place = PIPE ? blockIdx.y : blockIdx.x, places = PIPE ? gridDim.y : gridDim.x;
+  const int b = blockIdx.x;   // batch rows side by side (see kDecBlocksPerCu)
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -411,9 +410,9 @@ __global__ __launch_bounds__(kDecThreads) void decode_split_kernel(
 
   const RowChunks<CHUNK, false> row(head_valid + (int64_t)b * H, head_start + (int64_t)b * H, H, sumC, cap, 0);
 
-  if (MERGE && counters && place == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
+  if (MERGE && counters && blockIdx.y == 0) zero_empty_rings(row, o + (int64_t)b * H * G * D, H, G * D);
 
-  for (int w = place; w < row.total; w += places) {
+  for (int w = blockIdx.y; w < row.total; w += gridDim.y) {
     const Chunk ck = row.at(w, H);
     const int c = ck.index, n_chunks = ck.count;
     const int64_t bh = (int64_t)b * H + ck.head;
@@ -949,17 +948,22 @@ __global__ __launch_bounds__(kGqaThreads) void decode_gqa_kernel(
 }
 
 constexpr int kChunk = 512;           // cache rows per work-group step of the one-query-head kernel
-constexpr int kDecBlocksPerCu = 16;   // work-groups per CU over the whole grid
+// Work-groups per CU over the whole grid, never more per batch row than it can have chunks (8 leaves a visible tail, 32 is no
+// better).  The batch rows lie side by side, chunk numbers outside (see kGqaBlocksPerCu).  Row by row, with the work-groups
+// that find no chunk between the rows, it is a matter of luck which CUs those meet: where a row is a multiple of two, four
+// or eight of them, the same ones every time.  GPU time over 9400 random launches (batch 1 to 64, 4 to 40 rings of 64 and
+// 128, full and ragged) against row by row with work-groups for the shortest chunks: 0.99 of it below 256 chunks, 0.95 from
+// there to four work-groups per CU (0.63 to 1.25, at most 1.07 in 95 of 100), 0.98 above (0.65 to 1.10).  Row by row with
+// no more of them than chunks of 512 rows is 0.99 in the middle range, but up to 1.7 where those are an even few: batch 64
+// of rings of 700, 500, 200 and 162 rows of 128, 8 places to a row, 11.5 us, 18.9 and, side by side, 12.1.  32 full rings of 128, 157888 rows to a batch
+// row, batch 64: 815 -> 807 us, batch 16 210 -> 204.5, batch 8 102.5 -> 101.0.
+constexpr int kDecBlocksPerCu = 16;
 // Work-groups per CU (full-length chunks by the rings' capacity) below which the chunks are half as long, and from
 // which the waves pipeline their own loads.  Half-length chunks pay only where full ones leave CUs idle: 32 rings of 128,
 // 288 chunks 17.3 us with half-length, 15.9 with full ones, 469 chunks 26.4 and 23.6, 8 rings 445 chunks 30.6 and 24.5;
 // 160 chunks 11.3 with half-length ones.  Pipelining pays where several work-groups follow each other on a CU: 814 chunks of
 // 64-element rows 23.5 us with, 22.6 without, 864 of 128 40.2 and 39.6, 1152 49.5 and 49.4, 1440 59.2 both.
 constexpr int kDecSmallBelow = 1;
-// These launches also have the batch rows side by side in the grid (see kGqaBlocksPerCu): 32 full rings of 128, 157888 rows
-// to a batch row, batch 64 815 -> 807 us, batch 16 210 -> 204.5, batch 8 102.5 -> 101.0; smaller ones are as fast or faster
-// row by row (246 chunks 10.2 and 10.4 us), with no more work-groups to a row than it can have chunks (690 chunks 18.7 ->
-// 16.9 us).
 constexpr int kDecPipeFrom = 4;
 
 // From this many bytes of K and V per launch on they are read non-temporally.  What a step reads of one layer
@@ -1021,13 +1025,11 @@ static int launch_decode(const void* q, const void* kc, const void* vc, void* o,
   const int64_t chunks = (sumC + kChunk - 1) / kChunk + H;   // per batch row, at the normal chunk length
   const bool pipe = (int64_t)B * chunks >= (int64_t)256 * kDecPipeFrom;
   const bool small = (int64_t)B * chunks < (int64_t)256 * kDecSmallBelow;
-  // 16 work-groups per CU over the whole grid (measured: 8 leaves a visible tail, 32 is no better),
-  // never more per batch row than chunks exist
   int64_t bx = (256 * kDecBlocksPerCu + B - 1) / B;
   if (bx > (small ? cap : chunks)) bx = small ? cap : chunks;
   if (bx < 1) bx = 1;
   auto launch = [&](auto split, auto merge) {
-    hipLaunchKernelGGL(split, pipe && !small ? dim3(B, (unsigned)bx) : dim3((unsigned)bx, B), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
+    hipLaunchKernelGGL(split, dim3(B, (unsigned)bx), dim3(kDecThreads), 0, st, (const uint16_t*)q, (const uint16_t*)kc,
                        (const uint16_t*)vc, (uint16_t*)o, part_acc, part_ml, head_start, head_valid, H, sumC,
                        sm_scale * kLog2e, cap, counters);
     if (int rc = check_launch("moa_decode_fwd(split)")) return rc;
