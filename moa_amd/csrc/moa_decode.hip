@@ -955,8 +955,8 @@ constexpr int kChunk = 512;           // cache rows per work-group step of the o
 // 128, full and ragged) against row by row with work-groups for the shortest chunks: 0.99 of it below 256 chunks, 0.95 from
 // there to four work-groups per CU (0.63 to 1.25, at most 1.07 in 95 of 100), 0.98 above (0.65 to 1.10).  Row by row with
 // no more of them than chunks of 512 rows is 0.99 in the middle range, but up to 1.7 where those are an even few: batch 64
-// of rings of 700, 500, 200 and 162 rows of 128, 8 places to a row, 11.5 us, 18.9 and, side by side, 12.1.  32 full rings of 128, 157888 rows to a batch
-// row, batch 64: 815 -> 807 us, batch 16 210 -> 204.5, batch 8 102.5 -> 101.0.
+// of rings of 700, 500, 200 and 162 rows of 128, 8 places to a row, 11.5 us, 18.9 and, side by side, 12.1.  32 full rings
+// of 128, 157888 rows to a batch row, batch 64: 815 -> 807 us, batch 16 210 -> 204.5, batch 8 102.5 -> 101.0.
 constexpr int kDecBlocksPerCu = 16;
 // Work-groups per CU (full-length chunks by the rings' capacity) below which the chunks are half as long, and from
 // which the waves pipeline their own loads.  Half-length chunks pay only where full ones leave CUs idle: 32 rings of 128,
